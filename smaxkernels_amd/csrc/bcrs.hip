@@ -1059,69 +1059,185 @@ static int gather_blocks(smax_hip_ctx ctx, const smax_hip_bcrs_info &T,
     return SMAX_HIP_SUCCESS;
 }
 
-// Group of G lanes per block position; fixed xor-butterfly over the group.
-template <int VT, int G>
-__global__ __launch_bounds__(256) void bcrs_sddmm_kernel(
-    int64_t n_positions, int64_t n_block_rows, int b_h, int b_w, int h_pad, int w_pad,
-    int col_major, int64_t k, const int32_t *__restrict__ row_ptr,
-    const int32_t *__restrict__ col, const typename vt<VT>::vec_t *__restrict__ Gm,
-    const typename vt<VT>::vec_t *__restrict__ X,
-    typename vt<VT>::vec_t *__restrict__ dvals) {
-    using T = vt<VT>;
-    using A = typename T::vec_t;
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    const int64_t e = t / G;
-    const int lane = static_cast<int>(t % G);
-    const int64_t bs = static_cast<int64_t>(h_pad) * w_pad;
-    const int64_t j = e / bs, off = e - j * bs;
-    const int ix = static_cast<int>(col_major ? off % h_pad : off / w_pad);
-    const int jx = static_cast<int>(col_major ? off / h_pad : off % w_pad);
-    const bool real = e < n_positions && ix < b_h && jx < b_w;
-    A acc = 0;
-    if (real) {
-        int64_t lo = 0, hi = n_block_rows;  // block row of block j
-        while (hi - lo > 1) {
-            const int64_t mid = (lo + hi) >> 1;
-            if (row_ptr[mid] <= j) lo = mid; else hi = mid;
-        }
-        const A *gr = Gm + (lo * h_pad + ix) * k;
-        const A *xr = X + (static_cast<int64_t>(col[j]) * w_pad + jx) * k;
-        for (int64_t v = lane; v < k; v += G) acc = T::fma_(gr[v], xr[v], acc);
+// Last row r in [0, n_rows) with row_ptr[r] <= j: all 64 lanes of a wavefront
+// (same j) probe 64 rows at a time, so 10^6 rows take four dependent loads.
+__device__ __forceinline__ int64_t wave_row_of(const int32_t *__restrict__ row_ptr,
+                                               int64_t n_rows, int64_t j) {
+    const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+    int64_t lo = 0, hi = n_rows;  // row_ptr[lo] <= j < row_ptr[hi]
+    while (hi - lo > 1) {
+        const int64_t step = (hi - lo + kWave - 1) / kWave;
+        const int64_t r = lo + lane * step;
+        const bool below = r < hi && row_ptr[r] <= j;  // lane 0's always is
+        lo += (__popcll(__ballot(below)) - 1) * step;
+        hi = lo + step < hi ? lo + step : hi;
     }
+    return lo;
+}
+
+// VL entries from p in one access (VL * sizeof(A) is 16 with p 16-byte
+// aligned, or VL is 1), predicated per run on v < k.
+template <typename A, int KP, int VL>
+__device__ __forceinline__ void load_cols(const A *__restrict__ p, int64_t k, A (&out)[KP]) {
 #pragma unroll
-    for (int o = G / 2; o >= 1; o >>= 1) acc += __shfl_xor(acc, o, G);
-    if (e < n_positions && lane == 0) dvals[e] = real ? acc : A(0);
-}
-
-template <int VT, int G>
-static void launch_bcrs_sddmm_g(smax_hip_ctx ctx, const smax_hip_bcrs_info &in,
-                                int64_t k, const void *Gm, const void *X, void *dv) {
-    using T = vt<VT>;
-    const int64_t n = in.n_blocks * in.h_pad * in.w_pad;
-    hipLaunchKernelGGL((bcrs_sddmm_kernel<VT, G>), grid_for(n * G, 256), dim3(256), 0,
-                       ctx->stream, n, in.n_block_rows, static_cast<int>(in.b_h),
-                       static_cast<int>(in.b_w), static_cast<int>(in.h_pad),
-                       static_cast<int>(in.w_pad), static_cast<int>(in.block_col_major),
-                       k, in.row_ptr, in.col,
-                       static_cast<const typename T::vec_t *>(Gm),
-                       static_cast<const typename T::vec_t *>(X),
-                       static_cast<typename T::vec_t *>(dv));
-}
-
-template <int VT>
-static int launch_bcrs_sddmm(smax_hip_ctx ctx, const smax_hip_bcrs_info &in,
-                             int64_t k, int g, const void *Gm, const void *X,
-                             void *dv) {
-    switch (g) {
-    case 1: launch_bcrs_sddmm_g<VT, 1>(ctx, in, k, Gm, X, dv); break;
-    case 2: launch_bcrs_sddmm_g<VT, 2>(ctx, in, k, Gm, X, dv); break;
-    case 4: launch_bcrs_sddmm_g<VT, 4>(ctx, in, k, Gm, X, dv); break;
-    case 8: launch_bcrs_sddmm_g<VT, 8>(ctx, in, k, Gm, X, dv); break;
-    case 16: launch_bcrs_sddmm_g<VT, 16>(ctx, in, k, Gm, X, dv); break;
-    case 32: launch_bcrs_sddmm_g<VT, 32>(ctx, in, k, Gm, X, dv); break;
-    default: launch_bcrs_sddmm_g<VT, 64>(ctx, in, k, Gm, X, dv); break;
+    for (int v = 0; v < KP; v += VL) {
+        A run[VL];
+#pragma unroll
+        for (int i = 0; i < VL; ++i) run[i] = 0;
+        if (v < k) load_run<A, VL>(p + v, run);
+#pragma unroll
+        for (int i = 0; i < VL; ++i) out[v + i] = run[i];
     }
-    SMAX_HIP_LAUNCHED(ctx, "bcrs_sddmm_kernel");
+}
+
+// One thread per block line, the positions of a block that are contiguous in
+// memory: a row of a row-major block (its G row against the block's w_pad X
+// rows), a column of a column-major one (its X row against the h_pad G rows).
+// The thread keeps the line's own operand row in registers (k <= 32) and
+// forms each position's sum by itself, in the tree of a group of KP lanes (KP
+// the power of two >= k, at most 64): lane l's chain over v = l, l + KP, ...,
+// then the xor-butterfly's halves, KP/2 first.
+//
+// What bounds it: the vector memory path, 16 bytes a lane and load (b + 1
+// operand rows of k entries per line of b results), and the store of dvals.
+// The results do not depend on who computes them, so the split is free: with
+// a group of KP lanes per position (each lane searching the position's block
+// row in row_ptr, 20 dependent loads) the 96^3 matrix of 4x4 blocks took
+// 9.74 ms at k = 8, 4-byte entries.
+//
+// A workgroup takes `iters` x 256 consecutive lines, so stores are contiguous
+// whatever the block shape and block rows may have any length; it finds its
+// first block's row once (wave_row_of) and writes the row of each of its
+// blocks to LDS.
+constexpr int kSddmmIters = 8;  // at most: 2048 lines a workgroup
+
+template <typename A, int KP, int VL, int M>
+__global__ __launch_bounds__(256) void bcrs_sddmm_lines(
+    int64_t n_blocks, int64_t n_block_rows, int iters, int n_lines, int lines_real, int n_out,
+    int outs_real, int h_pad, int w_pad, int col_major, int64_t k,
+    const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col,
+    const A *__restrict__ Gm, const A *__restrict__ X, A *__restrict__ dvals) {
+    __shared__ int32_t row_of[256 * kSddmmIters + 1];
+    const int span = iters * 256;
+    const int64_t t0 = xcd_block(blockIdx.x, gridDim.x) * span;
+    const int64_t j0 = t0 / n_lines;
+    const int first = static_cast<int>(t0 - j0 * n_lines);
+    // blocks of this workgroup: [j0, j1)
+    const int64_t jn = j0 + (first + span - 1) / n_lines + 1;
+    const int64_t j1 = jn < n_blocks ? jn : n_blocks;
+    if (j0 >= n_blocks) return;  // whole workgroups
+    for (int64_t r = wave_row_of(row_ptr, n_block_rows, j0) + threadIdx.x;
+         r < n_block_rows; r += 256) {
+        const int64_t s = row_ptr[r], e = row_ptr[r + 1];
+        if (s >= j1) break;
+        for (int64_t j = s > j0 ? s : j0; j < (e < j1 ? e : j1); ++j)
+            row_of[j - j0] = static_cast<int32_t>(r);
+    }
+    __syncthreads();
+    constexpr bool kKeep = KP <= 32;  // the line's own operand row stays in registers
+    for (int it = 0; it < iters; ++it) {
+        const int q = first + it * 256 + static_cast<int>(threadIdx.x);
+        const int jl = q / n_lines, i = q - jl * n_lines;
+        const int64_t j = j0 + jl;
+        if (j >= n_blocks) break;
+        A *out = dvals + (j * n_lines + i) * n_out;
+        const int64_t r = row_of[jl], c = col[j];
+        const A *grow = Gm + r * h_pad * k, *xrow = X + c * w_pad * k;
+        const A *own = (col_major ? xrow : grow) + i * k;
+        const A *others = col_major ? grow : xrow;
+        A f[kKeep ? KP : 1];
+        if constexpr (kKeep)
+            if (i < lines_real) load_cols<A, KP, VL>(own, k, f);
+        auto position = [&](int m) -> A {
+            if (i >= lines_real || m >= outs_real) return 0;
+            const A *w = others + m * k;
+            A p[KP];
+            if constexpr (kKeep) {
+                A b[KP];
+                load_cols<A, KP, VL>(w, k, b);
+#pragma unroll
+                for (int v = 0; v < KP; ++v) p[v] = __builtin_elementwise_fma(f[v], b[v], A(0));
+            } else {
+#pragma unroll
+                for (int v = 0; v < KP; ++v) p[v] = 0;
+                for (int64_t v0 = 0; v0 < k; v0 += KP) {
+#pragma unroll
+                    for (int v = 0; v < KP; v += VL) {
+                        if (v0 + v >= k) continue;
+                        A a[VL], b[VL];
+                        load_run<A, VL>(own + v0 + v, a);
+                        load_run<A, VL>(w + v0 + v, b);
+#pragma unroll
+                        for (int u = 0; u < VL; ++u)
+                            p[v + u] = __builtin_elementwise_fma(a[u], b[u], p[v + u]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int off = KP / 2; off >= 1; off >>= 1)
+#pragma unroll
+                for (int v = 0; v < off; ++v) p[v] += p[v + off];
+            return p[0];
+        };
+        if constexpr (M > 0) {
+            A sums[M];
+#pragma unroll
+            for (int m = 0; m < M; ++m) sums[m] = position(m);
+            store_run<A, M>(out, sums);
+        } else {
+            for (int m = 0; m < n_out; ++m) out[m] = position(m);
+        }
+    }
+}
+
+template <typename A, int KP, int VL, int M>
+static void launch_bcrs_sddmm_lines(smax_hip_ctx ctx, const smax_hip_bcrs_info &in, int64_t k,
+                                    const void *Gm, const void *X, void *dv) {
+    const bool cm = in.block_col_major != 0;
+    const int64_t n_lines = cm ? in.w_pad : in.h_pad, lines = in.n_blocks * n_lines;
+    // fewer lines a workgroup while that leaves CUs idle
+    int64_t iters = lines / (256 * 2048);
+    iters = iters < 1 ? 1 : iters > kSddmmIters ? kSddmmIters : iters;
+    hipLaunchKernelGGL((bcrs_sddmm_lines<A, KP, VL, M>), grid_for(lines, static_cast<int>(256 * iters)),
+                       dim3(256), 0, ctx->stream, in.n_blocks, in.n_block_rows,
+                       static_cast<int>(iters), static_cast<int>(n_lines),
+                       static_cast<int>(cm ? in.b_w : in.b_h),
+                       static_cast<int>(cm ? in.h_pad : in.w_pad),
+                       static_cast<int>(cm ? in.b_h : in.b_w), static_cast<int>(in.h_pad),
+                       static_cast<int>(in.w_pad), cm ? 1 : 0, k, in.row_ptr, in.col,
+                       static_cast<const A *>(Gm), static_cast<const A *>(X),
+                       static_cast<A *>(dv));
+}
+
+// 16-byte loads when every operand row is 16-byte aligned; 16-byte stores for
+// lines of four results.
+template <typename A, int KP>
+static void launch_bcrs_sddmm(smax_hip_ctx ctx, const smax_hip_bcrs_info &in, int64_t k,
+                              const void *Gm, const void *X, void *dv) {
+    constexpr int Q = 16 / static_cast<int>(sizeof(A));
+    const bool four = (in.block_col_major ? in.h_pad : in.w_pad) == 4 && aligned16(dv, dv);
+    if constexpr (KP >= Q) {
+        if (k % Q == 0 && aligned16(Gm, X)) {
+            if (four) launch_bcrs_sddmm_lines<A, KP, Q, 4>(ctx, in, k, Gm, X, dv);
+            else launch_bcrs_sddmm_lines<A, KP, Q, 0>(ctx, in, k, Gm, X, dv);
+            return;
+        }
+    }
+    if (four) launch_bcrs_sddmm_lines<A, KP, 1, 4>(ctx, in, k, Gm, X, dv);
+    else launch_bcrs_sddmm_lines<A, KP, 1, 0>(ctx, in, k, Gm, X, dv);
+}
+
+template <typename A>
+static int bcrs_sddmm(smax_hip_ctx ctx, const smax_hip_bcrs_info &in, int64_t k, const void *Gm,
+                      const void *X, void *dv) {
+    if (k <= 1) launch_bcrs_sddmm<A, 1>(ctx, in, k, Gm, X, dv);
+    else if (k <= 2) launch_bcrs_sddmm<A, 2>(ctx, in, k, Gm, X, dv);
+    else if (k <= 4) launch_bcrs_sddmm<A, 4>(ctx, in, k, Gm, X, dv);
+    else if (k <= 8) launch_bcrs_sddmm<A, 8>(ctx, in, k, Gm, X, dv);
+    else if (k <= 16) launch_bcrs_sddmm<A, 16>(ctx, in, k, Gm, X, dv);
+    else if (k <= 32) launch_bcrs_sddmm<A, 32>(ctx, in, k, Gm, X, dv);
+    else launch_bcrs_sddmm<A, 64>(ctx, in, k, Gm, X, dv);
+    SMAX_HIP_LAUNCHED(ctx, "bcrs_sddmm_lines");
     return SMAX_HIP_SUCCESS;
 }
 
@@ -1213,11 +1329,8 @@ int smax_hip_bcrs_sddmm(smax_hip_ctx ctx, int value_type, smax_hip_bcrs A, int64
         return fail(ctx, SMAX_HIP_ERROR_OVERFLOW,
                     "smax_hip_bcrs_sddmm: k = %lld exceeds the launch limits", (long long)k);
     if (A->info.n_blocks == 0) return SMAX_HIP_SUCCESS;
-    int g = 1;
-    while (g < k && g < 64) g <<= 1;
-    SMAX_HIP_DISPATCH_VT(value_type,
-                         return launch_bcrs_sddmm<VT>(ctx, A->info, k, g, G, X, dvals));
-    return SMAX_HIP_ERROR_UNSUPPORTED;
+    return value_type == SMAX_HIP_F64 ? bcrs_sddmm<double>(ctx, A->info, k, G, X, dvals)
+                                      : bcrs_sddmm<float>(ctx, A->info, k, G, X, dvals);
 }
 
 }  // extern "C"

@@ -336,3 +336,62 @@ def test_bcrs_adjoint_transpose_spmm_sddmm(ctx, vt, cm):
     assert (np.abs(mine - ref) <= (np.log2(k) + 1) * u * scale + 1e-300).all()
     for h in (T, b, b2):
         h.destroy()
+
+
+@pytest.mark.parametrize("vt", [capi.F64, capi.BF16])
+@pytest.mark.parametrize("bh,bw,hp,wp,cm", [(1, 1, 1, 1, False), (4, 4, 4, 4, False),
+                                            (4, 4, 4, 4, True), (3, 2, 4, 4, False),
+                                            (2, 3, 2, 5, True), (5, 6, 5, 6, False)])
+@pytest.mark.parametrize("k,shift", [(1, 0), (2, 0), (3, 0), (8, 0), (8, 1), (20, 0), (32, 0),
+                                     (33, 0), (64, 0), (70, 0)])
+def test_bcrs_sddmm_block_lines(ctx, vt, bh, bw, hp, wp, cm, k, shift):
+    """Block SDDMM over ragged block rows (empty ones, runs of them, and one
+    that spans several workgroups) for every load width (k = 8 with G and X
+    one entry off their 16-byte alignment), against binary64 (binary128 for
+    FP64) sums.  Per position: KP chains of q = ceil(k / KP) terms (KP the
+    power of two >= k, at most 64) and log2 KP additions of partial sums, so
+    |d - d_exact| <= (q + log2 KP) u sum |g x|; padding positions are zero."""
+    rng = np.random.default_rng(hp * 100 + k)
+    nbr, nbc = 260, 2100
+    per = rng.integers(0, 6, nbr)
+    per[[0, 7, 8, 9, nbr - 1]] = 0
+    per[40] = nbc
+    brp = np.concatenate([[0], np.cumsum(per)]).astype(np.int64)
+    bcol = np.concatenate([np.sort(rng.choice(nbc, p, replace=False)) for p in per])
+    # scalar CRS with dense blocks
+    rp = np.concatenate([[0], np.cumsum(np.repeat(per * bw, bh))]).astype(np.int32)
+    col = np.concatenate([np.tile((bcol[s:e, None] * bw + np.arange(bw)).ravel(), bh)
+                          for s, e in zip(brp, brp[1:])]).astype(np.int32)
+    vec = np.float64 if vt == capi.F64 else np.float32
+    val = np.zeros(col.size, np.float64 if vt == capi.F64 else np.uint16)
+    b = gpu_bcrs(ctx, nbr * bh, nbc * bw, rp, col, val, bh, bw, hp, wp, cm)
+    assert b.info.n_blocks == brp[-1]
+    G = rng.uniform(-1, 1, (nbr * hp, k)).astype(vec)
+    X = rng.uniform(-1, 1, (nbc * wp, k)).astype(vec)
+    pad = np.zeros(shift, vec)
+    dG, dX = (ctx.upload(np.concatenate([pad, a.ravel()])) for a in (G, X))
+    n = int(brp[-1]) * hp * wp
+    dv = ctx.upload(np.full(n, 7, vec))
+    off = shift * vec().itemsize
+    b.sddmm(vt, k, dG.ptr + off, dX.ptr + off, dv)
+    got = ctx.download(dv).reshape((-1, wp, hp) if cm else (-1, hp, wp))
+    if cm:
+        got = got.transpose(0, 2, 1)
+    brow = np.repeat(np.arange(nbr), per)
+    wide = np.longdouble if vt == capi.F64 else np.float64
+    Gb = G.reshape(nbr, hp, k)[brow].astype(wide)
+    Xb = X.reshape(nbc, wp, k)[bcol].astype(wide)
+    want, scale = np.zeros((2, brow.size, hp, wp), wide)
+    for v in range(k):
+        t = Gb[:, :, None, v] * Xb[:, None, :, v]
+        want += t
+        scale += np.abs(t)
+    kp = min(64, 1 << (k - 1).bit_length())
+    bound = (-(-k // kp) + np.log2(kp)) * np.finfo(vec).eps / 2 * scale
+    real = np.zeros((hp, wp), bool)
+    real[:bh, :bw] = True
+    assert (np.abs(got - want) <= bound)[:, real].all()
+    assert (got[:, ~real] == 0).all()
+    for d in (dG, dX, dv):
+        d.free()
+    b.destroy()
