@@ -395,3 +395,32 @@ def test_bcrs_sddmm_block_lines(ctx, vt, bh, bw, hp, wp, cm, k, shift):
     for d in (dG, dX, dv):
         d.free()
     b.destroy()
+
+
+@pytest.mark.parametrize("vt", [capi.F64, capi.F32, capi.BF16])
+@pytest.mark.parametrize("bh,bw,hp,wp", [(1, 1, 1, 1), (2, 2, 2, 2), (3, 3, 3, 3), (3, 3, 4, 4),
+                                         (5, 1, 5, 1)])
+@pytest.mark.parametrize("shift", [0, 1, 2])
+def test_bcrs_transpose_refresh_unit_widths(ctx, vt, bh, bw, hp, wp, shift):
+    """The transpose's blocks are copied in the widest unit (16, 8, 4 or 2
+    bytes) that the block size and both addresses allow: block sizes of every
+    class, and source values 0, 1 or 2 entries off their alignment."""
+    n = 5
+    A = matgen.block7(n, 1)
+    nb = n ** 3
+    per = np.diff(A.row_ptr)
+    rp = np.concatenate([[0], np.cumsum(np.repeat(per * bw, bh))]).astype(np.int32)
+    col = np.concatenate([np.tile((A.col[s:e, None].astype(np.int64) * bw + np.arange(bw)).ravel(), bh)
+                          for s, e in zip(A.row_ptr, A.row_ptr[1:])]).astype(np.int32)
+    dt = {capi.F64: np.float64, capi.F32: np.float32, capi.BF16: np.uint16}[vt]
+    b = gpu_bcrs(ctx, nb * bh, nb * bw, rp, col, np.zeros(col.size, dt), bh, bw, hp, wp, False)
+    T = b.transpose()
+    src = np.random.default_rng(shift).integers(0, 1 << 14, (b.info.n_blocks, hp * wp)).astype(dt)
+    d = ctx.upload(np.concatenate([np.zeros(shift, dt), src.ravel()]))
+    T.refresh_values(d.ptr + shift * dt().itemsize)
+    order = ctx.download_ptr(T.info.src_block, T.info.n_blocks, np.int32)
+    assert np.array_equal(np.sort(order), np.arange(b.info.n_blocks))
+    assert_bitwise(T.arrays(dt)["val"], src[order].ravel())
+    d.free()
+    for h in (T, b):
+        h.destroy()
