@@ -44,7 +44,8 @@ int bind(smax_hip_ctx ctx);
 // Checks the launch that was just enqueued.
 int check_launch(smax_hip_ctx ctx, const char *kernel);
 
-// Allocation helpers that record failures.
+// Allocation helpers that record failures.  Blocks of 1 MB and more that are
+// freed are kept for reuse within a bound (context.hip).
 int dev_alloc(smax_hip_ctx ctx, void **p, size_t bytes, const char *what);
 void dev_free(void *p);
 

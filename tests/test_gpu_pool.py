@@ -1,0 +1,74 @@
+"""Device blocks kept between handles: rebuilding layouts in turn, from several
+threads and contexts, gives the same layouts as a first build, and the memory
+goes back with the last context."""
+from __future__ import annotations
+
+import threading
+
+import numpy as np
+import pytest
+
+from smaxkernels_amd import capi, matgen
+
+pytestmark = pytest.mark.gpu
+FIELDS = ("chunk_ptr", "chunk_lengths", "col", "val", "perm", "src_index")
+
+
+def layout(ctx, d, A, sigma):
+    s = ctx.scs_from_crs(A.n_rows, A.n_cols, A.nnz, *d, 8, 64, sigma)
+    a = s.arrays(np.float64)
+    s.destroy()
+    return a
+
+
+def test_rebuilt_layouts_in_reused_blocks(ctx):
+    """Two matrices of different sizes and two window lengths, rebuilt in turn:
+    every rebuild lands in blocks that held another layout."""
+    mats = [matgen.lomax_band(60_000), matgen.lomax_band(90_000, seed=5)]
+    dev = [[ctx.upload(a) for a in (A.row_ptr, A.col, A.val)] for A in mats]
+    first = {}
+    for _ in range(3):
+        for i, A in enumerate(mats):
+            for sigma in (4096, 65536):
+                got = layout(ctx, dev[i], A, sigma)
+                want = first.setdefault((i, sigma), got)
+                for f in FIELDS:
+                    assert np.array_equal(got[f], want[f]), (i, sigma, f)
+    for ds in dev:
+        for d in ds:
+            d.free()
+
+
+def test_threads_with_contexts_of_their_own():
+    A = matgen.lomax_band(60_000)
+    want, errors = [], []
+
+    def work(n):
+        try:
+            with capi.Context(0) as c:
+                d = [c.upload(a) for a in (A.row_ptr, A.col, A.val)]
+                for _ in range(n):
+                    got = layout(c, d, A, 4096)
+                    want.append(got)
+                    assert all(np.array_equal(got[f], want[0][f]) for f in FIELDS)
+        except Exception as e:  # reported in the test's thread
+            errors.append(e)
+
+    work(1)
+    threads = [threading.Thread(target=work, args=(4,)) for _ in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+
+
+def test_handle_destroyed_after_its_context():
+    """A handle may be destroyed without a context (null): its blocks are freed."""
+    A = matgen.lomax_band(60_000)
+    c = capi.Context(0)
+    s = c.scs_from_crs(A.n_rows, A.n_cols, A.nnz, c.upload(A.row_ptr), c.upload(A.col),
+                       c.upload(A.val), 8, 64, 4096)
+    lib, h = c.lib, s.handle
+    c.close()
+    assert lib.smax_hip_scs_destroy(None, h) == capi.SUCCESS
