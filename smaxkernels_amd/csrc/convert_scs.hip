@@ -5,7 +5,9 @@
 // (index, count) pairs by count descending (convert_formats.hpp:46-55).
 // std::sort is unstable, so tied rows end up in the order libstdc++'s
 // introsort leaves them; that order is reproduced exactly here by running the
-// introsort recursion level-synchronously over every window at once:
+// introsort recursion level-synchronously over every segment at once (windows
+// and segments of up to a few thousand rows inside LDS, k_sort_tiles; longer
+// ones level by level over global memory until they are that short):
 //
 //  * a segment [h, e) with e - h > 16 and depth > 0 is partitioned exactly as
 //    __unguarded_partition_pivot does (bits/stl_algo.h:1878-1907): the
@@ -35,15 +37,25 @@
 
 namespace smaxhip {
 
-enum : int32_t { SEG_ACTIVE = 0, SEG_LEAF = 1, SEG_HEAP = 2, SEG_NONE = 3 };
+// SEG_PARKED: short enough for k_sort_tiles, which runs the rest of it.
+enum : int32_t { SEG_ACTIVE = 0, SEG_LEAF = 1, SEG_HEAP = 2, SEG_NONE = 3, SEG_PARKED = 4 };
 constexpr int kThreshold = 16;  // _S_threshold, bits/stl_algo.h:1855
 constexpr int kThreads = 256;
+
+// k_sort_tiles: positions of a workgroup's tile, and the longest segment that
+// the level-by-level phase leaves to it (segments that start in the same
+// kParked positions end within 2 * kParked - 1 of the first, one tile).
+constexpr int kTile = 4096;
+constexpr int kTileThreads = 1024;
+constexpr int kTileItems = kTile / kTileThreads;
+constexpr int kParked = kTile / 2;
 
 __device__ __forceinline__ int32_t lg2(int64_t n) {
     return 63 - __clzll(static_cast<unsigned long long>(n));
 }
 
 // ------------------------------------------------------------ init
+// Windows longer than a tile: their segments and (index, count) pairs.
 __global__ void k_init(int64_t n, int64_t n_rows, int64_t sigma,
                        const int32_t *__restrict__ row_ptr,
                        int32_t *__restrict__ idx, int32_t *__restrict__ cnt,
@@ -61,12 +73,12 @@ __global__ void k_init(int64_t n, int64_t n_rows, int64_t sigma,
         int64_t len = e - h;
         end[q] = static_cast<int32_t>(e);
         depth[q] = 2 * lg2(len);  // std::__lg(last - first) * 2
-        if (len > kThreshold) {
+        if (len > kParked) {
             state[q] = SEG_ACTIVE;
             list[atomicAdd(reinterpret_cast<unsigned long long *>(nlist), 1ull)] =
                 static_cast<int32_t>(q);
         } else {
-            state[q] = SEG_LEAF;
+            state[q] = SEG_PARKED;
         }
     } else {
         state[q] = SEG_NONE;
@@ -259,9 +271,9 @@ __global__ void k_newsegs(int64_t nl, const int32_t *__restrict__ list,
     depth[c] = d;
     end[h] = c;
     depth[h] = d;
-    const bool right = e - c > kThreshold, left = c - h > kThreshold;
-    state[c] = right ? SEG_ACTIVE : SEG_LEAF;
-    state[h] = left ? SEG_ACTIVE : SEG_LEAF;
+    const bool right = e - c > kParked, left = c - h > kParked;
+    state[c] = right ? SEG_ACTIVE : SEG_PARKED;
+    state[h] = left ? SEG_ACTIVE : SEG_PARKED;
     unsigned long long *cntp = reinterpret_cast<unsigned long long *>(nnext);
     if (right) next[atomicAdd(cntp, 1ull)] = c;
     if (left) next[atomicAdd(cntp, 1ull)] = h;
@@ -270,8 +282,9 @@ __global__ void k_newsegs(int64_t nl, const int32_t *__restrict__ list,
 // ------------------------------------------------------------ heap fallback
 // make_heap + sort_heap of bits/stl_heap.h on (idx, cnt) pairs,
 // comp(a, b) = a.count > b.count.
-__device__ void push_heap_d(int32_t *I, int32_t *K, int64_t hole, int64_t top,
-                            int32_t vi, int32_t vk) {
+template <typename Index>
+__device__ void push_heap_d(Index *I, int32_t *K, int64_t hole, int64_t top,
+                            Index vi, int32_t vk) {
     int64_t parent = (hole - 1) / 2;
     while (hole > top && K[parent] > vk) {
         I[hole] = I[parent];
@@ -283,8 +296,9 @@ __device__ void push_heap_d(int32_t *I, int32_t *K, int64_t hole, int64_t top,
     K[hole] = vk;
 }
 
-__device__ void adjust_heap_d(int32_t *I, int32_t *K, int64_t hole,
-                              int64_t len, int32_t vi, int32_t vk) {
+template <typename Index>
+__device__ void adjust_heap_d(Index *I, int32_t *K, int64_t hole,
+                              int64_t len, Index vi, int32_t vk) {
     const int64_t top = hole;
     int64_t second = hole;
     while (second < (len - 1) / 2) {
@@ -303,15 +317,8 @@ __device__ void adjust_heap_d(int32_t *I, int32_t *K, int64_t hole,
     push_heap_d(I, K, hole, top, vi, vk);
 }
 
-__global__ void k_heapsort(int64_t n, const int32_t *__restrict__ head,
-                           const int32_t *__restrict__ state,
-                           const int32_t *__restrict__ end, int32_t *idx,
-                           int32_t *cnt) {
-    int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (q >= n || head[q] != q || state[q] != SEG_HEAP) return;
-    int32_t *I = idx + q;
-    int32_t *K = cnt + q;
-    const int64_t len = end[q] - q;
+template <typename Index>
+__device__ void heap_sort_d(Index *I, int32_t *K, int64_t len) {
     if (len >= 2) {  // __make_heap
         int64_t parent = (len - 2) / 2;
         for (;;) {
@@ -322,40 +329,268 @@ __global__ void k_heapsort(int64_t n, const int32_t *__restrict__ head,
     }
     for (int64_t last = len; last > 1;) {  // __sort_heap / __pop_heap
         --last;
-        const int32_t vi = I[last], vk = K[last];
+        const Index vi = I[last];
+        const int32_t vk = K[last];
         I[last] = I[0];
         K[last] = K[0];
         adjust_heap_d(I, K, 0, last, vi, vk);
     }
 }
 
-// Stable insertion sort (count descending) of every leaf segment.
-__global__ void k_leaf(int64_t n, const int32_t *__restrict__ head,
-                       const int32_t *__restrict__ state,
-                       const int32_t *__restrict__ end, int32_t *idx,
-                       int32_t *cnt) {
+// Where position p's pair ends up: slot p holds row `row` of `count` entries.
+__device__ __forceinline__ void emit_slot(int64_t p, int32_t row, int32_t count, int64_t n_rows,
+                                          int32_t *__restrict__ slot_row,
+                                          int32_t *__restrict__ slot_len,
+                                          int32_t *__restrict__ perm) {
+    slot_row[p] = row;
+    slot_len[p] = count;
+    if (row < n_rows) perm[row] = static_cast<int32_t>(p);
+}
+
+// Segments that ran out of depth while still too long for a tile.
+__global__ void k_heapsort(int64_t n, int64_t n_rows, const int32_t *__restrict__ head,
+                           const int32_t *__restrict__ state,
+                           const int32_t *__restrict__ end, int32_t *idx, int32_t *cnt,
+                           int32_t *__restrict__ slot_row, int32_t *__restrict__ slot_len,
+                           int32_t *__restrict__ perm) {
     int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (q >= n || head[q] != q || state[q] != SEG_LEAF) return;
-    const int len = static_cast<int>(end[q] - q);
-    int32_t I[kThreshold], K[kThreshold];
-    for (int i = 0; i < len; ++i) {
-        I[i] = idx[q + i];
-        K[i] = cnt[q + i];
+    if (q >= n || head[q] != q || state[q] != SEG_HEAP) return;
+    heap_sort_d(idx + q, cnt + q, end[q] - q);
+    for (int64_t p = q; p < end[q]; ++p) emit_slot(p, idx[p], cnt[p], n_rows, slot_row, slot_len, perm);
+}
+
+// ------------------------------------------------------------ tiles in LDS
+// The same recursion for every segment of one tile of up to kTile positions,
+// all levels in one launch, and the leaves; the result goes straight to
+// slot_row, slot_len and perm.
+//   WINDOWS: tile t holds the whole windows [t * span, t * span + span), span
+//     a multiple of sigma; counts come from row_ptr.
+//   otherwise: the parked segments that start in the t-th kParked positions,
+//     with their pairs in idx / cnt (segments longer than kParked are done by
+//     k_heapsort).
+//
+// A thread owns kTileItems neighbouring positions and keeps their segment
+// heads in registers.  Per level: pivots; stopper flags, both kinds in one
+// packed 16 + 16 bit prefix sum; stopper positions by rank, and the swap count
+// s, which the position where L(q) = min(L, R) ends writes (L(q) never falls
+// and R(q + 1) never rises, so max_q min(L(q), R(q + 1)) lies there); moves;
+// new segments.
+//
+// What bounds it: LDS latency between some six barriers a level, 72 KB a
+// workgroup, two workgroups a CU.  Level by level over global memory, ten
+// launches each, a conversion of 2,000,003 rows at sigma = 4096 spent 2.6 ms
+// here.
+template <bool WINDOWS>
+__global__ __launch_bounds__(kTileThreads, 8) void k_sort_tiles(
+    int64_t n, int64_t n_rows, int64_t sigma, int64_t span, const int32_t *__restrict__ row_ptr,
+    const int32_t *__restrict__ idx_in, const int32_t *__restrict__ cnt_in,
+    const int32_t *__restrict__ g_head, const int32_t *__restrict__ g_end,
+    const int32_t *__restrict__ g_depth, int32_t *__restrict__ slot_row,
+    int32_t *__restrict__ slot_len, int32_t *__restrict__ perm, int64_t *__restrict__ errflag) {
+    __shared__ __align__(16) int32_t cnt[kTile];
+    __shared__ __align__(16) uint32_t pre[kTile];  // inclusive prefix: left (low), right (high)
+    __shared__ uint16_t idx[kTile];
+    __shared__ uint16_t pos_l[kTile + 1], pos_r[kTile + 1];  // entry h: swap count, cut
+    __shared__ uint16_t seg_end[kTile];
+    __shared__ uint8_t seg_depth[kTile], seg_state[kTile];
+    __shared__ uint32_t wave_sum[kTileThreads / kWave];
+    const int tid = static_cast<int>(threadIdx.x);
+    const int q0 = tid * kTileItems;
+    int64_t base;
+    int w;  // positions of this tile
+    if (WINDOWS) {
+        base = static_cast<int64_t>(blockIdx.x) * span;
+        w = static_cast<int>(n - base < span ? n - base : span);
+    } else {
+        const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kParked;
+        const int64_t t1 = (t0 + kParked < n ? t0 + kParked : n) - 1;
+        const int64_t h0 = g_head[t0], h1 = g_head[t1];
+        base = h0 == t0 ? t0 : g_end[h0];
+        const int64_t stop = g_end[h1] - h1 > kParked ? h1 : g_end[h1];
+        if (stop <= base) return;
+        w = static_cast<int>(stop - base);
     }
-    for (int i = 1; i < len; ++i) {
-        const int32_t vi = I[i], vk = K[i];
-        int j = i;
-        while (j > 0 && vk > K[j - 1]) {
-            I[j] = I[j - 1];
-            K[j] = K[j - 1];
-            --j;
+    int head[kTileItems];
+#pragma unroll
+    for (int u = 0; u < kTileItems; ++u) {
+        const int q = q0 + u;
+        head[u] = -1;
+        if (q < w) {
+            const int64_t g = base + q;
+            int e, depth;
+            if (WINDOWS) {
+                cnt[q] = g < n_rows ? row_ptr[g + 1] - row_ptr[g] : 0;
+                head[u] = q - q % static_cast<int>(sigma);
+                e = head[u] + static_cast<int>(sigma) < w ? head[u] + static_cast<int>(sigma) : w;
+                depth = 2 * lg2(e - head[u]);
+            } else {
+                cnt[q] = cnt_in[g];
+                const int64_t h = g_head[g];
+                head[u] = static_cast<int>(h - base);
+                e = static_cast<int>(g_end[h] - base);
+                depth = g_depth[h];
+            }
+            idx[q] = static_cast<uint16_t>(q);
+            if (head[u] == q) {
+                seg_end[q] = static_cast<uint16_t>(e);
+                seg_depth[q] = static_cast<uint8_t>(depth);
+                seg_state[q] = e - q > kThreshold ? SEG_ACTIVE : SEG_LEAF;
+            }
         }
-        I[j] = vi;
-        K[j] = vk;
     }
-    for (int i = 0; i < len; ++i) {
-        idx[q + i] = I[i];
-        cnt[q + i] = K[i];
+    __syncthreads();
+    for (;;) {
+        bool any = false;
+#pragma unroll
+        for (int u = 0; u < kTileItems; ++u) {
+            const int h = q0 + u;
+            if (head[u] != h || seg_state[h] != SEG_ACTIVE) continue;
+            if (seg_depth[h] == 0) {  // __partial_sort fallback
+                seg_state[h] = SEG_HEAP;
+                continue;
+            }
+            any = true;
+            const int e = seg_end[h];
+            const int a = h + 1, b = h + (e - h) / 2, c = e - 1;
+            const int32_t ca = cnt[a], cb = cnt[b], cc = cnt[c];
+            int m;  // __move_median_to_first, comp(a, b) = a > b
+            if (ca > cb) m = cb > cc ? b : ca > cc ? c : a;
+            else m = ca > cc ? a : cb > cc ? c : b;
+            const int32_t tc = cnt[h];
+            const uint16_t ti = idx[h];
+            cnt[h] = cnt[m];
+            idx[h] = idx[m];
+            cnt[m] = tc;
+            idx[m] = ti;
+        }
+        if (!__syncthreads_or(any)) break;
+        uint32_t mine[kTileItems];  // flags, then inclusive prefix
+        bool active[kTileItems];
+        uint32_t sum = 0;
+#pragma unroll
+        for (int u = 0; u < kTileItems; ++u) {
+            const int q = q0 + u, h = head[u];
+            active[u] = h >= 0 && seg_state[h] == SEG_ACTIVE;
+            uint32_t f = 0;
+            if (active[u] && q > h) {
+                const int32_t c = cnt[q], p = cnt[h];
+                f = (c <= p ? 1u : 0u) | (c >= p ? 0x10000u : 0u);
+            }
+            sum += f;
+            mine[u] = sum;
+        }
+        const uint32_t incl = wave_incl_scan(sum);
+        if ((tid & (kWave - 1)) == kWave - 1) wave_sum[tid / kWave] = incl;
+        __syncthreads();
+        uint32_t before = incl - sum;
+        for (int v = 0; v < tid / kWave; ++v) before += wave_sum[v];
+#pragma unroll
+        for (int u = 0; u < kTileItems; ++u) {
+            mine[u] += before;
+            pre[q0 + u] = mine[u];
+        }
+        __syncthreads();
+        // stopper ranks: L(q) of (h, q], R(q) of [q, e)
+        int lq[kTileItems], rq1[kTileItems];
+#pragma unroll
+        for (int u = 0; u < kTileItems; ++u) {
+            const int q = q0 + u, h = head[u];
+            if (!active[u]) continue;
+            const int e = seg_end[h];
+            const uint32_t ph = pre[h], pe = pre[e - 1];
+            lq[u] = static_cast<int>((mine[u] & 0xffffu) - (ph & 0xffffu));
+            rq1[u] = static_cast<int>((pe >> 16) - (mine[u] >> 16));
+            if (q > h) {
+                const int32_t c = cnt[q], p = cnt[h];
+                if (c <= p) pos_l[h + lq[u]] = static_cast<uint16_t>(q);
+                if (c >= p) pos_r[h + rq1[u] + 1] = static_cast<uint16_t>(q);
+            }
+            if (lq[u] <= rq1[u]) {
+                int ln = INT32_MAX, rn = 0;
+                if (q + 1 < e) {
+                    const uint32_t pn = pre[q + 1];
+                    ln = static_cast<int>((pn & 0xffffu) - (ph & 0xffffu));
+                    rn = static_cast<int>((pe >> 16) - (pn >> 16));
+                }
+                if (ln > rn) pos_l[h] = static_cast<uint16_t>(lq[u] > rn ? lq[u] : rn);
+            }
+        }
+        __syncthreads();
+        int dest[kTileItems];
+        int32_t mc[kTileItems];
+        uint16_t mi[kTileItems];
+#pragma unroll
+        for (int u = 0; u < kTileItems; ++u) {
+            const int q = q0 + u, h = head[u];
+            dest[u] = q;
+            if (!active[u]) continue;
+            const int s = pos_l[h];
+            if (q == h) {
+                const int e = seg_end[h];
+                const int ltot = static_cast<int>((pre[e - 1] & 0xffffu) - (pre[h] & 0xffffu));
+                const int lnext = s + 1 <= ltot ? pos_l[h + s + 1] : e;
+                const int rs = s >= 1 ? pos_r[h + s] : e;
+                int cut = lnext < rs ? lnext : rs;
+                if (cut <= h || cut >= e) {  // cannot happen for a valid partition
+                    atomicAdd(reinterpret_cast<unsigned long long *>(errflag), 1ull);
+                    cut = h + 1;
+                }
+                pos_r[h] = static_cast<uint16_t>(cut);
+                continue;
+            }
+            mc[u] = cnt[q];
+            mi[u] = idx[q];
+            const int32_t p = cnt[h];
+            if (mc[u] <= p && lq[u] <= s) dest[u] = pos_r[h + lq[u]];
+            if (dest[u] == q && mc[u] >= p && rq1[u] + 1 <= s) dest[u] = pos_l[h + rq1[u] + 1];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < kTileItems; ++u) {
+            const int q = q0 + u, h = head[u];
+            if (!active[u]) continue;
+            if (dest[u] != q) {
+                cnt[dest[u]] = mc[u];
+                idx[dest[u]] = mi[u];
+            }
+            const int cut = pos_r[h];
+            if (q == h) {
+                const int e = seg_end[h];
+                const uint8_t d = static_cast<uint8_t>(seg_depth[h] - 1);
+                seg_end[cut] = static_cast<uint16_t>(e);
+                seg_depth[cut] = d;
+                seg_state[cut] = e - cut > kThreshold ? SEG_ACTIVE : SEG_LEAF;
+                seg_end[h] = static_cast<uint16_t>(cut);
+                seg_depth[h] = d;
+                seg_state[h] = cut - h > kThreshold ? SEG_ACTIVE : SEG_LEAF;
+            } else if (q >= cut) {
+                head[u] = cut;
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int u = 0; u < kTileItems; ++u) {
+        const int h = q0 + u;
+        if (head[u] == h && seg_state[h] == SEG_HEAP) heap_sort_d(idx + h, cnt + h, seg_end[h] - h);
+    }
+    __syncthreads();
+    // leaves: the stable order by count descending, each position counting
+    // the elements of its segment (at most 16) that come before it
+#pragma unroll
+    for (int u = 0; u < kTileItems; ++u) {
+        const int q = q0 + u, h = head[u];
+        if (h < 0) continue;
+        const int32_t c = cnt[q];
+        int p = q;
+        if (seg_state[h] == SEG_LEAF) {
+            p = h;
+            const int e = seg_end[h];
+            for (int t = h; t < e; ++t) p += cnt[t] > c || (cnt[t] == c && t < q);
+        }
+        const int64_t g = base + idx[q];
+        emit_slot(base + p, WINDOWS ? static_cast<int32_t>(g) : idx_in[g], c, n_rows, slot_row,
+                  slot_len, perm);
     }
 }
 
@@ -372,23 +607,14 @@ __global__ void k_chunk_len(int64_t n_chunks, int64_t C,
     chunk_elems[c] = static_cast<int64_t>(m) * C;
 }
 
+// chunk_ptr from the inclusive sums; the number of elements also to *total.
 __global__ void k_chunk_ptr(int64_t n_chunks,
                             const int64_t *__restrict__ incl,
-                            int32_t *__restrict__ chunk_ptr) {
+                            int32_t *__restrict__ chunk_ptr, int64_t *__restrict__ total) {
     int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (c > n_chunks) return;
     chunk_ptr[c] = c == 0 ? 0 : static_cast<int32_t>(incl[c - 1]);
-}
-
-__global__ void k_perm(int64_t n, int64_t n_rows,
-                       const int32_t *__restrict__ idx,
-                       int32_t *__restrict__ perm,
-                       int32_t *__restrict__ slot_row) {
-    int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int32_t old = idx[i];
-    slot_row[i] = old;
-    if (old < n_rows) perm[old] = static_cast<int32_t>(i);
+    if (c == n_chunks) *total = incl[c - 1];
 }
 
 __global__ void k_fill_i32(int64_t n, int32_t v, int32_t *__restrict__ p) {
@@ -556,14 +782,24 @@ void scs_free_arrays(smax_hip_scs_info &in) {
         SMAX_HIP_LAUNCHED(ctx, #kernel);                                      \
     } while (0)
 
-// Sorted (index, count) pairs of every sigma window, exactly as std::sort.
-int sell_sort_windows(smax_hip_ctx ctx, int64_t n, int64_t n_rows,
-                      int64_t sigma, const int32_t *row_ptr, int32_t **idx_out,
-                      int32_t **cnt_out, Scratch &S) {
+// Slots of every sigma window in std::sort's order: slot_row, slot_len and
+// perm.  A failed partition is counted in *errors (device, zero on entry).
+int sell_sort_windows(smax_hip_ctx ctx, int64_t n, int64_t n_rows, int64_t sigma,
+                      const int32_t *row_ptr, int32_t *slot_row, int32_t *slot_len,
+                      int32_t *perm, int64_t *errors, Scratch &S) {
+    if (sigma <= kTile) {
+        const int64_t span = kTile / sigma * sigma;
+        hipLaunchKernelGGL(k_sort_tiles<true>, grid_for(n, static_cast<int>(span)),
+                           dim3(kTileThreads), 0, ctx->stream, n, n_rows, sigma, span, row_ptr,
+                           nullptr, nullptr, nullptr, nullptr, nullptr, slot_row, slot_len, perm,
+                           errors);
+        SMAX_HIP_LAUNCHED(ctx, "k_sort_tiles");
+        return SMAX_HIP_SUCCESS;
+    }
     int32_t *idx, *cnt, *idx2, *cnt2, *head, *end, *depth, *state;
     int32_t *pv, *sw, *cut, *PL, *SR, *posL, *posR, *listA, *listB, *tmp;
-    int64_t *counters;
-    const int64_t nlist_cap = n / (kThreshold + 1) + 2;
+    int64_t *nlist;
+    const int64_t nlist_cap = n / (kParked + 1) + 2;
     int rc = 0;
     rc |= S.get(ctx, &idx, n, "sell sort");
     rc |= S.get(ctx, &cnt, n, "sell sort");
@@ -575,15 +811,15 @@ int sell_sort_windows(smax_hip_ctx ctx, int64_t n, int64_t n_rows,
     rc |= S.get(ctx, &state, n, "sell sort");
     rc |= S.get(ctx, &listA, nlist_cap, "sell sort");
     rc |= S.get(ctx, &listB, nlist_cap, "sell sort");
-    rc |= S.get(ctx, &counters, 4, "sell sort");
-    if (rc) return rc ? SMAX_HIP_ERROR_OUT_OF_MEMORY : 0;
-    rc = smax_hip_zero(ctx, counters, 4 * sizeof(int64_t));
+    rc |= S.get(ctx, &nlist, 1, "sell sort");
+    if (rc) return SMAX_HIP_ERROR_OUT_OF_MEMORY;
+    rc = smax_hip_zero(ctx, nlist, sizeof(int64_t));
     if (rc) return rc;
     const int64_t sig = sigma < n ? sigma : n;
     LAUNCH(k_init, n, n, n_rows, sig, row_ptr, idx, cnt, head, end, depth,
-           state, listA, counters + 0);
+           state, listA, nlist);
     int64_t nl = 0;
-    rc = read_i64(ctx, counters + 0, &nl);
+    rc = read_i64(ctx, nlist, &nl);
     if (rc) return rc;
     if (nl > 0) {
         rc |= S.get(ctx, &pv, n, "sell sort");
@@ -608,32 +844,24 @@ int sell_sort_windows(smax_hip_ctx ctx, int64_t n, int64_t n_rows,
         rc = scan_inclusive<int32_t, true>(ctx, SR, SR, n, tmp);
         if (rc) return rc;
         LAUNCH(k_rank, n, n, head, state, end, cnt, pv, PL, SR, posL, posR, sw);
-        LAUNCH(k_cut, nl, nl, listA, state, end, PL, posL, posR, sw, cut,
-               counters + 2);
+        LAUNCH(k_cut, nl, nl, listA, state, end, PL, posL, posR, sw, cut, errors);
         LAUNCH(k_move, n, n, head, state, end, pv, sw, PL, SR, posL, posR, idx,
                cnt, idx2, cnt2);
         std::swap(idx, idx2);
         std::swap(cnt, cnt2);
         LAUNCH(k_split, n, n, head, state, cut);
-        rc = smax_hip_zero(ctx, counters + 1, sizeof(int64_t));
+        rc = smax_hip_zero(ctx, nlist, sizeof(int64_t));
         if (rc) return rc;
-        LAUNCH(k_newsegs, nl, nl, listA, state, end, depth, cut, listB,
-               counters + 1);
-        rc = read_i64(ctx, counters + 1, &nl);
+        LAUNCH(k_newsegs, nl, nl, listA, state, end, depth, cut, listB, nlist);
+        rc = read_i64(ctx, nlist, &nl);
         if (rc) return rc;
         std::swap(listA, listB);
     }
-    int64_t errs = 0;
-    rc = read_i64(ctx, counters + 2, &errs);
-    if (rc) return rc;
-    if (errs)
-        return fail(ctx, SMAX_HIP_ERROR_RUNTIME,
-                    "sell sort: %lld partitions produced an invalid cut",
-                    static_cast<long long>(errs));
-    LAUNCH(k_heapsort, n, n, head, state, end, idx, cnt);
-    LAUNCH(k_leaf, n, n, head, state, end, idx, cnt);
-    *idx_out = idx;
-    *cnt_out = cnt;
+    LAUNCH(k_heapsort, n, n, n_rows, head, state, end, idx, cnt, slot_row, slot_len, perm);
+    hipLaunchKernelGGL(k_sort_tiles<false>, grid_for(n, kParked), dim3(kTileThreads), 0,
+                       ctx->stream, n, n_rows, sig, 0, nullptr, idx, cnt, head, end, depth,
+                       slot_row, slot_len, perm, errors);
+    SMAX_HIP_LAUNCHED(ctx, "k_sort_tiles");
     return SMAX_HIP_SUCCESS;
 }
 
@@ -663,10 +891,7 @@ int build_scs(smax_hip_ctx ctx, int64_t n_rows, int64_t n_cols, int64_t nnz,
                     "scs conversion: %lld padded rows exceed int32",
                     (long long)n);
     Scratch S(ctx);
-    int32_t *idx = nullptr, *cnt = nullptr;
-    int rc = sell_sort_windows(ctx, n, n_rows, sigma, row_ptr, &idx, &cnt, S);
-    if (rc) return rc;
-
+    int rc = 0;
     smax_hip_scs_info info{};
     info.C = C;
     info.sigma = sigma;
@@ -687,7 +912,8 @@ int build_scs(smax_hip_ctx ctx, int64_t n_rows, int64_t n_cols, int64_t nnz,
         }
     } guard{ctx, &info};
 
-    int64_t *elems, *incl, *tmp64;
+    int64_t *elems, *incl, *tmp64, *words;  // words: sort errors, SELL elements
+    rc |= S.get(ctx, &words, 2, "scs conversion");
     rc |= S.get(ctx, &elems, n_chunks, "scs conversion");
     rc |= S.get(ctx, &incl, n_chunks, "scs conversion");
     rc |= S.get(ctx, &tmp64, scan_tmp_elems(n_chunks), "scs conversion");
@@ -703,21 +929,28 @@ int build_scs(smax_hip_ctx ctx, int64_t n_rows, int64_t n_cols, int64_t nnz,
                     sizeof(int32_t) * n, "scs slot_len");
     if (rc) return SMAX_HIP_ERROR_OUT_OF_MEMORY;
 
-    LAUNCH(k_chunk_len, n_chunks, n_chunks, C, cnt, info.chunk_lengths, elems);
+    rc = smax_hip_zero(ctx, words, 2 * sizeof(int64_t));
+    if (!rc)
+        rc = sell_sort_windows(ctx, n, n_rows, sigma, row_ptr, info.slot_row, info.slot_len,
+                               info.perm, words, S);
+    if (rc) return rc;
+    LAUNCH(k_chunk_len, n_chunks, n_chunks, C, info.slot_len, info.chunk_lengths, elems);
     rc = scan_inclusive<int64_t, false>(ctx, elems, incl, n_chunks, tmp64);
     if (rc) return rc;
-    int64_t n_elements = 0;
-    rc = read_i64(ctx, incl + (n_chunks - 1), &n_elements);
-    if (rc) return rc;
+    LAUNCH(k_chunk_ptr, n_chunks + 1, n_chunks, incl, info.chunk_ptr, words + 1);
+    SMAX_HIP_CALL(ctx, hipMemcpyAsync(ctx->host_word, words, 2 * sizeof(int64_t),
+                                      hipMemcpyDeviceToHost, ctx->stream));
+    SMAX_HIP_CALL(ctx, hipStreamSynchronize(ctx->stream));
+    if (ctx->host_word[0])
+        return fail(ctx, SMAX_HIP_ERROR_RUNTIME,
+                    "sell sort: %lld partitions produced an invalid cut",
+                    static_cast<long long>(ctx->host_word[0]));
+    const int64_t n_elements = ctx->host_word[1];
     if (n_elements > INT32_MAX)
         return fail(ctx, SMAX_HIP_ERROR_OVERFLOW,
                     "scs conversion: %lld SELL elements exceed int32 chunk_ptr",
                     (long long)n_elements);
     info.n_elements = n_elements;
-    LAUNCH(k_chunk_ptr, n_chunks + 1, n_chunks, incl, info.chunk_ptr);
-    LAUNCH(k_perm, n, n, n_rows, idx, info.perm, info.slot_row);
-    SMAX_HIP_CALL(ctx, hipMemcpyAsync(info.slot_len, cnt, sizeof(int32_t) * n,
-                                      hipMemcpyDeviceToDevice, ctx->stream));
 
     rc |= dev_alloc(ctx, reinterpret_cast<void **>(&info.col),
                     sizeof(int32_t) * n_elements, "scs col");

@@ -643,3 +643,41 @@ def test_scs_from_sell_refusals(ctx):
         d.free()
     T.destroy()
     S.destroy()
+
+
+@pytest.mark.parametrize("n", [1, 17, 4095, 4096, 4097, 13001])
+@pytest.mark.parametrize("sigma", [16, 17, 100, 2047, 2048, 2049, 4095, 4096, 4097, 6000, 1 << 20])
+@pytest.mark.parametrize("kind", ["ties", "wide", "ascending", "descending"])
+def test_window_sort_tile_edges(ctx, sort_pin, tmp_path, n, sigma, kind):
+    """The order inside every sigma window equals libstdc++'s std::sort around
+    the sizes where the sort changes path: leaves (16), tiles of whole windows
+    (4096 positions), and the segments of longer windows that are short enough
+    (2048) to finish in a tile."""
+    rng = np.random.default_rng(n + sigma)
+    L = rng.integers(0, {"ties": 4}.get(kind, 60), n).astype(np.int32)
+    if kind in ("ascending", "descending"):
+        L = np.sort(L) if kind == "ascending" else np.sort(L)[::-1].copy()
+    rp = np.concatenate([[0], np.cumsum(L)]).astype(np.int32)
+    A = Csr(n, 64, rp, np.zeros(rp[-1], np.int32), np.ones(rp[-1], np.float32))
+    s = gpu_scs(ctx, A, 1, sigma)
+    got = s.arrays(np.float32)
+    order = std_sort_windows(sort_pin, L, min(sigma, n), tmp_path)
+    assert_bitwise(got["slot_row"], order, "std::sort order")
+    assert_bitwise(got["slot_len"], L[order], "slot_len")
+    assert_bitwise(got["perm"][order], np.arange(n, dtype=np.int32), "perm")
+    s.destroy()
+
+
+@pytest.mark.parametrize("n,sigma", [(3000, 3000), (4096, 4096), (6000, 6000), (9000, 4500)])
+def test_window_sort_heap_fallback_in_and_beyond_a_tile(ctx, sort_pin, tmp_path, n, sigma):
+    """McIlroy's adversary per window: the heap-sorted segment lies in a tile
+    (windows up to 4096) or is too long for one (its own kernel)."""
+    out = tmp_path / "k.bin"
+    subprocess.run([str(sort_pin), "killer", str(sigma), str(out)], check=True)
+    L = np.tile(np.fromfile(out, np.int32), n // sigma)
+    rp = np.concatenate([[0], np.cumsum(L)]).astype(np.int32)
+    A = Csr(n, 64, rp, np.zeros(rp[-1], np.int32), np.ones(rp[-1], np.float32))
+    s = gpu_scs(ctx, A, 1, sigma)
+    order = std_sort_windows(sort_pin, L, sigma, tmp_path)
+    assert_bitwise(s.arrays(np.float32)["slot_row"], order, "std::sort order")
+    s.destroy()
