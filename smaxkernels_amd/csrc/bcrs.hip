@@ -561,33 +561,12 @@ static void launch_bcrs_spmm(smax_hip_ctx ctx, int64_t threads, int64_t n_block_
 // past, in row order, so of two entries with the same column the later one
 // stays, as in the reference's fill loop.
 
-// c / b_w for 0 <= c < 2^31 as a multiply and shift: with l = ceil(log2
-// b_w) and m = ceil(2^(31+l) / b_w), m*b_w - 2^(31+l) < b_w <= 2^l, which
-// makes floor(c*m / 2^(31+l)) exact for every 31-bit c (Granlund and
-// Montgomery, "Division by invariant integers using multiplication", 1994,
-// Theorem 4.2).
-struct BlockDiv {
-    uint32_t m;
-    int shift;
-    __device__ int32_t operator()(int32_t c) const {
-        return static_cast<int32_t>(
-            (static_cast<uint64_t>(static_cast<uint32_t>(c)) * m) >> shift);
-    }
-};
-
-inline BlockDiv block_div(int64_t b_w) {
-    int l = 0;
-    while ((int64_t{1} << l) < b_w) ++l;
-    const uint64_t m = ((uint64_t{1} << (31 + l)) + b_w - 1) / b_w;
-    return {static_cast<uint32_t>(m), 31 + l};
-}
-
 template <typename V>
 struct BcrsBuild {
     int64_t nbr, n_cols;
     int b_h, b_w, h_pad, w_pad, col_major;
     int cap;  // entries the LDS tile holds
-    BlockDiv div;
+    FastDiv div;
     const int32_t *row_ptr, *col;
     const V *val;
     int64_t *cnt;        // count pass: blocks per block row
@@ -914,7 +893,7 @@ int smax_hip_bcrs_from_crs(smax_hip_ctx ctx, int64_t n_rows, int64_t n_cols,
     args.h_pad = static_cast<int>(h_pad);
     args.w_pad = static_cast<int>(w_pad);
     args.col_major = block_col_major ? 1 : 0;
-    args.div = block_div(b_w);
+    args.div = fast_div(b_w);
     args.row_ptr = row_ptr;
     args.col = col;
     args.cnt = cnt;
@@ -1086,22 +1065,6 @@ static int gather_blocks(smax_hip_ctx ctx, const smax_hip_bcrs_info &T,
         launch_gather_blocks<uint16_t>(ctx, T.n_blocks, bytes, T.src_block, src, T.val);
     SMAX_HIP_LAUNCHED(ctx, "bcrs_gather_blocks");
     return SMAX_HIP_SUCCESS;
-}
-
-// Last row r in [0, n_rows) with row_ptr[r] <= j: all 64 lanes of a wavefront
-// (same j) probe 64 rows at a time, so 10^6 rows take four dependent loads.
-__device__ __forceinline__ int64_t wave_row_of(const int32_t *__restrict__ row_ptr,
-                                               int64_t n_rows, int64_t j) {
-    const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
-    int64_t lo = 0, hi = n_rows;  // row_ptr[lo] <= j < row_ptr[hi]
-    while (hi - lo > 1) {
-        const int64_t step = (hi - lo + kWave - 1) / kWave;
-        const int64_t r = lo + lane * step;
-        const bool below = r < hi && row_ptr[r] <= j;  // lane 0's always is
-        lo += (__popcll(__ballot(below)) - 1) * step;
-        hi = lo + step < hi ? lo + step : hi;
-    }
-    return lo;
 }
 
 // VL entries from p in one access (VL * sizeof(A) is 16 with p 16-byte

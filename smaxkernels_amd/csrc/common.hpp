@@ -119,6 +119,42 @@ __device__ __forceinline__ int64_t xcd_block(int64_t bid, int64_t nblocks) {
     return xcd < r ? xcd * (q + 1) + local : r * (q + 1) + (xcd - r) * q + local;
 }
 
+// n / d for 0 <= n < 2^31 as a multiply and shift: with l = ceil(log2 d) and
+// m = ceil(2^(31+l) / d), m*d - 2^(31+l) < d <= 2^l, which makes
+// floor(n*m / 2^(31+l)) exact for every 31-bit n (Granlund and Montgomery,
+// "Division by invariant integers using multiplication", 1994, Theorem 4.2).
+struct FastDiv {
+    uint32_t m;
+    int shift;
+    __device__ int32_t operator()(int32_t n) const {
+        return static_cast<int32_t>(
+            (static_cast<uint64_t>(static_cast<uint32_t>(n)) * m) >> shift);
+    }
+};
+
+inline FastDiv fast_div(int64_t d) {
+    int l = 0;
+    while ((int64_t{1} << l) < d) ++l;
+    const uint64_t m = ((uint64_t{1} << (31 + l)) + d - 1) / d;
+    return {static_cast<uint32_t>(m), 31 + l};
+}
+
+// Last row r in [0, n_rows) with row_ptr[r] <= j: all 64 lanes of a wavefront
+// (same j) probe 64 rows at a time, so 10^6 rows take four dependent loads.
+__device__ __forceinline__ int64_t wave_row_of(const int32_t *__restrict__ row_ptr,
+                                               int64_t n_rows, int64_t j) {
+    const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+    int64_t lo = 0, hi = n_rows;  // row_ptr[lo] <= j < row_ptr[hi]
+    while (hi - lo > 1) {
+        const int64_t step = (hi - lo + kWave - 1) / kWave;
+        const int64_t r = lo + lane * step;
+        const bool below = r < hi && row_ptr[r] <= j;  // lane 0's always is
+        lo += (__popcll(__ballot(below)) - 1) * step;
+        hi = lo + step < hi ? lo + step : hi;
+    }
+    return lo;
+}
+
 // Lane U of each aligned group of 8 lanes, handed to the group (ds_swizzle
 // in bit mode: and-mask 0x18 keeps the group, or-mask U picks the lane).
 // Used where 8 lanes share one row or slot and would otherwise each load

@@ -681,3 +681,32 @@ def test_window_sort_heap_fallback_in_and_beyond_a_tile(ctx, sort_pin, tmp_path,
     order = std_sort_windows(sort_pin, L, sigma, tmp_path)
     assert_bitwise(s.arrays(np.float32)["slot_row"], order, "std::sort order")
     s.destroy()
+
+
+@pytest.mark.parametrize("C_", [1, 3, 32, 64, 300])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.uint16])
+def test_conversion_fill_runs_of_empty_chunks(ctx, C_, dtype):
+    """Elements a workgroup apart with many empty chunks between them, rows
+    longer than a workgroup's span, and padding, for chunk widths that divide
+    a wavefront and others."""
+    rng = np.random.default_rng(C_)
+    n = 9000
+    L = np.zeros(n, np.int64)
+    L[[0, 1, 5, 40, 41, n // 2, n - 1]] = [3, 1, 700, 2, 5000, 1, 9]
+    L[3000:3100] = rng.integers(0, 50, 100)
+    rp = np.concatenate([[0], np.cumsum(L)]).astype(np.int32)
+    col = rng.integers(0, n, rp[-1]).astype(np.int32)
+    A = Csr(n, n, rp, col, rng.integers(1, 1 << 14, rp[-1]).astype(dtype))
+    for sigma in (1, 1000):
+        s = gpu_scs(ctx, A, C_, sigma)
+        got = s.arrays(dtype)
+        src, real = got["src_index"], got["src_index"] >= 0
+        assert_bitwise(np.sort(src[real]), np.arange(A.nnz, dtype=np.int32), "every entry once")
+        assert_bitwise(got["col"], np.where(real, col[src], 0).astype(np.int32), "col")
+        assert_bitwise(got["val"], np.where(real, A.val[src], 0).astype(dtype), "val")
+        # element j of slot i sits at chunk_ptr + j*C + i, in row order
+        for i in (0, 1, 5, 40, 41, n // 2, n - 1):
+            p = int(got["perm"][i])
+            at = int(got["chunk_ptr"][p // C_]) + np.arange(L[i]) * C_ + p % C_
+            assert_bitwise(src[at], np.arange(rp[i], rp[i + 1], dtype=np.int32), f"row {i}")
+        s.destroy()
