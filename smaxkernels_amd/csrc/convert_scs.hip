@@ -636,13 +636,16 @@ __device__ __forceinline__ int64_t row_of(const int32_t *__restrict__ ptr, int64
 // j of slot i of chunk c, at chunk_ptr[c] + j*C + i, is entry j of the slot's
 // row, or padding (column 0, value 0, no source) past the row's end.
 //
-// What bounds it: the stores of the padded arrays, 8 bytes and the value each;
-// they are contiguous, while the reads go along 64 rows at once and are served
-// line by line from L1.  A workgroup takes kFillItems x 256 consecutive
-// elements wherever they lie, so rows of thousands of entries are shared out
-// too.  Scattering in CRS order instead (a 21-step search of each entry's row,
-// scattered 4- and 8-byte stores) after three passes that cleared the arrays
-// took 1.15 + 0.24 ms for 2,000,003 rows at sigma = 4096 (80 M elements).
+// What bounds it: the stores of the padded arrays, 8 bytes and the value each
+// (contiguous; 225 us for the 80 M elements of 2,000,003 rows at sigma = 4096
+// in FP64), and, not overlapped with them, the reads along 64 rows at once
+// (260 us).  A wavefront takes kFillItems x 64 consecutive elements wherever
+// they lie, so rows of thousands of entries are shared out too, and a lane
+// that keeps its slot reads kFillItems entries of one row while their lines
+// are in L1; the outputs pass the caches by.  0.65 ms with 4 elements at a time
+// and 256 apart, 0.56 this way.  Scattering in CRS order instead (a 21-step
+// search of each entry's row, scattered 4- and 8-byte stores) after three
+// passes that cleared the arrays took 1.15 + 0.24 ms.
 constexpr int kFillItems = 16;
 
 template <typename V>
@@ -653,62 +656,61 @@ __global__ __launch_bounds__(256) void k_fill(
     const int32_t *__restrict__ chunk_ptr, const int32_t *__restrict__ slot_row,
     const int32_t *__restrict__ slot_len, int32_t *__restrict__ out_col, V *__restrict__ out_val,
     int32_t *__restrict__ out_src) {
-    const int64_t e0 = static_cast<int64_t>(blockIdx.x) * (256 * kFillItems);
-    int64_t c = wave_row_of(chunk_ptr, n_chunks, e0);
+    // neighbouring workgroups, whose rows share lines, on one XCD
+    const int64_t w0 = (xcd_block(blockIdx.x, gridDim.x) * 256 + (threadIdx.x & ~(kWave - 1))) *
+                       kFillItems;
+    if (w0 >= n_elements) return;  // whole wavefronts
+    const int64_t e0 = w0 + (threadIdx.x & (kWave - 1));
+    int64_t c = wave_row_of(chunk_ptr, n_chunks, w0);
     int32_t begin = chunk_ptr[c], end = chunk_ptr[c + 1];
     int64_t at = -1;  // the slot whose row start and length are held
     int32_t start = 0, len = 0;
-    constexpr int U = 4;
-    for (int t = 0; t < kFillItems; t += U) {
-        int32_t from[U];  // the element's CRS position, -1 for padding
+    int32_t from[kFillItems];  // each element's CRS position, -1 for padding
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int64_t e = e0 + (t + u) * 256 + threadIdx.x;
-            from[u] = -1;
-            if (e >= n_elements) continue;
+    for (int u = 0; u < kFillItems; ++u) {
+        const int64_t e = e0 + u * kWave;
+        from[u] = -1;
+        if (e >= n_elements) continue;
+        if (e >= end) {
+            // the next chunks in turn; past a run of empty ones by search
+            for (int step = 0; e >= end && step < 8; ++step) end = chunk_ptr[++c + 1];
             if (e >= end) {
-                // the next chunks in turn; past a run of empty ones by search
-                for (int step = 0; e >= end && step < 8; ++step) end = chunk_ptr[++c + 1];
-                if (e >= end) {
-                    c = row_of(chunk_ptr, c, n_chunks, e);
-                    end = chunk_ptr[c + 1];
-                }
-                begin = chunk_ptr[c];
+                c = row_of(chunk_ptr, c, n_chunks, e);
+                end = chunk_ptr[c + 1];
             }
-            const int32_t off = static_cast<int32_t>(e - begin);
-            const int32_t j = by_c(off);
-            const int64_t slot = c * C + (off - j * C);
-            if (slot != at) {
-                at = slot;
-                len = slot_len[slot];
-                const int32_t r = slot_row[slot];
-                start = r < n_rows ? row_ptr[r] : 0;
-            }
-            if (j < len) from[u] = start + j;
+            begin = chunk_ptr[c];
         }
-        int32_t vc[U], vs[U];
-        V vv[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            vc[u] = 0;
-            vs[u] = from[u];
-            vv[u] = 0;
-            if (from[u] >= 0) {
-                vc[u] = col[from[u]];
-                if (src_map) vs[u] = src_map[from[u]];
-            }
+        const int32_t off = static_cast<int32_t>(e - begin);
+        const int32_t j = by_c(off);
+        const int64_t slot = c * C + (off - j * C);
+        if (slot != at) {
+            at = slot;
+            len = slot_len[slot];
+            const int32_t r = slot_row[slot];
+            start = r < n_rows ? row_ptr[r] : 0;
         }
+        if (j < len) from[u] = start + j;
+    }
+    int32_t vc[kFillItems], vs[kFillItems];
+    V vv[kFillItems];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (vs[u] >= 0) vv[u] = val[vs[u]];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int64_t e = e0 + (t + u) * 256 + threadIdx.x;
-            if (e >= n_elements) continue;
-            out_col[e] = vc[u];
-            out_val[e] = vv[u];
-            out_src[e] = vs[u];
+    for (int u = 0; u < kFillItems; ++u) {
+        vc[u] = 0;
+        vs[u] = from[u];
+        if (from[u] >= 0) {
+            vc[u] = col[from[u]];
+            if (src_map) vs[u] = src_map[from[u]];
         }
+    }
+#pragma unroll
+    for (int u = 0; u < kFillItems; ++u) vv[u] = vs[u] >= 0 ? val[vs[u]] : V(0);
+#pragma unroll
+    for (int u = 0; u < kFillItems; ++u) {
+        const int64_t e = e0 + u * kWave;
+        if (e >= n_elements) continue;
+        __builtin_nontemporal_store(vc[u], out_col + e);
+        __builtin_nontemporal_store(vv[u], out_val + e);
+        __builtin_nontemporal_store(vs[u], out_src + e);
     }
 }
 
