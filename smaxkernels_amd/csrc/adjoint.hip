@@ -4,8 +4,8 @@
 // A^T: the CRS positions j = 0..nnz-1 are already in row-major order, so a
 // *stable* sort of (col[j], j) by column yields A^T's CRS with every column's
 // entries in ascending original row order.  The sort is an LSD radix sort
-// with 4-bit digits whose scatter ranks come from prefix sums only (no
-// atomics decide an order), so the layout is deterministic.  The resulting
+// whose scatter ranks come from ballots and prefix sums only (no atomics
+// decide an order), so the layout is deterministic.  The resulting
 // CRS of A^T goes through the same GPU SELL conversion as A, with src_index
 // pointing back at A's CRS nonzeros.
 //
@@ -362,35 +362,18 @@ int smax_hip_scs_transpose_from_crs(smax_hip_ctx ctx, int64_t n_rows,
                     "smax_hip_scs_transpose_from_crs: %lld x %lld exceeds int32",
                     (long long)n_rows, (long long)n_cols);
     const int64_t m = nnz > 0 ? nnz : 1;
-    uint32_t *keys = nullptr;
-    int32_t *vals = nullptr, *t_row_ptr = nullptr, *t_col = nullptr;
+    int32_t *t_row_ptr = nullptr, *t_col = nullptr;
     RadixSort sorter(ctx);
     int rc = sorter.reserve(m);
     if (!rc)
         rc = dev_alloc(ctx, reinterpret_cast<void **>(&t_row_ptr),
                        4 * (n_cols + 1), "transpose");
     if (!rc) rc = dev_alloc(ctx, reinterpret_cast<void **>(&t_col), 4 * m, "transpose");
-    if (!rc && nnz > 0) {
-        hipLaunchKernelGGL(iota_keys, grid_for(nnz, 256), dim3(256), 0,
-                           ctx->stream, nnz, col, sorter.keys(), sorter.vals());
-        rc = check_launch(ctx, "iota_keys");
-        if (!rc) rc = sorter.sort(nnz, n_cols);
-    }
-    keys = sorter.keys();
-    vals = sorter.vals();
-    if (!rc) {
-        hipLaunchKernelGGL(transpose_row_ptr, grid_for(n_cols + 1, 256), dim3(256),
-                           0, ctx->stream, n_cols, nnz, keys, t_row_ptr);
-        rc = check_launch(ctx, "transpose_row_ptr");
-    }
-    if (!rc && nnz > 0) {
-        hipLaunchKernelGGL(transpose_cols, grid_for(nnz, 256), dim3(256), 0,
-                           ctx->stream, nnz, n_rows, row_ptr, vals, t_col);
-        rc = check_launch(ctx, "transpose_cols");
-    }
+    if (!rc) rc = sorter.sort(reinterpret_cast<const uint32_t *>(col), nnz, n_cols);
+    if (!rc) rc = sorter.transposed_pattern(n_rows, n_cols, nnz, row_ptr, t_row_ptr, t_col);
     if (!rc)
         rc = build_scs(ctx, n_cols, n_rows, nnz, t_row_ptr, t_col, val,
-                       val_bytes, vals, C, sigma, out);
+                       val_bytes, sorter.vals(), C, sigma, out);
     (void)hipStreamSynchronize(ctx->stream);
     dev_free(t_row_ptr);
     dev_free(t_col);

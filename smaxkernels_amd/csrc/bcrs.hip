@@ -1263,27 +1263,14 @@ int smax_hip_bcrs_transpose(smax_hip_ctx ctx, smax_hip_bcrs A, smax_hip_bcrs *ou
         rc = dev_alloc(ctx, reinterpret_cast<void **>(&t.src_block), 4 * m,
                        "bcrs transpose");
     if (!rc) rc = dev_alloc(ctx, &t.val, a.val_bytes * m * a.h_pad * a.w_pad, "bcrs transpose");
+    if (!rc) rc = sorter.sort(reinterpret_cast<const uint32_t *>(a.col), nb, a.n_block_cols);
+    if (!rc)
+        rc = sorter.transposed_pattern(a.n_block_rows, t.n_block_rows, nb, a.row_ptr, t.row_ptr,
+                                       t.col);
     if (!rc && nb > 0) {
-        hipLaunchKernelGGL(iota_keys, grid_for(nb, 256), dim3(256), 0, ctx->stream, nb,
-                           a.col, sorter.keys(), sorter.vals());
-        rc = check_launch(ctx, "iota_keys");
-        if (!rc) rc = sorter.sort(nb, a.n_block_cols);
-    }
-    if (!rc) {
-        hipLaunchKernelGGL(transpose_row_ptr, grid_for(t.n_block_rows + 1, 256),
-                           dim3(256), 0, ctx->stream, t.n_block_rows, nb, sorter.keys(),
-                           t.row_ptr);
-        rc = check_launch(ctx, "transpose_row_ptr");
-    }
-    if (!rc && nb > 0) {
-        hipLaunchKernelGGL(transpose_cols, grid_for(nb, 256), dim3(256), 0, ctx->stream,
-                           nb, a.n_block_rows, a.row_ptr, sorter.vals(), t.col);
-        rc = check_launch(ctx, "transpose_cols");
-        if (!rc) {
-            const hipError_t e = hipMemcpyAsync(t.src_block, sorter.vals(), 4 * nb,
-                                                hipMemcpyDeviceToDevice, ctx->stream);
-            if (e != hipSuccess) rc = hip_fail(ctx, e, "src_block copy");
-        }
+        const hipError_t e = hipMemcpyAsync(t.src_block, sorter.vals(), 4 * nb,
+                                            hipMemcpyDeviceToDevice, ctx->stream);
+        if (e != hipSuccess) rc = hip_fail(ctx, e, "src_block copy");
         if (!rc) rc = gather_blocks(ctx, t, a.val);
     }
     (void)hipStreamSynchronize(ctx->stream);

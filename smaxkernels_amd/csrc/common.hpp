@@ -139,6 +139,16 @@ inline FastDiv fast_div(int64_t d) {
     return {static_cast<uint32_t>(m), 31 + l};
 }
 
+// The last r in [lo, hi) with ptr[r] <= j, where ptr[lo] <= j < ptr[hi].
+__device__ __forceinline__ int64_t row_of(const int32_t *__restrict__ ptr, int64_t lo, int64_t hi,
+                                          int64_t j) {
+    while (hi - lo > 1) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (ptr[mid] <= j) lo = mid; else hi = mid;
+    }
+    return lo;
+}
+
 // Last row r in [0, n_rows) with row_ptr[r] <= j: all 64 lanes of a wavefront
 // (same j) probe 64 rows at a time, so 10^6 rows take four dependent loads.
 __device__ __forceinline__ int64_t wave_row_of(const int32_t *__restrict__ row_ptr,

@@ -622,16 +622,6 @@ __global__ void k_fill_i32(int64_t n, int32_t v, int32_t *__restrict__ p) {
     if (i < n) p[i] = v;
 }
 
-// The last r in [lo, hi) with ptr[r] <= j, where ptr[lo] <= j < ptr[hi].
-__device__ __forceinline__ int64_t row_of(const int32_t *__restrict__ ptr, int64_t lo, int64_t hi,
-                                          int64_t j) {
-    while (hi - lo > 1) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (ptr[mid] <= j) lo = mid; else hi = mid;
-    }
-    return lo;
-}
-
 // The SELL arrays (convert_formats.hpp:101-128), element by element: element
 // j of slot i of chunk c, at chunk_ptr[c] + j*C + i, is entry j of the slot's
 // row, or padding (column 0, value 0, no source) past the row's end.

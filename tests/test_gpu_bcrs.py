@@ -424,3 +424,38 @@ def test_bcrs_transpose_refresh_unit_widths(ctx, vt, bh, bw, hp, wp, shift):
     d.free()
     for h in (T, b):
         h.destroy()
+
+
+@pytest.mark.parametrize("n_cols", [1, 2, 255, 256, 257, 4097, 65536, 65537, (1 << 17) + 3])
+@pytest.mark.parametrize("nnz", [1, 63, 4095, 4096, 4097, 30011])
+def test_transposed_pattern_digit_and_tile_edges(ctx, n_cols, nnz):
+    """The sort behind the transposes, through 1x1 blocks: one to three digits
+    (1 to 18 bit keys), partial tiles, runs of empty rows and one row longer
+    than a wavefront's share, against a stable host sort by column."""
+    rng = np.random.default_rng(nnz)
+    n_rows = 700
+    cut = np.sort(rng.integers(0, nnz + 1, n_rows - 1))
+    cut[100:400] = cut[100]          # empty rows
+    cut[400:] = np.maximum(cut[400:], cut[100])
+    rp = np.concatenate([[0], cut, [nnz]]).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(n_cols, e - s, replace=e - s > n_cols))
+                          for s, e in zip(rp, rp[1:])]).astype(np.int32)
+    # a block row keeps each column once
+    keep = np.ones(nnz, bool)
+    keep[1:] = col[1:] != col[:-1]
+    keep[rp[:-1][rp[:-1] < nnz]] = True
+    rp = np.concatenate([[0], np.cumsum(keep)])[rp].astype(np.int32)
+    col = col[keep]
+    b = gpu_bcrs(ctx, n_rows, n_cols, rp, col, np.arange(col.size, dtype=np.float64), 1, 1, 1, 1,
+                 False)
+    T = b.transpose()
+    order = np.argsort(col, kind="stable").astype(np.int32)
+    rows = np.repeat(np.arange(n_rows), np.diff(rp)).astype(np.int32)
+    got = T.arrays(np.float64)
+    assert_bitwise(ctx.download_ptr(T.info.src_block, col.size, np.int32), order, "src_block")
+    assert_bitwise(got["col"], rows[order], "col")
+    assert_bitwise(got["row_ptr"], np.searchsorted(col[order], np.arange(n_cols + 1))
+                   .astype(np.int32), "row_ptr")
+    assert_bitwise(got["val"], order.astype(np.float64), "val")
+    for h in (T, b):
+        h.destroy()
