@@ -23,6 +23,8 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "common.hpp"
@@ -132,9 +134,12 @@ enum { kCol32 = 0, kRel16 = 1, kTab8 = 2 };
 constexpr int kColTable = 32;
 
 // (A x)[s]: sequential fma chain over the slot's SELL elements, then (DIAG)
-// the FP32 diagonal term.  With kTab8 every lane of the wavefront must run
-// this (one chunk per wavefront, all slots present).
-template <typename V, typename W, bool DIAG, int MODE>
+// the FP32 diagonal term; x_at(c) is entry c of x.  With kTab8 every lane of
+// the wavefront must run this (one chunk per wavefront, all slots present).
+// REST: the last, shorter group of elements is loaded at once too, instead of
+// one element after the other (for the small systems, whose chains are a few
+// memory round trips long; it costs registers, which slows large ones).
+template <typename V, typename W, bool DIAG, int MODE, bool REST, typename X>
 __device__ __forceinline__ W apply_slot(int64_t s, int64_t C,
                                         const int32_t *__restrict__ chunk_ptr,
                                         const int32_t *__restrict__ chunk_len,
@@ -144,8 +149,7 @@ __device__ __forceinline__ W apply_slot(int64_t s, int64_t C,
                                         const int64_t *__restrict__ idx_row,
                                         const int16_t *__restrict__ tab,
                                         const V *__restrict__ val,
-                                        const float *__restrict__ diag,
-                                        const W *__restrict__ x) {
+                                        const float *__restrict__ diag, X x_at) {
     const int64_t c = s / C;
     const int64_t base = static_cast<int64_t>(chunk_ptr[c]) + (s - c * C);
     const int len = chunk_len[c];
@@ -186,20 +190,51 @@ __device__ __forceinline__ W apply_slot(int64_t s, int64_t C,
         }
         W xv[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) xv[u] = x[cc[u]];
+        for (int u = 0; u < U; ++u) xv[u] = x_at(cc[u]);
 #pragma unroll
         for (int u = 0; u < U; ++u)
             acc = fma_w(static_cast<W>(widen_t<V>::f(vv[u])), xv[u], acc);
     }
-    for (; j < len; ++j) {
-        int64_t cj;
-        if constexpr (MODE == kTab8)
-            cj = tab_col(ld_stream(iw + (j >> 2) * kWave), j);
-        else
-            cj = col_at(base + j * C);
-        acc = fma_w(static_cast<W>(widen_t<V>::f(val[base + j * C])), x[cj], acc);
+    if constexpr (REST) {
+        if (j < len) {
+            V vv[U];
+            uint32_t w[U / 4];
+            int64_t cc[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (j + u < len) vv[u] = ld_stream(val + base + (j + u) * C);
+            if constexpr (MODE == kTab8) {
+#pragma unroll
+                for (int g = 0; g < U / 4; ++g)
+                    if (j + 4 * g < len) w[g] = ld_stream(iw + ((j >> 2) + g) * kWave);
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (j + u < len) cc[u] = tab_col(w[u >> 2], u);
+            } else {
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (j + u < len) cc[u] = col_at(base + (j + u) * C);
+            }
+            W xv[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (j + u < len) xv[u] = x_at(cc[u]);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (j + u < len)
+                    acc = fma_w(static_cast<W>(widen_t<V>::f(vv[u])), xv[u], acc);
+        }
+    } else {
+        for (; j < len; ++j) {
+            int64_t cj;
+            if constexpr (MODE == kTab8)
+                cj = tab_col(ld_stream(iw + (j >> 2) * kWave), j);
+            else
+                cj = col_at(base + j * C);
+            acc = fma_w(static_cast<W>(widen_t<V>::f(val[base + j * C])), x_at(cj), acc);
+        }
     }
-    if (DIAG) acc = fma_w(static_cast<W>(diag[s]), x[s], acc);
+    if (DIAG) acc = fma_w(static_cast<W>(diag[s]), x_at(s), acc);
     return acc;
 }
 
@@ -217,8 +252,9 @@ __global__ __launch_bounds__(kCgThreads) void k_spmv_dot(
     const int64_t s = static_cast<int64_t>(blockIdx.x) * kCgThreads + threadIdx.x;
     W prod = 0;
     if (s < n) {
-        const W v = apply_slot<V, W, DIAG, MODE>(s, C, chunk_ptr, chunk_len, col, rel, idx,
-                                                 idx_row, tab, val, diag, p);
+        const W v = apply_slot<V, W, DIAG, MODE, false>(
+            s, C, chunk_ptr, chunk_len, col, rel, idx, idx_row, tab, val, diag,
+            [&](int64_t c) { return p[c]; });
         q[s] = v;
         prod = p[s] * v;
     }
@@ -239,8 +275,9 @@ __global__ __launch_bounds__(kCgThreads) void k_residual(
     const int64_t s = static_cast<int64_t>(blockIdx.x) * kCgThreads + threadIdx.x;
     double sq = 0;
     if (s < n) {
-        const double ax = apply_slot<double, double, false, MODE>(
-            s, C, chunk_ptr, chunk_len, col, rel, idx, idx_row, tab, val, nullptr, x);
+        const double ax = apply_slot<double, double, false, MODE, false>(
+            s, C, chunk_ptr, chunk_len, col, rel, idx, idx_row, tab, val, nullptr,
+            [&](int64_t c) { return x[c]; });
         const double v = b[s] - ax;
         r[s] = v;
         sq = v * v;
@@ -313,6 +350,114 @@ __global__ __launch_bounds__(kCgThreads) void k_update_p(
     for (int64_t i = static_cast<int64_t>(blockIdx.x) * kCgThreads + threadIdx.x;
          i < n; i += static_cast<int64_t>(gridDim.x) * kCgThreads)
         p[i] = fma_w(beta, p[i], r[i]);
+}
+
+// Two launches an iteration for systems of at most kFewPartials x 256 slots.
+// Their iterations are launches and dependent memory round trips, not bytes:
+// with five launches (product, two reductions, two updates) 9,216 slots took
+// 19 us an iteration whatever the products cost.  Here every workgroup adds
+// the partial sums itself, in the order of k_reduce, and the update of p runs
+// inside the product: p_new[c] = r[c] + beta p_old[c] is formed where it is
+// gathered (the same fma, so the iterates are those of the five launches bit
+// for bit) and each slot's own one is written to the other buffer.  Larger
+// systems keep the five: the second gather costs them more than a launch.
+constexpr int64_t kFewPartials = 1024;
+
+// Sum of partial[0..m), m <= kFewPartials, in every thread of a 256-thread
+// workgroup, in k_reduce's order (a butterfly per 64, then those in turn).
+template <typename W>
+__device__ __forceinline__ W reduce_few(const W *__restrict__ partial, int64_t m) {
+    __shared__ W ws[kFewPartials / kWave];
+    constexpr int kWaves = kCgThreads / kWave;
+    const int wave = threadIdx.x / kWave;
+    const int groups = static_cast<int>((m + kWave - 1) / kWave);
+    for (int g = wave; g < groups; g += kWaves) {
+        const int64_t i = g * kWave + (threadIdx.x & (kWave - 1));
+        W v = i < m ? partial[i] : W(0);
+#pragma unroll
+        for (int off = kWave / 2; off >= 1; off >>= 1) v += __shfl_xor(v, off, kWave);
+        if ((threadIdx.x & (kWave - 1)) == 0) ws[g] = v;
+    }
+    __syncthreads();
+    W t = ws[0];
+    for (int g = 1; g < groups; ++g) t += ws[g];
+    __syncthreads();
+    return t;
+}
+
+// FIRST: q = A p, partial_pq = sum p.q.  Otherwise the last update's r.r is
+// added up first (the loop ends here when it is <= stop2), and
+// p_new = r + beta p_old takes the place of p.
+template <typename V, typename W, bool DIAG, int MODE, bool FIRST>
+__global__ __launch_bounds__(kCgThreads) void k_few_product(
+    int64_t n, int64_t C, const int32_t *__restrict__ chunk_ptr,
+    const int32_t *__restrict__ chunk_len, const int32_t *__restrict__ col,
+    const int16_t *__restrict__ rel, const uint32_t *__restrict__ idx,
+    const int64_t *__restrict__ idx_row, const int16_t *__restrict__ tab,
+    const V *__restrict__ val, const float *__restrict__ diag, const W *__restrict__ r,
+    const W *__restrict__ p, W *__restrict__ p_new, W *__restrict__ q,
+    const W *__restrict__ partial_rr, W *__restrict__ partial_pq, W *__restrict__ scal, int rr_new,
+    int rr_old, int64_t *__restrict__ ctl, W stop2) {
+    if (ctl[CTL_DONE]) return;
+    W beta = 0;
+    if constexpr (!FIRST) {
+        const W rr = reduce_few(partial_rr, static_cast<int64_t>(gridDim.x));
+        const bool done = !(rr > stop2);
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            scal[rr_new] = rr;
+            if (done) ctl[CTL_DONE] = 1;
+        }
+        if (done) return;  // the same in every workgroup
+        beta = rr / scal[rr_old];
+    }
+    const int64_t s = static_cast<int64_t>(blockIdx.x) * kCgThreads + threadIdx.x;
+    const auto p_at = [&](int64_t c) {
+        if constexpr (FIRST) return p[c];
+        else return fma_w(beta, p[c], r[c]);
+    };
+    W prod = 0;
+    if (s < n) {
+        const W v = apply_slot<V, W, DIAG, MODE, true>(s, C, chunk_ptr, chunk_len, col, rel, idx,
+                                                       idx_row, tab, val, diag, p_at);
+        const W mine = p_at(s);
+        if constexpr (!FIRST) p_new[s] = mine;
+        q[s] = v;
+        prod = mine * v;
+    }
+    const W t = block_sum(prod);
+    if (threadIdx.x == 0) partial_pq[blockIdx.x] = t;
+}
+
+// alpha = r.r / p.q (breakdown as in k_reduce_pq); x += alpha p,
+// r -= alpha q, partial_rr = sum r.r
+template <typename W>
+__global__ __launch_bounds__(kCgThreads) void k_few_update(
+    int64_t n, const W *__restrict__ scal, int rr, const W *__restrict__ partial_pq,
+    W *__restrict__ x, W *__restrict__ r, const W *__restrict__ p, const W *__restrict__ q,
+    W *__restrict__ partial_rr, int64_t *__restrict__ ctl) {
+    if (ctl[CTL_DONE]) return;
+    const W pq = reduce_few(partial_pq, static_cast<int64_t>(gridDim.x));
+    const bool bad = !(pq > W(0));
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (bad) {
+            ctl[CTL_DONE] = 1;
+            ctl[CTL_BREAK] = 1;
+        } else {
+            ctl[CTL_ITERS] += 1;
+        }
+    }
+    if (bad) return;  // the same in every workgroup
+    const W alpha = scal[rr] / pq;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kCgThreads + threadIdx.x;
+    W sq = 0;
+    if (i < n) {
+        x[i] = fma_w(alpha, p[i], x[i]);
+        const W v = fma_w(-alpha, q[i], r[i]);
+        r[i] = v;
+        sq = fma_w(v, v, sq);
+    }
+    const W t = block_sum(sq);
+    if (threadIdx.x == 0) partial_rr[blockIdx.x] = t;
 }
 
 // p = r, partial = sum r.r
@@ -628,54 +773,129 @@ static dim3 upd_grid(int64_t n) {
     return dim3(static_cast<unsigned>(g < kUpdBlocks ? (g > 0 ? g : 1) : kUpdBlocks));
 }
 
+// What one CG loop works on: the operator with values of type V, vectors of
+// type W (p2: the other buffer of p), partial sums, and the device words: ctl
+// (4 int64) followed by scal (8 W), read back together.
+template <typename V, typename W>
+struct Loop {
+    const Mat &A;
+    const V *val;
+    const float *diag;
+    W *x, *r, *p, *p2, *q, *partial;
+    int64_t *ctl;
+    W *scal() const { return reinterpret_cast<W *>(ctl + 4); }
+    bool few() const { return A.n <= kFewPartials * kCgThreads; }
+};
+constexpr int kLoopWords = 4 + 8;  // int64 words of ctl and scal
+
+// Enqueues nb iterations; scal[par] holds the current r.r.  The device stops
+// by itself once r.r <= stop2.
+template <bool DIAG, typename V, typename W>
+static int enqueue_iterations(smax_hip_ctx ctx, const Loop<V, W> &L, int par, int64_t nb,
+                              W stop2) {
+    const Mat &A = L.A;
+    const int64_t n = A.n;
+    const dim3 sg = grid_for(n, kCgThreads), ug = upd_grid(n);
+    W *scal = L.scal();
+    if (!L.few()) {
+        for (int64_t b = 0, pp = par; b < nb; ++b, pp = 1 - pp) {
+            const int cur = static_cast<int>(pp), nxt = 1 - cur;
+            launch_spmv_dot<V, W, DIAG>(ctx, sg, A, L.val, L.diag, L.p, L.q, L.partial, L.ctl);
+            hipLaunchKernelGGL((k_reduce_pq<W>), dim3(1), dim3(kReduceThreads), 0,
+                               ctx->stream, L.partial, static_cast<int64_t>(sg.x),
+                               scal + 2, L.ctl);
+            hipLaunchKernelGGL((k_update_xr<W>), ug, dim3(kCgThreads), 0, ctx->stream,
+                               n, scal, cur, 2, L.x, L.r, L.p, L.q, L.partial, L.ctl);
+            hipLaunchKernelGGL((k_reduce<W>), dim3(1), dim3(kReduceThreads), 0,
+                               ctx->stream, L.partial, static_cast<int64_t>(ug.x),
+                               scal + nxt, L.ctl, stop2);
+            hipLaunchKernelGGL((k_update_p<W>), ug, dim3(kCgThreads), 0, ctx->stream,
+                               n, scal, nxt, cur, L.r, L.p, L.ctl);
+        }
+        SMAX_HIP_LAUNCHED(ctx, "cg iteration");
+        return SMAX_HIP_SUCCESS;
+    }
+    // two launches an iteration; the partial sums of p.q and r.r lie apart
+    W *ppq = L.partial, *prr = L.partial + sg.x;
+    W *p = L.p, *p2 = L.p2;
+    int cur = par;
+    for (int64_t b = 0; b < nb; ++b) {
+#define SMAX_CG_FEW(MODE, FIRST)                                                             \
+    hipLaunchKernelGGL((k_few_product<V, W, DIAG, MODE, FIRST>), sg, dim3(kCgThreads), 0,    \
+                       ctx->stream, n, A.C, A.chunk_ptr, A.chunk_len, A.col, A.rel, A.idx,    \
+                       A.idx_row, A.tab, L.val, L.diag, L.r, p, p2, L.q, prr, ppq, scal,      \
+                       1 - cur, cur, L.ctl, stop2)
+        if (b == 0) {
+            switch (A.mode()) {
+            case kTab8: SMAX_CG_FEW(kTab8, true); break;
+            case kRel16: SMAX_CG_FEW(kRel16, true); break;
+            default: SMAX_CG_FEW(kCol32, true); break;
+            }
+        } else {
+            switch (A.mode()) {
+            case kTab8: SMAX_CG_FEW(kTab8, false); break;
+            case kRel16: SMAX_CG_FEW(kRel16, false); break;
+            default: SMAX_CG_FEW(kCol32, false); break;
+            }
+            std::swap(p, p2);
+            cur = 1 - cur;
+        }
+#undef SMAX_CG_FEW
+        hipLaunchKernelGGL((k_few_update<W>), sg, dim3(kCgThreads), 0, ctx->stream, n, scal, cur,
+                           ppq, L.x, L.r, p, L.q, prr, L.ctl);
+    }
+    // the last iteration's r.r and p, as after five launches
+    hipLaunchKernelGGL((k_reduce<W>), dim3(1), dim3(kReduceThreads), 0, ctx->stream, prr,
+                       static_cast<int64_t>(sg.x), scal + (1 - cur), L.ctl, stop2);
+    hipLaunchKernelGGL((k_update_p<W>), ug, dim3(kCgThreads), 0, ctx->stream, n, scal, 1 - cur,
+                       cur, L.r, p, L.ctl);
+    SMAX_HIP_LAUNCHED(ctx, "cg iteration");
+    return SMAX_HIP_SUCCESS;
+}
+
+// Waits for the enqueued iterations: ctl[0..3) to h, the newest r.r (at the
+// parity of the iterations done) to *rr, and p names the buffer that holds the
+// direction (before: iterations done when they were enqueued).
+template <typename V, typename W>
+static int finish_iterations(smax_hip_ctx ctx, Loop<V, W> &L, int64_t before, int64_t h[3],
+                             W *rr) {
+    int64_t words[kLoopWords];
+    const int rc = read_words(ctx, L.ctl, words, kLoopWords);
+    if (rc) return rc;
+    for (int i = 0; i < 3; ++i) h[i] = words[i];
+    *rr = reinterpret_cast<const W *>(words + 4)[h[CTL_ITERS] & 1];
+    const int64_t k = h[CTL_ITERS] - before;
+    if (L.few() && k > 0 && ((k - 1) & 1)) std::swap(L.p, L.p2);
+    return SMAX_HIP_SUCCESS;
+}
+
 // CG iterations from the current (x, r, p) with r.r in scal[0].  Stops once
 // sqrt(r.r) <= stop or after max_it iterations; the host looks at the device
 // every `batch` iterations.  Returns the iterations run and the final r.r.
-template <typename V, typename W, bool DIAG>
-static int cg_loop(smax_hip_ctx ctx, const Mat &A, const V *val, const float *diag,
-                   W *x, W *r, W *p, W *q, W *partial, W *scal, int64_t *ctl,
-                   double stop, int64_t max_it, int64_t batch, int64_t *iters,
-                   double *rr_out) {
-    const int64_t n = A.n;
-    const dim3 sg = grid_for(n, kCgThreads), ug = upd_grid(n);
+template <bool DIAG, typename V, typename W>
+static int cg_loop(smax_hip_ctx ctx, Loop<V, W> &L, double stop, int64_t max_it, int64_t batch,
+                   int64_t *iters, double *rr_out) {
     const W stop2 = static_cast<W>(stop * stop);
-    hipLaunchKernelGGL(k_zero_ctl, dim3(1), dim3(64), 0, ctx->stream, ctl);
-    int64_t h[2] = {0, 0};
+    W *scal = L.scal();
+    hipLaunchKernelGGL(k_zero_ctl, dim3(1), dim3(64), 0, ctx->stream, L.ctl);
+    int64_t h[3] = {0, 0, 0};
     W rr = 0;
     int rc = read_words(ctx, scal, &rr, 1);
     if (rc) return rc;
     int64_t done_it = 0;
     bool done = !(static_cast<double>(rr) > stop * stop);
-    int par = 0;  // scal[par] holds the current r.r
     while (!done && done_it < max_it) {
         const int64_t nb = std::min<int64_t>(batch, max_it - done_it);
-        for (int64_t b = 0, pp = par; b < nb; ++b, pp = 1 - pp) {
-            const int cur = static_cast<int>(pp), nxt = 1 - cur;
-            launch_spmv_dot<V, W, DIAG>(ctx, sg, A, val, diag, p, q, partial, ctl);
-            hipLaunchKernelGGL((k_reduce_pq<W>), dim3(1), dim3(kReduceThreads), 0,
-                               ctx->stream, partial, static_cast<int64_t>(sg.x),
-                               scal + 2, ctl);
-            hipLaunchKernelGGL((k_update_xr<W>), ug, dim3(kCgThreads), 0, ctx->stream,
-                               n, scal, cur, 2, x, r, p, q, partial, ctl);
-            hipLaunchKernelGGL((k_reduce<W>), dim3(1), dim3(kReduceThreads), 0,
-                               ctx->stream, partial, static_cast<int64_t>(ug.x),
-                               scal + nxt, ctl, stop2);
-            hipLaunchKernelGGL((k_update_p<W>), ug, dim3(kCgThreads), 0, ctx->stream,
-                               n, scal, nxt, cur, r, p, ctl);
-        }
-        SMAX_HIP_LAUNCHED(ctx, "cg iteration");
-        rc = read_words(ctx, ctl, h, 2);
+        rc = enqueue_iterations<DIAG>(ctx, L, static_cast<int>(done_it & 1), nb, stop2);
+        if (!rc) rc = finish_iterations(ctx, L, done_it, h, &rr);
         if (rc) return rc;
         done_it = h[CTL_ITERS];
-        par = static_cast<int>(done_it & 1);
-        rc = read_words(ctx, scal + par, &rr, 1);
-        if (rc) return rc;
         done = h[CTL_DONE] != 0 || !(rr == rr);
     }
     *iters = done_it;
     *rr_out = static_cast<double>(rr);
     // leave the current r.r in scal[0] for the caller
-    if (par == 1)
+    if (done_it & 1)
         SMAX_HIP_CALL(ctx, hipMemcpyAsync(scal, scal + 1, sizeof(W),
                                           hipMemcpyDeviceToDevice, ctx->stream));
     return SMAX_HIP_SUCCESS;
@@ -872,17 +1092,18 @@ static int prepare(smax_hip_ctx ctx, smax_hip_scs A, int lo_type, bool want_diag
 // FP64 residual is undone (x restored from `xbak`) and restarts the
 // iteration; after two such steps in a row `*gave_up` hands the rest of the
 // solve to restarted (defect-correction) refinement.
-template <typename V, bool DIAG>
-static int reliable_cg(smax_hip_ctx ctx, const Mat &M, const double *val64,
-                       const V *val, const float *diag, const double *bs,
+template <bool DIAG, typename V>
+static int reliable_cg(smax_hip_ctx ctx, Loop<V, float> &L, const double *val64, const double *bs,
                        double *xs, double *xbak, double *r64, double *partial64,
-                       double *scal64, float *xl, float *r, float *p, float *q,
-                       float *partial32, float *scal32, int64_t *ctl, double bnorm,
-                       const smax_hip_cg_params *prm, int64_t batch, int64_t max_inner,
-                       int64_t *iters, int64_t *steps, double *rr_out,
-                       bool *gave_up) {
+                       double *scal64, double bnorm, const smax_hip_cg_params *prm,
+                       int64_t batch, int64_t max_inner, int64_t *iters, int64_t *steps,
+                       double *rr_out, bool *gave_up) {
+    const Mat &M = L.A;
     const int64_t n = M.n;
-    const dim3 sg = grid_for(n, kCgThreads), ug = upd_grid(n);
+    const dim3 ug = upd_grid(n);
+    float *const xl = L.x, *const r = L.r, *const partial32 = L.partial;
+    float *const scal32 = L.scal();
+    int64_t *const ctl = L.ctl;
     const double target = prm->rel_tol * bnorm;
     const double delta = prm->inner_rel_tol;
     double rr64 = 0;
@@ -891,7 +1112,7 @@ static int reliable_cg(smax_hip_ctx ctx, const Mat &M, const double *val64,
     *rr_out = rr64;
     if (bnorm == 0 || std::sqrt(rr64) <= target) return SMAX_HIP_SUCCESS;
     hipLaunchKernelGGL(k_start_reliable, ug, dim3(kCgThreads), 0, ctx->stream, n, r64,
-                       r, p, xl, partial32);
+                       r, L.p, xl, partial32);
     hipLaunchKernelGGL((k_reduce<float>), dim3(1), dim3(kReduceThreads), 0, ctx->stream,
                        partial32, static_cast<int64_t>(ug.x), scal32 + 0, nullptr, -1.0f);
     hipLaunchKernelGGL(k_zero_ctl, dim3(1), dim3(64), 0, ctx->stream, ctl);
@@ -906,24 +1127,9 @@ static int reliable_cg(smax_hip_ctx ctx, const Mat &M, const double *val64,
         bool stopped = false;
         while (!stopped && done_it < cycle_end) {
             const int64_t nb = std::min<int64_t>(batch, cycle_end - done_it);
-            for (int64_t b = 0, pp = done_it & 1; b < nb; ++b, pp = 1 - pp) {
-                const int cur = static_cast<int>(pp), nxt = 1 - cur;
-                launch_spmv_dot<V, float, DIAG>(ctx, sg, M, val, diag, p, q, partial32,
-                                                ctl);
-                hipLaunchKernelGGL((k_reduce_pq<float>), dim3(1), dim3(kReduceThreads), 0,
-                                   ctx->stream, partial32, static_cast<int64_t>(sg.x),
-                                   scal32 + 2, ctl);
-                hipLaunchKernelGGL((k_update_xr<float>), ug, dim3(kCgThreads), 0,
-                                   ctx->stream, n, scal32, cur, 2, xl, r, p, q,
-                                   partial32, ctl);
-                hipLaunchKernelGGL((k_reduce<float>), dim3(1), dim3(kReduceThreads), 0,
-                                   ctx->stream, partial32, static_cast<int64_t>(ug.x),
-                                   scal32 + nxt, ctl, trig2);
-                hipLaunchKernelGGL((k_update_p<float>), ug, dim3(kCgThreads), 0,
-                                   ctx->stream, n, scal32, nxt, cur, r, p, ctl);
-            }
-            SMAX_HIP_LAUNCHED(ctx, "reliable iteration");
-            rc = read_words(ctx, ctl, h, 3);
+            float rr32 = 0;
+            rc = enqueue_iterations<DIAG>(ctx, L, static_cast<int>(done_it & 1), nb, trig2);
+            if (!rc) rc = finish_iterations(ctx, L, done_it, h, &rr32);
             if (rc) return rc;
             done_it = h[CTL_ITERS];
             stopped = h[CTL_DONE] != 0;
@@ -968,14 +1174,14 @@ static int reliable_cg(smax_hip_ctx ctx, const Mat &M, const double *val64,
                                n, r64, r, partial32);
         else
             hipLaunchKernelGGL(k_start_reliable, ug, dim3(kCgThreads), 0, ctx->stream,
-                               n, r64, r, p, xl, partial32);
+                               n, r64, r, L.p, xl, partial32);
         hipLaunchKernelGGL((k_reduce<float>), dim3(1), dim3(kReduceThreads), 0, ctx->stream,
                            partial32, static_cast<int64_t>(ug.x), scal32 + par, nullptr,
                            -1.0f);
         hipLaunchKernelGGL(k_clear_done, dim3(1), dim3(64), 0, ctx->stream, ctl);
         if (keep_p)
             hipLaunchKernelGGL((k_update_p<float>), ug, dim3(kCgThreads), 0, ctx->stream,
-                               n, scal32, par, 1 - par, r, p, ctl);
+                               n, scal32, par, 1 - par, r, L.p, ctl);
         SMAX_HIP_LAUNCHED(ctx, "refinement step");
     }
     *iters = done_it;
@@ -1036,12 +1242,15 @@ int smax_hip_cg_f64(smax_hip_ctx ctx, smax_hip_scs A, const double *b,
     const double *val = static_cast<const double *>(in.val);
     const int64_t n = M.n, batch = prm->check_every > 0 ? prm->check_every : 25;
     Work w(ctx);
-    double *bs, *xs, *r, *p, *q, *partial, *scal;
+    double *bs, *xs, *r, *p, *p2 = nullptr, *q, *partial;
     int64_t *ctl;
     rc = w.get(&bs, n) | w.get(&xs, n) | w.get(&r, n) | w.get(&p, n) |
          w.get(&q, n) | w.get(&partial, ceil_div(n, kCgThreads) + kUpdBlocks) |
-         w.get(&scal, 8) | w.get(&ctl, 4);
+         w.get(&ctl, kLoopWords);
+    if (n <= kFewPartials * kCgThreads) rc |= w.get(&p2, n);
     if (rc) return SMAX_HIP_ERROR_OUT_OF_MEMORY;
+    Loop<double, double> L{M, val, nullptr, xs, r, p, p2, q, partial, ctl};
+    double *const scal = L.scal();
     const auto t0 = std::chrono::steady_clock::now();
     hipLaunchKernelGGL(k_to_slots, grid_for(n, 256), dim3(256), 0, ctx->stream, n,
                        in.n_rows, in.slot_row, b, bs);
@@ -1058,12 +1267,10 @@ int smax_hip_cg_f64(smax_hip_ctx ctx, smax_hip_scs A, const double *b,
         if (rc) return rc;
         if (bnorm == 0 || std::sqrt(rr) <= stop || total >= prm->max_iters) break;
         hipLaunchKernelGGL((k_copy_dot<double>), upd_grid(n), dim3(kCgThreads), 0,
-                           ctx->stream, n, r, p, partial);
+                           ctx->stream, n, r, L.p, partial);
         int64_t it = 0;
         double rr_rec = 0;
-        rc = cg_loop<double, double, false>(ctx, M, val, nullptr, xs, r, p, q, partial,
-                                            scal, ctl, stop, prm->max_iters - total,
-                                            batch, &it, &rr_rec);
+        rc = cg_loop<false>(ctx, L, stop, prm->max_iters - total, batch, &it, &rr_rec);
         if (rc) return rc;
         total += it;
     }
@@ -1106,14 +1313,18 @@ int smax_hip_ircg(smax_hip_ctx ctx, smax_hip_scs A, const double *b, double *x,
     const int64_t max_inner = prm->max_inner > 0 ? prm->max_inner : prm->max_iters;
     Work w(ctx);
     double *bs, *xs, *xbak, *r64, *partial64, *scal64;
-    float *d, *r, *p, *q, *partial32, *scal32;
+    float *d, *r, *p, *p2 = nullptr, *q, *partial32;
     int64_t *ctl;
     const int64_t np = ceil_div(n, kCgThreads) + kUpdBlocks;
     rc = w.get(&bs, n) | w.get(&xs, n) | w.get(&xbak, n) | w.get(&r64, n) |
          w.get(&partial64, np) |
          w.get(&scal64, 8) | w.get(&d, n) | w.get(&r, n) | w.get(&p, n) |
-         w.get(&q, n) | w.get(&partial32, np) | w.get(&scal32, 8) | w.get(&ctl, 4);
+         w.get(&q, n) | w.get(&partial32, np) | w.get(&ctl, kLoopWords);
+    if (n <= kFewPartials * kCgThreads) rc |= w.get(&p2, n);
     if (rc) return SMAX_HIP_ERROR_OUT_OF_MEMORY;
+    Loop<float, float> Lf{M, A->val_f32, nullptr, d, r, p, p2, q, partial32, ctl};
+    Loop<uint16_t, float> Lb{M, A->val_bf16, A->diag_f32, d, r, p, p2, q, partial32, ctl};
+    float *const scal32 = Lf.scal();
     const auto t0 = std::chrono::steady_clock::now();
     hipLaunchKernelGGL(k_to_slots, grid_for(n, 256), dim3(256), 0, ctx->stream, n,
                        in.n_rows, in.slot_row, b, bs);
@@ -1126,22 +1337,14 @@ int smax_hip_ircg(smax_hip_ctx ctx, smax_hip_scs A, const double *b, double *x,
     int64_t total = 0, outer = 0;
     bool fallback = false;
     if (!prm->restart_inner) {
-        if (lo == SMAX_HIP_F32)
-            rc = reliable_cg<float, false>(ctx, M, val, A->val_f32, nullptr, bs, xs, xbak,
-                                           r64, partial64, scal64, d, r, p, q, partial32,
-                                           scal32, ctl, bnorm, prm, batch, max_inner,
-                                           &total, &outer, &rr, &fallback);
-        else if (diag)
-            rc = reliable_cg<uint16_t, true>(ctx, M, val, A->val_bf16, A->diag_f32, bs,
-                                             xs, xbak, r64, partial64, scal64, d, r, p,
-                                             q, partial32, scal32, ctl, bnorm, prm,
-                                             batch, max_inner, &total, &outer, &rr,
-                                             &fallback);
-        else
-            rc = reliable_cg<uint16_t, false>(ctx, M, val, A->val_bf16, nullptr, bs, xs,
-                                              xbak, r64, partial64, scal64, d, r, p, q,
-                                              partial32, scal32, ctl, bnorm, prm, batch,
-                                              max_inner, &total, &outer, &rr, &fallback);
+        const auto solve = [&](auto &L, auto with_diag) {
+            return reliable_cg<decltype(with_diag)::value>(
+                ctx, L, val, bs, xs, xbak, r64, partial64, scal64, bnorm, prm, batch, max_inner,
+                &total, &outer, &rr, &fallback);
+        };
+        if (lo == SMAX_HIP_F32) rc = solve(Lf, std::false_type{});
+        else if (diag) rc = solve(Lb, std::true_type{});
+        else rc = solve(Lb, std::false_type{});
         if (rc) return rc;
     } else {
         rc = residual(ctx, M, val, bs, xs, r64, partial64, scal64, 0, &rr);
@@ -1156,7 +1359,8 @@ int smax_hip_ircg(smax_hip_ctx ctx, smax_hip_scs A, const double *b, double *x,
         if (rel <= prm->rel_tol || total >= prm->max_iters) break;
         ++outer;
         hipLaunchKernelGGL(k_start_inner, upd_grid(n), dim3(kCgThreads), 0,
-                           ctx->stream, n, scal64, 0, r64, r, p, d, partial32);
+                           ctx->stream, n, scal64, 0, r64, r,
+                           lo == SMAX_HIP_F32 ? Lf.p : Lb.p, d, partial32);
         hipLaunchKernelGGL((k_reduce<float>), dim3(1), dim3(kReduceThreads), 0, ctx->stream,
                            partial32, static_cast<int64_t>(upd_grid(n).x), scal32 + 0,
                            nullptr, -1.0f);
@@ -1168,17 +1372,11 @@ int smax_hip_ircg(smax_hip_ctx ctx, smax_hip_scs A, const double *b, double *x,
         double rr_in = 0;
         const int64_t cap = std::min<int64_t>(max_inner, prm->max_iters - total);
         if (lo == SMAX_HIP_F32)
-            rc = cg_loop<float, float, false>(ctx, M, A->val_f32, nullptr, d, r, p, q,
-                                              partial32, scal32, ctl, inner_tol, cap,
-                                              batch, &it, &rr_in);
+            rc = cg_loop<false>(ctx, Lf, inner_tol, cap, batch, &it, &rr_in);
         else if (diag)
-            rc = cg_loop<uint16_t, float, true>(ctx, M, A->val_bf16, A->diag_f32, d, r,
-                                                p, q, partial32, scal32, ctl, inner_tol,
-                                                cap, batch, &it, &rr_in);
+            rc = cg_loop<true>(ctx, Lb, inner_tol, cap, batch, &it, &rr_in);
         else
-            rc = cg_loop<uint16_t, float, false>(ctx, M, A->val_bf16, nullptr, d, r, p,
-                                                 q, partial32, scal32, ctl, inner_tol,
-                                                 cap, batch, &it, &rr_in);
+            rc = cg_loop<false>(ctx, Lb, inner_tol, cap, batch, &it, &rr_in);
         if (rc) return rc;
         total += it;
         SMAX_HIP_CALL(ctx, hipMemcpyAsync(xbak, xs, sizeof(double) * n,

@@ -19,7 +19,7 @@ struct smax_hip_ctx_s {
     hipEvent_t ev_start = nullptr;
     hipEvent_t ev_stop = nullptr;
     std::string last_error;
-    // Small pinned host word used to read back device counters.
+    // kHostWords pinned words used to read back device counters.
     int64_t *host_word = nullptr;
     // Device workspace of entry points that stage operands (column-major
     // CRS SpMM), grown on demand.  A buffer that is outgrown is retired, not
@@ -57,6 +57,7 @@ int ctx_workspace(smax_hip_ctx ctx, size_t bytes, void **out);
 int read_i64(smax_hip_ctx ctx, const int64_t *dptr, int64_t *out);
 
 constexpr int kWave = 64;
+constexpr int kHostWords = 16;
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 

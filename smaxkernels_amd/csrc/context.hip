@@ -404,7 +404,7 @@ int smax_hip_ctx_create(int device, smax_hip_ctx *out) {
     if (e == hipSuccess) e = hipEventCreate(&ctx->ev_stop);
     if (e == hipSuccess)
         e = hipHostMalloc(reinterpret_cast<void **>(&ctx->host_word),
-                          sizeof(int64_t) * 8, hipHostMallocDefault);
+                          sizeof(int64_t) * kHostWords, hipHostMallocDefault);
     if (e != hipSuccess) {
         int st = hip_fail(nullptr, e, "smax_hip_ctx_create");
         smax_hip_ctx_destroy(ctx);
