@@ -133,12 +133,93 @@ __device__ __forceinline__ float fma_w(float a, float b, float c) {
 enum { kCol32 = 0, kRel16 = 1, kTab8 = 2 };
 constexpr int kColTable = 32;
 
+// The vector a product gathers from: a plain one, or (k_few_product) p formed
+// where it is gathered, r + beta p.  at_byte takes a byte offset.
+template <typename W>
+struct Plain {
+    const W *__restrict__ x;
+    __device__ __forceinline__ W at(int64_t c) const { return x[c]; }
+    __device__ __forceinline__ W at_byte(uint32_t o) const {
+        return *reinterpret_cast<const W *>(reinterpret_cast<const char *>(x) + o);
+    }
+};
+template <typename W>
+struct Updated {
+    const W *__restrict__ r, *__restrict__ p;
+    W beta;
+    __device__ __forceinline__ W at(int64_t c) const { return fma_w(beta, p[c], r[c]); }
+    __device__ __forceinline__ W at_byte(uint32_t o) const {
+        return fma_w(beta, Plain<W>{p}.at_byte(o), Plain<W>{r}.at_byte(o));
+    }
+};
+
+// kTab8: the chain of slot s, one chunk per wavefront, every lane present.
+// Everything about the chunk is the same in all lanes and stays scalar; a
+// column is a 32-bit byte offset (vectors below 2 GiB, checked by
+// slot_matrix), entry (lane t: table entry t) and own (slot s) in bytes too,
+// so an element costs two operations for its shuffle address, the shuffle, an
+// add, the gather and the fma.  The next group's words and values are
+// requested before this group's gathers, and the last, shorter group is
+// loaded at once like the others: a wavefront waits about one memory round
+// trip per eight elements.
+template <typename V, typename W, typename X>
+__device__ __forceinline__ W tab_chain(int len, const uint32_t *__restrict__ iw,
+                                       const V *__restrict__ val, int lane, int entry,
+                                       uint32_t own, const X &x) {
+    constexpr int U = 8;
+    struct Group {
+        uint32_t w[U / 4];
+        V v[U];
+    };
+    const auto load = [&](int j, int m, Group &g) {  // elements [j, j + m), m <= U
+#pragma unroll
+        for (int h = 0; h < U / 4; ++h)
+            if (4 * h < m) g.w[h] = ld_stream(iw + ((j >> 2) + h) * kWave + lane);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (u < m) g.v[u] = ld_stream(val + (j + u) * kWave + lane);
+    };
+    W acc = 0;
+    const auto chain = [&](int m, const Group &g) {
+        W xv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (u < m) {
+                // 4 x the element's byte of its word: the lane to read from
+                const uint32_t w = g.w[u >> 2];
+                const uint32_t from = ((u & 3) == 0 ? w << 2 : w >> (8 * (u & 3) - 2)) & 0x7cu;
+                const int off = __builtin_amdgcn_ds_bpermute(static_cast<int>(from), entry);
+                xv[u] = x.at_byte(own + static_cast<uint32_t>(off));
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (u < m) acc = fma_w(static_cast<W>(widen_t<V>::f(g.v[u])), xv[u], acc);
+    };
+    const int full = len & ~(U - 1);
+    Group a, b;
+    if (full) {
+        load(0, U, a);
+        for (int j = U; j < full; j += U) {
+            load(j, U, b);
+            chain(U, a);
+            a = b;
+        }
+        if (full < len) load(full, len - full, b);
+        chain(U, a);
+    } else if (len > 0) {
+        load(0, len, b);
+    }
+    if (full < len) chain(len - full, b);
+    return acc;
+}
+
 // (A x)[s]: sequential fma chain over the slot's SELL elements, then (DIAG)
-// the FP32 diagonal term; x_at(c) is entry c of x.  With kTab8 every lane of
-// the wavefront must run this (one chunk per wavefront, all slots present).
-// REST: the last, shorter group of elements is loaded at once too, instead of
-// one element after the other (for the small systems, whose chains are a few
-// memory round trips long; it costs registers, which slows large ones).
+// the FP32 diagonal term.  With kTab8 every lane of the wavefront must run
+// this (one chunk per wavefront, all slots present).
+// REST (kRel16 and kCol32): the last, shorter group of elements is loaded at
+// once too, instead of one element after the other (for the small systems,
+// whose chains are a few memory round trips long; it costs registers, which
+// slows large ones).
 template <typename V, typename W, bool DIAG, int MODE, bool REST, typename X>
 __device__ __forceinline__ W apply_slot(int64_t s, int64_t C,
                                         const int32_t *__restrict__ chunk_ptr,
@@ -149,92 +230,67 @@ __device__ __forceinline__ W apply_slot(int64_t s, int64_t C,
                                         const int64_t *__restrict__ idx_row,
                                         const int16_t *__restrict__ tab,
                                         const V *__restrict__ val,
-                                        const float *__restrict__ diag, X x_at) {
-    const int64_t c = s / C;
-    const int64_t base = static_cast<int64_t>(chunk_ptr[c]) + (s - c * C);
-    const int len = chunk_len[c];
-    int entry = 0;
-    const uint32_t *iw = nullptr;  // kTab8: this slot's index words, one per row
-    if constexpr (MODE == kTab8) {
-        entry = tab[c * kColTable + (threadIdx.x & (kColTable - 1))];
-        iw = idx + idx_row[c] * kWave + (s - c * C);
-    }
-    // kTab8: the column of element j, its index byte taken from word w
-    auto tab_col = [&](uint32_t w, int j) -> int64_t {
-        return s + __shfl(entry, static_cast<int>((w >> (8 * (j & 3))) & 0xffu));
-    };
-    auto col_at = [&](int64_t o) -> int64_t {
-        if constexpr (MODE == kRel16)
-            return s + ld_stream(rel + o);
-        else
-            return ld_stream(col + o);
-    };
+                                        const float *__restrict__ diag, const X &x) {
     W acc = 0;
-    constexpr int U = 8;
-    int j = 0;
-    for (; j + U <= len; j += U) {
-        int64_t cc[U];
-        V vv[U];
+    if constexpr (MODE == kTab8) {
+        const int c = __builtin_amdgcn_readfirstlane(static_cast<int>(s / kWave));
+        const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+        constexpr int kBytes = sizeof(W);
+        const int entry = tab[c * kColTable + (lane & (kColTable - 1))] * kBytes;
+        acc = tab_chain<V, W>(chunk_len[c], idx + idx_row[c] * kWave, val + chunk_ptr[c], lane,
+                              entry, static_cast<uint32_t>(s) * kBytes, x);
+    } else {
+        const int64_t c = C == kWave ? s / kWave : s / C;
+        const int64_t base = static_cast<int64_t>(chunk_ptr[c]) + (s - c * C);
+        const int len = chunk_len[c];
+        auto col_at = [&](int64_t o) -> int64_t {
+            if constexpr (MODE == kRel16)
+                return s + ld_stream(rel + o);
+            else
+                return ld_stream(col + o);
+        };
+        constexpr int U = 8;
+        int j = 0;
+        for (; j + U <= len; j += U) {
+            int64_t cc[U];
+            V vv[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) vv[u] = ld_stream(val + base + (j + u) * C);
-        if constexpr (MODE == kTab8) {
-            // j is a multiple of 8: two whole index words
-            uint32_t w[U / 4];
-#pragma unroll
-            for (int g = 0; g < U / 4; ++g) w[g] = ld_stream(iw + ((j >> 2) + g) * kWave);
-#pragma unroll
-            for (int u = 0; u < U; ++u) cc[u] = tab_col(w[u >> 2], u);
-        } else {
+            for (int u = 0; u < U; ++u) vv[u] = ld_stream(val + base + (j + u) * C);
 #pragma unroll
             for (int u = 0; u < U; ++u) cc[u] = col_at(base + (j + u) * C);
-        }
-        W xv[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) xv[u] = x_at(cc[u]);
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            acc = fma_w(static_cast<W>(widen_t<V>::f(vv[u])), xv[u], acc);
-    }
-    if constexpr (REST) {
-        if (j < len) {
-            V vv[U];
-            uint32_t w[U / 4];
-            int64_t cc[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (j + u < len) vv[u] = ld_stream(val + base + (j + u) * C);
-            if constexpr (MODE == kTab8) {
-#pragma unroll
-                for (int g = 0; g < U / 4; ++g)
-                    if (j + 4 * g < len) w[g] = ld_stream(iw + ((j >> 2) + g) * kWave);
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                    if (j + u < len) cc[u] = tab_col(w[u >> 2], u);
-            } else {
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                    if (j + u < len) cc[u] = col_at(base + (j + u) * C);
-            }
             W xv[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (j + u < len) xv[u] = x_at(cc[u]);
+            for (int u = 0; u < U; ++u) xv[u] = x.at(cc[u]);
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                if (j + u < len)
-                    acc = fma_w(static_cast<W>(widen_t<V>::f(vv[u])), xv[u], acc);
+                acc = fma_w(static_cast<W>(widen_t<V>::f(vv[u])), xv[u], acc);
         }
-    } else {
-        for (; j < len; ++j) {
-            int64_t cj;
-            if constexpr (MODE == kTab8)
-                cj = tab_col(ld_stream(iw + (j >> 2) * kWave), j);
-            else
-                cj = col_at(base + j * C);
-            acc = fma_w(static_cast<W>(widen_t<V>::f(val[base + j * C])), x_at(cj), acc);
+        if constexpr (REST) {
+            if (j < len) {
+                V vv[U];
+                int64_t cc[U];
+                W xv[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (j + u < len) {
+                        vv[u] = ld_stream(val + base + (j + u) * C);
+                        cc[u] = col_at(base + (j + u) * C);
+                    }
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (j + u < len) xv[u] = x.at(cc[u]);
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (j + u < len)
+                        acc = fma_w(static_cast<W>(widen_t<V>::f(vv[u])), xv[u], acc);
+            }
+        } else {
+            for (; j < len; ++j)
+                acc = fma_w(static_cast<W>(widen_t<V>::f(val[base + j * C])),
+                            x.at(col_at(base + j * C)), acc);
         }
     }
-    if (DIAG) acc = fma_w(static_cast<W>(diag[s]), x_at(s), acc);
+    if (DIAG) acc = fma_w(static_cast<W>(diag[s]), x.at(s), acc);
     return acc;
 }
 
@@ -253,8 +309,7 @@ __global__ __launch_bounds__(kCgThreads) void k_spmv_dot(
     W prod = 0;
     if (s < n) {
         const W v = apply_slot<V, W, DIAG, MODE, false>(
-            s, C, chunk_ptr, chunk_len, col, rel, idx, idx_row, tab, val, diag,
-            [&](int64_t c) { return p[c]; });
+            s, C, chunk_ptr, chunk_len, col, rel, idx, idx_row, tab, val, diag, Plain<W>{p});
         q[s] = v;
         prod = p[s] * v;
     }
@@ -277,7 +332,7 @@ __global__ __launch_bounds__(kCgThreads) void k_residual(
     if (s < n) {
         const double ax = apply_slot<double, double, false, MODE, false>(
             s, C, chunk_ptr, chunk_len, col, rel, idx, idx_row, tab, val, nullptr,
-            [&](int64_t c) { return x[c]; });
+            Plain<double>{x});
         const double v = b[s] - ax;
         r[s] = v;
         sq = v * v;
@@ -411,15 +466,14 @@ __global__ __launch_bounds__(kCgThreads) void k_few_product(
         beta = rr / scal[rr_old];
     }
     const int64_t s = static_cast<int64_t>(blockIdx.x) * kCgThreads + threadIdx.x;
-    const auto p_at = [&](int64_t c) {
-        if constexpr (FIRST) return p[c];
-        else return fma_w(beta, p[c], r[c]);
-    };
+    std::conditional_t<FIRST, Plain<W>, Updated<W>> p_at;
+    if constexpr (FIRST) p_at = {p};
+    else p_at = {r, p, beta};
     W prod = 0;
     if (s < n) {
         const W v = apply_slot<V, W, DIAG, MODE, true>(s, C, chunk_ptr, chunk_len, col, rel, idx,
                                                        idx_row, tab, val, diag, p_at);
-        const W mine = p_at(s);
+        const W mine = p_at.at(s);
         if constexpr (!FIRST) p_new[s] = mine;
         q[s] = v;
         prod = mine * v;
@@ -1213,7 +1267,7 @@ static Mat slot_matrix(smax_hip_scs A, int32_t coding) {
           A->col_slot ? A->col_slot : in.col, nullptr, nullptr, nullptr, nullptr};
     if (coding != SMAX_HIP_COLUMNS_32) M.rel = A->col_rel;
     if ((coding == SMAX_HIP_COLUMNS_AUTO || coding == SMAX_HIP_COLUMNS_8) && A->col_idx &&
-        in.n_rows_padded % kWave == 0) {
+        in.n_rows_padded % kWave == 0 && in.n_rows_padded <= INT32_MAX / 8) {
         M.idx = A->col_idx;
         M.idx_row = A->col_idx_row;
         M.tab = A->col_tab;
