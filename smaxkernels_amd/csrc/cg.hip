@@ -161,8 +161,9 @@ struct Updated {
 // add, the gather and the fma.  The next group's words and values are
 // requested before this group's gathers, and the last, shorter group is
 // loaded at once like the others: a wavefront waits about one memory round
-// trip per eight elements.
-template <typename V, typename W, typename X>
+// trip per eight elements.  KEEP: the matrix may stay in the caches
+// (kKeepBytes); otherwise it is streamed past them.
+template <typename V, typename W, bool KEEP, typename X>
 __device__ __forceinline__ W tab_chain(int len, const uint32_t *__restrict__ iw,
                                        const V *__restrict__ val, int lane, int entry,
                                        uint32_t own, const X &x) {
@@ -171,13 +172,14 @@ __device__ __forceinline__ W tab_chain(int len, const uint32_t *__restrict__ iw,
         uint32_t w[U / 4];
         V v[U];
     };
+    const auto ld = [](const auto *p) { return KEEP ? *p : ld_stream(p); };
     const auto load = [&](int j, int m, Group &g) {  // elements [j, j + m), m <= U
 #pragma unroll
         for (int h = 0; h < U / 4; ++h)
-            if (4 * h < m) g.w[h] = ld_stream(iw + ((j >> 2) + h) * kWave + lane);
+            if (4 * h < m) g.w[h] = ld(iw + ((j >> 2) + h) * kWave + lane);
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (u < m) g.v[u] = ld_stream(val + (j + u) * kWave + lane);
+            if (u < m) g.v[u] = ld(val + (j + u) * kWave + lane);
     };
     W acc = 0;
     const auto chain = [&](int m, const Group &g) {
@@ -219,8 +221,8 @@ __device__ __forceinline__ W tab_chain(int len, const uint32_t *__restrict__ iw,
 // REST (kRel16 and kCol32): the last, shorter group of elements is loaded at
 // once too, instead of one element after the other (for the small systems,
 // whose chains are a few memory round trips long; it costs registers, which
-// slows large ones).
-template <typename V, typename W, bool DIAG, int MODE, bool REST, typename X>
+// slows large ones).  KEEP (kTab8): as in tab_chain.
+template <typename V, typename W, bool DIAG, int MODE, bool REST, bool KEEP, typename X>
 __device__ __forceinline__ W apply_slot(int64_t s, int64_t C,
                                         const int32_t *__restrict__ chunk_ptr,
                                         const int32_t *__restrict__ chunk_len,
@@ -237,7 +239,7 @@ __device__ __forceinline__ W apply_slot(int64_t s, int64_t C,
         const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
         constexpr int kBytes = sizeof(W);
         const int entry = tab[c * kColTable + (lane & (kColTable - 1))] * kBytes;
-        acc = tab_chain<V, W>(chunk_len[c], idx + idx_row[c] * kWave, val + chunk_ptr[c], lane,
+        acc = tab_chain<V, W, KEEP>(chunk_len[c], idx + idx_row[c] * kWave, val + chunk_ptr[c], lane,
                               entry, static_cast<uint32_t>(s) * kBytes, x);
     } else {
         const int64_t c = C == kWave ? s / kWave : s / C;
@@ -294,8 +296,17 @@ __device__ __forceinline__ W apply_slot(int64_t s, int64_t C,
     return acc;
 }
 
+// Matrices (values and one-byte columns) of up to this size are read with
+// ordinary loads and neighbouring slots on one XCD: from one product to the
+// next they then stay in the 256 MB last-level cache.  Larger ones are streamed.
+// Solves of the 27-point stencil to 1e-12, kept / streamed, by matrix size:
+// BF16 values 167 MB 22.4 / 25.7 ms, 201 MB 27.8 / 31.5, 239 MB 39.3 / 37.3;
+// FP32 186 MB 19.6 / 22.6, 229 MB 23.4 / 26.0, 279 MB 31.3 / 30.1; FP64 211 MB
+// 14.5 / 18.3, 268 MB 22.6 / 23.5, 335 MB 31.9 / 30.0.
+constexpr int64_t kKeepBytes = int64_t(230) * 1000 * 1000;
+
 // q = A p, partial[block] = sum p.q
-template <typename V, typename W, bool DIAG, int MODE>
+template <typename V, typename W, bool DIAG, int MODE, bool KEEP>
 __global__ __launch_bounds__(kCgThreads) void k_spmv_dot(
     int64_t n, int64_t C, const int32_t *__restrict__ chunk_ptr,
     const int32_t *__restrict__ chunk_len, const int32_t *__restrict__ col,
@@ -305,16 +316,17 @@ __global__ __launch_bounds__(kCgThreads) void k_spmv_dot(
     const float *__restrict__ diag, const W *__restrict__ p, W *__restrict__ q,
     W *__restrict__ partial, const int64_t *__restrict__ ctl) {
     if (ctl[CTL_DONE]) return;
-    const int64_t s = static_cast<int64_t>(blockIdx.x) * kCgThreads + threadIdx.x;
+    const int64_t block = KEEP ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+    const int64_t s = block * kCgThreads + threadIdx.x;
     W prod = 0;
     if (s < n) {
-        const W v = apply_slot<V, W, DIAG, MODE, false>(
+        const W v = apply_slot<V, W, DIAG, MODE, false, KEEP>(
             s, C, chunk_ptr, chunk_len, col, rel, idx, idx_row, tab, val, diag, Plain<W>{p});
         q[s] = v;
         prod = p[s] * v;
     }
     const W t = block_sum(prod);
-    if (threadIdx.x == 0) partial[blockIdx.x] = t;
+    if (threadIdx.x == 0) partial[block] = t;
 }
 
 // r = b - A x, partial = sum r.r  (FP64 outer residual)
@@ -330,7 +342,7 @@ __global__ __launch_bounds__(kCgThreads) void k_residual(
     const int64_t s = static_cast<int64_t>(blockIdx.x) * kCgThreads + threadIdx.x;
     double sq = 0;
     if (s < n) {
-        const double ax = apply_slot<double, double, false, MODE, false>(
+        const double ax = apply_slot<double, double, false, MODE, false, false>(
             s, C, chunk_ptr, chunk_len, col, rel, idx, idx_row, tab, val, nullptr,
             Plain<double>{x});
         const double v = b[s] - ax;
@@ -471,8 +483,8 @@ __global__ __launch_bounds__(kCgThreads) void k_few_product(
     else p_at = {r, p, beta};
     W prod = 0;
     if (s < n) {
-        const W v = apply_slot<V, W, DIAG, MODE, true>(s, C, chunk_ptr, chunk_len, col, rel, idx,
-                                                       idx_row, tab, val, diag, p_at);
+        const W v = apply_slot<V, W, DIAG, MODE, true, true>(
+            s, C, chunk_ptr, chunk_len, col, rel, idx, idx_row, tab, val, diag, p_at);
         const W mine = p_at.at(s);
         if constexpr (!FIRST) p_new[s] = mine;
         q[s] = v;
@@ -766,7 +778,7 @@ __global__ void k_split_bf16(int64_t npad, int64_t C,
 
 // ------------------------------------------------------------ host driver
 struct Mat {
-    int64_t n, C;
+    int64_t n, C, elements;
     const int32_t *chunk_ptr, *chunk_len, *col;
     const int16_t *rel;   // 16-bit column offsets from the slot, or nullptr
     const uint32_t *idx;     // kTab8 index words (with idx_row and tab), or nullptr
@@ -783,14 +795,19 @@ template <typename V, typename W, bool DIAG>
 static void launch_spmv_dot(smax_hip_ctx ctx, dim3 sg, const Mat &M, const V *val,
                             const float *diag, const W *p, W *q, W *partial,
                             const int64_t *ctl) {
-#define SMAX_CG_SPMV(MODE)                                                                   \
-    hipLaunchKernelGGL((k_spmv_dot<V, W, DIAG, MODE>), sg, dim3(kCgThreads), 0, ctx->stream, \
+#define SMAX_CG_SPMV(MODE, KEEP)                                                             \
+    hipLaunchKernelGGL((k_spmv_dot<V, W, DIAG, MODE, KEEP>), sg, dim3(kCgThreads), 0, ctx->stream, \
                        M.n, M.C, M.chunk_ptr, M.chunk_len, M.col, M.rel, M.idx, M.idx_row,     \
                        M.tab, val, diag, p, q, partial, ctl)
     switch (M.mode()) {
-    case kTab8: SMAX_CG_SPMV(kTab8); break;
-    case kRel16: SMAX_CG_SPMV(kRel16); break;
-    default: SMAX_CG_SPMV(kCol32); break;
+    case kTab8:
+        if (M.elements * static_cast<int64_t>(sizeof(V) + 1) <= kKeepBytes)
+            SMAX_CG_SPMV(kTab8, true);
+        else
+            SMAX_CG_SPMV(kTab8, false);
+        break;
+    case kRel16: SMAX_CG_SPMV(kRel16, false); break;
+    default: SMAX_CG_SPMV(kCol32, false); break;
     }
 #undef SMAX_CG_SPMV
 }
@@ -1263,7 +1280,7 @@ static int check_solver_args(smax_hip_ctx ctx, const char *fn, smax_hip_scs A,
 // it, limited by params->column_coding (SMAX_HIP_COLUMNS_*).
 static Mat slot_matrix(smax_hip_scs A, int32_t coding) {
     const smax_hip_scs_info &in = A->info;
-    Mat M{in.n_rows_padded, in.C, in.chunk_ptr, in.chunk_lengths,
+    Mat M{in.n_rows_padded, in.C, in.n_elements, in.chunk_ptr, in.chunk_lengths,
           A->col_slot ? A->col_slot : in.col, nullptr, nullptr, nullptr, nullptr};
     if (coding != SMAX_HIP_COLUMNS_32) M.rel = A->col_rel;
     if ((coding == SMAX_HIP_COLUMNS_AUTO || coding == SMAX_HIP_COLUMNS_8) && A->col_idx &&
