@@ -1,0 +1,257 @@
+// What the CRS and the SELL SpMM share beyond the tuned power-of-two kernels:
+// runs of columns of any alignment, and the long-row path.
+#pragma once
+
+#include "common.hpp"
+
+namespace smaxhip {
+
+// Q consecutive entries at p, aligned only as an entry is (one 16-byte access
+// where Q entries are 16 bytes; the hardware takes dword-aligned ones).
+template <typename A, int Q>
+struct __attribute__((packed, aligned(4))) RunOf {
+    A e[Q];
+};
+template <typename A, int Q>
+__device__ __forceinline__ void load_cols_run(const A *__restrict__ p, A (&out)[Q]) {
+    const RunOf<A, Q> v = *reinterpret_cast<const RunOf<A, Q> *>(p);
+#pragma unroll
+    for (int i = 0; i < Q; ++i) out[i] = v.e[i];
+}
+template <typename A, int Q>
+__device__ __forceinline__ void store_cols_run(A *__restrict__ p, const A (&in)[Q]) {
+    RunOf<A, Q> v;
+#pragma unroll
+    for (int i = 0; i < Q; ++i) v.e[i] = in[i];
+    *reinterpret_cast<RunOf<A, Q> *>(p) = v;
+}
+
+// k columns in runs of Q <= k: lane l of a row's ceil(k / Q) lanes owns the
+// columns from run_start(l); the last run is moved back to end at k, so it may
+// share columns with the one before (both form the same chains).
+template <int Q>
+__device__ __forceinline__ int64_t run_start(int64_t l, int64_t k) {
+    return l * Q + Q <= k ? l * Q : k - Q;
+}
+inline int64_t run_lanes(int64_t k, int64_t q) { return ceil_div(k, q); }
+
+// Long rows: at least this many entries and eight times the mean length (so
+// that they are few).  They run in long_row, a wavefront each, from
+// kLongestRow entries on a workgroup each.
+constexpr int64_t kLongRow = 128, kLongestRow = 512;
+inline int64_t long_row_from(int64_t nnz, int64_t n_rows) {
+    const int64_t eight = (8 * nnz + n_rows - 1) / n_rows;
+    return eight > kLongRow ? eight : kLongRow;
+}
+
+// Long rows in front of a launch's other rows: the first `whole` workgroups
+// take one row each, the next ceil((count - whole) / 4) take four.
+struct LongRows {
+    int64_t whole = 0, count = 0;
+    __host__ __device__ int64_t blocks() const { return whole + (count - whole + 3) / 4; }
+};
+
+// One row's outputs by NT threads, a wavefront (64) or a workgroup (256).  A
+// row is one fma chain per column whatever its length, so a lane that gathers
+// and chains by itself pays a memory round trip every eight entries: a row of
+// 2000 entries took 128 us, longer than all other rows of a matrix of 40,013
+// (16 us).  Here all lanes gather X runs, a tile of R x NT runs (at most NT
+// entries) ahead, into LDS, and the row's lanes chain them from there, about
+// 20 cycles an entry; the next tile's gathers are in flight meanwhile.  The
+// chain's order, and so Y, is unchanged.  Wavefronts for the many rows that
+// are just long: three of a workgroup's four would only wait.  CRS SpMM with a
+// plan, 1,000,000- and 200,003-row band matrices, FP32 k = 32: 0.398 -> 0.349
+// and 0.212 -> 0.082 ms; every long row a workgroup 0.401 and 0.085, R = 4
+// 0.364 and 0.085, rows from 256 entries on only 0.372 and 0.086, workgroups
+// from 1024 on 0.349 and 0.085.
+//   entry j of the row: column col[base + j * stride], value val[...] alike;
+//   xs, vs: R * NT * Q and NT entries of LDS (xs 16-byte aligned).
+constexpr int kLongRuns = 2;
+
+template <int VT, int Q, int NT>
+__device__ __forceinline__ void long_row(
+    typename vt<VT>::vec_t *xs, typename vt<VT>::vec_t *vs, int tid, int32_t len, int64_t base,
+    int64_t stride, const int32_t *__restrict__ col, const typename vt<VT>::val_t *__restrict__ val,
+    int64_t k, const typename vt<VT>::vec_t *__restrict__ X, int64_t ldx,
+    typename vt<VT>::vec_t *__restrict__ y) {
+    using T = vt<VT>;
+    using A = typename T::vec_t;
+    constexpr int R = kLongRuns;
+    const auto barrier = [] {
+        if constexpr (NT > kWave) {
+            __syncthreads();
+        } else {  // one wavefront: its LDS accesses stay in order
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    };
+    const int64_t lanes = (k + Q - 1) / Q;
+    for (int64_t l0 = 0; l0 < lanes; l0 += NT) {
+        const int g = static_cast<int>(lanes - l0 < NT ? lanes - l0 : NT);
+        const int most = NT * R / g;
+        const int ept = most < NT ? most : NT;  // entries per tile
+        int eu[R];      // this thread's entries of a tile
+        int64_t off[R]; // and the first column of its run of each
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            const int f = u * NT + tid;
+            eu[u] = f / g;
+            off[u] = run_start<Q>(l0 + f % g, k);
+            if (eu[u] >= ept) eu[u] = INT32_MAX / 2;  // none
+        }
+        int32_t c[R];
+        A xr[R][Q];
+        A vr = 0;
+        const auto load_columns = [&](int32_t t0) {
+#pragma unroll
+            for (int u = 0; u < R; ++u)
+                if (t0 + eu[u] < len) c[u] = col[base + (t0 + eu[u]) * stride];
+        };
+        const auto gather = [&](int32_t t0) {
+#pragma unroll
+            for (int u = 0; u < R; ++u)
+                if (t0 + eu[u] < len)
+                    load_cols_run<A, Q>(X + static_cast<int64_t>(c[u]) * ldx + off[u], xr[u]);
+            if (tid < ept && t0 + tid < len) vr = T::widen(val[base + (t0 + tid) * stride]);
+        };
+        load_columns(0);
+        gather(0);
+        load_columns(ept);
+        A acc[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) acc[q] = 0;
+        for (int32_t t0 = 0; t0 < len; t0 += ept) {
+#pragma unroll
+            for (int u = 0; u < R; ++u)
+                if (t0 + eu[u] < len) store_run<A, Q>(xs + (u * NT + tid) * Q, xr[u]);
+            if (tid < ept) vs[tid] = vr;
+            barrier();
+            if (t0 + ept < len) {
+                gather(t0 + ept);
+                load_columns(t0 + 2 * ept);
+            }
+            if (tid < g) {
+                const int m = len - t0 < ept ? len - t0 : ept;
+                constexpr int U = 8;
+                int e = 0;
+                for (; e + U <= m; e += U) {
+                    A w[U], b[U][Q];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        w[u] = vs[e + u];
+                        load_run<A, Q>(xs + ((e + u) * g + tid) * Q, b[u]);
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+#pragma unroll
+                        for (int q = 0; q < Q; ++q) acc[q] = T::fma_(w[u], b[u][q], acc[q]);
+                }
+                for (; e < m; ++e) {
+                    A b[Q];
+                    load_run<A, Q>(xs + (e * g + tid) * Q, b);
+                    const A w = vs[e];
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) acc[q] = T::fma_(w, b[q], acc[q]);
+                }
+            }
+            barrier();
+        }
+        if (tid < g) store_cols_run<A, Q>(y + run_start<Q>(l0 + tid, k), acc);
+    }
+}
+
+// The long rows' workgroups of a launch of 256 threads: workgroup `block` of
+// rows.blocks().  row_at(i) gives the i-th long row's (length, first entry,
+// output row).
+template <int VT, int Q, typename RowAt>
+__device__ __forceinline__ void long_rows(
+    const LongRows &rows, int64_t block, const RowAt &row_at, int64_t stride,
+    const int32_t *__restrict__ col, const typename vt<VT>::val_t *__restrict__ val, int64_t k,
+    const typename vt<VT>::vec_t *__restrict__ X, int64_t ldx,
+    typename vt<VT>::vec_t *__restrict__ Y, int64_t ldy) {
+    using A = typename vt<VT>::vec_t;
+    __shared__ __align__(16) A xs[256 * kLongRuns * Q];
+    __shared__ A vs[256];
+    const int tid = static_cast<int>(threadIdx.x);
+    if (block < rows.whole) {
+        const auto r = row_at(block);
+        long_row<VT, Q, 256>(xs, vs, tid, r.len, r.base, stride, col, val, k, X, ldx,
+                             Y + r.row * ldy);
+        return;
+    }
+    const int wave = tid / kWave;
+    const int64_t i = rows.whole + (block - rows.whole) * 4 + wave;
+    if (i >= rows.count) return;  // whole wavefronts
+    const auto r = row_at(i);
+    long_row<VT, Q, kWave>(xs + wave * kWave * kLongRuns * Q, vs + wave * kWave,
+                           tid & (kWave - 1), r.len, r.base, stride, col, val, k, X, ldx,
+                           Y + r.row * ldy);
+}
+struct LongRowAt {
+    int32_t len;
+    int64_t base, row;
+};
+
+// One lane's chains over a row in groups of eight entries, the next group's
+// columns and values requested before this group's X runs; the last, shorter
+// group is loaded at once too.  Any k >= Q.
+template <int VT, int Q>
+__device__ __forceinline__ void run_chain(
+    int64_t base, int64_t stride, int32_t len, const int32_t *__restrict__ col,
+    const typename vt<VT>::val_t *__restrict__ val,
+    const typename vt<VT>::vec_t *__restrict__ X, int64_t ldx,
+    typename vt<VT>::vec_t (&acc)[Q]) {
+    using T = vt<VT>;
+    using A = typename T::vec_t;
+    using V = typename T::val_t;
+    constexpr int U = 8;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) acc[q] = 0;
+    const int32_t full = len & ~(U - 1);
+    int32_t c0[U], c1[U];
+    V w0[U], w1[U];
+    const auto load_full = [&](int32_t j, int32_t (&c)[U], V (&w)[U]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            c[u] = col[base + (j + u) * stride];
+            w[u] = val[base + (j + u) * stride];
+        }
+    };
+    if (full > 0) load_full(0, c0, w0);
+    for (int32_t j = 0; j < full; j += U) {
+        if (j + U < full) load_full(j + U, c1, w1);
+        A xv[U][Q];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            load_cols_run<A, Q>(X + static_cast<int64_t>(c0[u]) * ldx, xv[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int q = 0; q < Q; ++q) acc[q] = T::fma_(T::widen(w0[u]), xv[u][q], acc[q]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            c0[u] = c1[u];
+            w0[u] = w1[u];
+        }
+    }
+    if (full < len) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (full + u < len) {
+                c1[u] = col[base + (full + u) * stride];
+                w1[u] = val[base + (full + u) * stride];
+            }
+        A xv[U][Q];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (full + u < len)
+                load_cols_run<A, Q>(X + static_cast<int64_t>(c1[u]) * ldx, xv[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (full + u < len)
+#pragma unroll
+                for (int q = 0; q < Q; ++q) acc[q] = T::fma_(T::widen(w1[u]), xv[u][q], acc[q]);
+    }
+}
+
+}  // namespace smaxhip

@@ -29,13 +29,14 @@
 
 #include "common.hpp"
 #include "scan.hpp"
+#include "spmm_long.hpp"
 
 struct smax_hip_crs_plan_s {
     int64_t n_rows = 0, nnz = 0, n_blocks = 0;
     int32_t block_threads = 256;     // row-block geometry: 256 (wide) or 64 (narrow)
     int32_t *block_start = nullptr;  // n_blocks + 1 row indices
     int32_t *row_order = nullptr;    // row-major SpMM execution order (n_rows)
-    int64_t spmm_lds = 0;            // dynamic LDS per SpMM workgroup (occupancy cap)
+    smaxhip::LongRows long_rows;     // how many rows, first in row_order, are long
 };
 
 namespace smaxhip {
@@ -159,65 +160,93 @@ __global__ void crs_block_starts(int64_t n_rows,
 }
 
 // ------------------------------------------------------------ SpMM
-// Thread (row, v) with v fastest for row-major operands (k lanes share one
-// broadcast val/col load, X rows are read contiguously), row fastest for
-// column-major ones (Y columns are written contiguously).
-template <int VT, bool ROW_MAJOR>
-__global__ __launch_bounds__(kCrsThreads) void crs_spmm_kernel(
-    int64_t n_rows, int64_t k, const int32_t *__restrict__ order,
-    const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col,
-    const typename vt<VT>::val_t *__restrict__ val,
+struct OrderedRow {  // the i-th row of a plan's order
+    const int32_t *__restrict__ order, *__restrict__ row_ptr;
+    __device__ __forceinline__ LongRowAt operator()(int64_t i) const {
+        const int32_t r = order[i];
+        return {row_ptr[r + 1] - row_ptr[r], row_ptr[r], r};
+    }
+};
+
+// Row-major SpMM for any k: ceil(k / Q) lanes per row, each owning a run of Q
+// columns (16 bytes' worth where k allows) read with one access per entry,
+// `rows` rows a workgroup (none: one row over `parts` workgroups).  LONG: the
+// first workgroups take the plan's long rows.
+//
+// What bounds it: the X rows gathered through L2, and for small matrices the
+// longest row's chain.  One column per lane instead (k lanes a row, a 64-bit
+// division each, groups of four entries, no prefetch) took 347 us for 200,003
+// rows, k = 10, FP64; this way 82.
+template <int VT, int Q, bool LONG>
+__global__ __launch_bounds__(kCrsThreads) void crs_spmm_run(
+    int64_t n_rows, LongRows longs, int64_t k, int64_t lanes, int32_t rows, FastDiv by_lanes,
+    int64_t parts, const int32_t *__restrict__ order, const int32_t *__restrict__ row_ptr,
+    const int32_t *__restrict__ col, const typename vt<VT>::val_t *__restrict__ val,
     const typename vt<VT>::vec_t *__restrict__ X, int64_t ldx,
     typename vt<VT>::vec_t *__restrict__ Y, int64_t ldy) {
-    using T = vt<VT>;
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * kCrsThreads + threadIdx.x;
-    int64_t r, v;
-    if (ROW_MAJOR) {
-        r = t / k;
-        v = t - r * k;
-    } else {
-        v = t / n_rows;
-        r = t - v * n_rows;
-    }
-    if (r >= n_rows || v >= k) return;
-    if (ROW_MAJOR && order) r = order[r];
-    const int64_t s = row_ptr[r], e = row_ptr[r + 1];
-    typename T::vec_t acc = 0;
-    int64_t j = s;
-    constexpr int U = 4;
-    for (; j + U <= e; j += U) {
-        int32_t c[U];
-        typename T::val_t w[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            c[u] = col[j + u];
-            w[u] = val[j + u];
+    using A = typename vt<VT>::vec_t;
+    if constexpr (LONG) {
+        if (blockIdx.x < longs.blocks()) {
+            long_rows<VT, Q>(longs, blockIdx.x, OrderedRow{order, row_ptr}, 1, col, val, k, X, ldx,
+                             Y, ldy);
+            return;
         }
-        typename T::vec_t xv[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            xv[u] = ROW_MAJOR ? X[static_cast<int64_t>(c[u]) * ldx + v]
-                              : X[v * ldx + c[u]];
-#pragma unroll
-        for (int u = 0; u < U; ++u) acc = T::fma_(T::widen(w[u]), xv[u], acc);
     }
-    for (; j < e; ++j) {
-        const typename T::vec_t xv =
-            ROW_MAJOR ? X[static_cast<int64_t>(col[j]) * ldx + v] : X[v * ldx + col[j]];
-        acc = T::fma_(T::widen(val[j]), xv, acc);
+    const int64_t block = blockIdx.x - (LONG ? longs.blocks() : 0);
+    int64_t pos, l;
+    if (rows > 0) {
+        const int32_t rl = by_lanes(static_cast<int32_t>(threadIdx.x));
+        if (rl >= rows) return;
+        pos = block * rows + rl;
+        l = static_cast<int64_t>(threadIdx.x) - rl * lanes;
+    } else {
+        pos = block / parts;
+        l = (block - pos * parts) * kCrsThreads + threadIdx.x;
+        if (l >= lanes) return;
     }
-    if (ROW_MAJOR) Y[r * ldy + v] = acc;
-    else Y[v * ldy + r] = acc;
+    if (LONG) pos += longs.count;
+    if (pos >= n_rows) return;
+    const int64_t r = order ? static_cast<int64_t>(order[pos]) : pos;
+    const int64_t v = run_start<Q>(l, k);
+    const int32_t s = row_ptr[r];
+    A acc[Q];
+    run_chain<VT, Q>(s, 1, row_ptr[r + 1] - s, col, val, X + v, ldx, acc);
+    store_cols_run<A, Q>(Y + r * ldy + v, acc);
+}
+
+template <int VT, int Q>
+static void launch_crs_spmm_run(smax_hip_ctx ctx, int64_t n_rows, int64_t k, LongRows longs,
+                                const int32_t *order, const int32_t *row_ptr,
+                                const int32_t *col, const void *val, const void *X, int64_t ldx,
+                                void *Y, int64_t ldy) {
+    using T = vt<VT>;
+    const int64_t lanes = run_lanes(k, Q);
+    const int64_t rows = kCrsThreads / lanes;
+    const int64_t parts = rows > 0 ? 1 : ceil_div(lanes, kCrsThreads);
+    const int64_t rest = n_rows - longs.count;
+    const int64_t blocks = longs.blocks() + (rows > 0 ? ceil_div(rest, rows) : rest * parts);
+    auto v = static_cast<const typename T::val_t *>(val);
+    auto xv = static_cast<const typename T::vec_t *>(X);
+    auto yv = static_cast<typename T::vec_t *>(Y);
+    const FastDiv by = fast_div(rows > 0 ? lanes : 1);
+#define SMAX_CRS_RUN(L)                                                                      \
+    hipLaunchKernelGGL((crs_spmm_run<VT, Q, L>), dim3(static_cast<unsigned>(blocks)),        \
+                       dim3(kCrsThreads), 0, ctx->stream, n_rows, longs, k, lanes,           \
+                       static_cast<int32_t>(rows), by, parts, order, row_ptr, col, v, xv, ldx, \
+                       yv, ldy)
+    if (longs.count > 0) SMAX_CRS_RUN(true);
+    else SMAX_CRS_RUN(false);
+#undef SMAX_CRS_RUN
 }
 
 // Row-major SpMM with k = K a power of two and 16-byte aligned X/Y rows: a
 // lane owns Q = 16 / sizeof(vec) consecutive columns v (K / Q lanes per row),
 // reads its part of each X row with one 16-byte load and keeps Q fma chains;
 // the chain is software-pipelined U elements deep.  Every Y[r, v] is the
-// same sequential chain over the row as in crs_spmm_kernel.
-template <int VT, int K>
+// same sequential chain over the row as in crs_spmm_run.
+template <int VT, int K, bool LONG>
 __global__ __launch_bounds__(kCrsThreads) void crs_spmm_rowvec(
-    int64_t n_rows, const int32_t *__restrict__ order,
+    int64_t n_rows, LongRows longs, const int32_t *__restrict__ order,
     const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col,
     const typename vt<VT>::val_t *__restrict__ val,
     const typename vt<VT>::vec_t *__restrict__ X, int64_t ldx,
@@ -229,8 +258,16 @@ __global__ __launch_bounds__(kCrsThreads) void crs_spmm_rowvec(
     constexpr int GL = K / Q;
     constexpr int U = 8;
     static_assert(GL * Q == K, "K must be a multiple of the run length");
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * kCrsThreads + threadIdx.x;
-    int64_t r = t / GL;
+    if constexpr (LONG) {  // the plan's long rows, as in crs_spmm_run
+        if (blockIdx.x < longs.blocks()) {
+            long_rows<VT, Q>(longs, blockIdx.x, OrderedRow{order, row_ptr}, 1, col, val, K, X, ldx,
+                             Y, ldy);
+            return;
+        }
+    }
+    const int64_t t = (static_cast<int64_t>(blockIdx.x) - (LONG ? longs.blocks() : 0)) *
+                          kCrsThreads + threadIdx.x;
+    int64_t r = t / GL + (LONG ? longs.count : 0);
     const int l = static_cast<int>(t % GL);
     if (r >= n_rows) return;
     if (order) r = order[r];
@@ -326,7 +363,7 @@ __global__ __launch_bounds__(kCrsThreads) void crs_spmm_rowvec(
 // their row strides are 16-byte aligned; false otherwise.
 template <int VT>
 static bool launch_crs_spmm_rowvec(smax_hip_ctx ctx, int64_t n_rows, int64_t k,
-                                   const int32_t *order, unsigned lds, const int32_t *row_ptr,
+                                   LongRows longs, const int32_t *order, const int32_t *row_ptr,
                                    const int32_t *col,
                                    const void *val, const void *X, int64_t ldx, void *Y,
                                    int64_t ldy) {
@@ -337,15 +374,23 @@ static bool launch_crs_spmm_rowvec(smax_hip_ctx ctx, int64_t n_rows, int64_t k,
     if (k < 4 * Q || k > 64 || (k & (k - 1)) != 0 || !aligned16(X, Y) ||
         (ldx * sizeof(A)) % 16 != 0 || (ldy * sizeof(A)) % 16 != 0)
         return false;
-    const dim3 g = grid_for(n_rows * (k / Q), kCrsThreads);
+    const dim3 g(static_cast<unsigned>(
+        longs.blocks() + ceil_div((n_rows - longs.count) * (k / Q), kCrsThreads)));
     auto v = static_cast<const typename T::val_t *>(val);
     auto xv = static_cast<const A *>(X);
     auto yv = static_cast<A *>(Y);
 #define SMAX_CRS_ROWVEC(KK)                                                                  \
     case KK:                                                                                  \
-        if constexpr (KK >= Q)                                                                \
-            hipLaunchKernelGGL((crs_spmm_rowvec<VT, KK>), g, dim3(kCrsThreads), lds,            \
-                               ctx->stream, n_rows, order, row_ptr, col, v, xv, ldx, yv, ldy); \
+        if constexpr (KK >= Q) {                                                              \
+            if (longs.count > 0)                                                              \
+                hipLaunchKernelGGL((crs_spmm_rowvec<VT, KK, true>), g, dim3(kCrsThreads), 0, \
+                                   ctx->stream, n_rows, longs, order, row_ptr, col, v, xv,    \
+                                   ldx, yv, ldy);                                             \
+            else                                                                              \
+                hipLaunchKernelGGL((crs_spmm_rowvec<VT, KK, false>), g, dim3(kCrsThreads), 0, \
+                                   ctx->stream, n_rows, longs, order, row_ptr, col, v, xv,    \
+                                   ldx, yv, ldy);                                             \
+        }                                                                                     \
         return true;
     switch (k) {
         SMAX_CRS_ROWVEC(2)
@@ -361,28 +406,26 @@ static bool launch_crs_spmm_rowvec(smax_hip_ctx ctx, int64_t n_rows, int64_t k,
 }
 
 // Row-major SpMM execution order: every thread group runs one row's chains,
-// so a wave lasts as long as its longest row.  Rows of at least
-// max(128, 8 x mean) entries start first, longest first (they set the
-// critical path); the rest follow window by window (kSpmmWindow rows, so a
+// so a wave lasts as long as its longest row.  Long rows (long_row_from) come
+// first, longest first, and run in workgroups of their own; the rest follow window by window (kSpmmWindow rows, so a
 // window's X band stays together), longest first inside each window so that
 // the rows sharing a wave have similar lengths.  Results do not depend on
 // the order.
 constexpr int64_t kSpmmWindow = 65536;
-constexpr int64_t kSpmmCapLds = 53 * 1024;
 
 static int build_row_order(smax_hip_ctx ctx, int64_t n_rows, int64_t nnz,
-                           const std::vector<int32_t> &rp, int32_t **out, int64_t *n_long) {
+                           const std::vector<int32_t> &rp, int32_t **out, LongRows *longs) {
     *out = nullptr;
-    *n_long = 0;
-    const double mean = static_cast<double>(nnz) / static_cast<double>(n_rows);
-    const int64_t thr =
-        std::max<int64_t>(128, static_cast<int64_t>(std::ceil(8 * mean)));
+    *longs = LongRows{};
+    const int64_t thr = long_row_from(nnz, n_rows);
     auto len = [&](int32_t r) { return rp[r + 1] - rp[r]; };
     std::vector<int32_t> ord;
     ord.reserve(static_cast<size_t>(n_rows));
     for (int64_t r = 0; r < n_rows; ++r)
         if (len(static_cast<int32_t>(r)) >= thr) ord.push_back(static_cast<int32_t>(r));
-    *n_long = static_cast<int64_t>(ord.size());
+    longs->count = static_cast<int64_t>(ord.size());
+    longs->whole = std::count_if(ord.begin(), ord.end(),
+                                 [&](int32_t r) { return len(r) >= kLongestRow; });
     auto longer = [&](int32_t a, int32_t b) { return len(a) > len(b); };
     std::stable_sort(ord.begin(), ord.end(), longer);
     for (int64_t w = 0; w < n_rows; w += kSpmmWindow) {
@@ -640,8 +683,8 @@ int smax_hip_crs_plan_create(smax_hip_ctx ctx, int64_t n_rows, int64_t nnz,
     dev_free(flag);
     dev_free(tmp);
     int32_t *order = nullptr;
-    int64_t n_long = 0;
-    if (!rc) rc = build_row_order(ctx, n_rows, nnz, rp, &order, &n_long);
+    LongRows longs;
+    if (!rc) rc = build_row_order(ctx, n_rows, nnz, rp, &order, &longs);
     if (rc) {
         dev_free(starts);
         dev_free(order);
@@ -654,10 +697,7 @@ int smax_hip_crs_plan_create(smax_hip_ctx ctx, int64_t n_rows, int64_t nnz,
     p->block_threads = nt;
     p->block_start = starts;
     p->row_order = order;
-    // With long rows leading, three workgroups per CU (53 KB of LDS each out
-    // of 160 KB) run the row-major SpMM faster than full occupancy: 0.46 ->
-    // 0.40 ms on the 1M-row band matrix, k = 32.
-    p->spmm_lds = n_long > 0 ? kSpmmCapLds : 0;
+    p->long_rows = longs;
     *out = p;
     return SMAX_HIP_SUCCESS;
 }
@@ -772,30 +812,25 @@ int smax_hip_crs_spmm(smax_hip_ctx ctx, int value_type, int64_t n_rows,
         return SMAX_HIP_ERROR_UNSUPPORTED;
     }
     const int32_t *order = plan ? plan->row_order : nullptr;
-    const int64_t spmm_lds = plan ? plan->spmm_lds : 0;
-    const int64_t threads = n_rows * k;
+    const LongRows longs = plan ? plan->long_rows : LongRows{};
+    // one column (k = 1): both layouts are the row-major one with unit strides
+    if (!row_major) ldx = ldy = 1;
     SMAX_HIP_DISPATCH_VT(value_type, {
-        using T = vt<VT>;
-        auto v = static_cast<const typename T::val_t *>(val);
-        auto xv = static_cast<const typename T::vec_t *>(X);
-        auto yv = static_cast<typename T::vec_t *>(Y);
-        if (row_major && launch_crs_spmm_rowvec<VT>(ctx, n_rows, k, order,
-                                                    static_cast<unsigned>(spmm_lds), row_ptr,
-                                                    col, val, X, ldx, Y, ldy)) {
-            SMAX_HIP_LAUNCHED(ctx, "crs_spmm_rowvec");
-            return SMAX_HIP_SUCCESS;
+        constexpr int64_t Q = 16 / sizeof(typename vt<VT>::vec_t);
+        if (!launch_crs_spmm_rowvec<VT>(ctx, n_rows, k, longs, order, row_ptr, col, val, X,
+                                        ldx, Y, ldy)) {
+            // the widest runs that k columns hold
+            if (k >= Q)
+                launch_crs_spmm_run<VT, Q>(ctx, n_rows, k, longs, order, row_ptr, col, val,
+                                           X, ldx, Y, ldy);
+            else if (Q > 2 && k >= 2)
+                launch_crs_spmm_run<VT, 2>(ctx, n_rows, k, longs, order, row_ptr, col, val,
+                                           X, ldx, Y, ldy);
+            else
+                launch_crs_spmm_run<VT, 1>(ctx, n_rows, k, longs, order, row_ptr, col, val,
+                                           X, ldx, Y, ldy);
         }
-        if (row_major)
-            hipLaunchKernelGGL((crs_spmm_kernel<VT, true>),
-                               grid_for(threads, kCrsThreads), dim3(kCrsThreads),
-                               0, ctx->stream, n_rows, k, order, row_ptr, col, v, xv,
-                               ldx, yv, ldy);
-        else
-            hipLaunchKernelGGL((crs_spmm_kernel<VT, false>),
-                               grid_for(threads, kCrsThreads), dim3(kCrsThreads),
-                               0, ctx->stream, n_rows, k, nullptr, row_ptr, col, v, xv,
-                               ldx, yv, ldy);
-        SMAX_HIP_LAUNCHED(ctx, "crs_spmm_kernel");
+        SMAX_HIP_LAUNCHED(ctx, "crs_spmm");
         return SMAX_HIP_SUCCESS;
     });
     return SMAX_HIP_ERROR_UNSUPPORTED;

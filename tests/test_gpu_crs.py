@@ -328,3 +328,38 @@ def _graph_survives_growth(ctx, torch):
         ctx.set_stream(None)
     for d in (rp, col, v, dX, dY):
         d.free()
+
+
+@pytest.mark.parametrize("vt", [capi.F64, capi.F32, capi.BF16])
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 10, 16, 20, 32, 33, 64, 260, 1100])
+@pytest.mark.parametrize("planned", [True, False])
+def test_spmm_long_rows_and_any_width(ctx, vt, k, planned):
+    """Row-major SpMM around the sizes where its path changes: the plan's long
+    rows (128 entries and more run in a workgroup of their own, tile by tile)
+    next to rows of 0, 1, 7, 8, 9 and 127 entries, and every column count's
+    runs (a last run shared with the one before; several workgroups a row)."""
+    rng = np.random.default_rng(k)
+    L = rng.integers(0, 4, 900)
+    L[[0, 5, 6, 7, 8, 300, 301, 302, 303, 899]] = [2000, 127, 128, 129, 0, 255, 256, 257, 1025, 640]
+    L[[10, 11, 12]] = [7, 8, 9]
+    n_cols = 3000
+    rp = np.concatenate([[0], np.cumsum(L)]).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(n_cols, l, replace=False)) for l in L]).astype(np.int32)
+    val = matgen.uniform_f64(5, rp[-1])
+    val = val if vt == capi.F64 else val.astype(np.float32) if vt == capi.F32 else matgen.to_bf16(val)
+    vec = np.float64 if vt == capi.F64 else np.float32
+    ldx, ldy = k + 1, k + 3
+    X = matgen.uniform_f64(6, n_cols * ldx).astype(vec).reshape(n_cols, ldx)
+    d = [ctx.upload(a) for a in (rp, col, val, X)]
+    dY = ctx.upload(np.full(L.size * ldy, 7, vec))
+    plan = ctx.crs_plan(L.size, int(rp[-1]), d[0]) if planned else None
+    ctx.crs_spmm(vt, L.size, n_cols, int(rp[-1]), d[0], d[1], d[2], k, True, d[3], ldx, dY, ldy,
+                 plan)
+    got = ctx.download(dY).reshape(-1, ldy)
+    want = oracle.crs_spmm(rp, col, val, k, True, np.ascontiguousarray(X[:, :k]).ravel())
+    assert_bitwise(got[:, :k].ravel(), np.asarray(want).ravel(), "Y")
+    assert (got[:, k:] == 7).all()
+    if plan:
+        ctx.crs_plan_destroy(plan)
+    for a in (*d, dY):
+        a.free()
