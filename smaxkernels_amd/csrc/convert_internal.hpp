@@ -2,6 +2,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "spmm_long.hpp"
 
 // Execution schedule of the SELL kernels, built once from the chunk lengths.
 struct smax_hip_scs_sched {
@@ -41,8 +42,19 @@ struct smax_hip_scs_tails {
     int64_t n_slots = 0, n_waves = 0;
 };
 
+// Long slots of a converted layout, for the SpMM: slots of `from` entries and
+// more, those that take a whole workgroup from the front of the list, the
+// others from its back.
+struct smax_hip_scs_longs {
+    int32_t *list = nullptr;
+    int64_t cap = 0;
+    int32_t from = 0;
+    smaxhip::LongRows rows;
+};
+
 struct smax_hip_scs_s {
     smax_hip_scs_info info;
+    smax_hip_scs_longs longs;     // built with the conversion
     // Built on first use by the CG solvers, freed with the handle:
     int32_t *col_slot = nullptr;  // perm[col[e]]: columns in slot space
     float *val_f32 = nullptr;     // values rounded to binary32

@@ -617,6 +617,20 @@ __global__ void k_chunk_ptr(int64_t n_chunks,
     if (c == n_chunks) *total = incl[c - 1];
 }
 
+// Lists the slots of `from` entries and more (smax_hip_scs_longs); counts[0]
+// and [1] (zero on entry): whole-workgroup ones and the others.  Their order
+// is that of the atomics; only which workgroup runs which depends on it.
+__global__ void k_long_slots(int64_t n, int32_t from, const int32_t *__restrict__ slot_len,
+                             int32_t *__restrict__ list, int64_t cap,
+                             int64_t *__restrict__ counts) {
+    const int64_t s = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (s >= n || slot_len[s] < from) return;
+    const bool whole = slot_len[s] >= kLongestRow;
+    const int64_t i = static_cast<int64_t>(
+        atomicAdd(reinterpret_cast<unsigned long long *>(counts + (whole ? 0 : 1)), 1ull));
+    list[whole ? i : cap - 1 - i] = static_cast<int32_t>(s);
+}
+
 __global__ void k_fill_i32(int64_t n, int32_t v, int32_t *__restrict__ p) {
     int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
@@ -952,15 +966,25 @@ int build_scs(smax_hip_ctx ctx, int64_t n_rows, int64_t n_cols, int64_t nnz,
         smax_hip_ctx ctx;
         smax_hip_scs_info *p;
         bool keep = false;
+        smax_hip_scs_longs *longs;
         ~Guard() {
             if (keep) return;
             (void)hipStreamSynchronize(ctx->stream);
             scs_free_arrays(*p);
+            dev_free(longs->list);
         }
-    } guard{ctx, &info};
+    };
+    smax_hip_scs_longs longs;
+    const int64_t from = long_slot_from(nnz, n_rows);
+    longs.from = static_cast<int32_t>(from <= INT32_MAX ? from : INT32_MAX);
+    longs.cap = nnz / longs.from + 1;
+    Guard guard{ctx, &info, false, &longs};
 
-    int64_t *elems, *incl, *tmp64, *words;  // words: sort errors, SELL elements
-    rc |= S.get(ctx, &words, 2, "scs conversion");
+    // words: sort errors, SELL elements, long slots (two counts)
+    int64_t *elems, *incl, *tmp64, *words;
+    rc |= S.get(ctx, &words, 4, "scs conversion");
+    rc |= dev_alloc(ctx, reinterpret_cast<void **>(&longs.list), sizeof(int32_t) * longs.cap,
+                    "scs long slots");
     rc |= S.get(ctx, &elems, n_chunks, "scs conversion");
     rc |= S.get(ctx, &incl, n_chunks, "scs conversion");
     rc |= S.get(ctx, &tmp64, scan_tmp_elems(n_chunks), "scs conversion");
@@ -976,7 +1000,7 @@ int build_scs(smax_hip_ctx ctx, int64_t n_rows, int64_t n_cols, int64_t nnz,
                     sizeof(int32_t) * n, "scs slot_len");
     if (rc) return SMAX_HIP_ERROR_OUT_OF_MEMORY;
 
-    rc = smax_hip_zero(ctx, words, 2 * sizeof(int64_t));
+    rc = smax_hip_zero(ctx, words, 4 * sizeof(int64_t));
     if (!rc)
         rc = sell_sort_windows(ctx, n, n_rows, sigma, row_ptr, info.slot_row, info.slot_len,
                                info.perm, words, S);
@@ -985,7 +1009,8 @@ int build_scs(smax_hip_ctx ctx, int64_t n_rows, int64_t n_cols, int64_t nnz,
     rc = scan_inclusive<int64_t, false>(ctx, elems, incl, n_chunks, tmp64);
     if (rc) return rc;
     LAUNCH(k_chunk_ptr, n_chunks + 1, n_chunks, incl, info.chunk_ptr, words + 1);
-    SMAX_HIP_CALL(ctx, hipMemcpyAsync(ctx->host_word, words, 2 * sizeof(int64_t),
+    LAUNCH(k_long_slots, n, n, longs.from, info.slot_len, longs.list, longs.cap, words + 2);
+    SMAX_HIP_CALL(ctx, hipMemcpyAsync(ctx->host_word, words, 4 * sizeof(int64_t),
                                       hipMemcpyDeviceToHost, ctx->stream));
     SMAX_HIP_CALL(ctx, hipStreamSynchronize(ctx->stream));
     if (ctx->host_word[0])
@@ -993,6 +1018,8 @@ int build_scs(smax_hip_ctx ctx, int64_t n_rows, int64_t n_cols, int64_t nnz,
                     "sell sort: %lld partitions produced an invalid cut",
                     static_cast<long long>(ctx->host_word[0]));
     const int64_t n_elements = ctx->host_word[1];
+    longs.rows.whole = ctx->host_word[2];
+    longs.rows.count = longs.rows.whole + ctx->host_word[3];
     if (n_elements > INT32_MAX)
         return fail(ctx, SMAX_HIP_ERROR_OVERFLOW,
                     "scs conversion: %lld SELL elements exceed int32 chunk_ptr",
@@ -1024,6 +1051,7 @@ int build_scs(smax_hip_ctx ctx, int64_t n_rows, int64_t n_cols, int64_t nnz,
     SMAX_HIP_CALL(ctx, hipStreamSynchronize(ctx->stream));
     smax_hip_scs scs = new smax_hip_scs_s();
     scs->info = info;
+    scs->longs = longs;
     scs->src_consecutive = src_map == nullptr;
     guard.keep = true;
     rc = build_schedule(ctx, C, sigma, n, n_chunks, n_elements, nnz, info.chunk_lengths,
@@ -1217,6 +1245,7 @@ int smax_hip_scs_destroy(smax_hip_ctx ctx, smax_hip_scs scs) {
     dev_free(scs->diag_f32);
     free_schedule(scs->sched);
     free_tails(scs->tails);
+    dev_free(scs->longs.list);
     dev_free(scs->elem_row);
     delete scs;
     return SMAX_HIP_SUCCESS;

@@ -44,6 +44,19 @@ inline int64_t long_row_from(int64_t nnz, int64_t n_rows) {
     return eight > kLongRow ? eight : kLongRow;
 }
 
+// In SELL a long slot alone also pays for its columns and values, one line an
+// entry that the other slots of its chunk would share; in large matrices, where
+// the longest rows no longer decide the time, fewer slots are long.
+// 1,000,000 rows, from 128 / 512 / 1024 / 1400 entries on: FP32 k = 32 0.359 /
+// 0.337 / 0.322 / 0.329 ms (none: 0.371), FP64 k = 16 0.468 / 0.404 / 0.372 /
+// 0.362 (0.382); 200,003 rows, FP64 k = 10: 0.089 / 0.094 / 0.146 / 0.169
+// (0.343).
+inline int64_t long_slot_from(int64_t nnz, int64_t n_rows) {
+    const int64_t row = long_row_from(nnz, n_rows), part = nnz / 16000;
+    const int64_t most = part < 1024 ? part : 1024;
+    return row > most ? row : most;
+}
+
 // Long rows in front of a launch's other rows: the first `whole` workgroups
 // take one row each, the next ceil((count - whole) / 4) take four.
 struct LongRows {

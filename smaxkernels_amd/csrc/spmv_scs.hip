@@ -18,6 +18,7 @@
 
 #include "common.hpp"
 #include "convert_internal.hpp"
+#include "spmm_long.hpp"
 
 namespace smaxhip {
 
@@ -269,99 +270,104 @@ __global__ __launch_bounds__(kScsThreads) void scs_spmv_generic(
     }
 }
 
-// SpMM, X and Y row-major with k columns: thread (slot, v), v fastest, so k
-// consecutive lanes share a slot's val/col (one broadcast load) and read a
-// contiguous row of X.  Y in original row order.  Workgroups take whole
-// chunks (cpb chunks of C*k threads each, or one chunk in bpc parts), in the
-// optional execution `order`.  LEN: each slot stops at its row's length and
-// no padding term is applied, so Y equals the CRS SpMM bit for bit; without
-// it the chain runs over the padded chunk (padding adds 0 * X[0, v]).  The
-// chain is software-pipelined like slot_chain_pipe.
-template <int VT, bool LEN>
-__global__ __launch_bounds__(kScsThreads) void scs_spmm_kernel(
-    int64_t C, int64_t n_chunks, int64_t n_rows, int64_t k, int64_t cpb, int64_t bpc,
-    const int32_t *__restrict__ chunk_ptr, const int32_t *__restrict__ chunk_len,
-    const int32_t *__restrict__ slot_len, const int32_t *__restrict__ order,
-    const int32_t *__restrict__ col, const typename vt<VT>::val_t *__restrict__ val,
-    const int32_t *__restrict__ slot_row, const typename vt<VT>::vec_t *__restrict__ X,
-    typename vt<VT>::vec_t *__restrict__ Y) {
-    using T = vt<VT>;
-    using A = typename T::vec_t;
-    using V = typename T::val_t;
-    constexpr int U = 8;
-    const int64_t ck = C * k;
-    int64_t pos, li;
-    if (cpb > 1) {
-        if (threadIdx.x >= cpb * ck) return;
-        pos = static_cast<int64_t>(blockIdx.x) * cpb + threadIdx.x / ck;
-        li = threadIdx.x % ck;
-    } else {
-        pos = blockIdx.x / bpc;
-        li = (blockIdx.x % bpc) * kScsThreads + threadIdx.x;
+// The i-th long slot of a handle: the whole-workgroup ones are listed from
+// the front, the others from the back.
+struct ListedSlot {
+    const int32_t *__restrict__ list;
+    int64_t cap, whole;
+    int64_t C;
+    const int32_t *__restrict__ chunk_ptr, *__restrict__ slot_len, *__restrict__ slot_row;
+    __device__ __forceinline__ LongRowAt operator()(int64_t i) const {
+        const int64_t s = list[i < whole ? i : cap - 1 - (i - whole)];
+        const int64_t c = s / C;
+        return {slot_len[s], static_cast<int64_t>(chunk_ptr[c]) + (s - c * C), slot_row[s]};
     }
-    if (pos >= n_chunks || li >= ck) return;
-    const int64_t chunk = order ? static_cast<int64_t>(order[pos]) : pos;
-    const int64_t i = li / k, v = li - i * k;
-    const int64_t slot = chunk * C + i;
-    const int32_t r = slot_row[slot];
-    if (r >= n_rows) return;
-    const int64_t base = static_cast<int64_t>(chunk_ptr[chunk]) + i;
-    const int len = LEN ? slot_len[slot] : chunk_len[chunk];
-    A acc = 0;
-    int j = 0;
-    if (len >= U) {
-        int32_t c0[U];
-        V w0[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            c0[u] = col[base + u * C];
-            w0[u] = val[base + u * C];
-        }
-        for (; j + 2 * U <= len; j += U) {
-            int32_t c1[U];
-            V w1[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                c1[u] = col[base + (j + U + u) * C];
-                w1[u] = val[base + (j + U + u) * C];
-            }
-            A xv[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) xv[u] = X[static_cast<int64_t>(c0[u]) * k + v];
-#pragma unroll
-            for (int u = 0; u < U; ++u) acc = T::fma_(T::widen(w0[u]), xv[u], acc);
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                c0[u] = c1[u];
-                w0[u] = w1[u];
-            }
-        }
-        A xv[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) xv[u] = X[static_cast<int64_t>(c0[u]) * k + v];
-#pragma unroll
-        for (int u = 0; u < U; ++u) acc = T::fma_(T::widen(w0[u]), xv[u], acc);
-        j += U;
-    }
-    for (; j < len; ++j) {
-        const int64_t o = base + static_cast<int64_t>(j) * C;
-        acc = T::fma_(T::widen(val[o]), X[static_cast<int64_t>(col[o]) * k + v], acc);
-    }
-    Y[static_cast<int64_t>(r) * k + v] = acc;
+};
+
+// Long slots that are neighbours, whose columns and values share lines, on one
+// XCD: 1,000,000 rows, k = 32: 0.367 -> 0.359 ms, 200,003: 0.087 -> 0.082.
+__device__ __forceinline__ int64_t long_block(const LongRows &r, int64_t b) {
+    return b < r.whole ? xcd_block(b, r.whole)
+                       : r.whole + xcd_block(b - r.whole, r.blocks() - r.whole);
 }
 
-// As scs_spmm_kernel for k = K a power of two with 16-byte aligned X and Y:
+// What the two SpMM kernels take.  The launch's first longs.blocks()
+// workgroups run the long slots, the others `per` slots each, in the execution
+// order of their chunks, `lanes` threads a slot (or one slot in `parts`).
+struct ScsSpmmArgs {
+    int64_t C, n_slots, n_rows, k, lanes, per, parts;
+    FastDiv by_lanes, by_c;
+    LongRows longs;
+    int32_t long_from;        // slots of this length and more are long (LONG)
+    const int32_t *long_list;
+    int64_t long_cap;
+    const int32_t *chunk_ptr, *chunk_len, *slot_len, *order, *col, *slot_row;
+
+    __device__ __forceinline__ ListedSlot listed() const {
+        return {long_list, long_cap, longs.whole, C, chunk_ptr, slot_len, slot_row};
+    }
+    // This thread's chunk, slot of the chunk and lane of the slot; false: none.
+    __device__ __forceinline__ bool place(int64_t block, int64_t &chunk, int64_t &i,
+                                          int64_t &l) const {
+        int64_t at;
+        if (per > 0) {
+            const int32_t t = by_lanes(static_cast<int32_t>(threadIdx.x));
+            if (t >= per) return false;
+            at = block * per + t;
+            l = static_cast<int64_t>(threadIdx.x) - t * lanes;
+        } else {
+            at = block / parts;
+            l = (block - at * parts) * kScsThreads + threadIdx.x;
+        }
+        if (at >= n_slots || l >= lanes) return false;
+        const int32_t pos = by_c(static_cast<int32_t>(at));
+        chunk = order ? static_cast<int64_t>(order[pos]) : pos;
+        i = at - pos * C;
+        return true;
+    }
+};
+
+// SpMM, X and Y row-major with any k columns, in the lanes and runs of
+// crs_spmm_run; Y in original row order.  LEN: each slot stops at its row's
+// length and no padding term is applied, so Y equals the CRS SpMM bit for
+// bit; without it the chain runs over the padded chunk (padding adds
+// 0 * X[0, v]).  LONG (with LEN): long slots run in workgroups and wavefronts
+// of their own.  One column per lane, four bytes an access, and no such path
+// took 128 us for 40,013 rows, k = 20, BF16 values.
+template <int VT, bool LEN, int Q, bool LONG>
+__global__ __launch_bounds__(kScsThreads) void scs_spmm_run(
+    ScsSpmmArgs a, const typename vt<VT>::val_t *__restrict__ val,
+    const typename vt<VT>::vec_t *__restrict__ X, typename vt<VT>::vec_t *__restrict__ Y) {
+    using A = typename vt<VT>::vec_t;
+    if constexpr (LONG) {
+        if (blockIdx.x < a.longs.blocks()) {
+            long_rows<VT, Q>(a.longs, long_block(a.longs, blockIdx.x), a.listed(), a.C, a.col,
+                             val, a.k, X, a.k, Y, a.k);
+            return;
+        }
+    }
+    int64_t chunk, i, l;
+    if (!a.place(blockIdx.x - (LONG ? a.longs.blocks() : 0), chunk, i, l)) return;
+    const int64_t slot = chunk * a.C + i;
+    const int32_t r = a.slot_row[slot];
+    if (r >= a.n_rows) return;
+    const int len = LEN ? a.slot_len[slot] : a.chunk_len[chunk];
+    if (LONG && len >= a.long_from) return;
+    const int64_t v = run_start<Q>(l, a.k);
+    A acc[Q];
+    run_chain<VT, Q>(static_cast<int64_t>(a.chunk_ptr[chunk]) + i, a.C, len, a.col, val, X + v,
+                     a.k, acc);
+    store_cols_run<A, Q>(Y + static_cast<int64_t>(r) * a.k + v, acc);
+}
+
+// As scs_spmm_run for k = K a power of two with 16-byte aligned X and Y:
 // a lane owns Q = 16 / sizeof(vec) consecutive columns v (K / Q lanes per
 // slot), reads its part of each X row with one 16-byte load and keeps Q fma
-// chains, each the same sequential chain as in scs_spmm_kernel.
-template <int VT, bool LEN, int K>
+// chains, each the same sequential chain as in scs_spmm_run.
+template <int VT, bool LEN, int K, bool LONG>
 __global__ __launch_bounds__(kScsThreads) void scs_spmm_vec(
-    int64_t C, int64_t n_chunks, int64_t n_rows, int64_t cpb, int64_t bpc,
-    const int32_t *__restrict__ chunk_ptr, const int32_t *__restrict__ chunk_len,
-    const int32_t *__restrict__ slot_len, const int32_t *__restrict__ order,
-    const int32_t *__restrict__ col, const typename vt<VT>::val_t *__restrict__ val,
-    const int32_t *__restrict__ slot_row, const typename vt<VT>::vec_t *__restrict__ X,
-    typename vt<VT>::vec_t *__restrict__ Y) {
+    ScsSpmmArgs a, const typename vt<VT>::val_t *__restrict__ val,
+    const typename vt<VT>::vec_t *__restrict__ X, typename vt<VT>::vec_t *__restrict__ Y) {
     using T = vt<VT>;
     using A = typename T::vec_t;
     using V = typename T::val_t;
@@ -369,25 +375,24 @@ __global__ __launch_bounds__(kScsThreads) void scs_spmm_vec(
     constexpr int GL = K / Q;
     constexpr int U = 8;
     static_assert(GL * Q == K, "K must be a multiple of the run length");
-    const int64_t ck = C * GL;
-    int64_t pos, li;
-    if (cpb > 1) {
-        if (threadIdx.x >= cpb * ck) return;
-        pos = static_cast<int64_t>(blockIdx.x) * cpb + threadIdx.x / ck;
-        li = threadIdx.x % ck;
-    } else {
-        pos = blockIdx.x / bpc;
-        li = (blockIdx.x % bpc) * kScsThreads + threadIdx.x;
+    if constexpr (LONG) {
+        if (blockIdx.x < a.longs.blocks()) {
+            long_rows<VT, Q>(a.longs, long_block(a.longs, blockIdx.x), a.listed(), a.C, a.col,
+                             val, K, X, K, Y, K);
+            return;
+        }
     }
-    if (pos >= n_chunks || li >= ck) return;
-    const int64_t chunk = order ? static_cast<int64_t>(order[pos]) : pos;
-    const int64_t i = li / GL;
-    const int l = static_cast<int>(li % GL);
+    int64_t chunk, i, l64;
+    if (!a.place(blockIdx.x - (LONG ? a.longs.blocks() : 0), chunk, i, l64)) return;
+    const int l = static_cast<int>(l64);
+    const int64_t C = a.C;
     const int64_t slot = chunk * C + i;
-    const int32_t r = slot_row[slot];
-    if (r >= n_rows) return;
-    const int64_t base = static_cast<int64_t>(chunk_ptr[chunk]) + i;
-    const int len = LEN ? slot_len[slot] : chunk_len[chunk];
+    const int32_t r = a.slot_row[slot];
+    if (r >= a.n_rows) return;
+    const int64_t base = static_cast<int64_t>(a.chunk_ptr[chunk]) + i;
+    const int len = LEN ? a.slot_len[slot] : a.chunk_len[chunk];
+    if (LONG && len >= a.long_from) return;
+    const int32_t *__restrict__ col = a.col;
     A acc[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) acc[q] = 0;
@@ -481,43 +486,72 @@ __global__ __launch_bounds__(kScsThreads) void scs_spmm_vec(
 }
 
 template <int VT, int K>
-static void launch_scs_spmm_vec(smax_hip_ctx ctx, int64_t C, int64_t n_chunks, int64_t n_rows,
-                                int64_t cpb, int64_t bpc, int64_t blocks, int64_t lds_bytes,
-                                const int32_t *chunk_ptr, const int32_t *chunk_len,
-                                const int32_t *slot_len, const int32_t *order,
-                                const int32_t *col, const typename vt<VT>::val_t *val,
-                                const int32_t *slot_row, const typename vt<VT>::vec_t *X,
-                                typename vt<VT>::vec_t *Y) {
-    const unsigned lds = static_cast<unsigned>(lds_bytes);
-    if (slot_len)
-        hipLaunchKernelGGL((scs_spmm_vec<VT, true, K>), dim3(static_cast<unsigned>(blocks)),
-                           dim3(kScsThreads), lds, ctx->stream, C, n_chunks, n_rows, cpb, bpc,
-                           chunk_ptr, chunk_len, slot_len, order, col, val, slot_row, X, Y);
-    else
-        hipLaunchKernelGGL((scs_spmm_vec<VT, false, K>), dim3(static_cast<unsigned>(blocks)),
-                           dim3(kScsThreads), lds, ctx->stream, C, n_chunks, n_rows, cpb, bpc,
-                           chunk_ptr, chunk_len, slot_len, order, col, val, slot_row, X, Y);
+static void launch_scs_spmm_vec(smax_hip_ctx ctx, const ScsSpmmArgs &a, dim3 grid,
+                                const typename vt<VT>::val_t *val,
+                                const typename vt<VT>::vec_t *X, typename vt<VT>::vec_t *Y) {
+#define SMAX_SCS_VEC(LEN, LONG)                                                               \
+    hipLaunchKernelGGL((scs_spmm_vec<VT, LEN, K, LONG>), grid, dim3(kScsThreads), 0, ctx->stream, \
+                       a, val, X, Y)
+    if (a.longs.count > 0) SMAX_SCS_VEC(true, true);
+    else if (a.slot_len) SMAX_SCS_VEC(true, false);
+    else SMAX_SCS_VEC(false, false);
+#undef SMAX_SCS_VEC
 }
 
-// lds_bytes: dynamic LDS reserved per workgroup of the 16-byte-run kernel
-// (an occupancy cap, 0 = none).
+template <int VT, int Q>
+static void launch_scs_spmm_run(smax_hip_ctx ctx, const ScsSpmmArgs &a, dim3 grid,
+                                const typename vt<VT>::val_t *val,
+                                const typename vt<VT>::vec_t *X, typename vt<VT>::vec_t *Y) {
+#define SMAX_SCS_RUN(LEN, LONG)                                                               \
+    hipLaunchKernelGGL((scs_spmm_run<VT, LEN, Q, LONG>), grid, dim3(kScsThreads), 0, ctx->stream, \
+                       a, val, X, Y)
+    if (a.longs.count > 0) SMAX_SCS_RUN(true, true);
+    else if (a.slot_len) SMAX_SCS_RUN(true, false);
+    else SMAX_SCS_RUN(false, false);
+#undef SMAX_SCS_RUN
+}
+
+// longs: the handle's long slots (nullptr: none; needs slot_len).
 template <int VT>
 static int launch_scs_spmm(smax_hip_ctx ctx, int64_t C, int64_t n_chunks, int64_t n_rows,
                            int64_t k, const int32_t *chunk_ptr, const int32_t *chunk_len,
                            const int32_t *slot_len, const int32_t *order,
                            const int32_t *col, const void *val, const int32_t *slot_row,
-                           const void *X, void *Y, int64_t lds_bytes = 0) {
+                           const void *X, void *Y, const smax_hip_scs_longs *longs = nullptr) {
     using T = vt<VT>;
     using A = typename T::vec_t;
     constexpr int64_t Q = 16 / sizeof(A);
     // k a power of two in [4Q, 64] with 16-byte aligned operands: Q columns
     // per lane, at least 4 lanes per slot
     const bool vec = k >= 4 * Q && k <= 64 && (k & (k - 1)) == 0 && aligned16(X, Y);
-    const int64_t ck = C * (vec ? k / Q : k);
-    const int64_t cpb = ck <= kScsThreads ? kScsThreads / ck : 1;
-    const int64_t bpc = ck <= kScsThreads ? 1 : ceil_div(ck, kScsThreads);
-    const int64_t blocks = cpb > 1 ? ceil_div(n_chunks, cpb) : n_chunks * bpc;
+    const int64_t q = k >= Q ? Q : k >= 2 ? 2 : 1;  // columns per lane
+    const int64_t lanes = run_lanes(k, q);
+    ScsSpmmArgs a{};
+    a.C = C;
+    a.n_slots = n_chunks * C;
+    a.n_rows = n_rows;
+    a.k = k;
+    a.lanes = lanes;
+    a.per = kScsThreads / lanes;
+    a.parts = a.per > 0 ? 1 : ceil_div(lanes, kScsThreads);
+    a.by_lanes = fast_div(a.per > 0 ? lanes : 1);
+    a.by_c = fast_div(C);
+    if (longs && slot_len) {
+        a.longs = longs->rows;
+        a.long_from = longs->from;
+        a.long_list = longs->list;
+        a.long_cap = longs->cap;
+    }
+    a.chunk_ptr = chunk_ptr;
+    a.chunk_len = chunk_len;
+    a.slot_len = slot_len;
+    a.order = order;
+    a.col = col;
+    a.slot_row = slot_row;
+    const int64_t blocks =
+        a.longs.blocks() + (a.per > 0 ? ceil_div(a.n_slots, a.per) : a.n_slots * a.parts);
     SMAX_HIP_REQUIRE(ctx, blocks <= INT32_MAX, "scs spmm: grid too large");
+    const dim3 grid(static_cast<unsigned>(blocks));
     auto v = static_cast<const typename T::val_t *>(val);
     auto xv = static_cast<const typename T::vec_t *>(X);
     auto yv = static_cast<typename T::vec_t *>(Y);
@@ -525,13 +559,8 @@ static int launch_scs_spmm(smax_hip_ctx ctx, int64_t C, int64_t n_chunks, int64_
         switch (k) {
 #define SMAX_SCS_SPMM_VEC(KK)                                                                \
     case KK:                                                                                  \
-        if constexpr (KK >= Q)                                                                \
-            launch_scs_spmm_vec<VT, KK>(ctx, C, n_chunks, n_rows, cpb, bpc, blocks, lds_bytes, \
-                                        chunk_ptr, chunk_len, slot_len, order, col, v,         \
-                                        slot_row, xv, yv);                                     \
+        if constexpr (KK >= 4 * Q) launch_scs_spmm_vec<VT, KK>(ctx, a, grid, v, xv, yv);      \
         break;
-            SMAX_SCS_SPMM_VEC(2)
-            SMAX_SCS_SPMM_VEC(4)
             SMAX_SCS_SPMM_VEC(8)
             SMAX_SCS_SPMM_VEC(16)
             SMAX_SCS_SPMM_VEC(32)
@@ -541,17 +570,10 @@ static int launch_scs_spmm(smax_hip_ctx ctx, int64_t C, int64_t n_chunks, int64_
         SMAX_HIP_LAUNCHED(ctx, "scs_spmm_vec");
         return SMAX_HIP_SUCCESS;
     }
-    if (slot_len)
-        hipLaunchKernelGGL((scs_spmm_kernel<VT, true>), dim3(static_cast<unsigned>(blocks)),
-                           dim3(kScsThreads), 0, ctx->stream, C, n_chunks, n_rows, k, cpb,
-                           bpc, chunk_ptr, chunk_len, slot_len, order, col, v, slot_row,
-                           xv, yv);
-    else
-        hipLaunchKernelGGL((scs_spmm_kernel<VT, false>), dim3(static_cast<unsigned>(blocks)),
-                           dim3(kScsThreads), 0, ctx->stream, C, n_chunks, n_rows, k, cpb,
-                           bpc, chunk_ptr, chunk_len, slot_len, order, col, v, slot_row,
-                           xv, yv);
-    SMAX_HIP_LAUNCHED(ctx, "scs_spmm_kernel");
+    if (q == Q) launch_scs_spmm_run<VT, Q>(ctx, a, grid, v, xv, yv);
+    else if (q == 2) launch_scs_spmm_run<VT, 2>(ctx, a, grid, v, xv, yv);
+    else launch_scs_spmm_run<VT, 1>(ctx, a, grid, v, xv, yv);
+    SMAX_HIP_LAUNCHED(ctx, "scs_spmm_run");
     return SMAX_HIP_SUCCESS;
 }
 
@@ -1190,15 +1212,11 @@ int smax_hip_scs_apply_spmm(smax_hip_ctx ctx, int value_type, smax_hip_scs A,
         return fail(ctx, SMAX_HIP_ERROR_INVALID_VALUE,
                     "smax_hip_scs_apply_spmm: value type %d does not match %lld-byte "
                     "values", value_type, (long long)in.val_bytes);
-    // the SpMV's occupancy cap pays off for the SpMM too when long chunks lead
-    // (0.40 -> 0.37 ms on the 1M-row band matrix at sigma = 65536, k = 32);
-    // without long chunks it costs (0.27 -> 0.28 ms on its transpose)
-    const int64_t lds = A->sched.order_lf ? A->sched.lds_cap_bytes : 0;
     SMAX_HIP_DISPATCH_VT(value_type,
                          return launch_scs_spmm<VT>(ctx, in.C, in.n_chunks, in.n_rows, k,
                                                     in.chunk_ptr, in.chunk_lengths,
                                                     in.slot_len, A->sched.order_lf, in.col,
-                                                    in.val, in.slot_row, X, Y, lds));
+                                                    in.val, in.slot_row, X, Y, &A->longs));
     return SMAX_HIP_ERROR_UNSUPPORTED;
 }
 

@@ -710,3 +710,32 @@ def test_conversion_fill_runs_of_empty_chunks(ctx, C_, dtype):
             at = int(got["chunk_ptr"][p // C_]) + np.arange(L[i]) * C_ + p % C_
             assert_bitwise(src[at], np.arange(rp[i], rp[i + 1], dtype=np.int32), f"row {i}")
         s.destroy()
+
+
+@pytest.mark.parametrize("vt", [capi.F64, capi.F32, capi.BF16])
+@pytest.mark.parametrize("k", [1, 2, 3, 5, 8, 16, 20, 32, 33, 64, 260, 1100])
+@pytest.mark.parametrize("C_,sigma", [(64, 4096), (32, 1), (3, 50), (300, 600)])
+def test_scs_apply_spmm_long_rows_and_any_width(ctx, vt, k, C_, sigma):
+    """SELL SpMM around the sizes where its path changes: slots of 128 entries
+    and more run in a wavefront or (512 and more) a workgroup of their own,
+    next to short and empty ones; every column count's runs; chunks that share
+    a workgroup, fill one, or span several."""
+    rng = np.random.default_rng(k)
+    L = rng.integers(0, 4, 900)
+    L[[0, 5, 6, 7, 8, 300, 301, 302, 303, 899]] = [2000, 127, 128, 129, 0, 511, 512, 513, 1025, 640]
+    L[[10, 11, 12]] = [7, 8, 9]
+    n_cols = 3000
+    rp = np.concatenate([[0], np.cumsum(L)]).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(n_cols, l, replace=False)) for l in L]).astype(np.int32)
+    val = matgen.uniform_f64(5, rp[-1])
+    val = val if vt == capi.F64 else val.astype(np.float32) if vt == capi.F32 else matgen.to_bf16(val)
+    vec = np.float64 if vt == capi.F64 else np.float32
+    X = matgen.uniform_f64(6, n_cols * k).astype(vec)
+    A = Csr(L.size, n_cols, rp, col, val)
+    s = gpu_scs(ctx, A, C_, sigma, val)
+    dX, dY = ctx.upload(X), ctx.upload(np.full(L.size * k, 7, vec))
+    s.apply_spmm(vt, k, dX, dY)
+    assert_bitwise(ctx.download(dY), np.asarray(oracle.crs_spmm(rp, col, val, k, True, X)).ravel())
+    for a in (dX, dY):
+        a.free()
+    s.destroy()
