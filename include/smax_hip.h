@@ -467,8 +467,7 @@ int smax_hip_scs_transpose_from_crs(smax_hip_ctx ctx, int64_t n_rows,
  * Accumulates in the value type's accumulation precision with a tree that
  * depends only on k: g = clamp(P/4, 1, 64) partial sums (P the smallest
  * power of two >= k), partial l an fma chain over v in [l*q, min(k, l*q+q)),
- * q = ceil(k/g), then a butterfly over the g partials.  G and X aligned to
- * 16 bytes take a faster kernel with identical results.  No reference
+ * q = ceil(k/g), then a butterfly over the g partials.  No reference
  * counterpart.
  */
 int smax_hip_scs_sddmm(smax_hip_ctx ctx, int value_type, smax_hip_scs A,

@@ -13,13 +13,14 @@
 // element e of SELL row r.  The reduction tree depends only on k: with P the
 // smallest power of two >= k, g = clamp(P / 4, 1, 64) lanes share an element,
 // lane l sums v in [l*Q, min(k, l*Q + Q)), Q = ceil(k / g), with an fma chain
-// from zero, and an xor-butterfly adds the g partial sums.  For k a power of
-// two up to 64 the lanes of a group share one row (SpMM order): the G row is
-// read once per row and each element costs one coalesced X row with 16-byte
-// loads.  Other k take one group per stored element, with the row of each
-// element from a per-element row array built on first use.  Both kernels
-// evaluate the same tree, so dvals do not depend on which one runs.
+// from zero, and an xor-butterfly adds the g partial sums.  Up to k = 256 the
+// lanes of a group share one row (SpMM order): the G row is read once per row
+// and each element costs one coalesced X row.  Larger k take one group per
+// stored element, with the row of each element from a per-element row array
+// built on first use.  Both kernels evaluate the same tree, so dvals do not
+// depend on which one runs.
 #include <algorithm>
+#include <type_traits>
 #include <utility>
 
 #include "common.hpp"
@@ -63,19 +64,15 @@ template <int G, typename A> __device__ __forceinline__ A group_sum(A acc) {
     return acc;
 }
 
-// One group of G = sddmm_group(k) lanes per stored element.
-template <int VT, int G>
+// k > 256: one wavefront (sddmm_group(k) = 64 lanes) per stored element.
+template <typename A>
 __global__ __launch_bounds__(256) void scs_sddmm_kernel(
     int64_t n_elements, int64_t k, const int32_t *__restrict__ col,
     const int32_t *__restrict__ elem_row, const int32_t *__restrict__ src,
-    const typename vt<VT>::vec_t *__restrict__ Gm,
-    const typename vt<VT>::vec_t *__restrict__ X,
-    typename vt<VT>::vec_t *__restrict__ dvals) {
-    using T = vt<VT>;
-    using A = typename T::vec_t;
+    const A *__restrict__ Gm, const A *__restrict__ X, A *__restrict__ dvals) {
     const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    const int64_t e = t / G;
-    const int lane = static_cast<int>(t % G);
+    const int64_t e = t / kWave;
+    const int lane = static_cast<int>(t % kWave);
     const bool valid = e < n_elements;
     const int32_t s = valid ? src[e] : -1;
     A acc = 0;
@@ -84,24 +81,13 @@ __global__ __launch_bounds__(256) void scs_sddmm_kernel(
         const int64_t c = col[e];
         const int64_t q = sddmm_run(k);
         const int64_t v1 = (lane + 1) * q < k ? (lane + 1) * q : k;
-        for (int64_t v = lane * q; v < v1; ++v) acc = T::fma_(Gm[r * k + v], X[c * k + v], acc);
+        for (int64_t v = lane * q; v < v1; ++v)
+            acc = __builtin_elementwise_fma(Gm[r * k + v], X[c * k + v], acc);
     }
-    acc = group_sum<G>(acc);
+    acc = group_sum<kWave>(acc);
     if (s >= 0 && lane == 0) dvals[s] = acc;
 }
 
-// k = K a power of two <= 64: GL = sddmm_group(K) lanes per slot (row) in
-// SpMM order, long chunks first.  Lane l keeps G[r, l*Q .. l*Q+Q) in
-// registers for the whole row; each element costs one coalesced X row read
-// with 16-byte loads, Q fmas per lane and the butterfly over GL lanes.  The
-// chain over the row's elements is software-pipelined (the next U column and
-// src indices are loaded before this group's X rows; U = kSddmmChainGroup),
-// and the U results of a
-// group, consecutive CRS positions of one row, leave in one store
-// instruction from U lanes (U / GL instructions when GL < U).  The U
-// elements of a group share one butterfly (group_reduce_scatter; per GL
-// elements when GL < U) that ends with each element's sum on the lane that
-// stores it, and each lane loads only the src indices it stores to.
 // The same butterfly over GL >= U lanes for U elements at once: at each
 // offset (GL/2 first) a lane keeps the half of its live elements that its
 // lane bit selects and sends the other half to its partner, adding (own +
@@ -150,192 +136,205 @@ __device__ __forceinline__ A group_reduce_scatter(A (&cur)[U], int l) {
 }
 
 // Elements per pipelined group of the row kernel, measured at N = 1M (band
-// matrix, SELL-64-65536): 16 for k = 16 and 32 (FP64 k = 16 0.61 -> 0.51 ms,
-// k = 32 0.80 -> 0.69 ms; FP32 k = 32 0.403 -> 0.385 ms), 8 for k = 64 (FP32
-// 0.71 ms against 0.77 with 16) and for k <= 8, where a lane holds several
-// elements of a group and 16 would leave three or four waves per SIMD.
-template <int K>
-constexpr int kSddmmChainGroup = K == 16 || K == 32 ? 16 : 8;
+// matrix, SELL-64-65536): 16 for 4 and 8 lanes (FP64 k = 16 0.61 -> 0.51 ms,
+// k = 32 0.80 -> 0.69 ms; FP32 k = 32 0.403 -> 0.385 ms), 8 for 16 and more
+// (FP32 k = 64 0.71 ms against 0.77 with 16) and for 1 and 2, where a lane
+// holds several elements of a group and 16 would leave three or four waves per
+// SIMD.
+template <int GL>
+constexpr int kSddmmChainGroup = GL == 4 || GL == 8 ? 16 : 8;
 
-// SEQ: the handle's src_index is consecutive within a slot, so a slot's
-// destinations are its first element's src_index plus j (one src load per
-// slot instead of one per element).
-template <int VT, int K, bool SEQ>
-__global__ __launch_bounds__(256) void scs_sddmm_rows(
-    int64_t C, int64_t n_chunks, int64_t n_rows, int64_t cpb, int64_t bpc,
-    const int32_t *__restrict__ chunk_ptr, const int32_t *__restrict__ slot_len,
-    const int32_t *__restrict__ order, const int32_t *__restrict__ col,
-    const int32_t *__restrict__ slot_row, const int32_t *__restrict__ src,
-    const typename vt<VT>::vec_t *__restrict__ Gm,
-    const typename vt<VT>::vec_t *__restrict__ X,
-    typename vt<VT>::vec_t *__restrict__ dvals) {
-    using T = vt<VT>;
-    using A = typename T::vec_t;
-    constexpr int GL = static_cast<int>(sddmm_group(K));
-    constexpr int Q = K / GL;
-    constexpr int U = kSddmmChainGroup<K>;
-    static_assert(GL * Q == K, "K must be a power of two");
-    const int64_t ck = C * GL;
-    int64_t pos, li;
-    if (cpb > 1) {
-        if (threadIdx.x >= cpb * ck) return;
-        pos = static_cast<int64_t>(blockIdx.x) * cpb + threadIdx.x / ck;
-        li = threadIdx.x % ck;
+// What the row kernel takes (slots as in ScsSpmmArgs of the SpMM).
+struct SddmmArgs {
+    int64_t C, n_slots, n_rows, k;
+    FastDiv by_c;
+    int64_t n_long, long_whole, long_cap;  // long slots: count, listed from the front, list size
+    int32_t long_from;
+    bool seq;  // src_index is consecutive within a slot
+    const int32_t *long_list, *chunk_ptr, *slot_len, *order, *col, *slot_row, *src;
+};
+
+// k <= 256: GL = sddmm_group(k) lanes per slot (row), lane l with the Q =
+// sddmm_run(k) entries from l * Q on of the G row in registers for the whole
+// row (EXACT: GL * Q = k; otherwise the last lanes read the row's last Q
+// entries and skip those before their own, and lanes past the end skip all).
+// Each element costs one coalesced X row, Q fmas per lane and its share of a
+// butterfly: the elements of a group go through one butterfly together
+// (group_reduce_scatter) that leaves each element's sum on the lane that
+// stores it, consecutive CRS positions of the row.  Column indices are
+// requested a group ahead; what is left of a row goes four elements at a time
+// with the surplus ones computed and not stored.
+//
+// The elements of a row are independent, so a long slot is shared out over
+// all groups of a workgroup of its own, the first n_long ones: one group
+// alone took 177 us for the longest rows of a matrix of 20,000 (k = 8, FP64).
+template <typename A, int GL, int Q, bool EXACT>
+__global__ __launch_bounds__(256) void scs_sddmm_rows(SddmmArgs a, const A *__restrict__ Gm,
+                                                      const A *__restrict__ X,
+                                                      A *__restrict__ dvals) {
+    constexpr int U = kSddmmChainGroup<GL>;
+    constexpr int kSlots = 256 / GL;  // groups of a workgroup
+    const int l = static_cast<int>(threadIdx.x) % GL, group = static_cast<int>(threadIdx.x) / GL;
+    const int64_t C = a.C;
+    int64_t slot, base;
+    int j = 0, end;
+    if (blockIdx.x < a.n_long) {
+        const int64_t i = blockIdx.x;
+        slot = a.long_list[i < a.long_whole ? i : a.long_cap - 1 - (i - a.long_whole)];
+        const int64_t c = slot / C;
+        base = static_cast<int64_t>(a.chunk_ptr[c]) + (slot - c * C);
+        const int len = a.slot_len[slot];
+        const int part = (len + kSlots - 1) / kSlots;
+        j = group * part;
+        end = j + part < len ? j + part : len;
+        if (j >= len) return;  // whole groups
     } else {
-        pos = blockIdx.x / bpc;
-        li = (blockIdx.x % bpc) * 256 + threadIdx.x;
+        const int64_t at = (blockIdx.x - a.n_long) * kSlots + group;
+        if (at >= a.n_slots) return;
+        const int32_t pos = a.by_c(static_cast<int32_t>(at));
+        const int64_t chunk = a.order ? static_cast<int64_t>(a.order[pos]) : pos;
+        const int64_t i = at - pos * C;
+        slot = chunk * C + i;
+        base = static_cast<int64_t>(a.chunk_ptr[chunk]) + i;
+        end = a.slot_len[slot];
+        if (end >= a.long_from || end == 0) return;
     }
-    if (pos >= n_chunks || li >= ck) return;
-    const int64_t chunk = order ? static_cast<int64_t>(order[pos]) : pos;
-    const int64_t i = li / GL;
-    const int l = static_cast<int>(li % GL);
-    const int64_t slot = chunk * C + i;
-    const int32_t r = slot_row[slot];
-    if (r >= n_rows) return;
-    const int len = slot_len[slot];
-    const int64_t base = static_cast<int64_t>(chunk_ptr[chunk]) + i;
-    // SEQ: CRS position of the slot's element 0 (its row start)
-    const int64_t row0 = SEQ && len > 0 ? src[base] : 0;
+    const int64_t r = a.slot_row[slot];
+    if (r >= a.n_rows) return;
+    const int64_t k = a.k;
+    const int64_t v0 = EXACT ? l * Q : run_start<Q>(l, k);
+    const int skip = EXACT ? 0 : l * Q < k ? static_cast<int>(l * Q - v0) : Q;
+    const int64_t row0 = a.seq ? a.src[base] : 0;  // the row's first CRS position
     A g[Q];
-    load_run<A, Q>(Gm + static_cast<int64_t>(r) * K + l * Q, g);
-    int j = 0;
-    if (len >= U) {
-        // kPer lanes hold each result, each lane holds kNpl results: lane l
-        // stores elements n*GL + l/kPer (n < kNpl) of each group of U
-        constexpr int kPer = GL >= U ? GL / U : 1;
-        constexpr int kNpl = GL >= U ? 1 : U / GL;
-        const int lane_elem = l / kPer;
-        const bool stores = l % kPer == 0;
-        int32_t c0[U], s0[kNpl];
+    load_cols_run<A, Q>(Gm + r * k + v0, g);
+    const A *xcol = X + v0;
+    // m of the UU elements from position p on, with columns c
+    const auto elements = [&](auto uu, int p, int m, const int32_t *c) {
+        constexpr int UU = decltype(uu)::value;
+        // kPer lanes hold each result, each lane holds kNpl results
+        constexpr int kPer = GL >= UU ? GL / UU : 1;
+        constexpr int kNpl = GL >= UU ? 1 : UU / GL;
+        const int mine = l / kPer;
+        int64_t to[kNpl];
 #pragma unroll
-        for (int u = 0; u < U; ++u) c0[u] = col[base + u * C];
+        for (int n = 0; n < kNpl; ++n) {
+            const int e = n * GL + mine;
+            to[n] = -1;
+            if (l % kPer == 0 && e < m)
+                to[n] = a.seq ? row0 + p + e : a.src[base + static_cast<int64_t>(p + e) * C];
+        }
+        A xv[UU][Q];
 #pragma unroll
-        for (int n = 0; n < kNpl; ++n)
-            s0[n] = SEQ ? 0 : src[base + static_cast<int64_t>(n * GL + lane_elem) * C];
-        for (;;) {
-            const bool more = j + 2 * U <= len;
-            int32_t c1[U], s1[kNpl];
-            if (more) {
+        for (int u = 0; u < UU; ++u)
+            load_cols_run<A, Q>(xcol + static_cast<int64_t>(c[u]) * k, xv[u]);
+        A part[UU];
+#pragma unroll
+        for (int u = 0; u < UU; ++u) {
+            A acc = 0;
+#pragma unroll
+            for (int t = 0; t < Q; ++t) {
+                const A next = __builtin_elementwise_fma(g[t], xv[u][t], acc);
+                acc = EXACT || t >= skip ? next : acc;
+            }
+            part[u] = acc;
+        }
+        if constexpr (GL >= UU) {
+            const A sum = group_reduce_scatter<GL, UU>(part, l);
+            if (to[0] >= 0) dvals[to[0]] = sum;
+        } else {
+#pragma unroll
+            for (int n = 0; n < kNpl; ++n) {
+                A piece[GL];
+#pragma unroll
+                for (int i = 0; i < GL; ++i) piece[i] = part[n * GL + i];
+                const A sum = group_reduce_scatter<GL, GL>(piece, l);
+                if (to[n] >= 0) dvals[to[n]] = sum;
+            }
+        }
+    };
+    const int full = j + (end - j) / U * U;
+    if (j < full) {
+        int32_t c0[U], c1[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) c0[u] = a.col[base + static_cast<int64_t>(j + u) * C];
+        for (; j < full; j += U) {
+            if (j + U < full)
 #pragma unroll
                 for (int u = 0; u < U; ++u)
-                    c1[u] = col[base + static_cast<int64_t>(j + U + u) * C];
-#pragma unroll
-                for (int n = 0; n < kNpl; ++n)
-                    s1[n] = SEQ ? 0
-                                : src[base + static_cast<int64_t>(j + U + n * GL + lane_elem) * C];
-            }
-            A xv[U][Q];
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                load_run<A, Q>(X + static_cast<int64_t>(c0[u]) * K + l * Q, xv[u]);
-            A part[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                A acc = 0;
-#pragma unroll
-                for (int t = 0; t < Q; ++t) acc = T::fma_(g[t], xv[u][t], acc);
-                part[u] = acc;
-            }
-            if constexpr (GL >= U) {
-                const A sum = group_reduce_scatter<GL, U>(part, l);
-                if (stores) dvals[SEQ ? row0 + j + lane_elem : s0[0]] = sum;
-            } else {
-#pragma unroll
-                for (int n = 0; n < kNpl; ++n) {
-                    A piece[GL];
-#pragma unroll
-                    for (int i = 0; i < GL; ++i) piece[i] = part[n * GL + i];
-                    dvals[SEQ ? row0 + j + n * GL + lane_elem : s0[n]] =
-                        group_reduce_scatter<GL, GL>(piece, l);
-                }
-            }
-            j += U;
-            if (!more) break;
+                    c1[u] = a.col[base + static_cast<int64_t>(j + U + u) * C];
+            elements(std::integral_constant<int, U>{}, j, U, c0);
 #pragma unroll
             for (int u = 0; u < U; ++u) c0[u] = c1[u];
-            for (int n = 0; n < kNpl; ++n) s0[n] = s1[n];
         }
     }
-    for (; j < len; ++j) {
-        const int64_t e = base + static_cast<int64_t>(j) * C;
-        A xv[Q];
-        load_run<A, Q>(X + static_cast<int64_t>(col[e]) * K + l * Q, xv);
-        A acc = 0;
+    constexpr int R = 4;
+    for (; j < end; j += R) {
+        int32_t c[R];
 #pragma unroll
-        for (int t = 0; t < Q; ++t) acc = T::fma_(g[t], xv[t], acc);
-        acc = group_sum<GL>(acc);
-        if (l == 0) dvals[SEQ ? row0 + j : src[e]] = acc;
+        for (int u = 0; u < R; ++u)
+            c[u] = a.col[base + static_cast<int64_t>(j + u < end ? j + u : end - 1) * C];
+        elements(std::integral_constant<int, R>{}, j, end - j < R ? end - j : R, c);
     }
 }
 
-template <int VT, int K>
-static void launch_sddmm_rows(smax_hip_ctx ctx, smax_hip_scs A, const void *Gm,
+template <typename A, int GL, int Q>
+static void launch_sddmm_rows(smax_hip_ctx ctx, smax_hip_scs S, int64_t k, const void *Gm,
                               const void *X, void *dv) {
-    using T = vt<VT>;
-    const smax_hip_scs_info &in = A->info;
-    const int64_t ck = in.C * sddmm_group(K);
-    const int64_t cpb = ck <= 256 ? 256 / ck : 1;
-    const int64_t bpc = ck <= 256 ? 1 : ceil_div(ck, 256);
-    const int64_t blocks = cpb > 1 ? ceil_div(in.n_chunks, cpb) : in.n_chunks * bpc;
-    // the SpMV's occupancy cap, as for the SpMM, when long chunks lead
-    const unsigned lds =
-        static_cast<unsigned>(A->sched.order_lf ? A->sched.lds_cap_bytes : 0);
-#define SMAX_SDDMM_ROWS(SEQ)                                                               \
-    hipLaunchKernelGGL((scs_sddmm_rows<VT, K, SEQ>), dim3(static_cast<unsigned>(blocks)), \
-                       dim3(256), lds, ctx->stream, in.C, in.n_chunks, in.n_rows, cpb, bpc, \
-                       in.chunk_ptr, in.slot_len, A->sched.order_lf, in.col, in.slot_row,  \
-                       in.src_index, static_cast<const typename T::vec_t *>(Gm),           \
-                       static_cast<const typename T::vec_t *>(X),                          \
-                       static_cast<typename T::vec_t *>(dv))
-    if (A->src_consecutive)
-        SMAX_SDDMM_ROWS(true);
-    else
-        SMAX_SDDMM_ROWS(false);
+    const smax_hip_scs_info &in = S->info;
+    SddmmArgs a{};
+    a.C = in.C;
+    a.n_slots = in.n_rows_padded;
+    a.n_rows = in.n_rows;
+    a.k = k;
+    a.by_c = fast_div(in.C);
+    a.n_long = S->longs.rows.count;
+    a.long_whole = S->longs.rows.whole;
+    a.long_cap = S->longs.cap;
+    a.long_from = S->longs.from;
+    a.seq = S->src_consecutive;
+    a.long_list = S->longs.list;
+    a.chunk_ptr = in.chunk_ptr;
+    a.slot_len = in.slot_len;
+    a.order = S->sched.order_lf;
+    a.col = in.col;
+    a.slot_row = in.slot_row;
+    a.src = in.src_index;
+    const dim3 grid(static_cast<unsigned>(a.n_long + ceil_div(a.n_slots, 256 / GL)));
+    const auto g = static_cast<const A *>(Gm);
+    const auto x = static_cast<const A *>(X);
+    const auto d = static_cast<A *>(dv);
+    if (k == GL * Q)
+        hipLaunchKernelGGL((scs_sddmm_rows<A, GL, Q, true>), grid, dim3(256), 0, ctx->stream, a, g,
+                           x, d);
+    else if constexpr (GL > 1)
+        hipLaunchKernelGGL((scs_sddmm_rows<A, GL, Q, false>), grid, dim3(256), 0, ctx->stream, a,
+                           g, x, d);
+}
+
+// sddmm_group(k) and sddmm_run(k) as template arguments, 1 <= k <= 256.
+template <typename A>
+static void sddmm_rows(smax_hip_ctx ctx, smax_hip_scs S, int64_t k, const void *Gm, const void *X,
+                       void *dv) {
+#define SMAX_SDDMM_ROWS(GL)                                                                \
+    case GL:                                                                               \
+        if (sddmm_run(k) == 3) launch_sddmm_rows<A, GL, 3>(ctx, S, k, Gm, X, dv);          \
+        else launch_sddmm_rows<A, GL, 4>(ctx, S, k, Gm, X, dv);                            \
+        break;
+    switch (sddmm_group(k)) {
+        SMAX_SDDMM_ROWS(2)
+        SMAX_SDDMM_ROWS(4)
+        SMAX_SDDMM_ROWS(8)
+        SMAX_SDDMM_ROWS(16)
+        SMAX_SDDMM_ROWS(32)
+        SMAX_SDDMM_ROWS(64)
+    default:  // one lane: k <= 4
+        if (k == 1) launch_sddmm_rows<A, 1, 1>(ctx, S, k, Gm, X, dv);
+        else if (k == 2) launch_sddmm_rows<A, 1, 2>(ctx, S, k, Gm, X, dv);
+        else if (k == 3) launch_sddmm_rows<A, 1, 3>(ctx, S, k, Gm, X, dv);
+        else launch_sddmm_rows<A, 1, 4>(ctx, S, k, Gm, X, dv);
+        break;
+    }
 #undef SMAX_SDDMM_ROWS
-}
-
-template <int VT>
-static bool sddmm_rows(smax_hip_ctx ctx, smax_hip_scs A, int64_t k, const void *Gm,
-                       const void *X, void *dv) {
-    switch (k) {
-    case 1: launch_sddmm_rows<VT, 1>(ctx, A, Gm, X, dv); return true;
-    case 2: launch_sddmm_rows<VT, 2>(ctx, A, Gm, X, dv); return true;
-    case 4: launch_sddmm_rows<VT, 4>(ctx, A, Gm, X, dv); return true;
-    case 8: launch_sddmm_rows<VT, 8>(ctx, A, Gm, X, dv); return true;
-    case 16: launch_sddmm_rows<VT, 16>(ctx, A, Gm, X, dv); return true;
-    case 32: launch_sddmm_rows<VT, 32>(ctx, A, Gm, X, dv); return true;
-    case 64: launch_sddmm_rows<VT, 64>(ctx, A, Gm, X, dv); return true;
-    default: return false;
-    }
-}
-
-template <int VT, int G>
-static void launch_sddmm_g(smax_hip_ctx ctx, const smax_hip_scs_info &in,
-                           const int32_t *elem_row, int64_t k, const void *Gm,
-                           const void *X, void *dv) {
-    using T = vt<VT>;
-    hipLaunchKernelGGL((scs_sddmm_kernel<VT, G>), grid_for(in.n_elements * G, 256),
-                       dim3(256), 0, ctx->stream, in.n_elements, k, in.col, elem_row,
-                       in.src_index, static_cast<const typename T::vec_t *>(Gm),
-                       static_cast<const typename T::vec_t *>(X),
-                       static_cast<typename T::vec_t *>(dv));
-}
-
-template <int VT>
-static int launch_sddmm(smax_hip_ctx ctx, const smax_hip_scs_info &in,
-                        const int32_t *elem_row, int64_t k, int g, const void *Gm,
-                        const void *X, void *dv) {
-    switch (g) {
-    case 1: launch_sddmm_g<VT, 1>(ctx, in, elem_row, k, Gm, X, dv); break;
-    case 2: launch_sddmm_g<VT, 2>(ctx, in, elem_row, k, Gm, X, dv); break;
-    case 4: launch_sddmm_g<VT, 4>(ctx, in, elem_row, k, Gm, X, dv); break;
-    case 8: launch_sddmm_g<VT, 8>(ctx, in, elem_row, k, Gm, X, dv); break;
-    case 16: launch_sddmm_g<VT, 16>(ctx, in, elem_row, k, Gm, X, dv); break;
-    case 32: launch_sddmm_g<VT, 32>(ctx, in, elem_row, k, Gm, X, dv); break;
-    default: launch_sddmm_g<VT, 64>(ctx, in, elem_row, k, Gm, X, dv); break;
-    }
-    SMAX_HIP_LAUNCHED(ctx, "scs_sddmm_kernel");
-    return SMAX_HIP_SUCCESS;
 }
 
 }  // namespace smaxhip
@@ -396,16 +395,11 @@ int smax_hip_scs_sddmm(smax_hip_ctx ctx, int value_type, smax_hip_scs A,
         return fail(ctx, SMAX_HIP_ERROR_OVERFLOW,
                     "smax_hip_scs_sddmm: k = %lld exceeds the launch limits", (long long)k);
     if (in.n_elements == 0) return SMAX_HIP_SUCCESS;
-    // the row kernel's 16-byte loads need 16-byte aligned G and X rows
-    const int64_t run_bytes = sddmm_run(k) * (value_type == SMAX_HIP_F64 ? 8 : 4);
-    const bool aligned = run_bytes % 16 != 0 || aligned16(G, X);
-    if (aligned && (k & (k - 1)) == 0 && k <= 64 && in.C * sddmm_group(k) <= INT32_MAX) {
-        bool done = false;
-        SMAX_HIP_DISPATCH_VT(value_type, done = sddmm_rows<VT>(ctx, A, k, G, X, dvals));
-        if (done) {
-            SMAX_HIP_LAUNCHED(ctx, "scs_sddmm_rows");
-            return SMAX_HIP_SUCCESS;
-        }
+    if (k <= 256) {
+        if (value_type == SMAX_HIP_F64) sddmm_rows<double>(ctx, A, k, G, X, dvals);
+        else sddmm_rows<float>(ctx, A, k, G, X, dvals);
+        SMAX_HIP_LAUNCHED(ctx, "scs_sddmm_rows");
+        return SMAX_HIP_SUCCESS;
     }
     if (!A->elem_row) {
         int rc = dev_alloc(ctx, reinterpret_cast<void **>(&A->elem_row),
@@ -416,11 +410,19 @@ int smax_hip_scs_sddmm(smax_hip_ctx ctx, int value_type, smax_hip_scs A,
                            in.chunk_lengths, in.slot_len, in.slot_row, A->elem_row);
         SMAX_HIP_LAUNCHED(ctx, "k_elem_row");
     }
-    const int g = static_cast<int>(sddmm_group(k));
-    SMAX_HIP_DISPATCH_VT(value_type,
-                         return launch_sddmm<VT>(ctx, in, A->elem_row, k, g, G, X,
-                                                 dvals));
-    return SMAX_HIP_ERROR_UNSUPPORTED;
+    const dim3 grid = grid_for(in.n_elements * kWave, 256);
+    if (value_type == SMAX_HIP_F64)
+        hipLaunchKernelGGL(scs_sddmm_kernel<double>, grid, dim3(256), 0, ctx->stream,
+                           in.n_elements, k, in.col, A->elem_row, in.src_index,
+                           static_cast<const double *>(G), static_cast<const double *>(X),
+                           static_cast<double *>(dvals));
+    else
+        hipLaunchKernelGGL(scs_sddmm_kernel<float>, grid, dim3(256), 0, ctx->stream,
+                           in.n_elements, k, in.col, A->elem_row, in.src_index,
+                           static_cast<const float *>(G), static_cast<const float *>(X),
+                           static_cast<float *>(dvals));
+    SMAX_HIP_LAUNCHED(ctx, "scs_sddmm_kernel");
+    return SMAX_HIP_SUCCESS;
 }
 
 }  // extern "C"

@@ -232,3 +232,40 @@ def test_sddmm_on_transpose_layout_equals_sddmm_on_a(ctx, vt, k):
         d.free()
     S.destroy()
     T.destroy()
+
+
+@pytest.mark.parametrize("vt", [capi.F64, capi.F32])
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 8, 9, 12, 20, 31, 33, 48, 65, 100, 129, 200, 256,
+                               257, 300])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_sddmm_long_rows_and_any_width(ctx, vt, k, transposed):
+    """SDDMM over rows of 0 to 2000 entries (long ones are shared out over a
+    workgroup) for every lane count and run length, exact and partial, with
+    consecutive and scattered destinations (the transposed layout), against
+    binary64 (binary128 for FP64) sums: g lanes' chains of q terms and a
+    butterfly, so |d - d_exact| <= (q + log2 g) u sum |g x|."""
+    rng = np.random.default_rng(k)
+    L = rng.integers(0, 4, 700)
+    L[[0, 5, 6, 7, 8, 300, 301, 302, 699]] = [2000, 127, 128, 129, 0, 511, 513, 1025, 640]
+    L[10:26] = np.arange(1, 17)
+    n_cols = 2500
+    rp = np.concatenate([[0], np.cumsum(L)]).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(n_cols, l, replace=False)) for l in L]).astype(np.int32)
+    vec = np.float64 if vt == capi.F64 else np.float32
+    rows = np.repeat(np.arange(L.size), L)
+    G = rng.uniform(-1, 1, (L.size, k)).astype(vec)
+    X = rng.uniform(-1, 1, (n_cols, k)).astype(vec)
+    d = [ctx.upload(a) for a in (rp, col, np.zeros(rp[-1], vec), G, X)]
+    dv = ctx.upload(np.full(rp[-1], 7, vec))
+    build = ctx.scs_transpose_from_crs if transposed else ctx.scs_from_crs
+    S = build(L.size, n_cols, int(rp[-1]), d[0], d[1], d[2], vec().itemsize, 64, 512)
+    S.sddmm(vt, k, d[4] if transposed else d[3], d[3] if transposed else d[4], dv)
+    wide = np.longdouble if vt == capi.F64 else np.float64
+    t = G.astype(wide)[rows] * X.astype(wide)[col]
+    p = 1 << (k - 1).bit_length()
+    g = min(max(p // 4, 1), 64)
+    bound = (-(-k // g) + np.log2(g)) * np.finfo(vec).eps / 2 * np.abs(t).sum(1)
+    assert (np.abs(ctx.download(dv) - t.sum(1)) <= bound).all()
+    for a in (*d, dv):
+        a.free()
+    S.destroy()
