@@ -8,8 +8,8 @@
 //  * sequential: one lane per row reading straight from HBM (the reference's
 //    CUDA schedule, spmv_cuda_crs_impl.cu:5-22);
 //  * blocked: a plan cuts the rows into row blocks of at most T rows whose
-//    first nonzeros fall in one W-entry window; rows of 512 or more nonzeros
-//    form a block of their own.  Each workgroup of T threads streams its
+//    first nonzeros fall in one W-entry window; a long row (kCrsLongRow)
+//    forms a block of its own.  Each workgroup of T threads streams its
 //    block's values and column indices through LDS in coalesced W-entry tiles
 //    (gathering x on the way), and each row's lane then runs its fma chain out
 //    of LDS.  Short rows are thereby reduced lane-per-row while the loads stay
@@ -18,10 +18,10 @@
 //    band of neighbouring blocks is shared in one L2.  Two geometries:
 //    T = 256, W = 1024 for rows of even length, and single-wave blocks,
 //    T = 64, W = 512, when the longest row exceeds 4x the mean: a wave then
-//    waits at its own tiles' barriers only (4M-row band matrix, FP64:
-//    0.692 ms against 0.766; BF16 values 0.512 against 0.692; the 512^2
-//    Laplacian and a 27-point stencil run 6.0 / 25.5 us with the wide blocks
-//    against 6.5 / 28.2 us).
+//    waits at its own tiles' barriers only and pipelines its long rows (4M-row
+//    band matrix, FP64: 0.666 ms against 0.766; BF16 values 0.454 against
+//    0.692; the 512^2 Laplacian and a 27-point stencil run 6.0 / 25.5 us with
+//    the wide blocks against 6.5 / 28.2 us).
 #include <algorithm>
 #include <cmath>
 #include <mutex>
@@ -42,7 +42,12 @@ struct smax_hip_crs_plan_s {
 namespace smaxhip {
 
 constexpr int kCrsThreads = 256;
-constexpr int kCrsLongRow = 512;     // rows at least this long stream alone
+// Rows at least this long form a block of their own, by threads per block:
+// with one wavefront they then take long_row_sum (from 128 on: 1,000,000 rows
+// 150 us, from 256: 140, from 512: 147), with four a shorter one is done by
+// its thread while the other rows' threads run.
+template <int NT>
+constexpr int kCrsLongRow = NT == kWave ? 256 : 512;
 // row-block geometries: threads per block (= rows at most) and the tile and
 // block-start window in nonzeros
 constexpr int kBlkWideThreads = 256, kBlkWideTile = 1024;
@@ -82,6 +87,86 @@ __global__ __launch_bounds__(kCrsThreads) void crs_spmv_lane(
 }
 
 // ------------------------------------------------------------ blocked
+// One long row by one wavefront: tiles of TILE entries (half the arrays) go
+// through LDS as in crs_spmv_blocked, but the next tile's columns, values and
+// x entries are requested while this one's chain runs, and the chain reads LDS
+// 32 bytes ahead of its fmas instead of waiting for each entry's read.  What
+// bounds it is that chain, one fma after another in the row's order: 100+
+// cycles an entry when each waits, 31 (FP64) now.  Every lane runs the same
+// chain (broadcast reads).  20,000 rows with rows of up to 2000, FP64: 91 ->
+// 28 us; 300,007 rows, BF16: 117 -> 49; 4,000,000, FP64: 729 -> 666.  Tiles
+// of 512 need the registers of one more wavefront per SIMD (BF16, 4,000,000
+// rows: 482 us against 454), of 128 expose more of the gathers (FP64, 300,007:
+// 64 against 61); 64 bytes ahead take 25 us at 20,000 rows but 678 at
+// 4,000,000.
+template <typename A>
+constexpr int kChainAhead = 32 / static_cast<int>(sizeof(A));
+
+template <int VT, int TILE>
+__device__ __forceinline__ typename vt<VT>::vec_t long_row_sum(
+    typename vt<VT>::vec_t *sv, typename vt<VT>::vec_t *sx, int64_t s, int64_t e,
+    const int32_t *__restrict__ col, const typename vt<VT>::val_t *__restrict__ val,
+    const typename vt<VT>::vec_t *__restrict__ x) {
+    using T = vt<VT>;
+    using A = typename T::vec_t;
+    constexpr int PER = TILE / kWave, U = kChainAhead<A>;
+    const int tid = static_cast<int>(threadIdx.x);
+    int32_t c[PER];
+    typename T::val_t v[PER];
+    A xv[PER];
+    const auto load_columns = [&](int64_t t0) {
+#pragma unroll
+        for (int u = 0; u < PER; ++u)
+            if (t0 + tid + u * kWave < e) c[u] = ld_stream(col + t0 + tid + u * kWave);
+    };
+    const auto gather = [&](int64_t t0) {
+#pragma unroll
+        for (int u = 0; u < PER; ++u)
+            if (t0 + tid + u * kWave < e) {
+                v[u] = ld_stream(val + t0 + tid + u * kWave);
+                xv[u] = x[c[u]];
+            }
+    };
+    load_columns(s);
+    gather(s);
+    load_columns(s + TILE);
+    A acc = 0;
+    for (int64_t t0 = s; t0 < e; t0 += TILE) {
+#pragma unroll
+        for (int u = 0; u < PER; ++u)
+            if (t0 + tid + u * kWave < e) {
+                sv[tid + u * kWave] = T::widen(v[u]);
+                sx[tid + u * kWave] = xv[u];
+            }
+        __syncthreads();
+        if (t0 + TILE < e) {
+            gather(t0 + TILE);
+            load_columns(t0 + 2 * TILE);
+        }
+        const int nt = static_cast<int>(e - t0 < TILE ? e - t0 : TILE);
+        const int full = nt & ~(2 * U - 1);
+        A w0[U], b0[U], w1[U], b1[U];
+        load_run<A, U>(sv, w0);
+        load_run<A, U>(sx, b0);
+        for (int j = 0; j < full; j += 2 * U) {
+            load_run<A, U>(sv + j + U, w1);
+            load_run<A, U>(sx + j + U, b1);
+            __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the fmas
+#pragma unroll
+            for (int u = 0; u < U; ++u) acc = T::fma_(w0[u], b0[u], acc);
+            // The last pass reads U entries past the tile, of the arrays' other half.
+            load_run<A, U>(sv + j + 2 * U, w0);
+            load_run<A, U>(sx + j + 2 * U, b0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < U; ++u) acc = T::fma_(w1[u], b1[u], acc);
+        }
+        for (int j = full; j < nt; ++j) acc = T::fma_(sv[j], sx[j], acc);
+        __syncthreads();
+    }
+    return acc;
+}
+
 template <int VT, int NT, int TILE>
 __global__ __launch_bounds__(NT) void crs_spmv_blocked(
     const int32_t *__restrict__ block_start,
@@ -91,12 +176,19 @@ __global__ __launch_bounds__(NT) void crs_spmv_blocked(
     typename vt<VT>::vec_t *__restrict__ y) {
     using T = vt<VT>;
     using A = typename T::vec_t;
-    __shared__ A sv[TILE];
-    __shared__ A sx[TILE];
+    __shared__ __align__(16) A sv[TILE];
+    __shared__ __align__(16) A sx[TILE];
     const int tid = threadIdx.x;
     const int64_t b = xcd_block(blockIdx.x, gridDim.x);
     const int64_t r0 = block_start[b], r1 = block_start[b + 1];
     const int64_t s = row_ptr[r0], e = row_ptr[r1];
+    if constexpr (NT == kWave) {
+        if (r1 - r0 == 1 && e - s >= kCrsLongRow<NT>) {
+            const A sum = long_row_sum<VT, TILE / 2>(sv, sx, s, e, col, val, x);
+            if (tid == 0) y[r0] = sum;
+            return;
+        }
+    }
     const int64_t row = r0 + tid;
     const bool has = row < r1;
     const int64_t rs = has ? row_ptr[row] : 0, re = has ? row_ptr[row + 1] : 0;
@@ -138,13 +230,14 @@ __global__ __launch_bounds__(NT) void crs_spmv_blocked(
 // threads), when r's first nonzero enters a new window of `window` entries,
 // or when r or r-1 is a long row.
 __global__ void crs_block_flags(int64_t n_rows, const int32_t *__restrict__ row_ptr,
-                                int32_t *__restrict__ flag, int32_t nt, int32_t window) {
+                                int32_t *__restrict__ flag, int32_t nt, int32_t window,
+                                int32_t long_row) {
     const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (r >= n_rows) return;
     int32_t f = 1;
     if (r % nt != 0) {
         const int32_t a = row_ptr[r - 1], b = row_ptr[r], c = row_ptr[r + 1];
-        f = (a / window != b / window) || (b - a >= kCrsLongRow) || (c - b >= kCrsLongRow);
+        f = (a / window != b / window) || (b - a >= long_row) || (c - b >= long_row);
     }
     flag[r] = f;
 }
@@ -637,6 +730,8 @@ int smax_hip_crs_plan_create(smax_hip_ctx ctx, int64_t n_rows, int64_t nnz,
                         4.0 * static_cast<double>(nnz) / static_cast<double>(n_rows);
     const int32_t nt = narrow ? kBlkNarrowThreads : kBlkWideThreads;
     const int32_t window = narrow ? kBlkNarrowTile : kBlkWideTile;
+    const int32_t long_row =
+        narrow ? kCrsLongRow<kBlkNarrowThreads> : kCrsLongRow<kBlkWideThreads>;
     int32_t *flag = nullptr, *tmp = nullptr, *starts = nullptr;
     int rc = dev_alloc(ctx, reinterpret_cast<void **>(&flag),
                        sizeof(int32_t) * n_rows, "crs plan");
@@ -649,7 +744,7 @@ int smax_hip_crs_plan_create(smax_hip_ctx ctx, int64_t n_rows, int64_t nnz,
     int64_t n_blocks = 0;
     if (!rc) {
         hipLaunchKernelGGL(crs_block_flags, grid_for(n_rows, 256), dim3(256), 0,
-                           ctx->stream, n_rows, row_ptr, flag, nt, window);
+                           ctx->stream, n_rows, row_ptr, flag, nt, window, long_row);
         rc = check_launch(ctx, "crs_block_flags");
     }
     // flag -> inclusive positions (in place); tmp is the scan scratch.
@@ -669,7 +764,7 @@ int smax_hip_crs_plan_create(smax_hip_ctx ctx, int64_t n_rows, int64_t nnz,
                        sizeof(int32_t) * n_rows, "crs plan");
         if (!rc) {
             hipLaunchKernelGGL(crs_block_flags, grid_for(n_rows, 256), dim3(256),
-                               0, ctx->stream, n_rows, row_ptr, flag2, nt, window);
+                               0, ctx->stream, n_rows, row_ptr, flag2, nt, window, long_row);
             rc = check_launch(ctx, "crs_block_flags");
         }
         if (!rc) {

@@ -104,6 +104,30 @@ def test_crs_spmv_long_and_empty_rows(ctx, vt):
 
 
 @pytest.mark.parametrize("vt", VTS)
+@pytest.mark.parametrize("first", [0, 1])
+def test_crs_spmv_pipelined_long_rows(ctx, vt, first):
+    """Planned row blocks of one wavefront: rows around the length from which
+    one has a block of its own (256), around whole tiles of it and around the
+    entries its chain takes at once, behind 0 or 1 rows of odd length."""
+    rng = np.random.default_rng(12)
+    n = 3000
+    longs = [255, 256, 257, 259, 263, 264, 265, 271, 272, 273, 511, 512, 513, 520,
+             527, 767, 768, 769, 1024, 1031, 1536, 2999, 3000]
+    L = rng.integers(0, 4, n)
+    L[0] = 3 * first
+    L[1:1 + 5 * len(longs):5] = longs
+    L[-1] = 300
+    assert L.max() > 4 * L.mean()
+    rp = np.concatenate([[0], np.cumsum(L)]).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(n, l, replace=False)) for l in L]
+                         ).astype(np.int32)
+    A = Csr(n, n, rp, col, rng.uniform(-1, 1, rp[-1]))
+    val, x = operands(vt, A)
+    assert_bitwise(run_spmv(ctx, vt, A, val, x, True),
+                   oracle.crs_spmv(A.row_ptr, A.col, val, x))
+
+
+@pytest.mark.parametrize("vt", VTS)
 @pytest.mark.parametrize("k", [1, 4, 8, 32, 64])
 @pytest.mark.parametrize("row_major", [True, False])
 @pytest.mark.parametrize("planned", [False, True])
