@@ -16,6 +16,14 @@ struct smax_hip_scs_sched {
     // Dynamic LDS reserved by the C = 64 (and C = 32) SpMV launch to cap its
     // occupancy (0 = no cap).
     int64_t lds_cap_bytes = 0;
+    // C = 64 and C = 32 SpMV by slot lengths: the chunks of long_from columns
+    // and more by whole workgroups, a chunk's entry for each of its parts, dealt
+    // to the XCDs as `order` is (entry i on XCD i % 8; -1 = none); long_blocks =
+    // 0: none.  The list follows `order` in its allocation.
+    const int32_t *long_chunks = nullptr;
+    int64_t long_blocks = 0;
+    int32_t long_from = 0;
+    int32_t long_share = 0;
     // Longest chunk (-1: unknown).  Layouts whose chunks all fit one short
     // group run the C = 64 SpMV's single-group chains.
     int32_t max_chunk_len = -1;
@@ -40,6 +48,11 @@ struct smax_hip_scs_tails {
     int64_t n_blocks = 0;     // workgroups of tail waves (a multiple of 8; 0: none)
     int64_t n_elements = 0;   // storage of col / val
     int64_t n_slots = 0, n_waves = 0;
+    // The first n_wide waves, the longest, run by whole workgroups (as the
+    // schedule's long chunks; their list follows `slot` in its allocation).
+    const int32_t *wide = nullptr;
+    int64_t wide_blocks = 0;
+    int32_t n_wide = 0, share = 0;
 };
 
 // Long slots of a converted layout, for the SpMM: slots of `from` entries and

@@ -39,6 +39,30 @@ constexpr int kScsPipeUnroll = VT == SMAX_HIP_BF16 ? 8 : VT == SMAX_HIP_F32 ? 16
 // 7.16 -> 5.98 us kernel time; back to back 4.56 -> 4.68 us.
 constexpr int kShortChain = 8;
 
+template <int VT>
+__device__ __forceinline__ typename vt<VT>::vec_t
+slot_chain_short(const int32_t *__restrict__ col, const typename vt<VT>::val_t *__restrict__ val,
+                 const typename vt<VT>::vec_t *__restrict__ x, int64_t base, int len) {
+    using T = vt<VT>;
+    int32_t c[kShortChain];
+    typename T::val_t v[kShortChain];
+#pragma unroll
+    for (int u = 0; u < kShortChain; ++u)
+        if (u < len) {
+            c[u] = ld_stream(col + base + u * kWave);
+            v[u] = ld_stream(val + base + u * kWave);
+        }
+    typename T::vec_t xv[kShortChain];
+#pragma unroll
+    for (int u = 0; u < kShortChain; ++u)
+        if (u < len) xv[u] = x[c[u]];
+    typename T::vec_t acc = 0;
+#pragma unroll
+    for (int u = 0; u < kShortChain; ++u)
+        if (u < len) acc = T::fma_(T::widen(v[u]), xv[u], acc);
+    return acc;
+}
+
 // One slot's chain in groups of U: the next group's column indices and
 // values are requested before this group's x gathers (software pipelining),
 // so a long chain waits about one memory round trip per group instead of
@@ -97,6 +121,208 @@ slot_chain_pipe(const int32_t *__restrict__ col,
     return acc;
 }
 
+// A long chunk by a whole workgroup.  A chunk's longest rows are one lane's
+// chain each: by a wavefront, the chunk takes a memory round trip for every U
+// columns, with ever fewer of its lanes still at work.  Here all 256 threads
+// gather a tile of kLongTile entries, request the next tile's while its first
+// wavefront runs the chains out of LDS, and a tile's columns are as many as
+// its lanes that are still live leave room for (64 lanes: 32 columns, 5 lanes:
+// 256), each lane's entries side by side in LDS.  What is past a row's end is
+// stored as -0 * 0, which leaves every accumulator as it is, signed zeros
+// included.  Bound by the longest row's chain (up to some 100,000 rows) and by
+// the gathers beyond; rows of up to 2000 entries in a band, before and after:
+//   SELL-64-4096, FP64     20,000 rows   71 ->  36 us, 1,000,000  241 -> 169 us
+//   SELL-64-4096, BF16    300,007       174 ->  66
+//   SELL-64-65536, FP64   300,007       210 ->  70,    4,000,000  698 -> 680
+//   SELL-64-64, FP64       20,000       210 ->  37,    4,000,000 1124 -> 1066
+//   SELL-32-64, FP64      100,000       305 ->  52
+// Tiles of 1024: 300,007 rows at sigma = 65536 7% slower.
+constexpr int kLongTile = 2048;
+// A long chunk's lanes are split between up to kLongParts workgroups, as many
+// (a power of two) as leave each `share` entries or more.
+constexpr int kLongParts = 8;
+__host__ __device__ __forceinline__ int long_parts(int64_t entries, int64_t share) {
+    int parts = 1;
+    while (parts < kLongParts && 2 * parts * share <= entries) parts *= 2;
+    return parts;
+}
+
+template <int VT>
+struct LongChunk {
+    using A = typename vt<VT>::vec_t;
+    static constexpr int kAhead = 32 / static_cast<int>(sizeof(A));  // chain's LDS reads
+    static constexpr int kPad = 16 / static_cast<int>(sizeof(A));    // between lanes' runs
+    static constexpr int kStore = kLongTile + kWave * kPad + kAhead;
+    static constexpr int64_t kBytes = 2 * static_cast<int64_t>(sizeof(A)) * kStore;
+};
+
+// Columns j0 .. j0 + cols of the chunk for the lanes whose rows reach past j0.
+struct LongTile {
+    int32_t j0, cols, live;  // live: how many lanes
+    int32_t shift;           // cols = kLongTile >> shift
+    int32_t src, left;       // this thread's lane of the chunk, its row's entries from j0 on
+    int32_t row;             // the lane's place among the live ones, as a chain
+};
+
+template <int CS>
+__device__ __forceinline__ LongTile long_tile(int32_t j0, int32_t len) {
+    const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+    uint64_t live = __ballot(len > j0);
+    if constexpr (CS < kWave) live &= (1ull << CS) - 1;
+    LongTile t;
+    t.j0 = j0;
+    t.live = __popcll(live);
+    t.shift = t.live > 1 ? 32 - __clz(t.live - 1) : 0;
+    t.cols = kLongTile >> t.shift;
+    t.row = __popcll(live & ((1ull << lane) - 1));
+    // lane -> place, the others behind: a permutation of the wavefront
+    const int to = (live >> lane) & 1 ? t.row : t.live + lane - t.row;
+    const int from = __builtin_amdgcn_ds_permute(to * 4, lane);
+    const int s = static_cast<int>(threadIdx.x) & ((1 << t.shift) - 1);
+    t.src = __shfl(from, s);
+    const int32_t n = __shfl(len, t.src);
+    t.left = s < t.live ? n - j0 : 0;
+    return t;
+}
+
+template <int VT, int CS>
+__device__ __forceinline__ typename vt<VT>::vec_t long_chunk(
+    typename vt<VT>::vec_t *__restrict__ lds, const int32_t *__restrict__ col,
+    const typename vt<VT>::val_t *__restrict__ val,
+    const typename vt<VT>::vec_t *__restrict__ x, int64_t base, int32_t len) {
+    using T = vt<VT>;
+    using A = typename T::vec_t;
+    using L = LongChunk<VT>;
+    constexpr int PER = kLongTile / kScsThreads, U = L::kAhead;
+    A *const sv = lds, *const sx = lds + L::kStore;
+    const int tid = static_cast<int>(threadIdx.x);
+    int32_t c[PER];
+    typename T::val_t v[PER];
+    A xv[PER];
+    const auto at = [&](const LongTile &t, int u) {
+        return (tid >> t.shift) + u * (kScsThreads >> t.shift);
+    };
+    const auto load_columns = [&](const LongTile &t) {
+        const int32_t *p = col + base + static_cast<int64_t>(t.j0) * CS + t.src;
+#pragma unroll
+        for (int u = 0; u < PER; ++u)
+            if (at(t, u) < t.left) c[u] = ld_stream(p + at(t, u) * CS);
+    };
+    const auto gather = [&](const LongTile &t) {
+        const typename T::val_t *p = val + base + static_cast<int64_t>(t.j0) * CS + t.src;
+#pragma unroll
+        for (int u = 0; u < PER; ++u)
+            if (at(t, u) < t.left) {
+                v[u] = ld_stream(p + at(t, u) * CS);
+                xv[u] = x[c[u]];
+            }
+    };
+    A acc = 0;
+    LongTile t = long_tile<CS>(0, len);
+    load_columns(t);
+    gather(t);
+    LongTile next = long_tile<CS>(t.j0 + t.cols, len);
+    load_columns(next);
+    while (t.live > 0) {
+        const int run = t.cols + L::kPad;
+        const int own = (tid & ((1 << t.shift) - 1)) * run;
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+            const bool in = at(t, u) < t.left;
+            sv[own + at(t, u)] = in ? T::widen(v[u]) : A(-0.0);
+            sx[own + at(t, u)] = in ? xv[u] : A(0);
+        }
+        __syncthreads();
+        const LongTile now = t;
+        t = next;
+        if (t.live > 0) {
+            gather(t);
+            next = long_tile<CS>(t.j0 + t.cols, len);
+            load_columns(next);
+        }
+        if (tid < CS && len > now.j0) {
+            const A *pv = sv + now.row * run, *px = sx + now.row * run;
+            const int m = len - now.j0 < now.cols ? len - now.j0 : now.cols;
+            A w0[U], b0[U], w1[U], b1[U];
+            load_run<A, U>(pv, w0);
+            load_run<A, U>(px, b0);
+            // Up to 2U - 1 entries past the row's end are -0 * 0; the last
+            // pass reads U entries more.
+            for (int j = 0; j < m; j += 2 * U) {
+                load_run<A, U>(pv + j + U, w1);
+                load_run<A, U>(px + j + U, b1);
+                __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the fmas
+#pragma unroll
+                for (int u = 0; u < U; ++u) acc = T::fma_(w0[u], b0[u], acc);
+                load_run<A, U>(pv + j + 2 * U, w0);
+                load_run<A, U>(px + j + 2 * U, b0);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < U; ++u) acc = T::fma_(w1[u], b1[u], acc);
+            }
+        }
+        __syncthreads();
+    }
+    return acc;
+}
+
+// The launch's long chunks (see smax_hip_scs_sched), or with tails its long
+// tail waves (smax_hip_scs_tails).
+struct LongChunks {
+    const int32_t *list;  // kLongParts * chunk + part, -1: none
+    int64_t blocks;
+    int32_t from;   // chunks of this length and more, tail waves before this one
+    int32_t share;  // entries that a part has at least
+};
+
+// This workgroup's part of a long chunk of CS lanes: true if there is one and
+// the thread's lane of it is among them; `len` is then its row's length, 0 on
+// the other lanes.  Every thread of the workgroup comes here.
+template <int CS>
+__device__ __forceinline__ bool long_part(int32_t part, int32_t share, int32_t &len, bool &any) {
+    const int lane = static_cast<int>(threadIdx.x) & (CS - 1);
+    int64_t entries = len;
+#pragma unroll
+    for (int d = 1; d < CS; d *= 2) entries += __shfl_xor(entries, d);
+    const int parts = long_parts(entries, share);
+    any = part < parts;
+    const bool mine = any && lane * parts / CS == part;
+    if (!mine) len = 0;
+    return mine;
+}
+
+// What the SpMV kernels take, in one or two arguments: a launch costs the host
+// time for every argument it copies (small matrices back to back: 3.95 us a
+// product with 17 arguments, 3.70 with these).
+template <int VT>
+struct ScsSpmv {
+    int64_t n_chunks, n_rows;
+    const int32_t *chunk_ptr, *chunk_len, *slot_len, *order, *col;
+    const typename vt<VT>::val_t *val;
+    const int32_t *slot_row;
+    const typename vt<VT>::vec_t *x;
+    typename vt<VT>::vec_t *y;
+};
+
+// Tail waves (t_slot null: none) and long chunks; layouts of short chunks
+// have neither.
+template <int VT, bool SHORT>
+struct ScsParts {
+    const int32_t *t_head, *t_slot;
+    const int64_t *t_ptr;
+    const int32_t *t_col;
+    const typename vt<VT>::val_t *t_val;
+    int64_t t_blocks;
+    LongChunks longs;
+};
+template <int VT>
+struct ScsParts<VT, true> {
+    static constexpr const int32_t *t_head = nullptr, *t_slot = nullptr, *t_col = nullptr;
+    static constexpr const int64_t *t_ptr = nullptr;
+    static constexpr const typename vt<VT>::val_t *t_val = nullptr;
+    static constexpr int64_t t_blocks = 0;
+};
+
 // C == 64: one wavefront per chunk, one lane per slot.
 //   REMAP: XCD-contiguous workgroup order (see xcd_block).
 //   order: optional execution order, wave position -> chunk (-1: idle).
@@ -114,77 +340,99 @@ slot_chain_pipe(const int32_t *__restrict__ col,
 //          kinds of wave run the same chain code on their own arrays;
 //          t_blocks is a multiple of 8, so the chunks' workgroups keep their
 //          XCD alignment.
-template <int VT, bool UNPERM, bool REMAP, bool LEN, bool SHORT>
-__global__ __launch_bounds__(kScsThreads) void scs_spmv_w64(
-    int64_t n_chunks, int64_t n_rows, const int32_t *__restrict__ chunk_ptr,
-    const int32_t *__restrict__ chunk_len, const int32_t *__restrict__ slot_len,
-    const int32_t *__restrict__ order, const int32_t *__restrict__ col,
-    const typename vt<VT>::val_t *__restrict__ val,
-    const int32_t *__restrict__ slot_row,
-    const typename vt<VT>::vec_t *__restrict__ x,
-    typename vt<VT>::vec_t *__restrict__ y, const int32_t *__restrict__ t_head,
-    const int32_t *__restrict__ t_slot, const int64_t *__restrict__ t_ptr,
-    const int32_t *__restrict__ t_col, const typename vt<VT>::val_t *__restrict__ t_val,
-    int64_t t_blocks) {
+//   LONG (LEN only): the first longs.blocks workgroups (again a multiple of
+//          8) run the long chunks or, with tails, the long tail waves; the
+//          wavefronts leave those out.
+//   FP64 is held to 128 registers (4 wavefronts per SIMD; it takes 136 by
+//   itself): SELL-64-64 of 4,000,000 rows 1.16 -> 1.08 ms, SELL-32-4096 0.80
+//   -> 0.78, the 27-point stencil of 64^3 43 -> 29 us.
+template <int VT, bool UNPERM, bool REMAP, bool LEN, bool SHORT, bool LONG>
+__global__ __launch_bounds__(kScsThreads, !SHORT && VT == SMAX_HIP_F64 ? 4 : 1) void scs_spmv_w64(
+    ScsSpmv<VT> a, ScsParts<VT, SHORT> p) {
     using T = vt<VT>;
+    // All of a short layout's arguments at once: fetched as they come up, the
+    // later ones each add a wait (the 512^2 Laplacian, FP64: 4.37 us, not 4.57).
+    if constexpr (SHORT)
+        asm volatile("" ::"s"(a.x), "s"(a.y), "s"(a.slot_row), "s"(a.col), "s"(a.val),
+                     "s"(a.order), "s"(a.chunk_ptr), "s"(a.chunk_len), "s"(a.slot_len));
     const int lane = threadIdx.x & (kWave - 1);
-    const bool tails = !SHORT && LEN && t_slot != nullptr;
+    if constexpr (LONG) {
+        if (static_cast<int64_t>(blockIdx.x) < p.longs.blocks) {
+            extern __shared__ __align__(16) char long_lds[];
+            const int32_t id = p.longs.list[blockIdx.x];
+            if (id < 0) return;
+            const int64_t at = id / kLongParts;
+            const bool tail = p.t_slot != nullptr;
+            const int64_t slot = tail ? p.t_slot[at * kWave + lane] : at * kWave + lane;
+            const int32_t full = slot >= 0 ? a.slot_len[slot] : 0;
+            int32_t len = full;
+            bool any;
+            const bool mine = long_part<kWave>(id % kLongParts, p.longs.share, len, any);
+            if (!any) return;
+            typename T::vec_t acc = long_chunk<VT, kWave>(
+                reinterpret_cast<typename T::vec_t *>(long_lds), tail ? p.t_col : a.col,
+                tail ? p.t_val : a.val, a.x, tail ? p.t_ptr[at] : a.chunk_ptr[at], len);
+            if (!mine || slot < 0 || threadIdx.x >= kWave) return;
+            if (full < a.chunk_len[slot / kWave])
+                acc = T::fma_(T::widen(typename T::val_t(0)), a.x[0], acc);
+            if (!UNPERM) {
+                a.y[slot] = acc;
+            } else if (a.slot_row[slot] < a.n_rows) {
+                a.y[a.slot_row[slot]] = acc;
+            }
+            return;
+        }
+    }
+    const bool tails = !SHORT && LEN && p.t_slot != nullptr;
+    int64_t block = blockIdx.x, blocks = gridDim.x, from = 0;
+    if constexpr (LONG) {
+        block -= p.longs.blocks;
+        blocks -= p.longs.blocks;
+        from = p.longs.from;
+    }
     int64_t slot, base;
     int clen, len;
     const int32_t *cp;
     const typename T::val_t *vp;
-    if (tails && static_cast<int64_t>(blockIdx.x) < t_blocks) {
-        const int64_t w = static_cast<int64_t>(blockIdx.x) * (kScsThreads / kWave) +
-                          threadIdx.x / kWave;
-        const int32_t ts = t_slot[w * kWave + lane];
+    if (tails && block < p.t_blocks) {
+        const int64_t w = block * (kScsThreads / kWave) + threadIdx.x / kWave;
+        if (LONG && w < from) return;
+        const int32_t ts = p.t_slot[w * kWave + lane];
         if (ts < 0) return;
         slot = ts;
-        base = t_ptr[w] + lane;
-        clen = chunk_len[ts / kWave];
-        len = slot_len[ts];
-        cp = t_col;
-        vp = t_val;
+        base = p.t_ptr[w] + lane;
+        clen = a.chunk_len[ts / kWave];
+        len = a.slot_len[ts];
+        cp = p.t_col;
+        vp = p.t_val;
     } else {
-        const int64_t hb = tails ? blockIdx.x - t_blocks : blockIdx.x;
-        const int64_t hn = tails ? gridDim.x - t_blocks : gridDim.x;
+        const int64_t hb = tails ? block - p.t_blocks : block;
+        const int64_t hn = tails ? blocks - p.t_blocks : blocks;
         const int64_t blk = REMAP ? xcd_block(hb, hn) : hb;
         const int64_t pos = blk * (kScsThreads / kWave) + (threadIdx.x / kWave);
-        const int64_t chunk = order ? static_cast<int64_t>(order[pos]) : pos;
-        if (chunk < 0 || chunk >= n_chunks) return;
+        const int64_t chunk = a.order ? static_cast<int64_t>(a.order[pos]) : pos;
+        if (chunk < 0 || chunk >= a.n_chunks) return;
         slot = chunk * kWave + lane;
-        base = static_cast<int64_t>(chunk_ptr[chunk]) + lane;
-        clen = chunk_len[chunk];
-        len = LEN ? slot_len[slot] : clen;
-        if (tails && len > t_head[chunk]) return;
-        cp = col;
-        vp = val;
+        base = static_cast<int64_t>(a.chunk_ptr[chunk]) + lane;
+        clen = a.chunk_len[chunk];
+        if (LONG && !tails && clen >= from) return;
+        len = LEN ? a.slot_len[slot] : clen;
+        if (tails && len > p.t_head[chunk]) return;
+        cp = a.col;
+        vp = a.val;
     }
     typename T::vec_t acc = 0;
     if constexpr (SHORT) {
-        int32_t c[kShortChain];
-        typename T::val_t v[kShortChain];
-#pragma unroll
-        for (int u = 0; u < kShortChain; ++u)
-            if (u < len) {
-                c[u] = ld_stream(cp + base + u * kWave);
-                v[u] = ld_stream(vp + base + u * kWave);
-            }
-        typename T::vec_t xv[kShortChain];
-#pragma unroll
-        for (int u = 0; u < kShortChain; ++u)
-            if (u < len) xv[u] = x[c[u]];
-#pragma unroll
-        for (int u = 0; u < kShortChain; ++u)
-            if (u < len) acc = T::fma_(T::widen(v[u]), xv[u], acc);
+        acc = slot_chain_short<VT>(cp, vp, a.x, base, len);
     } else {
-        acc = slot_chain_pipe<VT, kScsPipeUnroll<VT>>(cp, vp, x, base, kWave, len);
+        acc = slot_chain_pipe<VT, kScsPipeUnroll<VT>>(cp, vp, a.x, base, kWave, len);
     }
-    if (LEN && len < clen) acc = T::fma_(T::widen(typename T::val_t(0)), x[0], acc);
+    if (LEN && len < clen) acc = T::fma_(T::widen(typename T::val_t(0)), a.x[0], acc);
     if (UNPERM) {
-        const int32_t r = slot_row[slot];
-        if (r < n_rows) y[r] = acc;
+        const int32_t r = a.slot_row[slot];
+        if (r < a.n_rows) a.y[r] = acc;
     } else {
-        y[slot] = acc;
+        a.y[slot] = acc;
     }
 }
 
@@ -197,44 +445,65 @@ __global__ __launch_bounds__(kScsThreads) void scs_spmv_w64(
 //   kernel's group size (4M-row band matrix, C = 32, FP64: sigma = 65536
 //   0.692 -> 0.660 ms, 0.640 with the occupancy cap; sigma = N 1.093 ->
 //   1.061 ms; BF16 values, sigma = 65536: 0.495 -> 0.477 ms).
-template <int VT, bool UNPERM, bool LEN, bool REMAP, int CS>
-__global__ __launch_bounds__(kScsThreads) void scs_spmv_generic(
-    int64_t C, int64_t n_chunks, int64_t n_rows, int64_t cpb, int64_t bpc,
-    const int32_t *__restrict__ chunk_ptr, const int32_t *__restrict__ chunk_len,
-    const int32_t *__restrict__ slot_len, const int32_t *__restrict__ order,
-    const int32_t *__restrict__ col,
-    const typename vt<VT>::val_t *__restrict__ val,
-    const int32_t *__restrict__ slot_row,
-    const typename vt<VT>::vec_t *__restrict__ x,
-    typename vt<VT>::vec_t *__restrict__ y, const int32_t *__restrict__ t_head,
-    const int32_t *__restrict__ t_slot, const int64_t *__restrict__ t_ptr,
-    const int32_t *__restrict__ t_col, const typename vt<VT>::val_t *__restrict__ t_val,
-    int64_t t_blocks) {
+template <int VT, bool UNPERM, bool LEN, bool REMAP, int CS, bool LONG>
+__global__ __launch_bounds__(kScsThreads, VT == SMAX_HIP_F64 ? 4 : 1) void scs_spmv_generic(
+    int64_t C, int64_t cpb, int64_t bpc, ScsSpmv<VT> a, ScsParts<VT, false> p) {
     using T = vt<VT>;
     if constexpr (CS > 0) C = CS;
-    const bool tails = CS == 0 && LEN && t_slot != nullptr;
+    if constexpr (LONG) {
+        if (static_cast<int64_t>(blockIdx.x) < p.longs.blocks) {
+            extern __shared__ __align__(16) char long_lds[];
+            // C = 32 chunks, or tail waves of any C
+            constexpr int LC = CS > 0 ? CS : kWave;
+            const int32_t id = p.longs.list[blockIdx.x];
+            if (id < 0) return;
+            const int64_t at = id / kLongParts;
+            const int lane = static_cast<int>(threadIdx.x) % LC;
+            const int64_t slot = CS == 0 ? p.t_slot[at * LC + lane] : at * LC + lane;
+            const int32_t full = slot >= 0 ? a.slot_len[slot] : 0;
+            int32_t len = full;
+            bool any;
+            const bool mine = long_part<LC>(id % kLongParts, p.longs.share, len, any);
+            if (!any) return;
+            typename T::vec_t acc = long_chunk<VT, LC>(
+                reinterpret_cast<typename T::vec_t *>(long_lds), CS == 0 ? p.t_col : a.col,
+                CS == 0 ? p.t_val : a.val, a.x, CS == 0 ? p.t_ptr[at] : a.chunk_ptr[at], len);
+            if (!mine || slot < 0 || static_cast<int>(threadIdx.x) >= LC) return;
+            if (full < a.chunk_len[slot / C])
+                acc = T::fma_(T::widen(typename T::val_t(0)), a.x[0], acc);
+            if (!UNPERM) {
+                a.y[slot] = acc;
+            } else if (a.slot_row[slot] < a.n_rows) {
+                a.y[a.slot_row[slot]] = acc;
+            }
+            return;
+        }
+    }
+    const bool tails = CS == 0 && LEN && p.t_slot != nullptr;
     int64_t slot, base, stride;
     int clen, len;
     const int32_t *cp;
     const typename T::val_t *vp;
-    if (tails && static_cast<int64_t>(blockIdx.x) < t_blocks) {
+    const int64_t block = LONG ? blockIdx.x - p.longs.blocks : blockIdx.x;
+    const int64_t blocks = LONG ? gridDim.x - p.longs.blocks : gridDim.x;
+    if (tails && block < p.t_blocks) {
         const int lane = threadIdx.x & (kWave - 1);
-        const int64_t w = static_cast<int64_t>(blockIdx.x) * (kScsThreads / kWave) +
-                          threadIdx.x / kWave;
-        const int32_t ts = t_slot[w * kWave + lane];
+        const int64_t w = block * (kScsThreads / kWave) + threadIdx.x / kWave;
+        if (LONG && w < p.longs.from) return;
+        const int32_t ts = p.t_slot[w * kWave + lane];
         if (ts < 0) return;
         slot = ts;
-        base = t_ptr[w] + lane;
+        base = p.t_ptr[w] + lane;
         stride = kWave;
-        clen = chunk_len[ts / C];
-        len = slot_len[ts];
-        cp = t_col;
-        vp = t_val;
+        clen = a.chunk_len[ts / C];
+        len = a.slot_len[ts];
+        cp = p.t_col;
+        vp = p.t_val;
     } else {
         int64_t pos, i;
         if (cpb > 0) {
-            const int64_t hb = tails ? blockIdx.x - t_blocks : blockIdx.x;
-            const int64_t hn = tails ? gridDim.x - t_blocks : gridDim.x;
+            const int64_t hb = tails ? block - p.t_blocks : block;
+            const int64_t hn = tails ? blocks - p.t_blocks : blocks;
             const int64_t blk = REMAP ? xcd_block(hb, hn) : hb;
             pos = blk * cpb + threadIdx.x / C;
             i = threadIdx.x % C;
@@ -244,29 +513,30 @@ __global__ __launch_bounds__(kScsThreads) void scs_spmv_generic(
             i = (blockIdx.x % bpc) * kScsThreads + threadIdx.x;
             if (i >= C) return;
         }
-        if (pos >= n_chunks) return;
-        const int64_t chunk = order ? static_cast<int64_t>(order[pos]) : pos;
+        if (pos >= a.n_chunks) return;
+        const int64_t chunk = a.order ? static_cast<int64_t>(a.order[pos]) : pos;
         if (chunk < 0) return;
         slot = chunk * C + i;
-        base = static_cast<int64_t>(chunk_ptr[chunk]) + i;
+        base = static_cast<int64_t>(a.chunk_ptr[chunk]) + i;
         stride = C;
-        clen = chunk_len[chunk];
-        len = LEN ? slot_len[slot] : clen;
-        if (tails && len > t_head[chunk]) return;
-        cp = col;
-        vp = val;
+        clen = a.chunk_len[chunk];
+        if (LONG && !tails && clen >= p.longs.from) return;
+        len = LEN ? a.slot_len[slot] : clen;
+        if (tails && len > p.t_head[chunk]) return;
+        cp = a.col;
+        vp = a.val;
     }
     typename T::vec_t acc;
     if constexpr (CS > 0)
-        acc = slot_chain_pipe<VT, kScsPipeUnroll<VT>>(cp, vp, x, base, CS, len);
+        acc = slot_chain_pipe<VT, kScsPipeUnroll<VT>>(cp, vp, a.x, base, CS, len);
     else
-        acc = slot_chain_pipe<VT, kScsUnroll>(cp, vp, x, base, stride, len);
-    if (LEN && len < clen) acc = T::fma_(T::widen(typename T::val_t(0)), x[0], acc);
+        acc = slot_chain_pipe<VT, kScsUnroll>(cp, vp, a.x, base, stride, len);
+    if (LEN && len < clen) acc = T::fma_(T::widen(typename T::val_t(0)), a.x[0], acc);
     if (UNPERM) {
-        const int32_t r = slot_row[slot];
-        if (r < n_rows) y[r] = acc;
+        const int32_t r = a.slot_row[slot];
+        if (r < a.n_rows) a.y[r] = acc;
     } else {
-        y[slot] = acc;
+        a.y[slot] = acc;
     }
 }
 
@@ -577,111 +847,126 @@ static int launch_scs_spmm(smax_hip_ctx ctx, int64_t C, int64_t n_chunks, int64_
     return SMAX_HIP_SUCCESS;
 }
 
-struct W64Args {
-    int64_t lds_bytes;  // dynamic LDS reserved per workgroup (occupancy cap)
-    int64_t n_chunks, n_rows;
-    const int32_t *chunk_ptr, *chunk_len, *slot_len, *order, *col;
-    const void *val;
-    const int32_t *slot_row;
-    const void *x;
-    void *y;
-    const smax_hip_scs_tails *tails;  // nullptr or n_blocks == 0: none
-    bool short_chains;                // every chunk at most kShortChain long
+template <int VT>
+struct ScsLaunch {
+    unsigned lds_bytes;  // dynamic LDS per workgroup (long chunks, occupancy cap)
+    ScsSpmv<VT> a;
+    ScsParts<VT, false> p;
 };
 
-template <int VT, bool UNPERM, bool REMAP, bool LEN, bool SHORT>
-static void launch_w64(smax_hip_ctx ctx, const W64Args &a) {
-    using T = vt<VT>;
-    const smax_hip_scs_tails *t =
-        !SHORT && LEN && a.tails && a.tails->n_blocks > 0 ? a.tails : nullptr;
-    const int64_t tb = t ? t->n_blocks : 0;
-    hipLaunchKernelGGL((scs_spmv_w64<VT, UNPERM, REMAP, LEN, SHORT>),
-                       dim3(static_cast<unsigned>(ceil_div(a.n_chunks, kScsThreads / kWave) + tb)),
-                       dim3(kScsThreads), static_cast<unsigned>(a.lds_bytes), ctx->stream,
-                       a.n_chunks, a.n_rows, a.chunk_ptr, a.chunk_len, a.slot_len, a.order, a.col,
-                       static_cast<const typename T::val_t *>(a.val), a.slot_row,
-                       static_cast<const typename T::vec_t *>(a.x),
-                       static_cast<typename T::vec_t *>(a.y), t ? t->head : nullptr,
-                       t ? t->slot : nullptr, t ? t->ptr : nullptr, t ? t->col : nullptr,
-                       static_cast<const typename T::val_t *>(t ? t->val : nullptr), tb);
+template <int VT, bool UNPERM, bool REMAP, bool LEN, bool SHORT, bool LONG>
+static void launch_w64(smax_hip_ctx ctx, const ScsLaunch<VT> &l) {
+    const int64_t blocks =
+        ceil_div(l.a.n_chunks, kScsThreads / kWave) + l.p.t_blocks + l.p.longs.blocks;
+    const dim3 grid(static_cast<unsigned>(blocks));
+    if constexpr (SHORT) {
+        hipLaunchKernelGGL((scs_spmv_w64<VT, UNPERM, REMAP, LEN, true, false>), grid,
+                           dim3(kScsThreads), l.lds_bytes, ctx->stream, l.a,
+                           ScsParts<VT, true>{});
+    } else {
+        hipLaunchKernelGGL((scs_spmv_w64<VT, UNPERM, REMAP, LEN, false, LONG>), grid,
+                           dim3(kScsThreads), l.lds_bytes, ctx->stream, l.a, l.p);
+    }
 }
 
 template <int VT, bool UNPERM, bool SHORT>
-static void launch_w64_len(smax_hip_ctx ctx, bool remap, const W64Args &a) {
-    const bool len = a.slot_len != nullptr;
+static void launch_w64_len(smax_hip_ctx ctx, bool remap, const ScsLaunch<VT> &l) {
+    const bool len = l.a.slot_len != nullptr;
+    if constexpr (!SHORT) {
+        if (l.p.longs.blocks > 0) {
+            if (remap)
+                launch_w64<VT, UNPERM, true, true, false, true>(ctx, l);
+            else
+                launch_w64<VT, UNPERM, false, true, false, true>(ctx, l);
+            return;
+        }
+    }
     if (remap && len)
-        launch_w64<VT, UNPERM, true, true, SHORT>(ctx, a);
+        launch_w64<VT, UNPERM, true, true, SHORT, false>(ctx, l);
     else if (remap)
-        launch_w64<VT, UNPERM, true, false, SHORT>(ctx, a);
+        launch_w64<VT, UNPERM, true, false, SHORT, false>(ctx, l);
     else if (len)
-        launch_w64<VT, UNPERM, false, true, SHORT>(ctx, a);
+        launch_w64<VT, UNPERM, false, true, SHORT, false>(ctx, l);
     else
-        launch_w64<VT, UNPERM, false, false, SHORT>(ctx, a);
-}
-
-// Short chains only without tail waves (a layout with them is padded more
-// than 6x, and its chunks then run their heads only).
-template <int VT, bool UNPERM>
-static void launch_w64_sched(smax_hip_ctx ctx, bool remap, const W64Args &a) {
-    const bool has_tails = a.slot_len && a.tails && a.tails->n_blocks > 0;
-    if (a.short_chains && !has_tails)
-        launch_w64_len<VT, UNPERM, true>(ctx, remap, a);
-    else
-        launch_w64_len<VT, UNPERM, false>(ctx, remap, a);
+        launch_w64<VT, UNPERM, false, false, SHORT, false>(ctx, l);
 }
 
 // remap: XCD-contiguous order (right when sigma-windows keep rows local);
 // slot_len: optional per-slot lengths (nullptr: full chunk chains);
-// order: optional execution order for C = 64 (nullptr: chunk order);
-// tails: the handle's tail waves (C = 64 with slot_len; nullptr: none);
-// max_chunk_len: the longest chunk when known (-1: unknown).
+// sched: the layout's schedule (nullptr: chunk order);
+// tails: the handle's tail waves (C = 64 with slot_len; nullptr: none).
 template <int VT>
 int launch_scs_spmv(smax_hip_ctx ctx, int64_t C, int64_t n_chunks,
                     int64_t n_rows, const int32_t *chunk_ptr,
                     const int32_t *chunk_len, const int32_t *col,
                     const void *val, const int32_t *slot_row, const void *x,
-                    void *y, bool unperm, bool remap = true,
+                    void *y, bool unperm, const smax_hip_scs_sched *sched = nullptr,
                     const int32_t *slot_len = nullptr,
-                    const int32_t *order = nullptr, int64_t lds_bytes = 0,
-                    const smax_hip_scs_tails *tails = nullptr, int32_t max_chunk_len = -1) {
-    using T = vt<VT>;
+                    const smax_hip_scs_tails *tails = nullptr) {
+    const bool remap = sched ? sched->remap : true;
+    ScsLaunch<VT> l{};
+    l.a = {n_chunks, n_rows, chunk_ptr, chunk_len, slot_len,
+           !sched ? nullptr : C <= kScsThreads ? sched->order : sched->order_lf, col,
+           static_cast<const typename vt<VT>::val_t *>(val), slot_row,
+           static_cast<const typename vt<VT>::vec_t *>(x),
+           static_cast<typename vt<VT>::vec_t *>(y)};
+    l.lds_bytes = sched ? static_cast<unsigned>(sched->lds_cap_bytes) : 0u;
+    const bool has_tails = slot_len && C <= kScsThreads && tails && tails->n_blocks > 0;
+    if (has_tails) {
+        l.p.t_head = tails->head;
+        l.p.t_slot = tails->slot;
+        l.p.t_ptr = tails->ptr;
+        l.p.t_col = tails->col;
+        l.p.t_val = static_cast<const typename vt<VT>::val_t *>(tails->val);
+        l.p.t_blocks = tails->n_blocks;
+        l.p.longs = {tails->wide, tails->wide_blocks, tails->n_wide, tails->share};
+    } else if (sched && slot_len && sched->long_blocks > 0) {
+        l.p.longs = {sched->long_chunks, sched->long_blocks, sched->long_from,
+                     sched->long_share};
+    }
+    if (l.p.longs.blocks > 0)
+        l.lds_bytes = std::max(l.lds_bytes, static_cast<unsigned>(LongChunk<VT>::kBytes));
     if (C == kWave) {
-        const bool short_chains = max_chunk_len >= 0 && max_chunk_len <= kShortChain;
-        const W64Args a{lds_bytes, n_chunks, n_rows, chunk_ptr, chunk_len, slot_len,
-                        order, col, val, slot_row, x, y, tails, short_chains};
-        if (unperm)
-            launch_w64_sched<VT, true>(ctx, remap, a);
+        // Short chains only without tail waves (a layout with them is padded
+        // more than 6x, and its chunks then run their heads only).
+        const bool short_chains = sched && !has_tails && sched->max_chunk_len >= 0 &&
+                                  sched->max_chunk_len <= kShortChain;
+        if (unperm && short_chains)
+            launch_w64_len<VT, true, true>(ctx, remap, l);
+        else if (unperm)
+            launch_w64_len<VT, true, false>(ctx, remap, l);
+        else if (short_chains)
+            launch_w64_len<VT, false, true>(ctx, remap, l);
         else
-            launch_w64_sched<VT, false>(ctx, remap, a);
+            launch_w64_len<VT, false, false>(ctx, remap, l);
         SMAX_HIP_LAUNCHED(ctx, "scs_spmv_w64");
         return SMAX_HIP_SUCCESS;
     }
-    auto v = static_cast<const typename T::val_t *>(val);
-    auto xv = static_cast<const typename T::vec_t *>(x);
-    auto yv = static_cast<typename T::vec_t *>(y);
     const int64_t cpb = C <= kScsThreads ? kScsThreads / C : 0;
     const int64_t bpc = C <= kScsThreads ? 1 : ceil_div(C, kScsThreads);
-    const smax_hip_scs_tails *t =
-        slot_len && cpb > 0 && tails && tails->n_blocks > 0 ? tails : nullptr;
-    const int64_t tb = t ? t->n_blocks : 0;
-    const int64_t blocks = (cpb > 0 ? ceil_div(n_chunks, cpb) : n_chunks * bpc) + tb;
+    const int64_t blocks = (cpb > 0 ? ceil_div(n_chunks, cpb) : n_chunks * bpc) +
+                           l.p.t_blocks + l.p.longs.blocks;
     SMAX_HIP_REQUIRE(ctx, blocks <= INT32_MAX, "scs spmv: grid too large");
     const dim3 grid(static_cast<unsigned>(blocks));
     const bool rm = remap && cpb > 0;
-    auto tv = static_cast<const typename T::val_t *>(t ? t->val : nullptr);
     // C = 32 without tail waves: the compile-time chunk width, and the
     // schedule's occupancy cap
-    const bool c32 = C == 32 && !t;
-    const unsigned lds = c32 ? static_cast<unsigned>(lds_bytes) : 0u;
-#define SMAX_SCS_GENERIC_CS(U, L, R, CS)                                                 \
-    hipLaunchKernelGGL((scs_spmv_generic<VT, U, L, R, CS>), grid, dim3(kScsThreads), lds, \
-                       ctx->stream, C, n_chunks, n_rows, cpb, bpc, chunk_ptr,           \
-                       chunk_len, slot_len, order, col, v, slot_row, xv, yv,            \
-                       t ? t->head : nullptr, t ? t->slot : nullptr, t ? t->ptr : nullptr, \
-                       t ? t->col : nullptr, tv, tb)
+    const bool c32 = C == 32 && !has_tails;
+    const unsigned lds = c32 || l.p.longs.blocks > 0 ? l.lds_bytes : 0u;
+#define SMAX_SCS_GENERIC_CS(U, L, R, CS, LONG)                                                \
+    hipLaunchKernelGGL((scs_spmv_generic<VT, U, L, R, CS, LONG>), grid, dim3(kScsThreads), lds, \
+                       ctx->stream, C, cpb, bpc, l.a, l.p)
 #define SMAX_SCS_GENERIC(U, L, R)                                                        \
-    if (c32) SMAX_SCS_GENERIC_CS(U, L, R, 32); else SMAX_SCS_GENERIC_CS(U, L, R, 0)
-    if (unperm && slot_len) {
+    if (c32) SMAX_SCS_GENERIC_CS(U, L, R, 32, false); else SMAX_SCS_GENERIC_CS(U, L, R, 0, false)
+#define SMAX_SCS_GENERIC_LONG(U, R)                                                      \
+    if (c32) SMAX_SCS_GENERIC_CS(U, true, R, 32, true); else SMAX_SCS_GENERIC_CS(U, true, R, 0, true)
+    if (l.p.longs.blocks > 0) {
+        if (unperm) {
+            if (rm) SMAX_SCS_GENERIC_LONG(true, true); else SMAX_SCS_GENERIC_LONG(true, false);
+        } else {
+            if (rm) SMAX_SCS_GENERIC_LONG(false, true); else SMAX_SCS_GENERIC_LONG(false, false);
+        }
+    } else if (unperm && slot_len) {
         if (rm) SMAX_SCS_GENERIC(true, true, true); else SMAX_SCS_GENERIC(true, true, false);
     } else if (unperm) {
         if (rm) SMAX_SCS_GENERIC(true, false, true); else SMAX_SCS_GENERIC(true, false, false);
@@ -691,6 +976,7 @@ int launch_scs_spmv(smax_hip_ctx ctx, int64_t C, int64_t n_chunks,
         if (rm) SMAX_SCS_GENERIC(false, false, true); else SMAX_SCS_GENERIC(false, false, false);
     }
 #undef SMAX_SCS_GENERIC
+#undef SMAX_SCS_GENERIC_LONG
 #undef SMAX_SCS_GENERIC_CS
     SMAX_HIP_LAUNCHED(ctx, "scs_spmv_generic");
     return SMAX_HIP_SUCCESS;
@@ -716,7 +1002,14 @@ int launch_scs_spmv(smax_hip_ctx ctx, int64_t C, int64_t n_chunks,
 // slot (and 8x the mean) start first, longest first, one per workgroup where
 // the range has room (each on its own CU, with its own miss queue); the rest
 // follow in chunk order.  Results do not depend on the order.
+//
+// Where the slots' lengths are at hand, chunks of at least kWideChunk entries
+// per slot (and 4x the mean) leave this order and are run by whole workgroups
+// (long_chunk).  With 128 and 8x instead: 1,000,000 rows, C = 32, sigma =
+// 65536, FP32 133 us against 127, 4,000,000 rows, C = 32, sigma = 4096, FP64
+// 803 against 760; no size measured slower with the lower line.
 constexpr int kLongChunk = 128;
+constexpr int kWideChunk = 64;
 constexpr int64_t kLdsPerCu = 160 * 1024;
 
 static int upload_order(smax_hip_ctx ctx, const std::vector<int32_t> &ord, int32_t **out) {
@@ -729,10 +1022,32 @@ static int upload_order(smax_hip_ctx ctx, const std::vector<int32_t> &ord, int32
     return SMAX_HIP_SUCCESS;
 }
 
+// Entries per workgroup of a long chunk: enough workgroups for the chip while
+// the matrix is small, whole chunks once there are many of them (1 / 2048 of the
+// entries: 1,000,000 rows, C = 32, sigma = 65536, FP32 142 us against 127).
+static int32_t long_share(int64_t nnz) {
+    return static_cast<int32_t>(std::max<int64_t>(2048, nnz / 1024));
+}
+
+// Appends the eight lists entry by entry, the i-th of list r at 8i + r, with
+// -1 behind the shorter ones; returns the number of entries.
+static size_t append_by_xcd(std::vector<int32_t> &out,
+                            const std::vector<std::vector<int32_t>> &lists) {
+    size_t most = 0;
+    for (const auto &l : lists) most = std::max(most, l.size());
+    const size_t at = out.size();
+    out.resize(at + 8 * most, -1);
+    for (size_t r = 0; r < lists.size(); ++r)
+        for (size_t i = 0; i < lists[r].size(); ++i) out[at + 8 * i + r] = lists[r][i];
+    return 8 * most;
+}
+
 void free_schedule(smax_hip_scs_sched &s) {
     dev_free(s.order);
     dev_free(s.order_lf);
     s.order = s.order_lf = nullptr;
+    s.long_chunks = nullptr;
+    s.long_blocks = 0;
 }
 
 // Row of each chunk's first slot, packed for one copy to the host (a strided
@@ -831,6 +1146,19 @@ int build_schedule(smax_hip_ctx ctx, int64_t C, int64_t sigma, int64_t n_rows_pa
     const int64_t per_block = kScsThreads / C;  // chunks per workgroup
     const int64_t nb = ceil_div(n, per_block);
     std::vector<int32_t> ord(static_cast<size_t>(nb * per_block), -1);
+    // The long chunks of each range, longest first.
+    std::vector<std::vector<int32_t>> longs;
+    const int64_t wide = std::max<int64_t>(kWideChunk, static_cast<int64_t>(std::ceil(4 * mean)));
+    auto list_longs = [&](int64_t a, int64_t b) {
+        std::vector<int32_t> l;
+        for (int64_t i = a; i < std::min(b, n); ++i) {
+            const int32_t c = sq ? (*sq)[i] : static_cast<int32_t>(i);
+            if (cl[c] >= wide) l.push_back(c);
+        }
+        std::stable_sort(l.begin(), l.end(),
+                         [&](int32_t p, int32_t q) { return cl[p] > cl[q]; });
+        longs.push_back(std::move(l));
+    };
     if (out->remap) {
         constexpr int64_t kXcd = 8;
         const int64_t q = nb / kXcd, rem = nb % kXcd;
@@ -838,9 +1166,36 @@ int build_schedule(smax_hip_ctx ctx, int64_t C, int64_t sigma, int64_t n_rows_pa
             const int64_t s = k < rem ? k * (q + 1) : rem * (q + 1) + (k - rem) * q;
             const int64_t len = k < rem ? q + 1 : q;
             fill(ord, s * per_block, (s + len) * per_block, per_block, sq);
+            list_longs(s * per_block, (s + len) * per_block);
         }
     } else {
         fill(ord, 0, nb * per_block, per_block, sq);
+        list_longs(0, nb * per_block);
+    }
+    if ((C == kWave || C == 32) && n_long > 0) {
+        // one range: dealt out in turn; eight: one range per XCD.  A chunk
+        // gets the workgroups that it needs if no lane of it is padded.  First
+        // parts come first: they hold the longest rows, and the hardware hands
+        // an XCD's workgroups to its CUs in turn (parts of a chunk side by side,
+        // 1,000,000 rows, sigma = 4096, FP64: 0.286 ms against 0.168).
+        const int32_t share = long_share(nnz);
+        std::vector<std::vector<int32_t>> parts(8);
+        for (int p = 0; p < kLongParts; ++p)
+            for (size_t r = 0; r < longs.size(); ++r)
+                for (size_t i = 0; i < longs[r].size(); ++i) {
+                    const int32_t c = longs[r][i];
+                    if (p < long_parts(C * cl[c], share))
+                        parts[longs.size() == 1 ? i % 8 : r].push_back(c * kLongParts + p);
+                }
+        const size_t at = ord.size();
+        const size_t blocks = append_by_xcd(ord, parts);
+        const int rc = upload_order(ctx, ord, &out->order);
+        if (rc) return rc;
+        out->long_chunks = out->order + at;
+        out->long_blocks = static_cast<int64_t>(blocks);
+        out->long_from = static_cast<int32_t>(std::min<int64_t>(wide, INT32_MAX));
+        out->long_share = share;
+        return SMAX_HIP_SUCCESS;
     }
     return upload_order(ctx, ord, &out->order);
 }
@@ -969,6 +1324,17 @@ int build_tails(smax_hip_ctx ctx, smax_hip_scs A) {
         tptr[w] = store;
         store += wave_len[w] * kWave;
     }
+    // The waves of kWideChunk columns and more, by whole workgroups.
+    const int32_t share = long_share(in.nnz);
+    std::vector<std::vector<int32_t>> parts(8);
+    int64_t wide = 0;
+    while (wide < n_waves && wave_len[wide] >= kWideChunk) ++wide;
+    for (int p = 0; p < kLongParts; ++p)
+        for (int64_t w = 0; w < wide; ++w)
+            if (p < long_parts(kWave * wave_len[w], share))
+                parts[w % 8].push_back(static_cast<int32_t>(w * kLongParts + p));
+    const size_t listed = tslot.size();
+    const int64_t wide_blocks = static_cast<int64_t>(append_by_xcd(tslot, parts));
     smax_hip_scs_tails t;
     t.n_elements = store;
     t.n_slots = static_cast<int64_t>(tail.size());
@@ -1005,6 +1371,10 @@ int build_tails(smax_hip_ctx ctx, smax_hip_scs A) {
             return hip_fail(ctx, e, "scs tails");
         }
     t.n_blocks = n_blocks;
+    t.wide = t.slot + listed;
+    t.wide_blocks = wide_blocks;
+    t.n_wide = static_cast<int32_t>(wide);
+    t.share = share;
     A->tails = t;  // freed with the handle from here on
     rc = tail_fill(ctx, A, true);
     if (rc) return rc;
@@ -1123,13 +1493,7 @@ int smax_hip_scs_spmv_plan(smax_hip_ctx ctx, int value_type, smax_hip_scs_plan p
     SMAX_HIP_DISPATCH_VT(value_type,
                          return launch_scs_spmv<VT>(ctx, plan->C, plan->n_chunks, npad,
                                                     chunk_ptr, chunk_lengths, col, val,
-                                                    nullptr, x, y, false,
-                                                    plan->sched.remap, nullptr,
-                                                    plan->C <= kScsThreads
-                                                        ? plan->sched.order
-                                                        : plan->sched.order_lf,
-                                                    plan->sched.lds_cap_bytes, nullptr,
-                                                    plan->sched.max_chunk_len));
+                                                    nullptr, x, y, false, &plan->sched));
     return SMAX_HIP_ERROR_UNSUPPORTED;
 }
 
@@ -1149,13 +1513,8 @@ int smax_hip_scs_apply(smax_hip_ctx ctx, int value_type, smax_hip_scs A,
                          return launch_scs_spmv<VT>(ctx, in.C, in.n_chunks, in.n_rows,
                                                     in.chunk_ptr, in.chunk_lengths,
                                                     in.col, in.val, in.slot_row, x, y,
-                                                    unpermuted != 0, A->sched.remap,
-                                                    in.slot_len,
-                                                    in.C <= kScsThreads
-                                                        ? A->sched.order
-                                                        : A->sched.order_lf,
-                                                    A->sched.lds_cap_bytes, &A->tails,
-                                                    A->sched.max_chunk_len));
+                                                    unpermuted != 0, &A->sched,
+                                                    in.slot_len, &A->tails));
     return SMAX_HIP_ERROR_UNSUPPORTED;
 }
 

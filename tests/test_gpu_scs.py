@@ -739,3 +739,49 @@ def test_scs_apply_spmm_long_rows_and_any_width(ctx, vt, k, C_, sigma):
     for a in (dX, dY):
         a.free()
     s.destroy()
+
+
+@pytest.mark.parametrize("vt", [capi.F64, capi.F32, capi.BF16])
+@pytest.mark.parametrize("C_,sigma,tails", [(64, 1 << 20, False), (64, 512, False),
+                                            (32, 256, False), (64, 1, True),
+                                            (32, 1, True), (16, 1, True)])
+@pytest.mark.parametrize("x0", [0.5, np.inf])
+def test_scs_apply_long_chunks_by_workgroups(ctx, vt, C_, sigma, tails, x0):
+    """Long chunks and long tail waves, run by workgroups that gather a tile of
+    2048 entries: chunk lengths around the one from which they are long (64),
+    rows around whole tiles of 64 lanes (32 columns) and of one lane (2048),
+    chunks of one, a few and many long rows (one to eight workgroups), the
+    padding term of an infinite x[0], both output orders."""
+    rng = np.random.default_rng(31)
+    n, m = 9000, 4200
+    L = rng.integers(0, 5, n)
+    many = np.r_[np.arange(60, 68), 96, 127, 128, 129, rng.integers(130, 400, 180)]
+    few = [4200, 4097, 4096, 4095, 2049, 2048, 2047, 1025, 1024, 513, 65, 64, 63, 33, 32, 31]
+    if tails:
+        L[::97][:len(many)] = many[:len(L[::97])]
+        L[50::301][:len(few)] = few
+    else:
+        L[600:600 + len(many)] = many
+        L[4000:4000 + len(few)] = few
+        L[7000] = 900
+    rp = np.concatenate([[0], np.cumsum(L)]).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(m, l, replace=False)) for l in L]).astype(np.int32)
+    A = Csr(n, m, rp, col, rng.uniform(-1, 1, rp[-1]))
+    val, x = values_for(vt, A)
+    x = x.copy()
+    x[0] = x0
+    s = gpu_scs(ctx, A, C_, sigma, val)
+    assert (s.tails()[1] > 0) == tails
+    want_s = oracle.crs_to_scs(A.row_ptr, A.col, val, C_, sigma)
+    want = oracle.scs_spmv(C_, want_s["n_chunks"], want_s["chunk_ptr"],
+                           want_s["chunk_lengths"], want_s["col"], want_s["val"], x)
+    dx = ctx.upload(x)
+    dy = ctx.zeros(s.info.n_rows_padded, x.dtype)
+    dy2 = ctx.zeros(A.n_rows, x.dtype)
+    s.apply(vt, dx, dy)
+    assert_same_values(ctx.download(dy), want, "long chunks")
+    s.apply(vt, dx, dy2, unpermuted=True)
+    assert_same_values(ctx.download(dy2), want[want_s["perm"]], "long chunks, original order")
+    for d in (dx, dy, dy2):
+        d.free()
+    s.destroy()
