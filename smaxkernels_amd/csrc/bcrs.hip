@@ -7,12 +7,14 @@
 // (row-major), accumulated per output in (j, jx) order exactly as
 // naive_bcrs_spmv does (spmv_cpu_bcrs_impl.hpp:45-74): bit-identical.
 //
-// SpMV stages the blocks of a range of block rows through LDS: the values
-// of 256/b_h block rows are contiguous in memory, so the workgroup streams
-// them (and the x entries their columns select) with coalesced loads, then
-// lane (r, ix) runs its fma chain out of LDS.
+// SpMV, b_w <= 8: a thread per output row reads its row of each block itself
+// (bcrs_spmv_rows).  Wider blocks are staged through LDS: the values of
+// 256/b_h block rows are contiguous in memory, so the workgroup streams them
+// (and the x entries their columns select) with coalesced loads, then lane
+// (r, ix) runs its fma chain out of LDS.
 #include "common.hpp"
 #include "scan.hpp"
+#include "spmm_long.hpp"
 
 #include <type_traits>
 #include <utility>
@@ -74,6 +76,74 @@ __global__ __launch_bounds__(kBThreads) void bcrs_spmv_lds(
         __syncthreads();
     }
     if (has) y[my_r * h_pad + ix] = acc;
+}
+
+// Q values side by side, aligned as a value is.
+template <typename V, int Q>
+__device__ __forceinline__ void load_vals(const V *__restrict__ p, V (&out)[Q]) {
+    if constexpr (sizeof(V) >= 4) {
+        load_cols_run<V, Q>(p, out);
+    } else {
+#pragma unroll
+        for (int i = 0; i < Q; ++i) out[i] = p[i];
+    }
+}
+
+// SpMV, b_w = BW <= 8: thread (r, ix) reads its row of each block itself, G
+// blocks at a time (their columns, then all their values and x entries, then
+// the fmas): no barrier between loading and the chains, and a block row's
+// lanes are neighbours, so a block's lines are read by one wavefront.  RM:
+// row-major blocks, the row's BW values side by side.  Bound by the blocks'
+// bytes (3x3 FP64, 48^3 block rows: 4.4 TB/s).  7-point block matrices,
+// staged in LDS -> so: 3x3 FP64 of 48^3 43.7 -> 12.8 us, 5x5 of 40^3 70 ->
+// 16.7, 6x6 89 -> 21.5, 6x6 BF16 of 32^3 38 -> 5.1; a thread per block row
+// -> so: 2x2 FP64 of 48^3 10.1 -> 6.2, 4x4 24.4 -> 16.7, 4x4 FP32 of 64^3
+// 28.7 -> 20.9, BF16 of 96^3 55.8 -> 46.7.  Half as many
+// blocks at a time: 3x3 13.8 us, 6x6 22.5.
+template <int VT, int BW, int G, bool RM>
+__global__ __launch_bounds__(kBThreads) void bcrs_spmv_rows(
+    int64_t n_rows, int b_h, FastDiv by_h, int h_pad, int w_pad,
+    const int32_t *__restrict__ col,
+    const int32_t *__restrict__ row_ptr, const typename vt<VT>::val_t *__restrict__ val,
+    const typename vt<VT>::vec_t *__restrict__ x, typename vt<VT>::vec_t *__restrict__ y) {
+    using T = vt<VT>;
+    using A = typename T::vec_t;
+    using V = typename T::val_t;
+    const int64_t t = xcd_block(blockIdx.x, gridDim.x) * kBThreads + threadIdx.x;
+    if (t >= n_rows) return;
+    const int32_t r = by_h(static_cast<int32_t>(t));
+    const int32_t ix = static_cast<int32_t>(t) - r * b_h;
+    const int64_t bs = static_cast<int64_t>(h_pad) * w_pad;
+    const V *vrow = val + (RM ? ix * w_pad : ix);
+    const int32_t je = row_ptr[r + 1];
+    A acc = 0;
+    for (int32_t j = row_ptr[r]; j < je; j += G) {
+        int32_t c[G];
+        V w[G][BW];
+        A xv[G][BW];
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+            if (j + g < je) c[g] = col[j + g];
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+            if (j + g < je) {
+                const V *blk = vrow + (j + g) * bs;
+                if constexpr (RM) {
+                    load_vals<V, BW>(blk, w[g]);
+                } else {
+#pragma unroll
+                    for (int jx = 0; jx < BW; ++jx) w[g][jx] = blk[jx * h_pad];
+                }
+                load_cols_run<A, BW>(x + static_cast<int64_t>(c[g]) * w_pad, xv[g]);
+            }
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+            if (j + g < je) {
+#pragma unroll
+                for (int jx = 0; jx < BW; ++jx) acc = T::fma_(T::widen(w[g][jx]), xv[g][jx], acc);
+            }
+    }
+    y[static_cast<int64_t>(r) * h_pad + ix] = acc;
 }
 
 // Thread (r, ix, v), v fastest: the k lanes of one output row share each
@@ -146,6 +216,76 @@ __global__ __launch_bounds__(kBThreads) void bcrs_spmm_kernel(
         for (int jx = 0; jx < BW; ++jx) acc = T::fma_(T::widen(w0[jx]), x0[jx], acc);
     }
     Y[(r * h_pad + ix) * k + v] = acc;
+}
+
+// SpMM in parts of a block, b_w = BW and b_h a multiple of H, X and Y of any
+// alignment and any k >= Q: thread (r, h, l) keeps H outputs of block row r in
+// one run of Q columns (the last run is moved back to end at k), G blocks at a
+// time.  RM: row-major blocks.  Bound by the blocks' lines, which each of a
+// block row's lanes reads through L1.  Against a thread per output (k = 8 /
+// 10 / 32): 3x3 FP64 of 48^3 63 / 78 / 225 -> 23 / 29 / 65 us, 5x5 of 40^3 87
+// / 110 / 327 -> 28 / 37 / 84, 6x6 121 / 153 / 523 -> 33 / 41 / 144, 6x6 BF16
+// of 32^3 44 / 72 / 175 -> 8.4 / 11.6 / 23.  One block at a time: 6x6 FP64 59
+// / 60 / 143.
+template <int VT, int H, int BW, int Q, int G, bool RM>
+__global__ __launch_bounds__(kBThreads) void bcrs_spmm_part(
+    int64_t n_threads, FastDiv by_lanes, int lanes, FastDiv by_parts, int parts, int h_pad,
+    int w_pad, int64_t k, const int32_t *__restrict__ col, const int32_t *__restrict__ row_ptr,
+    const typename vt<VT>::val_t *__restrict__ val, const typename vt<VT>::vec_t *__restrict__ X,
+    typename vt<VT>::vec_t *__restrict__ Y) {
+    using T = vt<VT>;
+    using A = typename T::vec_t;
+    using V = typename T::val_t;
+    const int64_t t = xcd_block(blockIdx.x, gridDim.x) * kBThreads + threadIdx.x;
+    if (t >= n_threads) return;
+    const int32_t rh = by_lanes(static_cast<int32_t>(t));
+    const int32_t l = static_cast<int32_t>(t) - rh * lanes;
+    const int32_t r = by_parts(rh);
+    const int32_t ix = (rh - r * parts) * H;
+    const int64_t v = run_start<Q>(l, k);
+    const int64_t bs = static_cast<int64_t>(h_pad) * w_pad;
+    const V *vpart = val + (RM ? ix * w_pad : ix);
+    const A *xpart = X + v;
+    A acc[H][Q];
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) acc[h][q] = 0;
+    const int32_t je = row_ptr[r + 1];
+    for (int32_t j = row_ptr[r]; j < je; j += G) {
+        int32_t c[G];
+        V w[G][RM ? H : BW][RM ? BW : H];
+        A xv[G][BW][Q];
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+            if (j + g < je) c[g] = col[j + g];
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+            if (j + g < je) {
+                const A *xr = xpart + static_cast<int64_t>(c[g]) * w_pad * k;
+#pragma unroll
+                for (int jx = 0; jx < BW; ++jx) load_cols_run<A, Q>(xr + jx * k, xv[g][jx]);
+                const V *blk = vpart + (j + g) * bs;
+#pragma unroll
+                for (int a = 0; a < (RM ? H : BW); ++a)
+                    load_vals<V, RM ? BW : H>(blk + a * (RM ? w_pad : h_pad), w[g][a]);
+            }
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+            if (j + g < je) {
+#pragma unroll
+                for (int h = 0; h < H; ++h)
+#pragma unroll
+                    for (int jx = 0; jx < BW; ++jx)
+#pragma unroll
+                        for (int q = 0; q < Q; ++q)
+                            acc[h][q] = T::fma_(T::widen(w[g][RM ? h : jx][RM ? jx : h]),
+                                                xv[g][jx][q], acc[h][q]);
+            }
+    }
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+        store_cols_run<A, Q>(Y + (static_cast<int64_t>(r) * h_pad + ix + h) * k + v, acc[h]);
 }
 
 // One block's values, widened to the accumulation type.  DENSE: h_pad == BH
@@ -502,30 +642,24 @@ static void launch_bcrs_spmm_reg(smax_hip_ctx ctx, int64_t n_block_rows, int64_t
         }
 #undef SMAX_BCRS_QUAD
     }
-    // block groups: 8 when a single thread holds the whole block row (k = 1),
-    // else 2 (measured on the 96^3 block matrix: k = 1 0.108 -> 0.058 ms,
-    // k = 8 0.173 -> 0.160 ms, k = 64 0.663 -> 0.649 ms in BF16).  Padded
-    // blocks load value by value, with an address each: groups of 8 would
-    // spill registers, so a single thread takes kPaddedGroup blocks at once.
-    constexpr int kPaddedGroup = 4;
-    const bool single = !runs && k == 1;
+    // block groups of 2 (measured on the 96^3 block matrix: k = 8 0.173 ->
+    // 0.160 ms, k = 64 0.663 -> 0.649 ms in BF16), of 8 where one thread has a
+    // whole block row of 2x2 BF16 values (see spmv_by_rows)
+    constexpr int GS = VT == SMAX_HIP_BF16 && BH == 2 && BW == 2 ? 8 : 2;
 #define SMAX_BCRS_REG_LAUNCH(QQ, DD, CC, GG)                                                \
     hipLaunchKernelGGL((bcrs_spmm_reg<VT, BH, BW, QQ, DD, CC, GG>), g, dim3(kBThreads), 0,  \
                        ctx->stream, n_block_rows, static_cast<int>(h_pad),                 \
                        static_cast<int>(w_pad), cm ? 1 : 0, k, col, row_ptr, v, xv, yv)
-#define SMAX_BCRS_REG_G(DD, CC, GS)                                                         \
-    if (single) SMAX_BCRS_REG_LAUNCH(1, DD, CC, GS);                                        \
-    else SMAX_BCRS_REG_LAUNCH(1, DD, CC, 2)
-    // runs imply k >= 4Q lanes' worth of columns, so never a single thread
     if (runs && dense && cm) { SMAX_BCRS_REG_LAUNCH(Q, true, true, 2); }
     else if (runs && dense) { SMAX_BCRS_REG_LAUNCH(Q, true, false, 2); }
     else if (runs) { SMAX_BCRS_REG_LAUNCH(Q, false, false, 2); }
     else if (pairs && cm) { SMAX_BCRS_REG_LAUNCH(2, true, true, 2); }
     else if (pairs) { SMAX_BCRS_REG_LAUNCH(2, true, false, 2); }
-    else if (dense && cm) { SMAX_BCRS_REG_G(true, true, 8); }
-    else if (dense) { SMAX_BCRS_REG_G(true, false, 8); }
-    else { SMAX_BCRS_REG_G(false, false, kPaddedGroup); }
-#undef SMAX_BCRS_REG_G
+    else if (dense && cm && k == 1) { SMAX_BCRS_REG_LAUNCH(1, true, true, GS); }
+    else if (dense && k == 1) { SMAX_BCRS_REG_LAUNCH(1, true, false, GS); }
+    else if (dense && cm) { SMAX_BCRS_REG_LAUNCH(1, true, true, 2); }
+    else if (dense) { SMAX_BCRS_REG_LAUNCH(1, true, false, 2); }
+    else { SMAX_BCRS_REG_LAUNCH(1, false, false, 2); }
 #undef SMAX_BCRS_REG_LAUNCH
 }
 
@@ -543,6 +677,94 @@ static void launch_bcrs_spmm(smax_hip_ctx ctx, int64_t threads, int64_t n_block_
                        col, row_ptr, static_cast<const typename T::val_t *>(val),
                        static_cast<const typename T::vec_t *>(X),
                        static_cast<typename T::vec_t *>(Y));
+}
+
+// False: more threads than the kernel's index arithmetic holds.
+template <int VT, int H, int BW, int G>
+static bool launch_bcrs_spmm_part(smax_hip_ctx ctx, int64_t n_block_rows, int64_t b_h,
+                                  int64_t h_pad, int64_t w_pad, bool cm, int64_t k,
+                                  const int32_t *col, const int32_t *row_ptr, const void *val,
+                                  const void *X, void *Y) {
+    using T = vt<VT>;
+    using A = typename T::vec_t;
+    constexpr int Q = 16 / sizeof(A);
+    const bool runs = k >= Q;
+    const int64_t lanes = runs ? run_lanes(k, Q) : k, parts = b_h / H;
+    const int64_t threads = n_block_rows * parts * lanes;
+    if (threads > INT32_MAX - kBThreads) return false;
+#define SMAX_BCRS_PART(QQ, RM)                                                               \
+    hipLaunchKernelGGL((bcrs_spmm_part<VT, H, BW, QQ, G, RM>), grid_for(threads, kBThreads), \
+                       dim3(kBThreads), 0, ctx->stream, threads, fast_div(lanes),            \
+                       static_cast<int>(lanes), fast_div(parts), static_cast<int>(parts),    \
+                       static_cast<int>(h_pad), static_cast<int>(w_pad), k, col, row_ptr,    \
+                       static_cast<const typename T::val_t *>(val), static_cast<const A *>(X), \
+                       static_cast<A *>(Y))
+    if (runs && cm) SMAX_BCRS_PART(Q, false);
+    else if (runs) SMAX_BCRS_PART(Q, true);
+    else if (cm) SMAX_BCRS_PART(1, false);
+    else SMAX_BCRS_PART(1, true);
+#undef SMAX_BCRS_PART
+    return true;
+}
+
+// Which block shapes take it: 3x3, 5x5, 6x6 and stacks of them; 2x2, except
+// BF16 values from k = 32 on (96^3: 0.182 ms against the register-blocked
+// kernel's 0.164, while k = 8 takes 0.044 against 0.050; FP64 of 48^3, k = 8
+// 13.4 us against 19.3, k = 32 34 against 39); 4x4 in FP64 from k = 8 on (48^3,
+// k = 8 29.5 us against 37.8, k = 32 117 both, k = 4 29.7 against 27.6; FP32
+// and BF16 values have broadcast kernels).
+static bool spmm_in_parts(smax_hip_ctx ctx, int value_type, int64_t n_block_rows, int64_t b_h,
+                          int64_t b_w, int64_t h_pad, int64_t w_pad, bool cm, int64_t k,
+                          const int32_t *col, const int32_t *row_ptr, const void *val,
+                          const void *X, void *Y) {
+#define SMAX_BCRS_PARTS(VT, H, W, G)                                                       \
+    return launch_bcrs_spmm_part<VT, H, W, G>(ctx, n_block_rows, b_h, h_pad, w_pad, cm, k, \
+                                              col, row_ptr, val, X, Y)
+    SMAX_HIP_DISPATCH_VT(value_type, {
+        if (b_w == 3 && b_h % 3 == 0) SMAX_BCRS_PARTS(VT, 3, 3, 4);
+        if (b_w == 5 && b_h % 5 == 0) SMAX_BCRS_PARTS(VT, 5, 5, 2);
+        if (b_w == 6 && b_h % 3 == 0) SMAX_BCRS_PARTS(VT, 3, 6, 2);
+        if (b_w == 2 && b_h == 2 && !(VT == SMAX_HIP_BF16 && (k == 1 || k >= 32)))
+            SMAX_BCRS_PARTS(VT, 2, 2, 4);
+        if (VT == SMAX_HIP_F64 && b_w == 4 && b_h == 4 && k >= 8)
+            SMAX_BCRS_PARTS(SMAX_HIP_F64, 4, 4, 2);
+    });
+#undef SMAX_BCRS_PARTS
+    return false;
+}
+
+// b_w <= 8, except unpadded 2x2 blocks of BF16 values, whose 8 bytes a thread
+// per block row reads at once (48^3: 4.4 us against 5.3, 96^3: 24.1 against
+// 24.8).  False also with more rows than the kernel's arithmetic holds.
+static bool spmv_by_rows(smax_hip_ctx ctx, int value_type, int64_t n_block_rows, int64_t b_h,
+                         int64_t b_w, int64_t h_pad, int64_t w_pad, bool cm, const int32_t *col,
+                         const int32_t *row_ptr, const void *val, const void *x, void *y) {
+    const int64_t rows = n_block_rows * b_h;
+    if (b_w > 8 || rows > INT32_MAX - kBThreads) return false;
+    if (value_type == SMAX_HIP_BF16 && h_pad == 2 && w_pad == 2 && b_h == 2 && b_w == 2)
+        return false;
+#define SMAX_BCRS_ROWS(W, RM)                                                                \
+    hipLaunchKernelGGL((bcrs_spmv_rows<VT, W, (W <= 3 ? 8 : 4), RM>), grid_for(rows, kBThreads), \
+                       dim3(kBThreads), 0, ctx->stream, rows, static_cast<int>(b_h),         \
+                       fast_div(b_h), static_cast<int>(h_pad), static_cast<int>(w_pad), col, \
+                       row_ptr, static_cast<const typename T::val_t *>(val),                 \
+                       static_cast<const typename T::vec_t *>(x),                            \
+                       static_cast<typename T::vec_t *>(y))
+#define SMAX_BCRS_ROWS_W(W)                                                    \
+    case W:                                                                    \
+        if (cm) SMAX_BCRS_ROWS(W, false); else SMAX_BCRS_ROWS(W, true);        \
+        break;
+    SMAX_HIP_DISPATCH_VT(value_type, {
+        using T = vt<VT>;
+        switch (b_w) {
+            SMAX_BCRS_ROWS_W(1) SMAX_BCRS_ROWS_W(2) SMAX_BCRS_ROWS_W(3) SMAX_BCRS_ROWS_W(4)
+            SMAX_BCRS_ROWS_W(5) SMAX_BCRS_ROWS_W(6) SMAX_BCRS_ROWS_W(7) SMAX_BCRS_ROWS_W(8)
+        }
+        return true;
+    });
+#undef SMAX_BCRS_ROWS_W
+#undef SMAX_BCRS_ROWS
+    return false;
 }
 
 // ------------------------------------------------------------ conversion
@@ -761,12 +983,15 @@ int smax_hip_bcrs_spmv(smax_hip_ctx ctx, int value_type,
                         b_h, b_w, h_pad, w_pad);
     if (rc) return rc;
     SMAX_HIP_REQUIRE(ctx, row_ptr && x && y, "smax_hip_bcrs_spmv: null pointer");
-    // b_h, b_w in {1, 2, 4}: the register-blocked product with one right-hand
-    // side (a thread per block row, the same chains; twice as fast as staging
-    // the blocks in LDS on the 96^3 block matrix)
+    // b_h, b_w in {1, 2, 4}: the SpMM with one right-hand side
     if ((b_h == 1 || b_h == 2 || b_h == 4) && (b_w == 1 || b_w == 2 || b_w == 4))
         return smax_hip_bcrs_spmm(ctx, value_type, n_block_rows, b_h, b_w, h_pad, w_pad, col,
                                   row_ptr, val, block_col_major, 1, x, y);
+    if (spmv_by_rows(ctx, value_type, n_block_rows, b_h, b_w, h_pad, w_pad,
+                     block_col_major != 0, col, row_ptr, val, x, y)) {
+        SMAX_HIP_LAUNCHED(ctx, "bcrs_spmv_rows");
+        return SMAX_HIP_SUCCESS;
+    }
     const int64_t rows_per_wg = kBThreads / b_h;
     SMAX_HIP_DISPATCH_VT(value_type, {
         using T = vt<VT>;
@@ -801,6 +1026,16 @@ int smax_hip_bcrs_spmm(smax_hip_ctx ctx, int value_type,
                     (long long)(n_block_rows * h_pad), (long long)k);
     const int64_t threads = n_block_rows * b_h * k;
     const bool cm = block_col_major != 0;
+    if (k == 1 && spmv_by_rows(ctx, value_type, n_block_rows, b_h, b_w, h_pad, w_pad, cm, col,
+                               row_ptr, val, X, Y)) {
+        SMAX_HIP_LAUNCHED(ctx, "bcrs_spmv_rows");
+        return SMAX_HIP_SUCCESS;
+    }
+    if (spmm_in_parts(ctx, value_type, n_block_rows, b_h, b_w, h_pad, w_pad, cm, k, col, row_ptr,
+                      val, X, Y)) {
+        SMAX_HIP_LAUNCHED(ctx, "bcrs_spmm_part");
+        return SMAX_HIP_SUCCESS;
+    }
     // register-blocked shapes: every (b_h, b_w) in {1, 2, 4} x {1, 2, 4}
     const bool reg = (b_h == 1 || b_h == 2 || b_h == 4) && (b_w == 1 || b_w == 2 || b_w == 4);
 #define SMAX_BCRS_REG(H, W)                                                            \

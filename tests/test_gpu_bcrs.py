@@ -459,3 +459,50 @@ def test_transposed_pattern_digit_and_tile_edges(ctx, n_cols, nnz):
     assert_bitwise(got["val"], order.astype(np.float64), "val")
     for h in (T, b):
         h.destroy()
+
+
+@pytest.mark.parametrize("vt", [capi.F64, capi.F32, capi.BF16])
+@pytest.mark.parametrize("cm", [True, False])
+@pytest.mark.parametrize("bh,bw,hp,wp", [(3, 3, 3, 3), (6, 3, 7, 4), (3, 6, 3, 8), (6, 6, 6, 6),
+                                         (5, 5, 5, 5), (10, 5, 11, 5), (7, 7, 7, 7),
+                                         (1, 8, 1, 8), (3, 2, 3, 2), (9, 9, 9, 9),
+                                         (2, 2, 2, 2), (4, 4, 4, 5)])
+def test_bcrs_products_of_any_block_shape(ctx, vt, cm, bh, bw, hp, wp):
+    """SpMV by rows (b_w <= 8) and SpMM in parts of a block: block rows of 0 to
+    9 and of 40 blocks (every remainder of the groups), padded blocks, k below,
+    at and past a run of columns, X and Y one entry past a 16-byte boundary;
+    bit for bit against the oracle."""
+    rng = np.random.default_rng(65)
+    nbr, nbc = 157, 90
+    lens = rng.integers(0, 10, nbr)
+    lens[3::17] = 40
+    row_ptr = np.zeros(nbr + 1, np.int32)
+    row_ptr[1:] = np.cumsum(lens)
+    col = np.concatenate([np.sort(rng.choice(nbc, n, replace=False)) for n in lens]
+                         ).astype(np.int32)
+    val = vals_for(vt, rng.uniform(-1.0, 1.0, int(row_ptr[-1]) * hp * wp))
+    xt = np.float64 if vt == capi.F64 else np.float32
+    d = [ctx.upload(a) for a in (col, row_ptr, val)]
+    rows = (np.arange(nbr * hp) % hp) < bh
+    x = rng.uniform(-1.0, 1.0, nbc * wp).astype(xt)
+    dx, dy = ctx.upload(x), ctx.zeros(nbr * hp, xt)
+    ctx.bcrs_spmv(vt, nbr, bh, bw, hp, wp, *d, cm, dx, dy)
+    want = oracle.bcrs_spmv(nbr, bh, bw, hp, wp, col, row_ptr, val, cm, x)
+    assert_bitwise(ctx.download(dy)[rows], want[rows], "spmv")
+    dx.free()
+    dy.free()
+    for k in (1, 2, 3, 4, 5, 8, 11, 32):
+        X = rng.uniform(-1.0, 1.0, nbc * wp * k).astype(xt)
+        dX = ctx.upload(np.concatenate([X[:1], X]))
+        dY = ctx.zeros(nbr * hp * k + 1, xt)
+        ctx.bcrs_spmm(vt, nbr, bh, bw, hp, wp, *d, cm, k, dX.ptr + X.itemsize,
+                      dY.ptr + X.itemsize)
+        want = oracle.bcrs_spmm(nbr, bh, bw, hp, wp, col, row_ptr, val, cm, k, X)
+        rk = np.repeat(rows, k)
+        got = ctx.download(dY)[1:]
+        assert_bitwise(got[rk], want[rk], f"spmm k={k}")
+        assert not got[~rk].any(), f"spmm k={k} wrote padding rows"
+        dX.free()
+        dY.free()
+    for a in d:
+        a.free()
