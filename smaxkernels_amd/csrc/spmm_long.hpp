@@ -69,27 +69,37 @@ struct LongRows {
 // and chains by itself pays a memory round trip every eight entries: a row of
 // 2000 entries took 128 us, longer than all other rows of a matrix of 40,013
 // (16 us).  Here all lanes gather X runs, a tile of R x NT runs (at most NT
-// entries) ahead, into LDS, and the row's lanes chain them from there, about
-// 20 cycles an entry; the next tile's gathers are in flight meanwhile.  The
+// entries) ahead, into LDS, column by column; a lane per column then chains
+// its entries from there, which lie side by side, at about 11 cycles an entry
+// (6 of them the fma), the next tile's gathers in flight meanwhile.  The
 // chain's order, and so Y, is unchanged.  Wavefronts for the many rows that
-// are just long: three of a workgroup's four would only wait.  CRS SpMM with a
-// plan, 1,000,000- and 200,003-row band matrices, FP32 k = 32: 0.398 -> 0.349
-// and 0.212 -> 0.082 ms; every long row a workgroup 0.401 and 0.085, R = 4
-// 0.364 and 0.085, rows from 256 entries on only 0.372 and 0.086, workgroups
-// from 1024 on 0.349 and 0.085.
+// are just long: three of a workgroup's four would only wait.
 //   entry j of the row: column col[base + j * stride], value val[...] alike;
-//   xs, vs: R * NT * Q and NT entries of LDS (xs 16-byte aligned).
-constexpr int kLongRuns = 2;
+//   lds: LongRowLds<A, Q, NT>::kStore elements, 16-byte aligned.
+constexpr int kLongRuns = 4;
+constexpr int kLongCols = 64;  // columns of a pass, a lane of one wavefront each
+
+template <typename A, int Q, int NT>
+struct LongRowLds {
+    static constexpr int kUnit = 16 / static_cast<int>(sizeof(A));
+    // Columns lie an odd number of 16-byte units apart: 16 lanes' reads take
+    // all banks once.
+    static constexpr int kXs = NT * kLongRuns * Q + (kLongCols + Q) * kUnit;
+    static constexpr int kStore = kXs + NT;
+};
 
 template <int VT, int Q, int NT>
 __device__ __forceinline__ void long_row(
-    typename vt<VT>::vec_t *xs, typename vt<VT>::vec_t *vs, int tid, int32_t len, int64_t base,
-    int64_t stride, const int32_t *__restrict__ col, const typename vt<VT>::val_t *__restrict__ val,
-    int64_t k, const typename vt<VT>::vec_t *__restrict__ X, int64_t ldx,
+    typename vt<VT>::vec_t *lds, int tid, int32_t len, int64_t base, int64_t stride,
+    const int32_t *__restrict__ col, const typename vt<VT>::val_t *__restrict__ val, int64_t k,
+    const typename vt<VT>::vec_t *__restrict__ X, int64_t ldx,
     typename vt<VT>::vec_t *__restrict__ y) {
     using T = vt<VT>;
     using A = typename T::vec_t;
-    constexpr int R = kLongRuns;
+    using V = typename T::val_t;
+    using L = LongRowLds<A, Q, NT>;
+    constexpr int R = kLongRuns, U = 8;
+    A *const xs = lds, *const vs = lds + L::kXs;
     const auto barrier = [] {
         if constexpr (NT > kWave) {
             __syncthreads();
@@ -98,78 +108,74 @@ __device__ __forceinline__ void long_row(
             __builtin_amdgcn_wave_barrier();
         }
     };
-    const int64_t lanes = (k + Q - 1) / Q;
-    for (int64_t l0 = 0; l0 < lanes; l0 += NT) {
-        const int g = static_cast<int>(lanes - l0 < NT ? lanes - l0 : NT);
-        const int most = NT * R / g;
-        const int ept = most < NT ? most : NT;  // entries per tile
-        int eu[R];      // this thread's entries of a tile
-        int64_t off[R]; // and the first column of its run of each
+    const int32_t passes = static_cast<int32_t>((k + kLongCols - 1) / kLongCols);
+    const int32_t width = static_cast<int32_t>((k + passes - 1) / passes);
+    const int32_t g = (width + Q - 1) / Q;
+    // Entries of a tile: whole groups of the chain, a value per thread.
+    const int32_t most = NT * R / g & ~(U - 1);
+    const int32_t ept = most < NT ? most : NT;
+    const int32_t run = ept + L::kUnit;  // a column's place; U is even in units
+    int32_t eu[R], at[R], off[R];        // this thread's entries, their LDS places, columns
 #pragma unroll
-        for (int u = 0; u < R; ++u) {
-            const int f = u * NT + tid;
-            eu[u] = f / g;
-            off[u] = run_start<Q>(l0 + f % g, k);
-            if (eu[u] >= ept) eu[u] = INT32_MAX / 2;  // none
-        }
+    for (int u = 0; u < R; ++u) {
+        const int32_t f = u * NT + tid;
+        eu[u] = f / g;
+        off[u] = static_cast<int32_t>(run_start<Q>(f - eu[u] * g, width));
+        at[u] = eu[u] < ept ? off[u] * run + eu[u] : -1;
+        if (eu[u] >= ept) eu[u] = 0;  // none: repeats a load
+    }
+    for (int32_t pass = 0; pass < passes; ++pass) {
+        const int64_t v0 = pass * width + width <= k ? pass * width : k - width;
         int32_t c[R];
         A xr[R][Q];
-        A vr = 0;
+        V vr;
+        // Past the row's end its last entry is loaded again: under conditions
+        // the loads would be waited for where their results merge.
         const auto load_columns = [&](int32_t t0) {
 #pragma unroll
             for (int u = 0; u < R; ++u)
-                if (t0 + eu[u] < len) c[u] = col[base + (t0 + eu[u]) * stride];
+                c[u] = col[base + (t0 + eu[u] < len ? t0 + eu[u] : len - 1) * stride];
         };
         const auto gather = [&](int32_t t0) {
 #pragma unroll
             for (int u = 0; u < R; ++u)
-                if (t0 + eu[u] < len)
-                    load_cols_run<A, Q>(X + static_cast<int64_t>(c[u]) * ldx + off[u], xr[u]);
-            if (tid < ept && t0 + tid < len) vr = T::widen(val[base + (t0 + tid) * stride]);
+                load_cols_run<A, Q>(X + static_cast<int64_t>(c[u]) * ldx + v0 + off[u], xr[u]);
+            vr = val[base + (t0 + tid < len ? t0 + tid : len - 1) * stride];
         };
         load_columns(0);
         gather(0);
         load_columns(ept);
-        A acc[Q];
-#pragma unroll
-        for (int q = 0; q < Q; ++q) acc[q] = 0;
+        A acc = 0;
         for (int32_t t0 = 0; t0 < len; t0 += ept) {
+            // What is past the row's end is -0 * 0, which leaves every
+            // accumulator as it is, signed zeros included.
 #pragma unroll
             for (int u = 0; u < R; ++u)
-                if (t0 + eu[u] < len) store_run<A, Q>(xs + (u * NT + tid) * Q, xr[u]);
-            if (tid < ept) vs[tid] = vr;
+                if (at[u] >= 0) {
+                    const bool in = t0 + eu[u] < len;
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) xs[at[u] + q * run] = in ? xr[u][q] : A(0);
+                }
+            if (tid < ept) vs[tid] = t0 + tid < len ? T::widen(vr) : A(-0.0);
             barrier();
             if (t0 + ept < len) {
                 gather(t0 + ept);
                 load_columns(t0 + 2 * ept);
             }
-            if (tid < g) {
-                const int m = len - t0 < ept ? len - t0 : ept;
-                constexpr int U = 8;
-                int e = 0;
-                for (; e + U <= m; e += U) {
-                    A w[U], b[U][Q];
+            if (tid < width) {
+                const A *px = xs + tid * run;
+                const int32_t m = len - t0 < ept ? len - t0 : ept;
+                for (int32_t e = 0; e < m; e += U) {
+                    A w[U], b[U];
+                    load_run<A, U>(vs + e, w);
+                    load_run<A, U>(px + e, b);
 #pragma unroll
-                    for (int u = 0; u < U; ++u) {
-                        w[u] = vs[e + u];
-                        load_run<A, Q>(xs + ((e + u) * g + tid) * Q, b[u]);
-                    }
-#pragma unroll
-                    for (int u = 0; u < U; ++u)
-#pragma unroll
-                        for (int q = 0; q < Q; ++q) acc[q] = T::fma_(w[u], b[u][q], acc[q]);
-                }
-                for (; e < m; ++e) {
-                    A b[Q];
-                    load_run<A, Q>(xs + (e * g + tid) * Q, b);
-                    const A w = vs[e];
-#pragma unroll
-                    for (int q = 0; q < Q; ++q) acc[q] = T::fma_(w, b[q], acc[q]);
+                    for (int u = 0; u < U; ++u) acc = T::fma_(w[u], b[u], acc);
                 }
             }
             barrier();
         }
-        if (tid < g) store_cols_run<A, Q>(y + run_start<Q>(l0 + tid, k), acc);
+        if (tid < width) y[v0 + tid] = acc;
     }
 }
 
@@ -183,12 +189,12 @@ __device__ __forceinline__ void long_rows(
     const typename vt<VT>::vec_t *__restrict__ X, int64_t ldx,
     typename vt<VT>::vec_t *__restrict__ Y, int64_t ldy) {
     using A = typename vt<VT>::vec_t;
-    __shared__ __align__(16) A xs[256 * kLongRuns * Q];
-    __shared__ A vs[256];
+    constexpr int kWhole = LongRowLds<A, Q, 256>::kStore, kPart = LongRowLds<A, Q, kWave>::kStore;
+    __shared__ __align__(16) A lds[kWhole > 4 * kPart ? kWhole : 4 * kPart];
     const int tid = static_cast<int>(threadIdx.x);
     if (block < rows.whole) {
         const auto r = row_at(block);
-        long_row<VT, Q, 256>(xs, vs, tid, r.len, r.base, stride, col, val, k, X, ldx,
+        long_row<VT, Q, 256>(lds, tid, r.len, r.base, stride, col, val, k, X, ldx,
                              Y + r.row * ldy);
         return;
     }
@@ -196,9 +202,8 @@ __device__ __forceinline__ void long_rows(
     const int64_t i = rows.whole + (block - rows.whole) * 4 + wave;
     if (i >= rows.count) return;  // whole wavefronts
     const auto r = row_at(i);
-    long_row<VT, Q, kWave>(xs + wave * kWave * kLongRuns * Q, vs + wave * kWave,
-                           tid & (kWave - 1), r.len, r.base, stride, col, val, k, X, ldx,
-                           Y + r.row * ldy);
+    long_row<VT, Q, kWave>(lds + wave * kPart, tid & (kWave - 1), r.len, r.base, stride, col, val,
+                           k, X, ldx, Y + r.row * ldy);
 }
 struct LongRowAt {
     int32_t len;
@@ -232,7 +237,10 @@ __device__ __forceinline__ void run_chain(
     };
     if (full > 0) load_full(0, c0, w0);
     for (int32_t j = 0; j < full; j += U) {
-        if (j + U < full) load_full(j + U, c1, w1);
+        // 2-byte values loaded under a condition are waited for at once; the
+        // last group loads itself again (40,013 rows, k = 20: 30.4 -> 26.9 us;
+        // 8-byte values 82 -> 89 us at 200,003 rows, k = 10).
+        if (sizeof(V) == 2 || j + U < full) load_full(j + U < full ? j + U : j, c1, w1);
         A xv[U][Q];
 #pragma unroll
         for (int u = 0; u < U; ++u)

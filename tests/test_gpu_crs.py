@@ -387,3 +387,10 @@ def test_spmm_long_rows_and_any_width(ctx, vt, k, planned):
         ctx.crs_plan_destroy(plan)
     for a in (*d, dY):
         a.free()
+
+
+@pytest.mark.parametrize("vt", [capi.F64, capi.F32, capi.BF16])
+@pytest.mark.parametrize("k", [61, 63, 65, 127, 129])
+def test_spmm_long_rows_pass_edges(ctx, vt, k):
+    """Widths around the 64 columns that one pass over a long row covers."""
+    test_spmm_long_rows_and_any_width(ctx, vt, k, True)
