@@ -19,7 +19,7 @@
 //    T = 256, W = 1024 for rows of even length, and single-wave blocks,
 //    T = 64, W = 512, when the longest row exceeds 4x the mean: a wave then
 //    waits at its own tiles' barriers only and pipelines its long rows (4M-row
-//    band matrix, FP64: 0.666 ms against 0.766; BF16 values 0.454 against
+//    band matrix, FP64: 0.657 ms against 0.766; BF16 values 0.443 against
 //    0.692; the 512^2 Laplacian and a 27-point stencil run 6.0 / 25.5 us with
 //    the wide blocks against 6.5 / 28.2 us).
 #include <algorithm>
@@ -31,12 +31,21 @@
 #include "scan.hpp"
 #include "spmm_long.hpp"
 
+namespace smaxhip {
+// The rows of `from` entries and more, first in the plan's row order: the
+// SpMV's first `blocks` (a multiple of 8) workgroups take one each.
+struct FirstRows {
+    int32_t count = 0, blocks = 0, from = INT32_MAX;
+};
+}  // namespace smaxhip
+
 struct smax_hip_crs_plan_s {
     int64_t n_rows = 0, nnz = 0, n_blocks = 0;
     int32_t block_threads = 256;     // row-block geometry: 256 (wide) or 64 (narrow)
     int32_t *block_start = nullptr;  // n_blocks + 1 row indices
     int32_t *row_order = nullptr;    // row-major SpMM execution order (n_rows)
     smaxhip::LongRows long_rows;     // how many rows, first in row_order, are long
+    smaxhip::FirstRows first;        // the SpMV's share of them
 };
 
 namespace smaxhip {
@@ -89,19 +98,15 @@ __global__ __launch_bounds__(kCrsThreads) void crs_spmv_lane(
 // ------------------------------------------------------------ blocked
 // One long row by one wavefront: tiles of TILE entries (half the arrays) go
 // through LDS as in crs_spmv_blocked, but the next tile's columns, values and
-// x entries are requested while this one's chain runs, and the chain reads LDS
-// 32 bytes ahead of its fmas instead of waiting for each entry's read.  What
-// bounds it is that chain, one fma after another in the row's order: 100+
-// cycles an entry when each waits, 31 (FP64) now.  Every lane runs the same
-// chain (broadcast reads).  20,000 rows with rows of up to 2000, FP64: 91 ->
-// 28 us; 300,007 rows, BF16: 117 -> 49; 4,000,000, FP64: 729 -> 666.  Tiles
-// of 512 need the registers of one more wavefront per SIMD (BF16, 4,000,000
-// rows: 482 us against 454), of 128 expose more of the gathers (FP64, 300,007:
-// 64 against 61); 64 bytes ahead take 25 us at 20,000 rows but 678 at
-// 4,000,000.
-template <typename A>
-constexpr int kChainAhead = 32 / static_cast<int>(sizeof(A));
-
+// x entries are requested while this one's chain runs.  What bounds it is that
+// chain, one fma after another in the row's order: 6 cycles an entry from
+// registers, 11 (FP32) to 15 (FP64) with groups of eight read from LDS, which
+// the compiler overlaps better than reads placed a group ahead by hand (13 and
+// 23).  Every lane runs the same chain (broadcast reads).  20,000 rows with
+// rows of up to 2000, FP64: 91 us with one entry at a time, 19 now.  FP64
+// takes two groups at once (one: 23 us); with 4-byte entries the registers are
+// worth more (two: BF16, 300,007 rows 44 us against 42).  Tiles of 512: BF16,
+// 4,000,000 rows 12% slower.
 template <int VT, int TILE>
 __device__ __forceinline__ typename vt<VT>::vec_t long_row_sum(
     typename vt<VT>::vec_t *sv, typename vt<VT>::vec_t *sx, int64_t s, int64_t e,
@@ -109,59 +114,55 @@ __device__ __forceinline__ typename vt<VT>::vec_t long_row_sum(
     const typename vt<VT>::vec_t *__restrict__ x) {
     using T = vt<VT>;
     using A = typename T::vec_t;
-    constexpr int PER = TILE / kWave, U = kChainAhead<A>;
+    constexpr int PER = TILE / kWave, U = 8, kAtOnce = sizeof(A) == 8 ? 2 : 1;
     const int tid = static_cast<int>(threadIdx.x);
     int32_t c[PER];
     typename T::val_t v[PER];
     A xv[PER];
+    // Past the row's end its last entry is loaded again: under conditions the
+    // loads would be waited for where their results merge.
+    const auto at = [&](int64_t t0, int u) {
+        const int64_t j = t0 + tid + u * kWave;
+        return j < e ? j : e - 1;
+    };
     const auto load_columns = [&](int64_t t0) {
 #pragma unroll
-        for (int u = 0; u < PER; ++u)
-            if (t0 + tid + u * kWave < e) c[u] = ld_stream(col + t0 + tid + u * kWave);
+        for (int u = 0; u < PER; ++u) c[u] = ld_stream(col + at(t0, u));
     };
     const auto gather = [&](int64_t t0) {
 #pragma unroll
-        for (int u = 0; u < PER; ++u)
-            if (t0 + tid + u * kWave < e) {
-                v[u] = ld_stream(val + t0 + tid + u * kWave);
-                xv[u] = x[c[u]];
-            }
+        for (int u = 0; u < PER; ++u) {
+            v[u] = ld_stream(val + at(t0, u));
+            xv[u] = x[c[u]];
+        }
     };
     load_columns(s);
     gather(s);
     load_columns(s + TILE);
     A acc = 0;
     for (int64_t t0 = s; t0 < e; t0 += TILE) {
+        // What is past the row's end is -0 * 0, which leaves the accumulator
+        // as it is, signed zeros included.
 #pragma unroll
-        for (int u = 0; u < PER; ++u)
-            if (t0 + tid + u * kWave < e) {
-                sv[tid + u * kWave] = T::widen(v[u]);
-                sx[tid + u * kWave] = xv[u];
-            }
+        for (int u = 0; u < PER; ++u) {
+            const bool in = t0 + tid + u * kWave < e;
+            sv[tid + u * kWave] = in ? T::widen(v[u]) : A(-0.0);
+            sx[tid + u * kWave] = in ? xv[u] : A(0);
+        }
         __syncthreads();
         if (t0 + TILE < e) {
             gather(t0 + TILE);
             load_columns(t0 + 2 * TILE);
         }
         const int nt = static_cast<int>(e - t0 < TILE ? e - t0 : TILE);
-        const int full = nt & ~(2 * U - 1);
-        A w0[U], b0[U], w1[U], b1[U];
-        load_run<A, U>(sv, w0);
-        load_run<A, U>(sx, b0);
-        for (int j = 0; j < full; j += 2 * U) {
-            load_run<A, U>(sv + j + U, w1);
-            load_run<A, U>(sx + j + U, b1);
-            __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the fmas
+#pragma unroll kAtOnce
+        for (int j = 0; j < nt; j += U) {
+            A w[U], b[U];
+            load_run<A, U>(sv + j, w);
+            load_run<A, U>(sx + j, b);
 #pragma unroll
-            for (int u = 0; u < U; ++u) acc = T::fma_(w0[u], b0[u], acc);
-            // The last pass reads U entries past the tile, of the arrays' other half.
-            load_run<A, U>(sv + j + 2 * U, w0);
-            load_run<A, U>(sx + j + 2 * U, b0);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = 0; u < U; ++u) acc = T::fma_(w1[u], b1[u], acc);
+            for (int u = 0; u < U; ++u) acc = T::fma_(w[u], b[u], acc);
         }
-        for (int j = full; j < nt; ++j) acc = T::fma_(sv[j], sx[j], acc);
         __syncthreads();
     }
     return acc;
@@ -173,17 +174,28 @@ __global__ __launch_bounds__(NT) void crs_spmv_blocked(
     const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col,
     const typename vt<VT>::val_t *__restrict__ val,
     const typename vt<VT>::vec_t *__restrict__ x,
-    typename vt<VT>::vec_t *__restrict__ y) {
+    typename vt<VT>::vec_t *__restrict__ y, FirstRows first, const int32_t *__restrict__ order) {
     using T = vt<VT>;
     using A = typename T::vec_t;
     __shared__ __align__(16) A sv[TILE];
     __shared__ __align__(16) A sx[TILE];
     const int tid = threadIdx.x;
-    const int64_t b = xcd_block(blockIdx.x, gridDim.x);
-    const int64_t r0 = block_start[b], r1 = block_start[b + 1];
+    int64_t r0, r1;
+    bool ahead = false;
+    if (NT == kWave && static_cast<int32_t>(blockIdx.x) < first.blocks) {
+        if (static_cast<int32_t>(blockIdx.x) >= first.count) return;
+        r0 = order[blockIdx.x];
+        r1 = r0 + 1;
+        ahead = true;
+    } else {
+        const int64_t b = xcd_block(blockIdx.x - first.blocks, gridDim.x - first.blocks);
+        r0 = block_start[b];
+        r1 = block_start[b + 1];
+    }
     const int64_t s = row_ptr[r0], e = row_ptr[r1];
     if constexpr (NT == kWave) {
         if (r1 - r0 == 1 && e - s >= kCrsLongRow<NT>) {
+            if (!ahead && e - s >= first.from) return;
             const A sum = long_row_sum<VT, TILE / 2>(sv, sx, s, e, col, val, x);
             if (tid == 0) y[r0] = sum;
             return;
@@ -218,8 +230,25 @@ __global__ __launch_bounds__(NT) void crs_spmv_blocked(
         if (has) {
             const int64_t lo = rs > t0 ? rs : t0;
             const int64_t hi = re < t0 + nt ? re : t0 + nt;
-            for (int64_t j = lo; j < hi; ++j)
-                acc = T::fma_(sv[j - t0], sx[j - t0], acc);
+            int j = static_cast<int>(lo - t0);
+            const int m = static_cast<int>(hi - t0);
+            if constexpr (NT == kWave) {
+                // Four entries' LDS reads at once.  A block waits for its
+                // longest row, which waited for each entry: 300,007 rows, FP64
+                // 51 -> 44 us, BF16 42 -> 36; 1,000,000, FP64 139 -> 126.
+                constexpr int U = 4;
+                for (; j + U <= m; j += U) {
+                    A w[U], b[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        w[u] = sv[j + u];
+                        b[u] = sx[j + u];
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u) acc = T::fma_(w[u], b[u], acc);
+                }
+            }
+            for (; j < m; ++j) acc = T::fma_(sv[j], sx[j], acc);
         }
         __syncthreads();
     }
@@ -536,6 +565,22 @@ static int build_row_order(smax_hip_ctx ctx, int64_t n_rows, int64_t nnz,
     return SMAX_HIP_SUCCESS;
 }
 
+// Which rows' workgroups come first in the one-wavefront SpMV.  In row order a
+// long row may start when the others are nearly done, and its chain then adds
+// to their time; in large matrices (`from` is an entry for every 16,000) the
+// longest row no longer decides it and the row order's shared x band does:
+// 300,007 rows, FP64 61 -> 52 us, 1,000,000 143 -> 137; with an entry for
+// every 64,000, 4,000,000 rows took 684 us instead of 666.
+static FirstRows first_rows(int64_t nnz, int64_t n_rows, const std::vector<int32_t> &rp) {
+    FirstRows f;
+    const int64_t from = std::max({kLongestRow, long_row_from(nnz, n_rows), nnz / 16000});
+    for (int64_t r = 0; r < n_rows; ++r) f.count += rp[r + 1] - rp[r] >= from;
+    if (f.count == 0) return f;
+    f.blocks = (f.count + 7) / 8 * 8;
+    f.from = static_cast<int32_t>(from);
+    return f;
+}
+
 }  // namespace smaxhip
 
 using namespace smaxhip;
@@ -793,6 +838,7 @@ int smax_hip_crs_plan_create(smax_hip_ctx ctx, int64_t n_rows, int64_t nnz,
     p->block_start = starts;
     p->row_order = order;
     p->long_rows = longs;
+    if (narrow) p->first = first_rows(nnz, n_rows, rp);
     *out = p;
     return SMAX_HIP_SUCCESS;
 }
@@ -834,15 +880,15 @@ int smax_hip_crs_spmv(smax_hip_ctx ctx, int value_type, int64_t n_rows,
         auto xv = static_cast<const typename T::vec_t *>(x);
         auto yv = static_cast<typename T::vec_t *>(y);
         if (plan) {
-            const dim3 g(static_cast<unsigned>(plan->n_blocks));
+            const dim3 g(static_cast<unsigned>(plan->n_blocks + plan->first.blocks));
             if (plan->block_threads == kBlkNarrowThreads)
                 hipLaunchKernelGGL((crs_spmv_blocked<VT, kBlkNarrowThreads, kBlkNarrowTile>), g,
                                    dim3(kBlkNarrowThreads), 0, ctx->stream, plan->block_start,
-                                   row_ptr, col, v, xv, yv);
+                                   row_ptr, col, v, xv, yv, plan->first, plan->row_order);
             else
                 hipLaunchKernelGGL((crs_spmv_blocked<VT, kBlkWideThreads, kBlkWideTile>), g,
                                    dim3(kBlkWideThreads), 0, ctx->stream, plan->block_start,
-                                   row_ptr, col, v, xv, yv);
+                                   row_ptr, col, v, xv, yv, FirstRows{}, nullptr);
             SMAX_HIP_LAUNCHED(ctx, "crs_spmv_blocked");
         } else {
             hipLaunchKernelGGL((crs_spmv_lane<VT>), grid_for(n_rows, kCrsThreads),
