@@ -1338,6 +1338,13 @@ __device__ __forceinline__ void load_cols(const A *__restrict__ p, int64_t k, A 
 // blocks to LDS.
 constexpr int kSddmmIters = 8;  // at most: 2048 lines a workgroup
 
+// Lines of M results load all their operand rows before the sums where 64
+// bytes a row or less leave the registers for it; by itself the compiler keeps
+// two or three loads in flight (96^3, 4x4, 4-byte entries, k = 8: 302 -> 266
+// us; 64^3, 3x3, FP64, k = 8: 89 -> 77).
+template <typename A, int KP>
+constexpr bool kSddmmAtOnce = KP * sizeof(A) <= 64;
+
 template <typename A, int KP, int VL, int M>
 __global__ __launch_bounds__(256) void bcrs_sddmm_lines(
     int64_t n_blocks, int64_t n_block_rows, int iters, int n_lines, int lines_real, int n_out,
@@ -1362,6 +1369,7 @@ __global__ __launch_bounds__(256) void bcrs_sddmm_lines(
     }
     __syncthreads();
     constexpr bool kKeep = KP <= 32;  // the line's own operand row stays in registers
+    constexpr bool kAtOnce = kSddmmAtOnce<A, KP>;
     for (int it = 0; it < iters; ++it) {
         const int q = first + it * 256 + static_cast<int>(threadIdx.x);
         const int jl = q / n_lines, i = q - jl * n_lines;
@@ -1375,6 +1383,12 @@ __global__ __launch_bounds__(256) void bcrs_sddmm_lines(
         A f[kKeep ? KP : 1];
         if constexpr (kKeep)
             if (i < lines_real) load_cols<A, KP, VL>(own, k, f);
+        const auto halve = [](A (&p)[KP]) {
+#pragma unroll
+            for (int off = KP / 2; off >= 1; off >>= 1)
+#pragma unroll
+                for (int v = 0; v < off; ++v) p[v] += p[v + off];
+        };
         auto position = [&](int m) -> A {
             if (i >= lines_real || m >= outs_real) return 0;
             const A *w = others + m * k;
@@ -1400,13 +1414,29 @@ __global__ __launch_bounds__(256) void bcrs_sddmm_lines(
                     }
                 }
             }
-#pragma unroll
-            for (int off = KP / 2; off >= 1; off >>= 1)
-#pragma unroll
-                for (int v = 0; v < off; ++v) p[v] += p[v + off];
+            halve(p);
             return p[0];
         };
-        if constexpr (M > 0) {
+        if constexpr (M > 0 && kAtOnce) {
+            A sums[M] = {};
+            if (i < lines_real) {
+                A b[M][KP];
+#pragma unroll
+                for (int m = 0; m < M; ++m)
+                    load_cols<A, KP, VL>(others + (m < outs_real ? m : 0) * k, k, b[m]);
+                __builtin_amdgcn_sched_barrier(0);  // every row requested before the sums
+#pragma unroll
+                for (int m = 0; m < M; ++m) {
+                    A p[KP];
+#pragma unroll
+                    for (int v = 0; v < KP; ++v)
+                        p[v] = __builtin_elementwise_fma(f[v], b[m][v], A(0));
+                    halve(p);
+                    if (m < outs_real) sums[m] = p[0];
+                }
+            }
+            store_run<A, M>(out, sums);
+        } else if constexpr (M > 0) {
             A sums[M];
 #pragma unroll
             for (int m = 0; m < M; ++m) sums[m] = position(m);
@@ -1438,20 +1468,27 @@ static void launch_bcrs_sddmm_lines(smax_hip_ctx ctx, const smax_hip_bcrs_info &
 
 // 16-byte loads when every operand row is 16-byte aligned; 16-byte stores for
 // lines of four results.
+template <typename A, int KP, int VL>
+static void launch_bcrs_sddmm_vl(smax_hip_ctx ctx, const smax_hip_bcrs_info &in, int64_t k,
+                                 const void *Gm, const void *X, void *dv) {
+    const int64_t out = aligned16(dv, dv) ? (in.block_col_major ? in.h_pad : in.w_pad) : 0;
+    if constexpr (kSddmmAtOnce<A, KP>) {
+        if (out == 2) return launch_bcrs_sddmm_lines<A, KP, VL, 2>(ctx, in, k, Gm, X, dv);
+        if (out == 3) return launch_bcrs_sddmm_lines<A, KP, VL, 3>(ctx, in, k, Gm, X, dv);
+    }
+    if (out == 4) return launch_bcrs_sddmm_lines<A, KP, VL, 4>(ctx, in, k, Gm, X, dv);
+    launch_bcrs_sddmm_lines<A, KP, VL, 0>(ctx, in, k, Gm, X, dv);
+}
+
 template <typename A, int KP>
 static void launch_bcrs_sddmm(smax_hip_ctx ctx, const smax_hip_bcrs_info &in, int64_t k,
                               const void *Gm, const void *X, void *dv) {
     constexpr int Q = 16 / static_cast<int>(sizeof(A));
-    const bool four = (in.block_col_major ? in.h_pad : in.w_pad) == 4 && aligned16(dv, dv);
     if constexpr (KP >= Q) {
-        if (k % Q == 0 && aligned16(Gm, X)) {
-            if (four) launch_bcrs_sddmm_lines<A, KP, Q, 4>(ctx, in, k, Gm, X, dv);
-            else launch_bcrs_sddmm_lines<A, KP, Q, 0>(ctx, in, k, Gm, X, dv);
-            return;
-        }
+        if (k % Q == 0 && aligned16(Gm, X))
+            return launch_bcrs_sddmm_vl<A, KP, Q>(ctx, in, k, Gm, X, dv);
     }
-    if (four) launch_bcrs_sddmm_lines<A, KP, 1, 4>(ctx, in, k, Gm, X, dv);
-    else launch_bcrs_sddmm_lines<A, KP, 1, 0>(ctx, in, k, Gm, X, dv);
+    launch_bcrs_sddmm_vl<A, KP, 1>(ctx, in, k, Gm, X, dv);
 }
 
 template <typename A>
