@@ -785,3 +785,25 @@ def test_scs_apply_long_chunks_by_workgroups(ctx, vt, C_, sigma, tails, x0):
     for d in (dx, dy, dy2):
         d.free()
     s.destroy()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.uint16])
+@pytest.mark.parametrize("extra", [0, 1, 63])
+def test_refresh_values_around_the_wide_kernel(ctx, dtype, extra):
+    """Layouts of just under and just over 2^20 elements, where a lane takes
+    eight elements instead of one, with an uneven last workgroup."""
+    for n in ((1 << 15) - 64, (1 << 15) + extra):
+        L = np.full(n, 32)
+        L[5] = 40
+        L[7::64] = 0
+        rp = np.concatenate([[0], np.cumsum(L)]).astype(np.int32)
+        col = (np.arange(rp[-1]) % n).astype(np.int32)
+        s = gpu_scs(ctx, Csr(n, n, rp, col, np.zeros(rp[-1], dtype)), 64, 256)
+        new = np.random.default_rng(n).integers(1, 1 << 14, rp[-1]).astype(dtype)
+        d = ctx.upload(new)
+        s.refresh_values(d)
+        got = s.arrays(dtype)
+        src = got["src_index"]
+        assert_bitwise(got["val"], np.where(src >= 0, new[src], 0).astype(dtype), "values")
+        d.free()
+        s.destroy()
