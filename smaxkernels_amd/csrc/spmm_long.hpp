@@ -46,8 +46,9 @@ inline int64_t long_row_from(int64_t nnz, int64_t n_rows) {
 
 // In SELL a long slot alone also pays for its columns and values, one line an
 // entry that the other slots of its chunk would share; in large matrices, where
-// the longest rows no longer decide the time, fewer slots are long.
-// 1,000,000 rows, from 128 / 512 / 1024 / 1400 entries on: FP32 k = 32 0.359 /
+// the longest rows no longer decide the time, fewer slots are long.  Measured
+// with 16-byte runs in LDS, before a lane took one column (now 0.312, 0.355 and
+// 0.082 ms with this rule): 1,000,000 rows, from 128 / 512 / 1024 / 1400 entries on: FP32 k = 32 0.359 /
 // 0.337 / 0.322 / 0.329 ms (none: 0.371), FP64 k = 16 0.468 / 0.404 / 0.372 /
 // 0.362 (0.382); 200,003 rows, FP64 k = 10: 0.089 / 0.094 / 0.146 / 0.169
 // (0.343).
