@@ -32,17 +32,19 @@
 #include "spmm_long.hpp"
 
 namespace smaxhip {
-// The rows of `from` entries and more, first in the plan's row order: the
-// SpMV's first `blocks` (a multiple of 8) workgroups take one each.
+// The first `count` rows of the plan's row order, its longest: the SpMV's first
+// `blocks` (a multiple of 8) workgroups take one each.  Their own blocks are
+// marked in block_start when the plan is made, so that each row is run once
+// whatever row_ptr says by then.
 struct FirstRows {
-    int32_t count = 0, blocks = 0, from = INT32_MAX;
+    int32_t count = 0, blocks = 0;
 };
 }  // namespace smaxhip
 
 struct smax_hip_crs_plan_s {
     int64_t n_rows = 0, nnz = 0, n_blocks = 0;
     int32_t block_threads = 256;     // row-block geometry: 256 (wide) or 64 (narrow)
-    int32_t *block_start = nullptr;  // n_blocks + 1 row indices
+    int32_t *block_start = nullptr;  // n_blocks + 1 row indices, ~row: a first row's block
     int32_t *row_order = nullptr;    // row-major SpMM execution order (n_rows)
     smaxhip::LongRows long_rows;     // how many rows, first in row_order, are long
     smaxhip::FirstRows first;        // the SpMV's share of them
@@ -181,21 +183,20 @@ __global__ __launch_bounds__(NT) void crs_spmv_blocked(
     __shared__ __align__(16) A sx[TILE];
     const int tid = threadIdx.x;
     int64_t r0, r1;
-    bool ahead = false;
     if (NT == kWave && static_cast<int32_t>(blockIdx.x) < first.blocks) {
         if (static_cast<int32_t>(blockIdx.x) >= first.count) return;
         r0 = order[blockIdx.x];
         r1 = r0 + 1;
-        ahead = true;
     } else {
         const int64_t b = xcd_block(blockIdx.x - first.blocks, gridDim.x - first.blocks);
-        r0 = block_start[b];
-        r1 = block_start[b + 1];
+        const int32_t b0 = block_start[b], b1 = block_start[b + 1];
+        if (NT == kWave && b0 < 0) return;  // one of the first workgroups' rows
+        r0 = b0;
+        r1 = NT == kWave && b1 < 0 ? ~b1 : b1;
     }
     const int64_t s = row_ptr[r0], e = row_ptr[r1];
     if constexpr (NT == kWave) {
         if (r1 - r0 == 1 && e - s >= kCrsLongRow<NT>) {
-            if (!ahead && e - s >= first.from) return;
             const A sum = long_row_sum<VT, TILE / 2>(sv, sx, s, e, col, val, x);
             if (tid == 0) y[r0] = sum;
             return;
@@ -271,13 +272,17 @@ __global__ void crs_block_flags(int64_t n_rows, const int32_t *__restrict__ row_
     flag[r] = f;
 }
 
+// first_from: rows of so many entries, each a block of its own, are first rows.
 __global__ void crs_block_starts(int64_t n_rows,
+                                 const int32_t *__restrict__ row_ptr, int64_t first_from,
                                  const int32_t *__restrict__ flag,
                                  const int32_t *__restrict__ pos,
                                  int32_t *__restrict__ block_start) {
     const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (r >= n_rows) return;
-    if (flag[r]) block_start[pos[r] - 1] = static_cast<int32_t>(r);
+    const int32_t start = static_cast<int32_t>(r);
+    if (flag[r])
+        block_start[pos[r] - 1] = row_ptr[r + 1] - row_ptr[r] >= first_from ? ~start : start;
     if (r == n_rows - 1) block_start[pos[r]] = static_cast<int32_t>(n_rows);
 }
 
@@ -571,14 +576,8 @@ static int build_row_order(smax_hip_ctx ctx, int64_t n_rows, int64_t nnz,
 // longest row no longer decides it and the row order's shared x band does:
 // 300,007 rows, FP64 61 -> 52 us, 1,000,000 143 -> 137; with an entry for
 // every 64,000, 4,000,000 rows took 684 us instead of 666.
-static FirstRows first_rows(int64_t nnz, int64_t n_rows, const std::vector<int32_t> &rp) {
-    FirstRows f;
-    const int64_t from = std::max({kLongestRow, long_row_from(nnz, n_rows), nnz / 16000});
-    for (int64_t r = 0; r < n_rows; ++r) f.count += rp[r + 1] - rp[r] >= from;
-    if (f.count == 0) return f;
-    f.blocks = (f.count + 7) / 8 * 8;
-    f.from = static_cast<int32_t>(from);
-    return f;
+static int64_t first_from(int64_t nnz, int64_t n_rows) {
+    return std::max({kLongestRow, long_row_from(nnz, n_rows), nnz / 16000});
 }
 
 }  // namespace smaxhip
@@ -777,6 +776,16 @@ int smax_hip_crs_plan_create(smax_hip_ctx ctx, int64_t n_rows, int64_t nnz,
     const int32_t window = narrow ? kBlkNarrowTile : kBlkWideTile;
     const int32_t long_row =
         narrow ? kCrsLongRow<kBlkNarrowThreads> : kCrsLongRow<kBlkWideThreads>;
+    int64_t from = INT64_MAX;  // first rows: this long and more
+    FirstRows first;
+    if (narrow) {
+        const int64_t line = first_from(nnz, n_rows);
+        for (int64_t r = 0; r < n_rows; ++r) first.count += rp[r + 1] - rp[r] >= line;
+        if (first.count > 0) {
+            from = line;
+            first.blocks = (first.count + 7) / 8 * 8;
+        }
+    }
     int32_t *flag = nullptr, *tmp = nullptr, *starts = nullptr;
     int rc = dev_alloc(ctx, reinterpret_cast<void **>(&flag),
                        sizeof(int32_t) * n_rows, "crs plan");
@@ -814,7 +823,8 @@ int smax_hip_crs_plan_create(smax_hip_ctx ctx, int64_t n_rows, int64_t nnz,
         }
         if (!rc) {
             hipLaunchKernelGGL(crs_block_starts, grid_for(n_rows, 256), dim3(256),
-                               0, ctx->stream, n_rows, flag2, flag, starts);
+                               0, ctx->stream, n_rows, row_ptr, from,
+                               flag2, flag, starts);
             rc = check_launch(ctx, "crs_block_starts");
         }
         (void)hipStreamSynchronize(ctx->stream);
@@ -838,7 +848,7 @@ int smax_hip_crs_plan_create(smax_hip_ctx ctx, int64_t n_rows, int64_t nnz,
     p->block_start = starts;
     p->row_order = order;
     p->long_rows = longs;
-    if (narrow) p->first = first_rows(nnz, n_rows, rp);
+    p->first = first;
     *out = p;
     return SMAX_HIP_SUCCESS;
 }

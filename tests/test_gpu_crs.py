@@ -394,3 +394,49 @@ def test_spmm_long_rows_and_any_width(ctx, vt, k, planned):
 def test_spmm_long_rows_pass_edges(ctx, vt, k):
     """Widths around the 64 columns that one pass over a long row covers."""
     test_spmm_long_rows_and_any_width(ctx, vt, k, True)
+
+
+def pattern(L, n_cols, vt, seed):
+    rng = np.random.default_rng(seed)
+    rp = np.concatenate([[0], np.cumsum(L)]).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(n_cols, l, replace=False)) for l in L]).astype(np.int32)
+    val = matgen.uniform_f64(seed, rp[-1])
+    val = val if vt == capi.F64 else val.astype(np.float32) if vt == capi.F32 else matgen.to_bf16(val)
+    return rp, col, val
+
+
+def other_patterns():
+    """Row lengths, and the same ones in other orders: two rows exchanged, the
+    long rows permuted among themselves, all rows reversed, every row moved on
+    by one (rows that were long are then empty or short)."""
+    rng = np.random.default_rng(3)
+    L = rng.integers(0, 6, 6000)
+    L[[0, 40, 41, 900, 901, 902, 2500, 5999]] = [600, 300, 1500, 511, 512, 513, 2000, 700]
+    L[1] = 0
+    swapped = L.copy()
+    swapped[[0, 40]] = L[[40, 0]]
+    long = np.flatnonzero(L >= 256)
+    permuted = L.copy()
+    permuted[long] = L[rng.permutation(long)]
+    return L, [swapped, permuted, L[::-1].copy(), np.roll(L, 1)]
+
+
+@pytest.mark.parametrize("vt", VTS)
+def test_crs_spmv_plan_of_another_pattern(ctx, vt):
+    """A plan decides who runs a row, not whether: with the plan of another
+    pattern of the same size every row is still written."""
+    L, others = other_patterns()
+    n, n_cols = L.size, 3000
+    rp = ctx.upload(np.concatenate([[0], np.cumsum(L)]).astype(np.int32))
+    plan = ctx.crs_plan(n, int(L.sum()), rp)
+    vec = np.float64 if vt == capi.F64 else np.float32
+    x = matgen.uniform_f64(8, n_cols).astype(vec)
+    for i, other in enumerate(others):
+        arrays = pattern(other, n_cols, vt, 30 + i)
+        d = [ctx.upload(a) for a in (*arrays, x, np.full(n, np.nan, vec))]
+        ctx.crs_spmv(vt, n, n_cols, int(L.sum()), *d, plan)
+        assert_bitwise(ctx.download(d[4]), oracle.crs_spmv(*arrays, x), f"pattern {i}")
+        for a in d:
+            a.free()
+    ctx.crs_plan_destroy(plan)
+    rp.free()
