@@ -100,6 +100,12 @@ __device__ __forceinline__ void long_row(
     using V = typename T::val_t;
     using L = LongRowLds<A, Q, NT>;
     constexpr int R = kLongRuns, U = 8;
+    // A row that was long when the list was made may be empty by now (a plan
+    // used with another pattern): it has no last entry to load.
+    if (len <= 0) {
+        for (int64_t v = tid; v < k; v += NT) y[v] = 0;
+        return;
+    }
     A *const xs = lds, *const vs = lds + L::kXs;
     const auto barrier = [] {
         if constexpr (NT > kWave) {

@@ -440,3 +440,30 @@ def test_crs_spmv_plan_of_another_pattern(ctx, vt):
             a.free()
     ctx.crs_plan_destroy(plan)
     rp.free()
+
+
+@pytest.mark.parametrize("vt", VTS)
+@pytest.mark.parametrize("k", [1, 3, 10, 32, 70])
+def test_crs_spmm_plan_of_another_pattern(ctx, vt, k):
+    """As for the SpMV; the rows that the plan lists as long have any length
+    here, none included."""
+    L, others = other_patterns()
+    empty = L.copy()  # the entries of all long rows in one other row
+    long = np.flatnonzero(L >= 256)
+    empty[long] = 0
+    empty[7] += L[long].sum()
+    n, n_cols = L.size, 8000
+    rp = ctx.upload(np.concatenate([[0], np.cumsum(L)]).astype(np.int32))
+    plan = ctx.crs_plan(n, int(L.sum()), rp)
+    vec = np.float64 if vt == capi.F64 else np.float32
+    X = matgen.uniform_f64(9, n_cols * k).astype(vec)
+    for i, other in enumerate(others + [empty]):
+        arrays = pattern(other, n_cols, vt, 40 + i)
+        d = [ctx.upload(a) for a in (*arrays, X, np.full(n * k, np.nan, vec))]
+        ctx.crs_spmm(vt, n, n_cols, int(L.sum()), *d[:3], k, True, d[3], k, d[4], k, plan)
+        assert_bitwise(ctx.download(d[4]), np.asarray(oracle.crs_spmm(*arrays, k, True, X)).ravel(),
+                       f"pattern {i}")
+        for a in d:
+            a.free()
+    ctx.crs_plan_destroy(plan)
+    rp.free()
