@@ -38,19 +38,45 @@ inline size_t value_bytes(FloatType t) {
 }
 inline size_t vector_bytes(FloatType t) { return t == FloatType::FLOAT64 ? 8 : 4; }
 
+// A CRS plan, kept from one initialize to the next while the row pointers are
+// the same: by what they hold, since a caller may change them in place or
+// register others at an address used before.
+struct RowPlan {
+    smax_hip_crs_plan plan = nullptr;
+    std::vector<int32_t> row_ptr;  // what it was built for
+    ULL nnz = 0;
+
+    int update(smax_hip_ctx ctx, const CRSMatrix &A, const int32_t *device_row_ptr) {
+        const int32_t *rp = static_cast<const int32_t *>(A.row_ptr);
+        if (plan && nnz == A.nnz && row_ptr.size() == A.n_rows + 1 &&
+            std::equal(row_ptr.begin(), row_ptr.end(), rp))
+            return 0;
+        destroy(ctx);
+        const int rc = report(ctx, smax_hip_crs_plan_create(ctx, A.n_rows, A.nnz, device_row_ptr,
+                                                            &plan),
+                              "CRS plan");
+        if (rc) return rc;
+        row_ptr.assign(rp, rp + A.n_rows + 1);
+        nnz = A.nnz;
+        return 0;
+    }
+    void destroy(smax_hip_ctx ctx) {
+        if (plan) smax_hip_crs_plan_destroy(ctx, plan);
+        plan = nullptr;
+    }
+};
+
 struct DeviceState {
     PLATFORM::HIP::Stream stream;
     DeviceBuffer a0, a1, a2, a3, a4;  // format arrays (see initialize)
     DeviceBuffer x, y;
-    smax_hip_crs_plan plan = nullptr;
-    const void *plan_row_ptr = nullptr;  // host row_ptr the plan was built for
-    ULL plan_rows = 0, plan_nnz = 0;
-    bool use_plan = false;               // CRS: row blocks chosen at initialize
+    RowPlan plan;
+    bool use_plan = false;  // CRS: row blocks chosen at initialize
     // SELL: a handle over the uploaded arrays (slot lengths, execution
     // schedule, tail waves), rebuilt at every initialize
     smax_hip_scs scs = nullptr;
     ~DeviceState() {
-        if (plan) smax_hip_crs_plan_destroy(stream.get(), plan);
+        plan.destroy(stream.get());
         if (scs) smax_hip_scs_destroy(stream.get(), scs);
     }
 };
@@ -134,18 +160,7 @@ inline int initialize(Timers *timers, KernelContext *k, Args *args, Flags *flags
                                                          static_cast<double>(A.n_rows);
         }
         d.use_plan = blocked;
-        if (!rc && blocked &&
-            (!d.plan || d.plan_row_ptr != A.row_ptr || d.plan_rows != A.n_rows ||
-             d.plan_nnz != A.nnz)) {
-            if (d.plan) smax_hip_crs_plan_destroy(ctx, d.plan);
-            d.plan = nullptr;
-            rc |= report(ctx, smax_hip_crs_plan_create(ctx, A.n_rows, A.nnz,
-                                                       d.a0.as<int32_t>(), &d.plan),
-                         "CRS row-block plan");
-            d.plan_row_ptr = A.row_ptr;
-            d.plan_rows = A.n_rows;
-            d.plan_nnz = A.nnz;
-        }
+        if (!rc && blocked) rc |= d.plan.update(ctx, A, d.a0.as<int32_t>());
     }
     x_size = std::max(x_size, args->x.n_rows);
     y_size = std::max(y_size, args->y.n_rows);
@@ -181,7 +196,7 @@ inline int apply(Timers *timers, KernelContext *k, Args *args, Flags *flags,
         const CRSMatrix &A = *args->A.crs;
         st = smax_hip_crs_spmv(ctx, vt, A.n_rows, A.n_cols, A.nnz,
                                d.a0.as<int32_t>(), d.a1.as<int32_t>(), d.a2.get(),
-                               x, y, d.use_plan ? d.plan : nullptr);
+                               x, y, d.use_plan ? d.plan.plan : nullptr);
     }
     return report(ctx, st, "SpMV launch");
 }

@@ -422,6 +422,66 @@ TEST(gpu, spmm_kats) {  // spmm_test.hpp (column-major), spmm_rowmaj_test.hpp
     }
 }
 
+TEST(gpu, pattern_changed_in_place) {
+    // The rows of the registered arrays exchanged in place between two runs:
+    // same pointers, rows and entries, but long rows where short or empty
+    // ones were.  SpMV (row blocks) and row-major SpMM (k = 3), each y whole.
+    const int n = 3000, k = 3;
+    std::vector<int> len(n);
+    for (int r = 0; r < n; ++r) len[r] = (r * 7) % 6;
+    const int at[] = {3, 40, 41, 900, 2500, 2999}, is[] = {600, 300, 1500, 512, 2000, 700};
+    for (int i = 0; i < 6; ++i) len[at[i]] = is[i];
+    std::vector<int> rp(n + 1), col;
+    std::vector<double> val;
+    const auto fill = [&] {
+        col.clear();
+        val.clear();
+        for (int r = 0; r < n; ++r) {
+            rp[r] = static_cast<int>(col.size());
+            for (int j = 0; j < len[r]; ++j) {
+                col.push_back((r + j) % n);
+                val.push_back(1.0 + j % 5);
+            }
+        }
+        rp[n] = static_cast<int>(col.size());
+    };
+    fill();
+    std::vector<double> x(n), y(n), X(n * k), Y(n * k);
+    for (int i = 0; i < n; ++i) x[i] = i % 9 - 4;
+    for (int i = 0; i < n * k; ++i) X[i] = i % 7 - 3;
+    SMAX::Interface smax;
+    smax.register_kernel("spmv", KernelType::SPMV, PlatformType::HIP);
+    smax.register_kernel("spmm", KernelType::SPMM, PlatformType::HIP);
+    auto *v = smax.kernel("spmv"), *m = smax.kernel("spmm");
+    v->register_A(n, n, col.size(), col.data(), rp.data(), val.data());
+    v->register_B(n, x.data());
+    v->register_C(n, y.data());
+    m->register_A(n, n, col.size(), col.data(), rp.data(), val.data());
+    m->register_B(n, k, X.data());
+    m->register_C(n, k, Y.data());
+    m->set_vec_row_major(true);
+    const size_t nnz = col.size();
+    for (int step = 0; step < 3; ++step) {
+        if (step == 1) std::swap(len[3], len[40]);
+        if (step == 2) std::reverse(len.begin(), len.end());
+        const auto *where = col.data();
+        fill();
+        check(col.size() == nnz && col.data() == where, "same arrays");
+        std::fill(y.begin(), y.end(), std::nan(""));
+        std::fill(Y.begin(), Y.end(), std::nan(""));
+        check(v->run() == 0 && m->run() == 0, "run");
+        for (int r = 0; r < n; ++r) {  // small whole numbers: exact
+            double s = 0, S[k] = {};
+            for (int j = rp[r]; j < rp[r + 1]; ++j) {
+                s += val[j] * x[col[j]];
+                for (int q = 0; q < k; ++q) S[q] += val[j] * X[col[j] * k + q];
+            }
+            check(y[r] == s, "SpMV row " + std::to_string(r));
+            for (int q = 0; q < k; ++q) check(Y[r * k + q] == S[q], "SpMM row " + std::to_string(r));
+        }
+    }
+}
+
 TEST(gpu, spmm_column_major_refuses_overrun) {
     // 5 x 3 matrix, column-major with the reference's leading dimension
     // n_rows = 5: X (3 x k) would be read up to (k-1)*5 + 3 > 3k entries, so
