@@ -432,10 +432,17 @@ constexpr int64_t kFewPartials = 1024;
 
 // Sum of partial[0..m), m <= kFewPartials, in every thread of a 256-thread
 // workgroup, in k_reduce's order (a butterfly per 64, then those in turn).
+// *done: ctl[CTL_DONE], the same in every thread.  One thread reads it, since
+// another workgroup of the same launch may store it meanwhile: wavefronts that
+// each read it for themselves could part, and those that stayed would add up
+// what the others had not written.
 template <typename W>
-__device__ __forceinline__ W reduce_few(const W *__restrict__ partial, int64_t m) {
+__device__ __forceinline__ W reduce_few(const W *__restrict__ partial, int64_t m,
+                                        const int64_t *ctl, bool *done) {
     __shared__ W ws[kFewPartials / kWave];
+    __shared__ int stop;
     constexpr int kWaves = kCgThreads / kWave;
+    if (threadIdx.x == 0) stop = ctl[CTL_DONE] != 0;
     const int wave = threadIdx.x / kWave;
     const int groups = static_cast<int>((m + kWave - 1) / kWave);
     for (int g = wave; g < groups; g += kWaves) {
@@ -446,6 +453,7 @@ __device__ __forceinline__ W reduce_few(const W *__restrict__ partial, int64_t m
         if ((threadIdx.x & (kWave - 1)) == 0) ws[g] = v;
     }
     __syncthreads();
+    *done = stop != 0;
     W t = ws[0];
     for (int g = 1; g < groups; ++g) t += ws[g];
     __syncthreads();
@@ -465,10 +473,13 @@ __global__ __launch_bounds__(kCgThreads) void k_few_product(
     const W *__restrict__ p, W *__restrict__ p_new, W *__restrict__ q,
     const W *__restrict__ partial_rr, W *__restrict__ partial_pq, W *__restrict__ scal, int rr_new,
     int rr_old, int64_t *__restrict__ ctl, W stop2) {
-    if (ctl[CTL_DONE]) return;
     W beta = 0;
-    if constexpr (!FIRST) {
-        const W rr = reduce_few(partial_rr, static_cast<int64_t>(gridDim.x));
+    if constexpr (FIRST) {
+        if (ctl[CTL_DONE]) return;  // this launch does not store it
+    } else {
+        bool before;
+        const W rr = reduce_few(partial_rr, static_cast<int64_t>(gridDim.x), ctl, &before);
+        if (before) return;
         const bool done = !(rr > stop2);
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             scal[rr_new] = rr;
@@ -501,8 +512,9 @@ __global__ __launch_bounds__(kCgThreads) void k_few_update(
     int64_t n, const W *__restrict__ scal, int rr, const W *__restrict__ partial_pq,
     W *__restrict__ x, W *__restrict__ r, const W *__restrict__ p, const W *__restrict__ q,
     W *__restrict__ partial_rr, int64_t *__restrict__ ctl) {
-    if (ctl[CTL_DONE]) return;
-    const W pq = reduce_few(partial_pq, static_cast<int64_t>(gridDim.x));
+    bool before;
+    const W pq = reduce_few(partial_pq, static_cast<int64_t>(gridDim.x), ctl, &before);
+    if (before) return;
     const bool bad = !(pq > W(0));
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (bad) {

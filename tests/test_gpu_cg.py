@@ -186,3 +186,57 @@ def test_not_converged_is_reported(ctx):
     rep, _, _ = solve(ctx, A, 64, 1, mixed=False, max_iters=5)
     assert rep.status == capi.ERROR_NOT_CONVERGED
     assert rep.rel_residual > 1e-10
+
+
+def run(ctx, A, b, prm, mixed):
+    rp, col, v = ctx.upload(A.row_ptr), ctx.upload(A.col), ctx.upload(A.val)
+    S = ctx.scs_from_crs(A.n_rows, A.n_cols, A.nnz, rp, col, v, 8, 64, 1)
+    db, dx = ctx.upload(b), ctx.zeros(A.n_rows, np.float64)
+    rep = ctx.cg(S, db, dx, prm, mixed)
+    x = ctx.download(dx)
+    S.destroy()
+    for d in (rp, col, v, db, dx):
+        d.free()
+    return rep, x
+
+
+def params(lo=capi.F64, **k):
+    base = dict(rel_tol=1e-10, max_iters=20000, check_every=10, inner_rel_tol=0.1, max_inner=5000,
+                inner_value_type=lo, keep_diag_f32=int(lo == capi.BF16))
+    return capi.CgParams(**{**base, **k})
+
+
+def assert_same_solve(a, b, n=None):
+    (ra, xa), (rb, xb) = a, b
+    assert (ra.iterations, ra.outer_iterations) == (rb.iterations, rb.outer_iterations)
+    assert ra.rel_residual == rb.rel_residual or n is not None
+    assert np.array_equal(xa[:n].view(np.uint64), xb[:n].view(np.uint64))
+
+
+@pytest.mark.parametrize("n", [9216, 262_144, 262_400])
+@pytest.mark.parametrize("negative,every,iterations", [(-0.2, 64, 9), (-0.5, 64, 5), (-1.0, 1, 0)])
+def test_breakdown_leaves_the_last_iterate(ctx, n, negative, every, iterations):
+    """p.q <= 0 (an indefinite diagonal): each of the solver's four starts ends
+    there without the step, whichever place of a batch it is.  A host CG with
+    the same starts gives the iterate; p.q is at least a fifth of the sum of
+    its terms' magnitudes wherever its sign decides, so rounding decides none,
+    and of ten steps' rounding (1e-16 each, amplified by the step sizes, below
+    10) 1e-9 is far off."""
+    d = 1 + np.arange(n) % 7 / 4.0
+    d[::every] = negative
+    A = matgen.CRS(n, n, np.arange(n + 1, dtype=np.int32), np.arange(n, dtype=np.int32), d)
+    b = matgen.uniform_f64(matgen.SEED_B, n)
+    x, total = np.zeros(n), 0
+    for _ in range(4):
+        r = b - d * x
+        p, rr = r.copy(), r @ r
+        while (pq := p @ (d * p)) > 0:
+            x, r = x + rr / pq * p, r - rr / pq * (d * p)
+            p, rr = r + r @ r / rr * p, r @ r
+            total += 1
+    assert total == iterations
+    runs = [run(ctx, A, b, params(check_every=c), False) for c in (1, 2, 3, 25)]
+    for rep, got in runs:
+        assert rep.status == capi.ERROR_NOT_CONVERGED and rep.iterations == total
+        assert np.abs(got - x).max() <= 1e-9 * max(np.abs(x).max(), 1)
+        assert_same_solve((rep, got), runs[0])
