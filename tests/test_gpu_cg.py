@@ -213,6 +213,45 @@ def assert_same_solve(a, b, n=None):
     assert np.array_equal(xa[:n].view(np.uint64), xb[:n].view(np.uint64))
 
 
+@pytest.mark.parametrize("lo", [capi.F64, capi.F32, capi.BF16])
+@pytest.mark.parametrize("stop", [{}, {"rel_tol": 1e-7}] + [{"max_iters": m} for m in range(1, 9)])
+def test_iterates_do_not_depend_on_the_batch(ctx, lo, stop):
+    """The host looks every check_every iterations; two buffers take turns as
+    p within a batch.  Batches of any length, stops by the residual and by the
+    iteration limit at every place of a batch: the same iterates."""
+    A = matgen.poisson2d(40)
+    b = matgen.uniform_f64(matgen.SEED_B, A.n_rows)
+    runs = [run(ctx, A, b, params(lo, check_every=c, **stop), lo != capi.F64)
+            for c in (1, 2, 3, 7, 10)]
+    for other in runs[1:]:
+        assert_same_solve(other, runs[0])
+
+
+def with_identity_rows(A, more):
+    """diag(A, I): `more` rows with a one on the diagonal after A's."""
+    n = A.n_rows
+    rp = np.concatenate([A.row_ptr, A.row_ptr[-1] + 1 + np.arange(more)]).astype(np.int32)
+    col = np.concatenate([A.col, n + np.arange(more)]).astype(np.int32)
+    return matgen.CRS(n + more, n + more, rp, col, np.concatenate([A.val, np.ones(more)]))
+
+
+@pytest.mark.parametrize("lo", [capi.F64, capi.F32, capi.BF16])
+@pytest.mark.parametrize("grid,more,limit", [(512, 256, 40), (96, 300_000, 20000)])
+def test_small_and_large_loops_give_the_same_iterates(ctx, lo, grid, more, limit):
+    """Systems of up to 262,144 slots run two launches an iteration, larger
+    ones five.  Identity rows with a zero right-hand side add only zeros to
+    every sum, so the first rows' iterates are those of the small system bit
+    for bit: 512^2 is the largest that takes two, 256 rows more take five."""
+    A = matgen.poisson2d(grid)
+    b = matgen.uniform_f64(matgen.SEED_B, A.n_rows)
+    prm = params(lo, max_iters=limit)
+    small = run(ctx, A, b, prm, lo != capi.F64)
+    large = run(ctx, with_identity_rows(A, more), np.concatenate([b, np.zeros(more)]), prm,
+                lo != capi.F64)
+    assert_same_solve(small, large, A.n_rows)
+    assert (large[1][A.n_rows:] == 0).all()
+
+
 @pytest.mark.parametrize("n", [9216, 262_144, 262_400])
 @pytest.mark.parametrize("negative,every,iterations", [(-0.2, 64, 9), (-0.5, 64, 5), (-1.0, 1, 0)])
 def test_breakdown_leaves_the_last_iterate(ctx, n, negative, every, iterations):
