@@ -166,6 +166,18 @@ int dev_alloc(smax_hip_ctx ctx, void **p, size_t bytes, const char *what) {
     return SMAX_HIP_SUCCESS;
 }
 
+// Waits until the current device is idle the way hipFree does, by it: also
+// while a stream is captured in relaxed mode, where hipDeviceSynchronize would
+// end the capture.
+static bool wait_idle() {
+    void *word = nullptr;
+    if (hipMalloc(&word, 1) != hipSuccess) {
+        (void)hipGetLastError();  // not for the next launch's check
+        return false;
+    }
+    return hipFree(word) == hipSuccess;
+}
+
 void dev_free(void *p) {
     if (!p) return;
     BlockPool &pl = pool();
@@ -188,7 +200,7 @@ void dev_free(void *p) {
     int cur = b.device;
     bool idle = hipGetDevice(&cur) == hipSuccess;
     if (idle && cur != b.device) idle = hipSetDevice(b.device) == hipSuccess;
-    if (idle) idle = hipDeviceSynchronize() == hipSuccess;
+    if (idle) idle = wait_idle();
     if (cur != b.device) (void)hipSetDevice(cur);
     if (!idle) {
         (void)hipFree(p);

@@ -72,3 +72,34 @@ def test_handle_destroyed_after_its_context():
     lib, h = c.lib, s.handle
     c.close()
     assert lib.smax_hip_scs_destroy(None, h) == capi.SUCCESS
+
+
+def test_handle_destroyed_during_a_capture(ctx):
+    """In relaxed mode freeing memory is allowed while a stream is captured:
+    a handle that goes then, as by garbage collection, leaves the capture be."""
+    import torch
+    A = matgen.lomax_band(60_000)
+    d = [ctx.upload(a) for a in (A.row_ptr, A.col, A.val)]
+    S, T = (ctx.scs_from_crs(A.n_rows, A.n_cols, A.nnz, *d, 8, 64, 4096) for _ in range(2))
+    x, y = ctx.upload(matgen.uniform_f64(3, A.n_cols)), ctx.zeros(A.n_rows, np.float64)
+    S.apply(capi.F64, x, y, unpermuted=True)
+    want = ctx.download(y)
+    st, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    ctx.set_stream(st.cuda_stream)
+    try:
+        with torch.cuda.graph(g, stream=st, capture_error_mode="relaxed"):
+            S.apply(capi.F64, x, y, unpermuted=True)
+            # without the context: its stream, which is being captured, is not waited for
+            assert ctx.lib.smax_hip_scs_destroy(None, T.handle) == capi.SUCCESS
+            S.apply(capi.F64, x, y, unpermuted=True)
+        for _ in range(3):
+            ctx._check(ctx.lib.smax_hip_zero(ctx.handle, y.ptr, y.nbytes))
+            ctx.sync()
+            g.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(ctx.download(y), want)
+    finally:
+        ctx.set_stream(None)
+    S.destroy()
+    for a in (*d, x, y):
+        a.free()
