@@ -113,6 +113,12 @@ int smax_hip_set_stream(smax_hip_ctx ctx, void *stream);
 void *smax_hip_get_stream(smax_hip_ctx ctx);
 int smax_hip_sync(smax_hip_ctx ctx);
 
+/* Gives back the device memory that the library keeps for its next handles on
+ * the context's device (blocks of 1 MB and more of destroyed handles, at most
+ * 4 GiB).  Other allocators of the process do not see those blocks as free:
+ * call it when one of them runs short.  Waits for the device. */
+int smax_hip_trim(smax_hip_ctx ctx);
+
 /* -------------------------------------------------------------- memory */
 /* Replace transfer_HtoD / transfer_DtoH (src/platforms/cuda/cuda.cuh:12-82);
  * copies are complete when they return. */

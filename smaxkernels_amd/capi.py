@@ -78,6 +78,7 @@ _SIGS = {
     "smax_hip_set_stream": ([vp, vp], C.c_int),
     "smax_hip_get_stream": ([vp], vp),
     "smax_hip_sync": ([vp], C.c_int),
+    "smax_hip_trim": ([vp], C.c_int),
     "smax_hip_malloc": ([vp, C.POINTER(vp), C.c_size_t], C.c_int),
     "smax_hip_free": ([vp, vp], C.c_int),
     "smax_hip_memcpy_h2d": ([vp, vp, vp, C.c_size_t], C.c_int),
@@ -241,6 +242,10 @@ class Context:
 
     def sync(self) -> None:
         self._check(self.lib.smax_hip_sync(self.handle))
+
+    def trim(self) -> None:
+        """Gives back the device memory kept for the next handles."""
+        self._check(self.lib.smax_hip_trim(self.handle))
 
     def empty(self, shape, dtype) -> DeviceArray:
         dtype = np.dtype(dtype)

@@ -64,7 +64,7 @@ int check_launch(smax_hip_ctx ctx, const char *kernel) {
 // A block comes in only after its device is idle, as hipFree would wait for
 // (no stream can still use it, whichever takes it next).  At most kPoolCap
 // bytes a device are held, the oldest leave first; all leave when an
-// allocation fails and with the device's last context.
+// allocation fails, by smax_hip_trim and with the device's last context.
 constexpr size_t kPoolMin = size_t(1) << 20;
 constexpr size_t kPoolCap = size_t(4) << 30;
 constexpr int kPoolDevices = 64;
@@ -462,6 +462,12 @@ void *smax_hip_get_stream(smax_hip_ctx ctx) {
 int smax_hip_sync(smax_hip_ctx ctx) {
     SMAX_HIP_CHECK_CTX(ctx);
     SMAX_HIP_CALL(ctx, hipStreamSynchronize(ctx->stream));
+    return SMAX_HIP_SUCCESS;
+}
+
+int smax_hip_trim(smax_hip_ctx ctx) {
+    SMAX_HIP_CHECK_CTX(ctx);
+    pool_trim(ctx->device);
     return SMAX_HIP_SUCCESS;
 }
 

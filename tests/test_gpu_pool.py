@@ -3,7 +3,10 @@ threads and contexts, gives the same layouts as a first build, and the memory
 goes back with the last context."""
 from __future__ import annotations
 
+import subprocess
+import sys
 import threading
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -103,3 +106,70 @@ def test_handle_destroyed_during_a_capture(ctx):
     S.destroy()
     for a in (*d, x, y):
         a.free()
+
+
+# Its own process: no other context of the device keeps the blocks.
+MEMORY = """
+import sys, torch
+sys.path.insert(0, sys.argv[1])
+from smaxkernels_amd import capi
+
+MB, GB = 1 << 20, 1 << 30
+free = lambda: torch.cuda.mem_get_info()[0]
+
+def handle(c, n):  # 28 bytes a row, and the conversion's scratch
+    ptr = torch.arange(n + 1, dtype=torch.int32, device="cuda")
+    col, val = ptr[:n], torch.ones(n, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    h = c.scs_from_crs(n, n, n, ptr, col, val, 8, 64, 4096)
+    del ptr, col, val
+    torch.cuda.empty_cache()
+    return h
+
+with capi.Context(0) as c:  # what the first use of everything takes
+    handle(c, 4_000_000).destroy()
+
+start = free()
+def held():
+    return start - free()
+def back(what):
+    assert held() < 64 * MB, (what, held())
+def keep(c):
+    handle(c, 8_000_000).destroy()
+    assert held() > 200 * MB, held()
+
+with capi.Context(0) as c:
+    back("a new context")
+    keep(c)
+    c.trim()
+    back("trim")
+    keep(c)
+    p = capi.vp()
+    assert c.lib.smax_hip_malloc(c.handle, capi.C.byref(p), 1 << 50) == capi.ERROR_OUT_OF_MEMORY
+    back("a failed allocation")
+    keep(c)
+    d = capi.Context(0)
+assert held() > 200 * MB, "the other context"
+d.close()
+back("the last context")
+
+with capi.Context(0) as c:
+    hs = [handle(c, 70_000_000) for _ in range(3)]
+    in_use = held()
+    assert in_use > 5.5 * GB, in_use
+    for h in hs:
+        h.destroy()
+    assert 2 * GB < held() < 4 * GB + 64 * MB, held()
+back("the last context")
+print("done")
+"""
+
+
+def test_memory_goes_back():
+    """By free device memory: kept blocks go by trim, a failed allocation (of
+    a size that no device has) and the last context, and what is kept stays
+    within 4 GiB when 5.5 GB are freed."""
+    root = Path(__file__).resolve().parents[1]
+    p = subprocess.run([sys.executable, "-c", MEMORY, str(root)], capture_output=True, text=True,
+                       timeout=100)
+    assert p.returncode == 0 and "done" in p.stdout, p.stdout + p.stderr
