@@ -1243,34 +1243,47 @@ int smax_hip_bcrs_destroy(smax_hip_ctx ctx, smax_hip_bcrs bcrs) {
 namespace smaxhip {
 
 // Block p of `out` = block src_block[p] of `src`, a block being `per` units of
-// type U.  A thread moves kGatherUnits units, 256 apart, with the block of
-// each from a 32-bit division by its workgroup's base.
+// type U.  A thread moves UNITS units, 256 apart; one unit's index is below
+// 2^31, with more the block of each is counted from its workgroup's first.
+// Past the end the last unit is loaded again: the loads are requested
+// together, not one after another.
 //
-// What bounds it: one read and one write of the blocks.  Units of 16 bytes
-// where the block size and alignment allow (value by value, with a 64-bit
-// division each, the 96^3 matrix of 4x4 BF16 blocks took 272 us; now 126; its
-// 417 MB take 75 at the copy rate).
+// What bounds it: one read and one write of the blocks (96^3 matrix of 4x4
+// BF16 blocks, 417 MB: 97 us, 75 at the copy rate), in units of 16 bytes where
+// the block size and alignment allow; in small matrices two dependent loads
+// (10^3: 2.3 us).  Value by value with a 64-bit division each: 278 and 2.3 us.
+// Four units a thread pay below 16 bytes once there are enough of them: 5x5
+// FP32 of 32^3 (5.6 M units) 15.0 -> 12.5 us, 3x3 FP64 (2.0 M) 9.0 -> 8.3,
+// 3x3 BF16 of 16^3 (0.2 M) 2.4 -> 2.6; with 16-byte units they change nothing.
+// (Quad is a built-in vector: an array of HIP's uint4 is kept in LDS, which
+// made 24^3 of 2x2 FP64 blocks 14.9 us, 2.8 now.)
+typedef uint32_t Quad __attribute__((ext_vector_type(4)));
 constexpr int kGatherUnits = 4;
+constexpr int64_t kGatherWide = 1 << 20;
 
-template <typename U>
+template <typename U, int UNITS>
 __global__ __launch_bounds__(256) void bcrs_gather_blocks(
-    int64_t total, int32_t per, const int32_t *__restrict__ src_block,
+    int64_t total, int32_t per, FastDiv by_per, const int32_t *__restrict__ src_block,
     const U *__restrict__ src, U *__restrict__ out) {
-    const int64_t base = static_cast<int64_t>(blockIdx.x) * (256 * kGatherUnits);
-    const int64_t p0 = base / per;
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * (256 * UNITS);
+    const int64_t p0 = UNITS == 1 ? 0 : base / per;
     const int32_t first = static_cast<int32_t>(base - p0 * per);
-    U v[kGatherUnits];
+    const int32_t left = static_cast<int32_t>(total - base < 256 * UNITS ? total - base : 256 * UNITS);
+    int32_t at[UNITS], blk[UNITS];
 #pragma unroll
-    for (int u = 0; u < kGatherUnits; ++u) {
+    for (int u = 0; u < UNITS; ++u) {
         const int32_t q = u * 256 + static_cast<int32_t>(threadIdx.x);
-        if (base + q >= total) break;
-        const int32_t pl = (first + q) / per, t = first + q - pl * per;
-        v[u] = src[static_cast<int64_t>(src_block[p0 + pl]) * per + t];
+        const int32_t i = first + (q < left ? q : left - 1), p = by_per(i);
+        at[u] = i - p * per;
+        blk[u] = src_block[p0 + p];
     }
+    U v[UNITS];
 #pragma unroll
-    for (int u = 0; u < kGatherUnits; ++u) {
-        const int64_t i = base + u * 256 + threadIdx.x;
-        if (i < total) out[i] = v[u];
+    for (int u = 0; u < UNITS; ++u) v[u] = src[static_cast<int64_t>(blk[u]) * per + at[u]];
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+        const int32_t q = u * 256 + static_cast<int32_t>(threadIdx.x);
+        if (q < left) out[base + q] = v[u];
     }
 }
 
@@ -1278,9 +1291,14 @@ template <typename U>
 static void launch_gather_blocks(smax_hip_ctx ctx, int64_t n_blocks, int64_t block_bytes,
                                  const int32_t *src_block, const void *src, void *out) {
     const int64_t per = block_bytes / static_cast<int64_t>(sizeof(U)), total = n_blocks * per;
-    hipLaunchKernelGGL(bcrs_gather_blocks<U>, grid_for(total, 256 * kGatherUnits), dim3(256), 0,
-                       ctx->stream, total, static_cast<int32_t>(per), src_block,
-                       static_cast<const U *>(src), static_cast<U *>(out));
+    const bool one = total < (sizeof(U) == 16 ? INT32_MAX : kGatherWide);
+    const auto launch = [&](auto kernel, int units) {
+        hipLaunchKernelGGL(kernel, grid_for(total, 256 * units), dim3(256), 0, ctx->stream, total,
+                           static_cast<int32_t>(per), fast_div(per), src_block,
+                           static_cast<const U *>(src), static_cast<U *>(out));
+    };
+    if (one) launch(bcrs_gather_blocks<U, 1>, 1);
+    else launch(bcrs_gather_blocks<U, kGatherUnits>, kGatherUnits);
 }
 
 static int gather_blocks(smax_hip_ctx ctx, const smax_hip_bcrs_info &T,
@@ -1291,7 +1309,7 @@ static int gather_blocks(smax_hip_ctx ctx, const smax_hip_bcrs_info &T,
     const uintptr_t all = reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(T.val) |
                           static_cast<uintptr_t>(bytes);
     if (all % 16 == 0)
-        launch_gather_blocks<uint4>(ctx, T.n_blocks, bytes, T.src_block, src, T.val);
+        launch_gather_blocks<Quad>(ctx, T.n_blocks, bytes, T.src_block, src, T.val);
     else if (all % 8 == 0)
         launch_gather_blocks<uint64_t>(ctx, T.n_blocks, bytes, T.src_block, src, T.val);
     else if (all % 4 == 0)

@@ -426,6 +426,29 @@ def test_bcrs_transpose_refresh_unit_widths(ctx, vt, bh, bw, hp, wp, shift):
         h.destroy()
 
 
+@pytest.mark.parametrize("vt", [capi.F64, capi.F32, capi.BF16])
+@pytest.mark.parametrize("b,n_blocks", [(3, 116_508), (3, 116_509), (5, 41_943), (5, 41_944),
+                                        (4, 140_001)])
+def test_bcrs_transpose_refresh_around_four_units(ctx, vt, b, n_blocks):
+    """From 2^20 units of 8 bytes and less a thread moves four: one block below
+    and above that (9 and 25 units a block), and 16-byte units, one a thread."""
+    dt = {capi.F64: np.float64, capi.F32: np.float32, capi.BF16: np.uint16}[vt]
+    rng = np.random.default_rng(b)
+    rp = np.arange(n_blocks * b + 1, dtype=np.int32) * b
+    col = (rng.permutation(n_blocks)[:, None, None] * b + np.zeros((1, b, 1), int)
+           + np.arange(b)).ravel().astype(np.int32)
+    A = gpu_bcrs(ctx, n_blocks * b, n_blocks * b, rp, col, np.zeros(col.size, dt), b, b, b, b, False)
+    T = A.transpose()
+    src = rng.integers(0, 1 << 14, (n_blocks, b * b)).astype(dt)
+    d = ctx.upload(src)
+    T.refresh_values(d)
+    order = ctx.download_ptr(T.info.src_block, n_blocks, np.int32)
+    assert_bitwise(T.arrays(dt)["val"], src[order].ravel())
+    d.free()
+    for h in (T, A):
+        h.destroy()
+
+
 @pytest.mark.parametrize("n_cols", [1, 2, 255, 256, 257, 4097, 65536, 65537, (1 << 17) + 3])
 @pytest.mark.parametrize("nnz", [1, 63, 4095, 4096, 4097, 30011])
 def test_transposed_pattern_digit_and_tile_edges(ctx, n_cols, nnz):
