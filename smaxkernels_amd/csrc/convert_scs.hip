@@ -725,9 +725,12 @@ __global__ __launch_bounds__(256) void k_fill(
 // items: 100,000 rows 14.1 -> 9.8 us, 1,000,000 82 -> 55, transposed 188 ->
 // 182; 200,000 rows, FP64, transposed 33 -> 24.  Below kRefreshWide elements
 // that leaves CUs idle (transposed, 40,013 rows: 4.3 us with one item, 4.9).
+// STREAM: not where the tail waves' copy reads the values next, whose lanes
+// follow one slot each and wait for every entry: 50,000 rows, SELL-32-1, FP64
+// 1043 us for that copy after streaming stores, 609 otherwise.
 constexpr int64_t kRefreshWide = 1 << 20;
 
-template <typename V, int ITEMS>
+template <typename V, int ITEMS, bool STREAM>
 __global__ __launch_bounds__(256) void k_refresh(int64_t n_elem, const int32_t *__restrict__ src,
                                                  const V *__restrict__ crs_val,
                                                  V *__restrict__ val) {
@@ -744,22 +747,21 @@ __global__ __launch_bounds__(256) void k_refresh(int64_t n_elem, const int32_t *
 #pragma unroll
     for (int u = 0; u < ITEMS; ++u)
         if (e0 + u * kWave < n_elem) {
-            if constexpr (ITEMS > 1) __builtin_nontemporal_store(v[u], val + e0 + u * kWave);
+            if constexpr (STREAM) __builtin_nontemporal_store(v[u], val + e0 + u * kWave);
             else val[e0 + u * kWave] = v[u];
         }
 }
 
 template <typename V>
 static int launch_refresh(smax_hip_ctx ctx, int64_t m, const int32_t *src, const void *crs_val,
-                          void *val) {
-    const auto from = static_cast<const V *>(crs_val);
-    const auto to = static_cast<V *>(val);
-    if (m >= kRefreshWide)
-        hipLaunchKernelGGL((k_refresh<V, 8>), grid_for(m, 256 * 8), dim3(256), 0, ctx->stream, m,
-                           src, from, to);
-    else
-        hipLaunchKernelGGL((k_refresh<V, 1>), grid_for(m, 256), dim3(256), 0, ctx->stream, m,
-                           src, from, to);
+                          void *val, bool stream) {
+    const auto launch = [&](auto kernel, int items) {
+        hipLaunchKernelGGL(kernel, grid_for(m, 256 * items), dim3(256), 0, ctx->stream, m, src,
+                           static_cast<const V *>(crs_val), static_cast<V *>(val));
+    };
+    if (m < kRefreshWide) launch(k_refresh<V, 1, false>, 1);
+    else if (stream) launch(k_refresh<V, 8, true>, 8);
+    else launch(k_refresh<V, 8, false>, 8);
     SMAX_HIP_LAUNCHED(ctx, "k_refresh");
     return SMAX_HIP_SUCCESS;
 }
@@ -1310,9 +1312,13 @@ int smax_hip_scs_refresh_values(smax_hip_ctx ctx, smax_hip_scs scs,
         scs->bf16_split = -1;
     }
     if (m == 0) return SMAX_HIP_SUCCESS;
-    const int rc = in.val_bytes == 8   ? launch_refresh<uint64_t>(ctx, m, in.src_index, crs_val, in.val)
-                   : in.val_bytes == 4 ? launch_refresh<uint32_t>(ctx, m, in.src_index, crs_val, in.val)
-                                       : launch_refresh<uint16_t>(ctx, m, in.src_index, crs_val, in.val);
+    const bool stream = scs->tails.n_blocks == 0;
+    int rc;
+    switch (in.val_bytes) {
+    case 8: rc = launch_refresh<uint64_t>(ctx, m, in.src_index, crs_val, in.val, stream); break;
+    case 4: rc = launch_refresh<uint32_t>(ctx, m, in.src_index, crs_val, in.val, stream); break;
+    default: rc = launch_refresh<uint16_t>(ctx, m, in.src_index, crs_val, in.val, stream); break;
+    }
     if (rc) return rc;
     // the tail waves hold copies of their slots' values
     return refresh_tail_values(ctx, scs);

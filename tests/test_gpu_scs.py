@@ -807,3 +807,25 @@ def test_refresh_values_around_the_wide_kernel(ctx, dtype, extra):
         assert_bitwise(got["val"], np.where(src >= 0, new[src], 0).astype(dtype), "values")
         d.free()
         s.destroy()
+
+
+@pytest.mark.parametrize("vt", [capi.F64, capi.F32, capi.BF16])
+@pytest.mark.parametrize("n", [5000, 20_000])
+def test_refresh_of_a_large_layout_with_tail_waves(ctx, vt, n):
+    """SELL-32-1 of heavy-tailed rows: the copy for the tail waves is taken
+    from the values that the refresh has just stored, below and above the
+    2^20 elements from which a lane takes eight."""
+    A = matgen.lomax_band(n)
+    cast = {capi.F64: lambda v: v, capi.F32: lambda v: v.astype(np.float32), capi.BF16: matgen.to_bf16}[vt]
+    val, new = cast(A.val), cast(matgen.uniform_f64(77, A.nnz))
+    d = [ctx.upload(a) for a in (A.row_ptr, A.col, val, new)]
+    S = ctx.scs_from_crs(A.n_rows, A.n_cols, A.nnz, *d[:3], val.dtype.itemsize, 32, 1)
+    assert S.tails()[0] > 0 and (S.info.n_elements >= 1 << 20) == (n == 20_000)
+    S.refresh_values(d[3])
+    x = matgen.uniform_f64(3, A.n_cols).astype(np.float64 if vt == capi.F64 else np.float32)
+    dx, dy = ctx.upload(x), ctx.zeros(A.n_rows, x.dtype)
+    S.apply(vt, dx, dy, unpermuted=True)
+    assert_bitwise(ctx.download(dy), oracle.crs_spmv(A.row_ptr, A.col, new, x))
+    S.destroy()
+    for a in (*d, dx, dy):
+        a.free()
