@@ -144,9 +144,9 @@ __device__ __forceinline__ A group_reduce_scatter(A (&cur)[U], int l) {
 template <int GL>
 constexpr int kSddmmChainGroup = GL == 4 || GL == 8 ? 16 : 8;
 
-// What the row kernel takes (slots as in ScsSpmmArgs of the SpMM).
+// What the two kernels for k <= 256 take (slots as in ScsSpmmArgs of the SpMM).
 struct SddmmArgs {
-    int64_t C, n_slots, n_rows, k;
+    int64_t C, n_slots, n_rows, k, n_chunks, n_elements;
     FastDiv by_c;
     int64_t n_long, long_whole, long_cap;  // long slots: count, listed from the front, list size
     int32_t long_from;
@@ -289,12 +289,70 @@ __global__ __launch_bounds__(256) void scs_sddmm_rows(SddmmArgs a, const A *__re
     }
 }
 
+// k <= 256, small layouts: a group of GL lanes per stored element (padding
+// included), in the tree of the row kernel.  A wavefront finds its first
+// element's chunk by search, a lane goes on from there as in the conversion's
+// fill.  Bound by dependent loads: a slot's elements are independent, and here
+// no lane runs more than one, where the row kernel's slots of up to 128 take
+// 16 to 30 us (5000 rows of a heavy-tailed band, k = 5, FP64: 22 us by rows,
+// 4.6 so; 2000 rows, k = 100: 17 and 9).
+template <typename A, int GL, int Q, bool EXACT>
+__global__ __launch_bounds__(256) void scs_sddmm_elements(SddmmArgs a, const A *__restrict__ Gm,
+                                                          const A *__restrict__ X,
+                                                          A *__restrict__ dvals) {
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const int64_t first = (t & ~static_cast<int64_t>(kWave - 1)) / GL, e = t / GL;
+    if (first >= a.n_elements) return;  // whole wavefronts
+    const int l = static_cast<int>(threadIdx.x) % GL;
+    const bool valid = e < a.n_elements;
+    const int32_t to = valid ? a.src[e] : -1;
+    const int64_t k = a.k;
+    const int64_t v0 = EXACT ? l * Q : run_start<Q>(l, k);
+    const int skip = EXACT ? 0 : l * Q < k ? static_cast<int>(l * Q - v0) : Q;
+    A x[Q], g[Q];
+    if (to >= 0) load_cols_run<A, Q>(X + static_cast<int64_t>(a.col[e]) * k + v0, x);
+    int64_t c = wave_row_of(a.chunk_ptr, a.n_chunks, first);
+    A acc = 0;
+    if (to >= 0) {
+        int32_t end = a.chunk_ptr[c + 1];
+        for (int step = 0; e >= end && step < 8; ++step) end = a.chunk_ptr[++c + 1];
+        if (e >= end) c = row_of(a.chunk_ptr, c, a.n_chunks, e);
+        const int32_t off = static_cast<int32_t>(e - a.chunk_ptr[c]);
+        const int64_t slot = c * a.C + (off - a.by_c(off) * a.C);
+        load_cols_run<A, Q>(Gm + static_cast<int64_t>(a.slot_row[slot]) * k + v0, g);
+#pragma unroll
+        for (int i = 0; i < Q; ++i) {
+            const A next = __builtin_elementwise_fma(g[i], x[i], acc);
+            acc = EXACT || i >= skip ? next : acc;
+        }
+    }
+    acc = group_sum<GL>(acc);
+    if (to >= 0 && l == 0) dvals[to] = acc;
+}
+
+// Below this many threads, padding included, one group an element.  Each
+// element then reads its own G row and a lane one store, so the rows win once
+// the chip is full; with one lane an element the larger share of the row
+// kernel's long chains carries further.  By element against by rows, us, on a
+// heavy-tailed band (1.6 elements stored per entry):
+//   k = 3, FP64   220,000 rows 81 / 138, 700,000 (18 M threads) 356 / 357
+//   k = 5         100,000 rows (5.2 M)  52 / 61, 130,000  72 / 69
+//   k = 9          14,000 rows (1.5 M)  14 / 18,  30,000  32 / 28
+//   k = 20         10,000 rows (2.1 M)  15 / 17,  14,000  26 / 18
+//   k = 48          5000 rows (2.1 M)   13 / 17,   7000   21 / 19
+//   k = 200         2000 rows (3.3 M)   18 / 20,   5000   64 / 56
+static bool sddmm_by_element(int64_t n_elements, int64_t lanes) {
+    return n_elements * lanes < (lanes == 1 ? 1 << 24 : lanes == 2 ? 5 << 20 : 1 << 21);
+}
+
 template <typename A, int GL, int Q>
 static void launch_sddmm_rows(smax_hip_ctx ctx, smax_hip_scs S, int64_t k, const void *Gm,
                               const void *X, void *dv) {
     const smax_hip_scs_info &in = S->info;
     SddmmArgs a{};
     a.C = in.C;
+    a.n_chunks = in.n_chunks;
+    a.n_elements = in.n_elements;
     a.n_slots = in.n_rows_padded;
     a.n_rows = in.n_rows;
     a.k = k;
@@ -315,6 +373,16 @@ static void launch_sddmm_rows(smax_hip_ctx ctx, smax_hip_scs S, int64_t k, const
     const auto g = static_cast<const A *>(Gm);
     const auto x = static_cast<const A *>(X);
     const auto d = static_cast<A *>(dv);
+    if (sddmm_by_element(in.n_elements, GL)) {
+        const dim3 per_element = grid_for(in.n_elements * GL, 256);
+        if (k == GL * Q)
+            hipLaunchKernelGGL((scs_sddmm_elements<A, GL, Q, true>), per_element, dim3(256), 0,
+                               ctx->stream, a, g, x, d);
+        else if constexpr (GL > 1)
+            hipLaunchKernelGGL((scs_sddmm_elements<A, GL, Q, false>), per_element, dim3(256), 0,
+                               ctx->stream, a, g, x, d);
+        return;
+    }
     if (k == GL * Q)
         hipLaunchKernelGGL((scs_sddmm_rows<A, GL, Q, true>), grid, dim3(256), 0, ctx->stream, a, g,
                            x, d);

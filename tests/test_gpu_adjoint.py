@@ -269,3 +269,46 @@ def test_sddmm_long_rows_and_any_width(ctx, vt, k, transposed):
     for a in (*d, dv):
         a.free()
     S.destroy()
+
+
+@pytest.mark.parametrize("vt", [capi.F64, capi.F32])
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 8, 9, 12, 13, 16, 20, 31, 32, 33, 48, 64, 65, 100,
+                               128, 129, 200, 256])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_sddmm_by_rows_and_by_element_agree(ctx, vt, k, transposed):
+    """Small layouts take a group of lanes per stored element, large ones a
+    slot's lanes over its elements, in the same tree.  In chunks of 32,768
+    slots the padding makes this matrix large: the same values bit for bit,
+    with rows of 0 to 2000 entries and a column of 650, exact and partial
+    runs, consecutive and scattered destinations."""
+    rng = np.random.default_rng(100 + k)
+    L = rng.integers(0, 4, 700)
+    L[:17] = np.arange(17)
+    L[[20, 21, 22, 23, 300, 301, 302, 699]] = [2000, 127, 128, 129, 511, 513, 1025, 640]
+    L[40:690] = np.maximum(L[40:690], 1)
+    n_cols = 2500
+    rp = np.concatenate([[0], np.cumsum(L)]).astype(np.int32)
+    col = np.concatenate([np.sort(np.concatenate([[7][:l], 8 + rng.choice(n_cols - 8, max(l - 1, 0),
+                                                                          replace=False)]))
+                          for l in L]).astype(np.int32)
+    vec = np.float64 if vt == capi.F64 else np.float32
+    G, X = (rng.uniform(-1, 1, n * k).astype(vec) for n in (L.size, n_cols))
+    d = [ctx.upload(a) for a in (rp, col, np.zeros(rp[-1], vec), G, X)]
+    build = ctx.scs_transpose_from_crs if transposed else ctx.scs_from_crs
+    out = []
+    for C_ in (4, 32768):
+        dv = ctx.upload(np.full(rp[-1], 7, vec))
+        S = build(L.size, n_cols, int(rp[-1]), *d[:3], vec().itemsize, C_, 4096)
+        # below and above every lane count's line
+        lanes = min(max((1 << (k - 1).bit_length()) // 4, 1), 64)
+        if C_ == 4:
+            assert S.info.n_elements * lanes < 1 << 21
+        else:
+            assert S.info.n_elements * lanes >= 1 << 24
+        S.sddmm(vt, k, d[4] if transposed else d[3], d[3] if transposed else d[4], dv)
+        out.append(ctx.download(dv))
+        S.destroy()
+        dv.free()
+    assert_bitwise(out[0], out[1])
+    for a in d:
+        a.free()
