@@ -218,9 +218,15 @@ struct LongRowAt {
 };
 
 // One lane's chains over a row in groups of eight entries, the next group's
-// columns and values requested before this group's X runs; the last, shorter
-// group is loaded at once too.  Any k >= Q.
-template <int VT, int Q>
+// columns and values requested before this group's X runs (LATE: after them);
+// the last, shorter group is loaded at once too.  Any k >= Q.
+//
+// Loads return in order, so X runs requested last are also waited for until
+// the next group has come: where a row's few lanes are all that is left, the
+// longer wait (BF16 without a plan, 5000 rows, k = 8: 80 us, LATE 71).  Where
+// long rows run elsewhere and the others are many, it keeps more requests in
+// flight (FP32 with a plan, 50,000 rows, 2%).
+template <int VT, int Q, bool LATE>
 __device__ __forceinline__ void run_chain(
     int64_t base, int64_t stride, int32_t len, const int32_t *__restrict__ col,
     const typename vt<VT>::val_t *__restrict__ val,
@@ -247,11 +253,15 @@ __device__ __forceinline__ void run_chain(
         // 2-byte values loaded under a condition are waited for at once; the
         // last group loads itself again (40,013 rows, k = 20: 30.4 -> 26.9 us;
         // 8-byte values 82 -> 89 us at 200,003 rows, k = 10).
-        if (sizeof(V) == 2 || j + U < full) load_full(j + U < full ? j + U : j, c1, w1);
+        const auto load_next = [&] {
+            if (sizeof(V) == 2 || j + U < full) load_full(j + U < full ? j + U : j, c1, w1);
+        };
+        if constexpr (!LATE) load_next();
         A xv[U][Q];
 #pragma unroll
         for (int u = 0; u < U; ++u)
             load_cols_run<A, Q>(X + static_cast<int64_t>(c0[u]) * ldx, xv[u]);
+        if constexpr (LATE) load_next();
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll

@@ -337,7 +337,7 @@ __global__ __launch_bounds__(kCrsThreads) void crs_spmm_run(
     const int64_t v = run_start<Q>(l, k);
     const int32_t s = row_ptr[r];
     A acc[Q];
-    run_chain<VT, Q>(s, 1, row_ptr[r + 1] - s, col, val, X + v, ldx, acc);
+    run_chain<VT, Q, !LONG && VT != SMAX_HIP_F64>(s, 1, row_ptr[r + 1] - s, col, val, X + v, ldx, acc);
     store_cols_run<A, Q>(Y + r * ldy + v, acc);
 }
 
@@ -970,8 +970,12 @@ int smax_hip_crs_spmm(smax_hip_ctx ctx, int value_type, int64_t n_rows,
         constexpr int64_t Q = 16 / sizeof(typename vt<VT>::vec_t);
         if (!launch_crs_spmm_rowvec<VT>(ctx, n_rows, k, longs, order, row_ptr, col, val, X,
                                         ldx, Y, ldy)) {
-            // the widest runs that k columns hold
-            if (k >= Q)
+            // the widest runs that k columns hold; narrower ones, and so more
+            // lanes, where no plan takes the long rows out and the chip is not
+            // full (5000 rows, k = 4, FP32 64 -> 56 us, BF16 70 -> 57; 10,000
+            // rows, k = 8 (20,000 lanes), 79 both)
+            const bool few = longs.count == 0 && n_rows * run_lanes(k, Q) < 16384;
+            if (k >= Q && !few)
                 launch_crs_spmm_run<VT, Q>(ctx, n_rows, k, longs, order, row_ptr, col, val,
                                            X, ldx, Y, ldy);
             else if (Q > 2 && k >= 2)

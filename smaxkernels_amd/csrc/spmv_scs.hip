@@ -625,7 +625,7 @@ __global__ __launch_bounds__(kScsThreads) void scs_spmm_run(
     if (LONG && len >= a.long_from) return;
     const int64_t v = run_start<Q>(l, a.k);
     A acc[Q];
-    run_chain<VT, Q>(static_cast<int64_t>(a.chunk_ptr[chunk]) + i, a.C, len, a.col, val, X + v,
+    run_chain<VT, Q, false>(static_cast<int64_t>(a.chunk_ptr[chunk]) + i, a.C, len, a.col, val, X + v,
                      a.k, acc);
     store_cols_run<A, Q>(Y + static_cast<int64_t>(r) * a.k + v, acc);
 }

@@ -467,3 +467,19 @@ def test_crs_spmm_plan_of_another_pattern(ctx, vt, k):
             a.free()
     ctx.crs_plan_destroy(plan)
     rp.free()
+
+
+@pytest.mark.parametrize("vt", VTS)
+@pytest.mark.parametrize("n,k", [(16383, 4), (16384, 4), (16383, 3), (8191, 5), (8192, 8)])
+def test_crs_spmm_unplanned_around_the_narrow_runs(ctx, vt, n, k):
+    """Without a plan, below 16,384 lanes of 16-byte runs a lane takes fewer
+    columns (5 of FP32: two lanes' runs of four, or three of two)."""
+    L = np.random.default_rng(n).integers(0, 12, n)
+    L[[0, 5, n - 1]] = [300, 0, 70]
+    rp, col, val = pattern(L, 2000, vt, 50 + k)
+    X = matgen.uniform_f64(9, 2000 * k).astype(np.float64 if vt == capi.F64 else np.float32)
+    d = [ctx.upload(a) for a in (rp, col, val, X, np.full(n * k, np.nan, X.dtype))]
+    ctx.crs_spmm(vt, n, 2000, int(rp[-1]), *d[:3], k, True, d[3], k, d[4], k)
+    assert_bitwise(ctx.download(d[4]), np.asarray(oracle.crs_spmm(rp, col, val, k, True, X)).ravel())
+    for a in d:
+        a.free()
