@@ -225,7 +225,8 @@ struct LongRowAt {
 // the next group has come: where a row's few lanes are all that is left, the
 // longer wait (BF16 without a plan, 5000 rows, k = 8: 80 us, LATE 71).  Where
 // long rows run elsewhere and the others are many, it keeps more requests in
-// flight (FP32 with a plan, 50,000 rows, 2%).
+// flight (FP32 with a plan, 50,000 rows, 2%), except in FP32 SELL, whose slots
+// share lines (600,000 rows, k = 8: 203 and 172 us).
 template <int VT, int Q, bool LATE>
 __device__ __forceinline__ void run_chain(
     int64_t base, int64_t stride, int32_t len, const int32_t *__restrict__ col,

@@ -602,16 +602,16 @@ struct ScsSpmmArgs {
 // length and no padding term is applied, so Y equals the CRS SpMM bit for
 // bit; without it the chain runs over the padded chunk (padding adds
 // 0 * X[0, v]).  LONG (with LEN): long slots run in workgroups and wavefronts
-// of their own.  One column per lane, four bytes an access, and no such path
-// took 128 us for 40,013 rows, k = 20, BF16 values.
-template <int VT, bool LEN, int Q, bool LONG>
+// of their own, in runs of LQ columns.  One column per lane, four bytes an
+// access, and no such path took 128 us for 40,013 rows, k = 20, BF16 values.
+template <int VT, bool LEN, int Q, int LQ, bool LONG>
 __global__ __launch_bounds__(kScsThreads) void scs_spmm_run(
     ScsSpmmArgs a, const typename vt<VT>::val_t *__restrict__ val,
     const typename vt<VT>::vec_t *__restrict__ X, typename vt<VT>::vec_t *__restrict__ Y) {
     using A = typename vt<VT>::vec_t;
     if constexpr (LONG) {
         if (blockIdx.x < a.longs.blocks()) {
-            long_rows<VT, Q>(a.longs, long_block(a.longs, blockIdx.x), a.listed(), a.C, a.col,
+            long_rows<VT, LQ>(a.longs, long_block(a.longs, blockIdx.x), a.listed(), a.C, a.col,
                              val, a.k, X, a.k, Y, a.k);
             return;
         }
@@ -625,7 +625,7 @@ __global__ __launch_bounds__(kScsThreads) void scs_spmm_run(
     if (LONG && len >= a.long_from) return;
     const int64_t v = run_start<Q>(l, a.k);
     A acc[Q];
-    run_chain<VT, Q, false>(static_cast<int64_t>(a.chunk_ptr[chunk]) + i, a.C, len, a.col, val, X + v,
+    run_chain<VT, Q, VT == SMAX_HIP_F32>(static_cast<int64_t>(a.chunk_ptr[chunk]) + i, a.C, len, a.col, val, X + v,
                      a.k, acc);
     store_cols_run<A, Q>(Y + static_cast<int64_t>(r) * a.k + v, acc);
 }
@@ -768,12 +768,12 @@ static void launch_scs_spmm_vec(smax_hip_ctx ctx, const ScsSpmmArgs &a, dim3 gri
 #undef SMAX_SCS_VEC
 }
 
-template <int VT, int Q>
+template <int VT, int Q, int LQ>
 static void launch_scs_spmm_run(smax_hip_ctx ctx, const ScsSpmmArgs &a, dim3 grid,
                                 const typename vt<VT>::val_t *val,
                                 const typename vt<VT>::vec_t *X, typename vt<VT>::vec_t *Y) {
 #define SMAX_SCS_RUN(LEN, LONG)                                                               \
-    hipLaunchKernelGGL((scs_spmm_run<VT, LEN, Q, LONG>), grid, dim3(kScsThreads), 0, ctx->stream, \
+    hipLaunchKernelGGL((scs_spmm_run<VT, LEN, Q, LONG ? LQ : Q, LONG>), grid, dim3(kScsThreads), 0, ctx->stream, \
                        a, val, X, Y)
     if (a.longs.count > 0) SMAX_SCS_RUN(true, true);
     else if (a.slot_len) SMAX_SCS_RUN(true, false);
@@ -794,7 +794,12 @@ static int launch_scs_spmm(smax_hip_ctx ctx, int64_t C, int64_t n_chunks, int64_
     // k a power of two in [4Q, 64] with 16-byte aligned operands: Q columns
     // per lane, at least 4 lanes per slot
     const bool vec = k >= 4 * Q && k <= 64 && (k & (k - 1)) == 0 && aligned16(X, Y);
-    const int64_t q = k >= Q ? Q : k >= 2 ? 2 : 1;  // columns per lane
+    // Columns per lane: 16 bytes where that leaves three lanes a slot or more.
+    // A wavefront lasts as long as its longest slot, and with one or two lanes
+    // a slot it holds many (1,000,000 rows, SELL-64-4096, FP32, k = 4: 292 us
+    // with four columns a lane, 228 with two, 207 with one; k = 8: 266 and 257,
+    // k = 12: 346 and 407; FP64, k = 4: 301 and 287 with one).
+    const int64_t q = vec || k >= 3 * Q ? Q : k > 4 ? 2 : 1;
     const int64_t lanes = run_lanes(k, q);
     ScsSpmmArgs a{};
     a.C = C;
@@ -803,6 +808,11 @@ static int launch_scs_spmm(smax_hip_ctx ctx, int64_t C, int64_t n_chunks, int64_
     a.k = k;
     a.lanes = lanes;
     a.per = kScsThreads / lanes;
+    // Slots are sorted in windows of a power of two; 42, 18 or 14 of them a
+    // workgroup fall in step with those, one less does not (600,000 rows,
+    // SELL-64-4096, k = 24, FP32, 42 slots 362 us, 41: 263; FP64, k = 28, 18
+    // and 17: 503 and 465; SELL-64-65536: 240 and 239).
+    if (a.per % 4 == 2 && a.per > 2) --a.per;
     a.parts = a.per > 0 ? 1 : ceil_div(lanes, kScsThreads);
     a.by_lanes = fast_div(a.per > 0 ? lanes : 1);
     a.by_c = fast_div(C);
@@ -840,9 +850,11 @@ static int launch_scs_spmm(smax_hip_ctx ctx, int64_t C, int64_t n_chunks, int64_
         SMAX_HIP_LAUNCHED(ctx, "scs_spmm_vec");
         return SMAX_HIP_SUCCESS;
     }
-    if (q == Q) launch_scs_spmm_run<VT, Q>(ctx, a, grid, v, xv, yv);
-    else if (q == 2) launch_scs_spmm_run<VT, 2>(ctx, a, grid, v, xv, yv);
-    else launch_scs_spmm_run<VT, 1>(ctx, a, grid, v, xv, yv);
+    if (q == Q) launch_scs_spmm_run<VT, Q, Q>(ctx, a, grid, v, xv, yv);
+    else if (q == 2) launch_scs_spmm_run<VT, 2, Q>(ctx, a, grid, v, xv, yv);
+    else if (k >= Q) launch_scs_spmm_run<VT, 1, Q>(ctx, a, grid, v, xv, yv);
+    else if (k >= 2) launch_scs_spmm_run<VT, 1, 2>(ctx, a, grid, v, xv, yv);
+    else launch_scs_spmm_run<VT, 1, 1>(ctx, a, grid, v, xv, yv);
     SMAX_HIP_LAUNCHED(ctx, "scs_spmm_run");
     return SMAX_HIP_SUCCESS;
 }

@@ -829,3 +829,12 @@ def test_refresh_of_a_large_layout_with_tail_waves(ctx, vt, n):
     S.destroy()
     for a in (*d, dx, dy):
         a.free()
+
+
+@pytest.mark.parametrize("vt", [capi.F64, capi.F32, capi.BF16])
+@pytest.mark.parametrize("k", [4, 6, 7, 9, 11, 12, 13, 21, 24, 28, 36, 56])
+def test_scs_apply_spmm_lanes_and_runs(ctx, vt, k):
+    """Columns per lane by width (1, 2 or 16 bytes' worth, long slots always in
+    the widest runs), and lane counts whose workgroups leave a slot's lanes out
+    (6, 14: 41 and 17 slots)."""
+    test_scs_apply_spmm_long_rows_and_any_width(ctx, vt, k, 64, 4096)
