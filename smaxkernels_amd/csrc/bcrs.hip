@@ -679,6 +679,7 @@ static void launch_bcrs_spmm(smax_hip_ctx ctx, int64_t threads, int64_t n_block_
                        static_cast<typename T::vec_t *>(Y));
 }
 
+
 // False: more threads than the kernel's index arithmetic holds.
 template <int VT, int H, int BW, int G>
 static bool launch_bcrs_spmm_part(smax_hip_ctx ctx, int64_t n_block_rows, int64_t b_h,
@@ -692,6 +693,21 @@ static bool launch_bcrs_spmm_part(smax_hip_ctx ctx, int64_t n_block_rows, int64_
     const int64_t lanes = runs ? run_lanes(k, Q) : k, parts = b_h / H;
     const int64_t threads = n_block_rows * parts * lanes;
     if (threads > INT32_MAX - kBThreads) return false;
+    if constexpr (H > 1) {
+        // Fewer threads than fill the chip: one output row each instead of H.
+        // us at H and at one, 7-point matrices, k = 4: 5x5 BF16 of 10^3 10.2 and
+        // 4.7, 3x3 FP64 of 16^3 5.6 and 3.7; from 2^14 threads on the block
+        // values that H rows share count again (5x5 FP64 of 24^3, k = 8, 28,000
+        // threads: 9.0 and 12.2).  BF16 values are loaded one by one, which
+        // moves the line for the smaller blocks (3x3 of 16^3, k = 16, 16,400
+        // threads: 5.8 and 4.0; 6x3 of 16^3, k = 3, 24,600: 5.4 and 4.0), and so
+        // do 2x2 blocks with 4-byte X (32^3, k = 4, 32,800: 4.1 and 3.7).
+        const bool small = (sizeof(A) == 4 && BW == 2) || (VT == SMAX_HIP_BF16 && BW == 3);
+        const int64_t few = !small ? 1 << 14 : BW == 2 || runs || parts == 1 ? 3 << 14 : 1 << 18;
+        if (threads < few)
+            return launch_bcrs_spmm_part<VT, 1, BW, G>(ctx, n_block_rows, b_h, h_pad, w_pad, cm, k,
+                                                       col, row_ptr, val, X, Y);
+    }
 #define SMAX_BCRS_PART(QQ, RM)                                                               \
     hipLaunchKernelGGL((bcrs_spmm_part<VT, H, BW, QQ, G, RM>), grid_for(threads, kBThreads), \
                        dim3(kBThreads), 0, ctx->stream, threads, fast_div(lanes),            \
@@ -707,12 +723,16 @@ static bool launch_bcrs_spmm_part(smax_hip_ctx ctx, int64_t n_block_rows, int64_
     return true;
 }
 
-// Which block shapes take it: 3x3, 5x5, 6x6 and stacks of them; 2x2, except
-// BF16 values from k = 32 on (96^3: 0.182 ms against the register-blocked
-// kernel's 0.164, while k = 8 takes 0.044 against 0.050; FP64 of 48^3, k = 8
-// 13.4 us against 19.3, k = 32 34 against 39); 4x4 in FP64 from k = 8 on (48^3,
-// k = 8 29.5 us against 37.8, k = 32 117 both, k = 4 29.7 against 27.6; FP32
-// and BF16 values have broadcast kernels).
+// Which block shapes take it: 3x3, 5x5, 6x6 and stacks of them; 2x2 and, in FP64
+// from k = 8 on, 4x4 (FP32 and BF16 values have broadcast kernels), except where
+// the register-blocked kernel is faster (us, this against that):
+//   2x2, 16-byte runs (k >= 16) once Y is 90 MB (FP64 of 64^3, k = 20, 84 MB 61
+//     / 64, of 72^3, k = 16, 96 MB 86 / 81) or, with 4-byte X, 100 MB (FP32 of
+//     80^3, k = 24, 98 MB 83 / 91, k = 32, 131 MB 110 / 105)
+//   2x2 BF16 values for k < 4 (96^3, k = 3 49 / 40, k = 4 33 / 39) and from k =
+//     32 on (96^3 182 / 164)
+//   4x4 FP64, even k, once Y is 64 MB (48^3, k = 16, 57 MB 48 / 53, 64^3, k = 8,
+//     67 MB 95 / 92; 56^3, k = 13, 73 MB 101 / 138)
 static bool spmm_in_parts(smax_hip_ctx ctx, int value_type, int64_t n_block_rows, int64_t b_h,
                           int64_t b_w, int64_t h_pad, int64_t w_pad, bool cm, int64_t k,
                           const int32_t *col, const int32_t *row_ptr, const void *val,
@@ -724,9 +744,14 @@ static bool spmm_in_parts(smax_hip_ctx ctx, int value_type, int64_t n_block_rows
         if (b_w == 3 && b_h % 3 == 0) SMAX_BCRS_PARTS(VT, 3, 3, 4);
         if (b_w == 5 && b_h % 5 == 0) SMAX_BCRS_PARTS(VT, 5, 5, 2);
         if (b_w == 6 && b_h % 3 == 0) SMAX_BCRS_PARTS(VT, 3, 6, 2);
-        if (b_w == 2 && b_h == 2 && !(VT == SMAX_HIP_BF16 && (k == 1 || k >= 32)))
+        constexpr int64_t kItem = sizeof(typename vt<VT>::vec_t);
+        const int64_t y_bytes = n_block_rows * b_h * k * kItem;
+        const bool wide = k >= 16 && k * kItem % 16 == 0 &&
+                          y_bytes >= (kItem == 8 ? 90'000'000 : 100'000'000);
+        if (b_w == 2 && b_h == 2 && !wide && !(VT == SMAX_HIP_BF16 && (k < 4 || k >= 32)))
             SMAX_BCRS_PARTS(VT, 2, 2, 4);
-        if (VT == SMAX_HIP_F64 && b_w == 4 && b_h == 4 && k >= 8)
+        if (VT == SMAX_HIP_F64 && b_w == 4 && b_h == 4 && k >= 8 &&
+            (k % 2 != 0 || y_bytes < 64'000'000))
             SMAX_BCRS_PARTS(SMAX_HIP_F64, 4, 4, 2);
     });
 #undef SMAX_BCRS_PARTS

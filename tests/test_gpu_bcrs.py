@@ -529,3 +529,37 @@ def test_bcrs_products_of_any_block_shape(ctx, vt, cm, bh, bw, hp, wp):
         dY.free()
     for a in d:
         a.free()
+
+
+@pytest.mark.parametrize("vt", [capi.F64, capi.F32, capi.BF16])
+@pytest.mark.parametrize("cm", [False, True])
+@pytest.mark.parametrize("bh,bw,n,k", [
+    # one output row a thread below 2^14 (3 x 2^14, 2^18) threads of several rows
+    (3, 3, 16383, 4), (3, 3, 16384, 4), (3, 3, 8192, 8), (5, 5, 4096, 13), (5, 5, 16384, 2),
+    (6, 6, 8192, 4), (6, 6, 8191, 4), (6, 3, 24576, 4), (9, 3, 43691, 2), (2, 2, 49151, 4),
+    (2, 2, 49152, 4), (4, 4, 4096, 8),
+    # the register-blocked kernel once Y is 90 or 100 MB (2x2), 64 MB (4x4, even k)
+    (2, 2, 351_562, 16), (2, 2, 351_563, 16), (2, 2, 781_250, 16), (2, 2, 351_563, 17),
+    (4, 4, 250_000, 8), (4, 4, 249_999, 8), (4, 4, 222_223, 9)])
+def test_bcrs_spmm_around_the_kernel_choices(ctx, vt, cm, bh, bw, n, k):
+    """Whole numbers, so that every order gives the exact product."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(n + k)
+    per = rng.integers(0, 3, n)
+    per[rng.integers(0, n, 3)] = 40
+    rp = np.concatenate([[0], np.cumsum(per)]).astype(np.int32)
+    n_cols = 5000
+    col = np.concatenate([np.sort(rng.choice(n_cols, p, replace=False)) if p > 2 else
+                          np.arange(p) * 2000 for p in per]).astype(np.int32)
+    blocks = rng.integers(-3, 4, (rp[-1], bh, bw)).astype(np.float64)
+    vec = np.float64 if vt == capi.F64 else np.float32
+    X = rng.integers(-4, 5, (n_cols * bw, k)).astype(vec)
+    stored = (blocks.transpose(0, 2, 1) if cm else blocks).ravel()
+    val = stored if vt == capi.F64 else stored.astype(np.float32) if vt == capi.F32 else matgen.to_bf16(stored)
+    d = [ctx.upload(a) for a in (col, rp, val, X)]
+    Y = ctx.zeros(n * bh * k, vec)
+    ctx.bcrs_spmm(vt, n, bh, bw, bh, bw, *d[:3], cm, k, d[3], Y)
+    want = sp.bsr_matrix((blocks, col, rp), shape=(n * bh, n_cols * bw)) @ X.astype(np.float64)
+    assert_bitwise(ctx.download(Y), want.astype(vec).ravel())
+    for a in (*d, Y):
+        a.free()
