@@ -227,21 +227,31 @@ __global__ __launch_bounds__(kBThreads) void bcrs_spmm_kernel(
 // / 110 / 327 -> 28 / 37 / 84, 6x6 121 / 153 / 523 -> 33 / 41 / 144, 6x6 BF16
 // of 32^3 44 / 72 / 175 -> 8.4 / 11.6 / 23.  One block at a time: 6x6 FP64 59
 // / 60 / 143.
+// One argument: a launch costs the host time for each (the four launches of a
+// training step of 12^3 3x3 BF16 blocks, k = 4: 18.7 us, 18.1 this way and with
+// LineSizes).
+struct PartSizes {
+    int64_t n_threads, k;
+    FastDiv by_lanes, by_parts;
+    int lanes, parts, h_pad, w_pad;
+};
+
 template <int VT, int H, int BW, int Q, int G, bool RM>
 __global__ __launch_bounds__(kBThreads) void bcrs_spmm_part(
-    int64_t n_threads, FastDiv by_lanes, int lanes, FastDiv by_parts, int parts, int h_pad,
-    int w_pad, int64_t k, const int32_t *__restrict__ col, const int32_t *__restrict__ row_ptr,
+    PartSizes a, const int32_t *__restrict__ col, const int32_t *__restrict__ row_ptr,
     const typename vt<VT>::val_t *__restrict__ val, const typename vt<VT>::vec_t *__restrict__ X,
     typename vt<VT>::vec_t *__restrict__ Y) {
     using T = vt<VT>;
     using A = typename T::vec_t;
     using V = typename T::val_t;
     const int64_t t = xcd_block(blockIdx.x, gridDim.x) * kBThreads + threadIdx.x;
-    if (t >= n_threads) return;
-    const int32_t rh = by_lanes(static_cast<int32_t>(t));
-    const int32_t l = static_cast<int32_t>(t) - rh * lanes;
-    const int32_t r = by_parts(rh);
-    const int32_t ix = (rh - r * parts) * H;
+    if (t >= a.n_threads) return;
+    const int h_pad = a.h_pad, w_pad = a.w_pad;
+    const int64_t k = a.k;
+    const int32_t rh = a.by_lanes(static_cast<int32_t>(t));
+    const int32_t l = static_cast<int32_t>(t) - rh * a.lanes;
+    const int32_t r = a.by_parts(rh);
+    const int32_t ix = (rh - r * a.parts) * H;
     const int64_t v = run_start<Q>(l, k);
     const int64_t bs = static_cast<int64_t>(h_pad) * w_pad;
     const V *vpart = val + (RM ? ix * w_pad : ix);
@@ -267,8 +277,8 @@ __global__ __launch_bounds__(kBThreads) void bcrs_spmm_part(
                 for (int jx = 0; jx < BW; ++jx) load_cols_run<A, Q>(xr + jx * k, xv[g][jx]);
                 const V *blk = vpart + (j + g) * bs;
 #pragma unroll
-                for (int a = 0; a < (RM ? H : BW); ++a)
-                    load_vals<V, RM ? BW : H>(blk + a * (RM ? w_pad : h_pad), w[g][a]);
+                for (int i = 0; i < (RM ? H : BW); ++i)
+                    load_vals<V, RM ? BW : H>(blk + i * (RM ? w_pad : h_pad), w[g][i]);
             }
 #pragma unroll
         for (int g = 0; g < G; ++g)
@@ -708,11 +718,17 @@ static bool launch_bcrs_spmm_part(smax_hip_ctx ctx, int64_t n_block_rows, int64_
             return launch_bcrs_spmm_part<VT, 1, BW, G>(ctx, n_block_rows, b_h, h_pad, w_pad, cm, k,
                                                        col, row_ptr, val, X, Y);
     }
+    const PartSizes sizes{threads,
+                          k,
+                          fast_div(lanes),
+                          fast_div(parts),
+                          static_cast<int>(lanes),
+                          static_cast<int>(parts),
+                          static_cast<int>(h_pad),
+                          static_cast<int>(w_pad)};
 #define SMAX_BCRS_PART(QQ, RM)                                                               \
     hipLaunchKernelGGL((bcrs_spmm_part<VT, H, BW, QQ, G, RM>), grid_for(threads, kBThreads), \
-                       dim3(kBThreads), 0, ctx->stream, threads, fast_div(lanes),            \
-                       static_cast<int>(lanes), fast_div(parts), static_cast<int>(parts),    \
-                       static_cast<int>(h_pad), static_cast<int>(w_pad), k, col, row_ptr,    \
+                       dim3(kBThreads), 0, ctx->stream, sizes, col, row_ptr,                 \
                        static_cast<const typename T::val_t *>(val), static_cast<const A *>(X), \
                        static_cast<A *>(Y))
     if (runs && cm) SMAX_BCRS_PART(Q, false);
@@ -1388,12 +1404,20 @@ constexpr int kSddmmIters = 8;  // at most: 2048 lines a workgroup
 template <typename A, int KP>
 constexpr bool kSddmmAtOnce = KP * sizeof(A) <= 64;
 
+struct LineSizes {  // one argument, as PartSizes
+    int64_t n_blocks, n_block_rows, k;
+    int iters, n_lines, lines_real, n_out, outs_real, h_pad, w_pad, col_major;
+};
+
 template <typename A, int KP, int VL, int M>
 __global__ __launch_bounds__(256) void bcrs_sddmm_lines(
-    int64_t n_blocks, int64_t n_block_rows, int iters, int n_lines, int lines_real, int n_out,
-    int outs_real, int h_pad, int w_pad, int col_major, int64_t k,
-    const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col,
+    LineSizes sizes, const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col,
     const A *__restrict__ Gm, const A *__restrict__ X, A *__restrict__ dvals) {
+    const int64_t n_blocks = sizes.n_blocks, n_block_rows = sizes.n_block_rows, k = sizes.k;
+    const int iters = sizes.iters, n_lines = sizes.n_lines, lines_real = sizes.lines_real;
+    const int n_out = sizes.n_out, outs_real = sizes.outs_real;
+    const int h_pad = sizes.h_pad, w_pad = sizes.w_pad;
+    const bool col_major = sizes.col_major != 0;
     __shared__ int32_t row_of[256 * kSddmmIters + 1];
     const int span = iters * 256;
     const int64_t t0 = xcd_block(blockIdx.x, gridDim.x) * span;
@@ -1498,15 +1522,21 @@ static void launch_bcrs_sddmm_lines(smax_hip_ctx ctx, const smax_hip_bcrs_info &
     // fewer lines a workgroup while that leaves CUs idle
     int64_t iters = lines / (256 * 2048);
     iters = iters < 1 ? 1 : iters > kSddmmIters ? kSddmmIters : iters;
-    hipLaunchKernelGGL((bcrs_sddmm_lines<A, KP, VL, M>), grid_for(lines, static_cast<int>(256 * iters)),
-                       dim3(256), 0, ctx->stream, in.n_blocks, in.n_block_rows,
-                       static_cast<int>(iters), static_cast<int>(n_lines),
-                       static_cast<int>(cm ? in.b_w : in.b_h),
-                       static_cast<int>(cm ? in.h_pad : in.w_pad),
-                       static_cast<int>(cm ? in.b_h : in.b_w), static_cast<int>(in.h_pad),
-                       static_cast<int>(in.w_pad), cm ? 1 : 0, k, in.row_ptr, in.col,
-                       static_cast<const A *>(Gm), static_cast<const A *>(X),
-                       static_cast<A *>(dv));
+    const LineSizes sizes{in.n_blocks,
+                          in.n_block_rows,
+                          k,
+                          static_cast<int>(iters),
+                          static_cast<int>(n_lines),
+                          static_cast<int>(cm ? in.b_w : in.b_h),
+                          static_cast<int>(cm ? in.h_pad : in.w_pad),
+                          static_cast<int>(cm ? in.b_h : in.b_w),
+                          static_cast<int>(in.h_pad),
+                          static_cast<int>(in.w_pad),
+                          cm ? 1 : 0};
+    hipLaunchKernelGGL((bcrs_sddmm_lines<A, KP, VL, M>),
+                       grid_for(lines, static_cast<int>(256 * iters)), dim3(256), 0, ctx->stream,
+                       sizes, in.row_ptr, in.col, static_cast<const A *>(Gm),
+                       static_cast<const A *>(X), static_cast<A *>(dv));
 }
 
 // 16-byte loads when every operand row is 16-byte aligned; 16-byte stores for
