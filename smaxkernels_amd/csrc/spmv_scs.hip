@@ -343,11 +343,13 @@ struct ScsParts<VT, true> {
 //   LONG (LEN only): the first longs.blocks workgroups (again a multiple of
 //          8) run the long chunks or, with tails, the long tail waves; the
 //          wavefronts leave those out.
-//   FP64 is held to 128 registers (4 wavefronts per SIMD; it takes 136 by
-//   itself): SELL-64-64 of 4,000,000 rows 1.16 -> 1.08 ms, SELL-32-4096 0.80
-//   -> 0.78, the 27-point stencil of 64^3 43 -> 29 us.
-template <int VT, bool UNPERM, bool REMAP, bool LEN, bool SHORT, bool LONG>
-__global__ __launch_bounds__(kScsThreads, !SHORT && VT == SMAX_HIP_F64 ? 4 : 1) void scs_spmv_w64(
+//   FOUR: held to 128 registers, 4 wavefronts per SIMD.  FP64 takes 136 by
+//   itself, which leaves three, 768 workgroups on the chip: larger grids then
+//   run in two rounds (the 27-point stencil of 64^3, 1024 workgroups, 44 -> 30
+//   us, SELL-64-64 of 4,000,000 rows 1.16 -> 1.08 ms), smaller ones are slower
+//   held to 128 (24^3 13.1 -> 13.7 us).
+template <int VT, bool UNPERM, bool REMAP, bool LEN, bool SHORT, bool LONG, bool FOUR>
+__global__ __launch_bounds__(kScsThreads, FOUR ? 4 : 1) void scs_spmv_w64(
     ScsSpmv<VT> a, ScsParts<VT, SHORT> p) {
     using T = vt<VT>;
     // All of a short layout's arguments at once: fetched as they come up, the
@@ -444,9 +446,11 @@ __global__ __launch_bounds__(kScsThreads, !SHORT && VT == SMAX_HIP_F64 ? 4 : 1) 
 //   then addresses its elements with constant offsets and runs the C = 64
 //   kernel's group size (4M-row band matrix, C = 32, FP64: sigma = 65536
 //   0.692 -> 0.660 ms, 0.640 with the occupancy cap; sigma = N 1.093 ->
-//   1.061 ms; BF16 values, sigma = 65536: 0.495 -> 0.477 ms).
+//   1.061 ms; BF16 values, sigma = 65536: 0.495 -> 0.477 ms).  FP64 is held to
+//   128 registers as above except in this form without long chunks (27-point
+//   stencil of 24^3 14.5 us held, 13.9 not, of 128^3 225 and 222).
 template <int VT, bool UNPERM, bool LEN, bool REMAP, int CS, bool LONG>
-__global__ __launch_bounds__(kScsThreads, VT == SMAX_HIP_F64 ? 4 : 1) void scs_spmv_generic(
+__global__ __launch_bounds__(kScsThreads, VT == SMAX_HIP_F64 && (LONG || CS == 0) ? 4 : 1) void scs_spmv_generic(
     int64_t C, int64_t cpb, int64_t bpc, ScsSpmv<VT> a, ScsParts<VT, false> p) {
     using T = vt<VT>;
     if constexpr (CS > 0) C = CS;
@@ -871,12 +875,17 @@ static void launch_w64(smax_hip_ctx ctx, const ScsLaunch<VT> &l) {
     const int64_t blocks =
         ceil_div(l.a.n_chunks, kScsThreads / kWave) + l.p.t_blocks + l.p.longs.blocks;
     const dim3 grid(static_cast<unsigned>(blocks));
+    constexpr bool kFour = VT == SMAX_HIP_F64;
+    constexpr int64_t kCus = 256;
     if constexpr (SHORT) {
-        hipLaunchKernelGGL((scs_spmv_w64<VT, UNPERM, REMAP, LEN, true, false>), grid,
+        hipLaunchKernelGGL((scs_spmv_w64<VT, UNPERM, REMAP, LEN, true, false, false>), grid,
                            dim3(kScsThreads), l.lds_bytes, ctx->stream, l.a,
                            ScsParts<VT, true>{});
+    } else if (kFour && !LONG && blocks <= 3 * kCus) {
+        hipLaunchKernelGGL((scs_spmv_w64<VT, UNPERM, REMAP, LEN, false, false, false>), grid,
+                           dim3(kScsThreads), l.lds_bytes, ctx->stream, l.a, l.p);
     } else {
-        hipLaunchKernelGGL((scs_spmv_w64<VT, UNPERM, REMAP, LEN, false, LONG>), grid,
+        hipLaunchKernelGGL((scs_spmv_w64<VT, UNPERM, REMAP, LEN, false, LONG, kFour>), grid,
                            dim3(kScsThreads), l.lds_bytes, ctx->stream, l.a, l.p);
     }
 }

@@ -838,3 +838,25 @@ def test_scs_apply_spmm_lanes_and_runs(ctx, vt, k):
     the widest runs), and lane counts whose workgroups leave a slot's lanes out
     (6, 14: 41 and 17 slots)."""
     test_scs_apply_spmm_long_rows_and_any_width(ctx, vt, k, 64, 4096)
+
+
+@pytest.mark.parametrize("vt", [capi.F64, capi.F32])
+@pytest.mark.parametrize("C_", [64, 32])
+@pytest.mark.parametrize("chunks", [3071, 3072, 3073])
+def test_scs_apply_around_three_workgroups_a_cu(ctx, vt, C_, chunks):
+    """Up to 768 workgroups of four 64-row chunks the FP64 kernel keeps its
+    registers: rows of 9 to 60 entries (no long chunk), the last chunk partial."""
+    n = chunks * 64 - 5
+    L = 9 + np.arange(n) % 52
+    rp = np.concatenate([[0], np.cumsum(L)]).astype(np.int32)
+    first = np.random.default_rng(chunks).integers(0, 4000, n)
+    col = (np.repeat(first, L) + np.arange(rp[-1]) - np.repeat(rp[:-1], L)).astype(np.int32)
+    val = matgen.uniform_f64(4, rp[-1]).astype(np.float64 if vt == capi.F64 else np.float32)
+    x = matgen.uniform_f64(5, n).astype(val.dtype)
+    S = gpu_scs(ctx, Csr(n, n, rp, col, val), C_, 1, val)
+    dx, dy = ctx.upload(x), ctx.zeros(n, x.dtype)
+    S.apply(vt, dx, dy, unpermuted=True)
+    assert_bitwise(ctx.download(dy), oracle.crs_spmv(rp, col, val, x))
+    S.destroy()
+    for a in (dx, dy):
+        a.free()
