@@ -15,10 +15,11 @@
 // lane l sums v in [l*Q, min(k, l*Q + Q)), Q = ceil(k / g), with an fma chain
 // from zero, and an xor-butterfly adds the g partial sums.  Up to k = 256 the
 // lanes of a group share one row (SpMM order): the G row is read once per row
-// and each element costs one coalesced X row.  Larger k take one group per
-// stored element, with the row of each element from a per-element row array
-// built on first use.  Both kernels evaluate the same tree, so dvals do not
-// depend on which one runs.
+// and each element costs one coalesced X row; layouts too small for that to fill
+// the chip take a group of lanes per stored element, its row from its chunk.
+// Larger k take one group per stored element, with the row of each element from
+// a per-element row array built on first use.  All kernels evaluate the same
+// tree, so dvals do not depend on which one runs.
 #include <algorithm>
 #include <type_traits>
 #include <utility>

@@ -653,20 +653,25 @@ static void launch_bcrs_spmm_reg(smax_hip_ctx ctx, int64_t n_block_rows, int64_t
 #undef SMAX_BCRS_QUAD
     }
     // block groups of 2 (measured on the 96^3 block matrix: k = 8 0.173 ->
-    // 0.160 ms, k = 64 0.663 -> 0.649 ms in BF16), of 8 where one thread has a
-    // whole block row of 2x2 BF16 values (see spmv_by_rows)
-    constexpr int GS = VT == SMAX_HIP_BF16 && BH == 2 && BW == 2 ? 8 : 2;
+    // 0.160 ms, k = 64 0.663 -> 0.649 ms in BF16)
 #define SMAX_BCRS_REG_LAUNCH(QQ, DD, CC, GG)                                                \
     hipLaunchKernelGGL((bcrs_spmm_reg<VT, BH, BW, QQ, DD, CC, GG>), g, dim3(kBThreads), 0,  \
                        ctx->stream, n_block_rows, static_cast<int>(h_pad),                 \
                        static_cast<int>(w_pad), cm ? 1 : 0, k, col, row_ptr, v, xv, yv)
+    // of 8 where one thread has a whole block row of 2x2 BF16 values, the one
+    // shape of which spmv_by_rows leaves k = 1 to this kernel
+    if constexpr (VT == SMAX_HIP_BF16 && BH == 2 && BW == 2) {
+        if (dense && k == 1) {
+            if (cm) { SMAX_BCRS_REG_LAUNCH(1, true, true, 8); }
+            else { SMAX_BCRS_REG_LAUNCH(1, true, false, 8); }
+            return;
+        }
+    }
     if (runs && dense && cm) { SMAX_BCRS_REG_LAUNCH(Q, true, true, 2); }
     else if (runs && dense) { SMAX_BCRS_REG_LAUNCH(Q, true, false, 2); }
     else if (runs) { SMAX_BCRS_REG_LAUNCH(Q, false, false, 2); }
     else if (pairs && cm) { SMAX_BCRS_REG_LAUNCH(2, true, true, 2); }
     else if (pairs) { SMAX_BCRS_REG_LAUNCH(2, true, false, 2); }
-    else if (dense && cm && k == 1) { SMAX_BCRS_REG_LAUNCH(1, true, true, GS); }
-    else if (dense && k == 1) { SMAX_BCRS_REG_LAUNCH(1, true, false, GS); }
     else if (dense && cm) { SMAX_BCRS_REG_LAUNCH(1, true, true, 2); }
     else if (dense) { SMAX_BCRS_REG_LAUNCH(1, true, false, 2); }
     else { SMAX_BCRS_REG_LAUNCH(1, false, false, 2); }
@@ -1077,7 +1082,10 @@ int smax_hip_bcrs_spmm(smax_hip_ctx ctx, int value_type,
         SMAX_HIP_LAUNCHED(ctx, "bcrs_spmm_part");
         return SMAX_HIP_SUCCESS;
     }
-    // register-blocked shapes: every (b_h, b_w) in {1, 2, 4} x {1, 2, 4}
+    // What the two kernels above leave of (b_h, b_w) in {1, 2, 4} x {1, 2, 4}
+    // runs in registers: for one right-hand side 2x2 BF16 blocks, for more the
+    // shapes that spmm_in_parts does not take (it takes square ones, up to the
+    // sizes of Y named there).
     const bool reg = (b_h == 1 || b_h == 2 || b_h == 4) && (b_w == 1 || b_w == 2 || b_w == 4);
 #define SMAX_BCRS_REG(H, W)                                                            \
     if (b_h == H && b_w == W) {                                                        \

@@ -46,12 +46,16 @@ inline int64_t long_row_from(int64_t nnz, int64_t n_rows) {
 
 // In SELL a long slot alone also pays for its columns and values, one line an
 // entry that the other slots of its chunk would share; in large matrices, where
-// the longest rows no longer decide the time, fewer slots are long.  Measured
-// with 16-byte runs in LDS, before a lane took one column (now 0.312, 0.355 and
-// 0.082 ms with this rule): 1,000,000 rows, from 128 / 512 / 1024 / 1400 entries on: FP32 k = 32 0.359 /
-// 0.337 / 0.322 / 0.329 ms (none: 0.371), FP64 k = 16 0.468 / 0.404 / 0.372 /
-// 0.362 (0.382); 200,003 rows, FP64 k = 10: 0.089 / 0.094 / 0.146 / 0.169
-// (0.343).
+// the longest rows no longer decide the time, fewer slots are long.  Band
+// matrices with rows of up to 2000 entries, us with this rule, then with a line
+// of 128 / 256 / 512 / 1024 entries and without long slots:
+//   40,013 rows, FP64 k = 10       32 |  32 /  34 /  56 / 100, 208
+//   200,003, FP64 k = 10           78 |  78 /  79 / 103 / 133, 274
+//   200,003, FP32 k = 32           62 |  65 /  63 /  76 / 117, 205
+//   500,009, FP64 k = 16          166 | 169 / 171 / 165 / 169, 258
+//   1,000,000, FP32 k = 32        315 | 329 / 323 / 323 / 317, 427
+//   1,000,000, FP64 k = 16        356 | 377 / 368 / 367 / 358, 381
+//   2,000,003, FP64 k = 8         615 | 661 / 631 / 644 / 615, 655
 inline int64_t long_slot_from(int64_t nnz, int64_t n_rows) {
     const int64_t row = long_row_from(nnz, n_rows), part = nnz / 16000;
     const int64_t most = part < 1024 ? part : 1024;

@@ -1028,7 +1028,10 @@ int launch_scs_spmv(smax_hip_ctx ctx, int64_t C, int64_t n_chunks,
 // per slot (and 4x the mean) leave this order and are run by whole workgroups
 // (long_chunk).  With 128 and 8x instead: 1,000,000 rows, C = 32, sigma =
 // 65536, FP32 133 us against 127, 4,000,000 rows, C = 32, sigma = 4096, FP64
-// 803 against 760; no size measured slower with the lower line.
+// 803 against 760.  Against the order alone, 4,000,000 rows, FP32: C = 64, sigma
+// = 1024 609 us and 644, C = 32, sigma = 65536 489 and 504, but C = 64, sigma =
+// 4096 534 and 528, sigma = 65536 479 and 471 (BF16 458 and 457; 2,000,000 rows
+// 227 and 235).
 constexpr int kLongChunk = 128;
 constexpr int kWideChunk = 64;
 constexpr int64_t kLdsPerCu = 160 * 1024;
