@@ -752,6 +752,9 @@ static bool launch_bcrs_spmm_part(smax_hip_ctx ctx, int64_t n_block_rows, int64_
 //     80^3, k = 24, 98 MB 83 / 91, k = 32, 131 MB 110 / 105)
 //   2x2 BF16 values for k < 4 (96^3, k = 3 49 / 40, k = 4 33 / 39) and from k =
 //     32 on (96^3 182 / 164)
+//   2x2 FP32, k = 3, from 2^13 block rows to a Y of 5 MB (24^3 3.8 / 3.7, 40^3
+//     5.8 / 5.3, 56^3, 4.2 MB 12.9 / 12.6, 64^3, 6.3 MB 16.9 / 17.5; its three
+//     lanes a block row of one column each save too little)
 //   4x4 FP64, even k, once Y is 64 MB (48^3, k = 16, 57 MB 48 / 53, 64^3, k = 8,
 //     67 MB 95 / 92; 56^3, k = 13, 73 MB 101 / 138)
 static bool spmm_in_parts(smax_hip_ctx ctx, int value_type, int64_t n_block_rows, int64_t b_h,
@@ -769,7 +772,10 @@ static bool spmm_in_parts(smax_hip_ctx ctx, int value_type, int64_t n_block_rows
         const int64_t y_bytes = n_block_rows * b_h * k * kItem;
         const bool wide = k >= 16 && k * kItem % 16 == 0 &&
                           y_bytes >= (kItem == 8 ? 90'000'000 : 100'000'000);
-        if (b_w == 2 && b_h == 2 && !wide && !(VT == SMAX_HIP_BF16 && (k < 4 || k >= 32)))
+        const bool three = VT == SMAX_HIP_F32 && k == 3 && n_block_rows >= 1 << 13 &&
+                           y_bytes < 5'000'000;
+        if (b_w == 2 && b_h == 2 && !wide && !three &&
+            !(VT == SMAX_HIP_BF16 && (k < 4 || k >= 32)))
             SMAX_BCRS_PARTS(VT, 2, 2, 4);
         if (VT == SMAX_HIP_F64 && b_w == 4 && b_h == 4 && k >= 8 &&
             (k % 2 != 0 || y_bytes < 64'000'000))

@@ -540,7 +540,9 @@ def test_bcrs_products_of_any_block_shape(ctx, vt, cm, bh, bw, hp, wp):
     (2, 2, 49152, 4), (4, 4, 4096, 8),
     # the register-blocked kernel once Y is 90 or 100 MB (2x2), 64 MB (4x4, even k)
     (2, 2, 351_562, 16), (2, 2, 351_563, 16), (2, 2, 781_250, 16), (2, 2, 351_563, 17),
-    (4, 4, 250_000, 8), (4, 4, 249_999, 8), (4, 4, 222_223, 9)])
+    (4, 4, 250_000, 8), (4, 4, 249_999, 8), (4, 4, 222_223, 9),
+    # and for k = 3 in FP32 (2x2) from 2^13 block rows to 5 MB
+    (2, 2, 8191, 3), (2, 2, 8192, 3), (2, 2, 208_333, 3), (2, 2, 208_334, 3)])
 def test_bcrs_spmm_around_the_kernel_choices(ctx, vt, cm, bh, bw, n, k):
     """Whole numbers, so that every order gives the exact product."""
     import scipy.sparse as sp
