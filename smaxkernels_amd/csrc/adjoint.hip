@@ -306,19 +306,29 @@ __global__ __launch_bounds__(256) void scs_sddmm_elements(SddmmArgs a, const A *
     if (first >= a.n_elements) return;  // whole wavefronts
     const int l = static_cast<int>(threadIdx.x) % GL;
     const bool valid = e < a.n_elements;
-    const int32_t to = valid ? a.src[e] : -1;
+    // Loaded together, so that X does not wait for one after the other; a
+    // wavefront of padding alone ends here.
+    const int64_t at = valid ? e : a.n_elements - 1;
+    const int32_t from = a.src[at], col = a.col[at], to = valid ? from : -1;
+    if (__ballot(to >= 0) == 0) return;
     const int64_t k = a.k;
     const int64_t v0 = EXACT ? l * Q : run_start<Q>(l, k);
     const int skip = EXACT ? 0 : l * Q < k ? static_cast<int>(l * Q - v0) : Q;
     A x[Q], g[Q];
-    if (to >= 0) load_cols_run<A, Q>(X + static_cast<int64_t>(a.col[e]) * k + v0, x);
+    load_cols_run<A, Q>(X + static_cast<int64_t>(col) * k + v0, x);
     int64_t c = wave_row_of(a.chunk_ptr, a.n_chunks, first);
     A acc = 0;
     if (to >= 0) {
-        int32_t end = a.chunk_ptr[c + 1];
-        for (int step = 0; e >= end && step < 8; ++step) end = a.chunk_ptr[++c + 1];
-        if (e >= end) c = row_of(a.chunk_ptr, c, a.n_chunks, e);
-        const int32_t off = static_cast<int32_t>(e - a.chunk_ptr[c]);
+        int32_t base = a.chunk_ptr[c], end = a.chunk_ptr[c + 1];
+        for (int step = 0; e >= end && step < 8; ++step) {
+            base = end;
+            end = a.chunk_ptr[++c + 1];
+        }
+        if (e >= end) {
+            c = row_of(a.chunk_ptr, c, a.n_chunks, e);
+            base = a.chunk_ptr[c];
+        }
+        const int32_t off = static_cast<int32_t>(e) - base;
         const int64_t slot = c * a.C + (off - a.by_c(off) * a.C);
         load_cols_run<A, Q>(Gm + static_cast<int64_t>(a.slot_row[slot]) * k + v0, g);
 #pragma unroll
@@ -331,19 +341,28 @@ __global__ __launch_bounds__(256) void scs_sddmm_elements(SddmmArgs a, const A *
     if (to >= 0 && l == 0) dvals[to] = acc;
 }
 
-// Below this many threads, padding included, one group an element.  Each
-// element then reads its own G row and a lane one store, so the rows win once
-// the chip is full; with one lane an element the larger share of the row
-// kernel's long chains carries further.  By element against by rows, us, on a
-// heavy-tailed band (1.6 elements stored per entry):
-//   k = 3, FP64   220,000 rows 81 / 138, 700,000 (18 M threads) 356 / 357
-//   k = 5         100,000 rows (5.2 M)  52 / 61, 130,000  72 / 69
-//   k = 9          14,000 rows (1.5 M)  14 / 18,  30,000  32 / 28
-//   k = 20         10,000 rows (2.1 M)  15 / 17,  14,000  26 / 18
-//   k = 48          5000 rows (2.1 M)   13 / 17,   7000   21 / 19
-//   k = 200         2000 rows (3.3 M)   18 / 20,   5000   64 / 56
-static bool sddmm_by_element(int64_t n_elements, int64_t lanes) {
-    return n_elements * lanes < (lanes == 1 ? 1 << 24 : lanes == 2 ? 5 << 20 : 1 << 21);
+// Whether a group an element is the faster one.  By rows a launch takes some 12
+// us for its long chains and then a time per entry; by element a time per entry
+// that a few lanes make the shorter one, but many a longer one (each entry reads
+// its own G row), and a quarter of it per padding element.  In threads (lanes an
+// entry), the difference is `more` eighths of the entries' and a quarter of the
+// padding's; `fixed` is what the chains cost in that measure.  By element / by
+// rows, us, heavy-tailed bands of 16 entries a row, rows in sort windows of 4096
+// (2.5 elements an entry) and unsorted (17):
+//   k = 3    FP64 400,000 rows 154 / 204, 700,000  334 / 309; unsorted 20,000 34 / 19
+//   k = 5    FP64 120,000  56 / 70, FP32  49 / 49;            unsorted 20,000 52 / 19
+//   k = 12   FP64 18,000   16 / 20, FP32  12 / 13;            unsorted 5000 16 / 17, 15 / 14
+//   k = 24   FP64 9000     13 / 20, FP32  11 / 13;            unsorted 3000 12 / 15, 11 / 12
+//   k = 48   FP64 5000     12 / 16, FP32  11 / 13;            unsorted 5000 41 / 17, 30 / 15
+//   k = 100  FP64 4000     18 / 22, 5000  28.6 / 28.6
+//   k = 200  FP64 4000     35 / 45, 5000  56 / 56;            unsorted 1000 14 / 15, 2000 39 / 22
+static bool sddmm_by_element(int64_t nnz, int64_t n_elements, int64_t lanes, bool f64) {
+    const int64_t more = lanes == 1 ? -3 : lanes == 2 ? -1 : lanes < 32 ? 4 : lanes == 32 ? 2 : 0;
+    const int64_t fixed = lanes == 1   ? 11 << 16
+                          : lanes == 2 ? (f64 ? 3 << 19 : 7 << 17)
+                          : lanes < 32 ? (f64 ? 7 << 18 : 5 << 18)
+                                       : 9 << 17;
+    return nnz < 10'000'000 && (nnz * more + (n_elements - nnz) * 2) * lanes < fixed * 8;
 }
 
 template <typename A, int GL, int Q>
@@ -374,7 +393,7 @@ static void launch_sddmm_rows(smax_hip_ctx ctx, smax_hip_scs S, int64_t k, const
     const auto g = static_cast<const A *>(Gm);
     const auto x = static_cast<const A *>(X);
     const auto d = static_cast<A *>(dv);
-    if (sddmm_by_element(in.n_elements, GL)) {
+    if (sddmm_by_element(in.nnz, in.n_elements, GL, sizeof(A) == 8)) {
         const dim3 per_element = grid_for(in.n_elements * GL, 256);
         if (k == GL * Q)
             hipLaunchKernelGGL((scs_sddmm_elements<A, GL, Q, true>), per_element, dim3(256), 0,
